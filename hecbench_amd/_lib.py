@@ -9,6 +9,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libhq.so")
+OPS_PATH = os.path.join(_HERE, "_ops.so")
 
 # Every symbol include/hq.h declares, with its ctypes signature.
 _c = ctypes
@@ -78,6 +79,25 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def native_ops():
+    """The module of the operators' host path (csrc/pyops.cpp, linked against libhq.so).  Where it is not built, an
+    object that raises at the first operator call, as load() does: importing the package needs no build."""
+    if os.path.exists(OPS_PATH):
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries are what the module is linked against)
+        spec = importlib.util.spec_from_file_location("hecbench_amd._ops", OPS_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        return module
+
+    class NotBuilt:
+        def __getattr__(self, name):
+            raise ImportError(f"{OPS_PATH} is not built; run `python -m hecbench_amd.build` (needs hipcc)")
+
+    return NotBuilt()
 
 
 class HqError(RuntimeError):

@@ -14,6 +14,8 @@
 namespace {
 std::mutex g_mu;
 std::map<int, HqDevice> g_devices;
+constexpr int kListedDevices = 64;
+std::atomic<const HqDevice*> g_known[kListedDevices];  // entries of g_devices that are gfx950 parts
 std::map<std::pair<int, hipStream_t>, HqWorkspace> g_workspaces;
 std::vector<std::pair<int, void*>> g_retired;  // outgrown buffers, freed by hq_shutdown()
 }  // namespace
@@ -64,6 +66,14 @@ extern "C" int hq_set_tunable(const char* name, int value, int clear) {
 int hq_current_device(const HqDevice** out) {
   int dev = 0;
   HQ_HIP_TRY(hipGetDevice(&dev));
+  // every call passes here: a device seen before costs one load, no lock (map nodes stay where they are)
+  const bool listed = dev >= 0 && dev < kListedDevices;
+  if (listed) {
+    if (const HqDevice* known = g_known[dev].load(std::memory_order_acquire)) {
+      *out = known;
+      return HQ_OK;
+    }
+  }
   std::lock_guard<std::mutex> lk(g_mu);
   auto it = g_devices.find(dev);
   if (it == g_devices.end()) {
@@ -78,6 +88,7 @@ int hq_current_device(const HqDevice** out) {
   }
   if (!it->second.ok) return HQ_ERR_UNSUPPORTED_DEVICE;
   *out = &it->second;
+  if (listed) g_known[dev].store(&it->second, std::memory_order_release);
   return HQ_OK;
 }
 
