@@ -77,3 +77,24 @@ def test_zero_block_and_midpoint_ties(hq, oracle):
     codes = np.stack([wp >> 4, wp & 15], 1).reshape(-1)
     assert (codes[:64] == 7).all() and codes[64] == 15
     assert np.array_equal(codes[65:80], np.arange(15))
+
+
+@pytest.mark.parametrize("table", [0, 1])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("n,blocksize", [(1, 8), (8, 8), (513, 8), (2047, 16), (511, 512), (2049, 512), (1025, 1024), (6001, 2048),
+                                        (4096, 4096), (20003, 4096), (2 ** 24 + 77, 64), (3000, 48)])
+def test_quantize_4bit_units(hq, oracle, n, blocksize, dtype, table):
+    """Edges of the lane units, of the waves and of blocks longer than a unit row, zero and denormal blocks, NaN and
+    infinite values (codes as the comparisons of the definition give them): byte for byte the oracle's."""
+    import torch
+    rng = np.random.default_rng(n + blocksize)
+    x = (rng.standard_normal(n) * 0.3).astype(dtype)
+    if 2000 < n < 100000:
+        x[5], x[17], x[70], x[n - 1] = np.nan, np.inf, -np.inf, -0.0
+        x[100:n // 2] = 0
+        x[n // 2:n // 2 + 64] = 1e-40 if dtype == np.float32 else 6e-8
+    packed, absmax = hq.quantize_4bit(_t(x), blocksize, table)
+    torch.cuda.synchronize()
+    wp, wa = oracle.quantize_4bit(x, blocksize, table)
+    assert np.array_equal(absmax.cpu().numpy(), wa)
+    assert np.array_equal(packed.cpu().numpy(), wp)
