@@ -27,7 +27,7 @@ std::vector<std::pair<int, void*>> g_retired;  // outgrown buffers, freed by hq_
 namespace {
 const char* const kTunableNames[HQ_TUNE_COUNT] = {
     "HQ_Q3_WAVES", "HQ_Q3_STEPS", "HQ_Q3_KSPLIT", "HQ_Q3_TILE", "HQ_Q3_SMALL_BATCH", "HQ_Q3_ROW_BLOCKS", "HQ_LUT_PATH", "HQ_LUT_KSPLIT", "HQ_NF4_PIPE",
-    "HQ_AQLM_ROWS", "HQ_Q8_WGS", "HQ_Q8_FAST", "HQ_GEMV_LDS", "HQ_GEMV_SPLIT", "HQ_SPLITK_FENCES"};
+    "HQ_AQLM_ROWS", "HQ_Q8_WGS", "HQ_Q8_FAST", "HQ_GEMV_LDS", "HQ_GEMV_SPLIT", "HQ_SPLITK_FENCES", "HQ_Q3_TILES"};
 constexpr int kUnset = INT_MIN;
 std::atomic<int> g_tunables[HQ_TUNE_COUNT];
 std::once_flag g_tunables_once;
@@ -146,8 +146,13 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   // 8192 of them whatever the shape
   if ((size_t)8192 * 64 > split_floats) split_floats = (size_t)8192 * 64;
   *floats = gemm_floats > split_floats ? gemm_floats : split_floats;
+  // many rows: the tiled kernels
+  size_t tile_floats = 0, tile_counters = 0;
+  hq_q3_tiles_bound(cus, max_K, &tile_floats, &tile_counters);
+  if (tile_floats > *floats) *floats = tile_floats;
   // arrival counters: one per column tile, narrow tiles four per 64 columns, row blocks sixteen per tile
   *counters = tiles > 1 ? tiles * 16 : 16;
+  if (tile_counters > *counters) *counters = tile_counters;
 }
 
 extern "C" int hq_reserve_need(int compute_units, int max_K, int max_N, int64_t* floats, int64_t* counters) {

@@ -57,6 +57,14 @@ struct HqQ3Scratch {
 int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const float* scales, const float* zeros,
                       float* y, int K, int N, int batch_M, unsigned flags, hipStream_t stream,
                       const HqQ3Scratch* fixed);
+// Batched 3-bit GEMM: the pre-pass (activations [M][K] -> operand-slot order of Mpad rows and Gpad k-groups, row sums and
+// 1 / row scale), and the tiled kernels for many rows.
+int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad, hipStream_t stream);
+bool hq_q3_tiles_serve(int N, int M);
+int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
+void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);
+int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
+                       int M, unsigned flags, hipStream_t stream);
 // Resolves the current device's copy of the fixed scratch array (once per device).
 int hq_noalloc_setup(void);
 
@@ -65,7 +73,7 @@ int hq_noalloc_setup(void);
 // one relaxed atomic load.
 enum HqTunable {
   HQ_TUNE_Q3_WAVES, HQ_TUNE_Q3_STEPS, HQ_TUNE_Q3_KSPLIT, HQ_TUNE_Q3_TILE, HQ_TUNE_Q3_SMALL_BATCH, HQ_TUNE_Q3_ROW_BLOCKS, HQ_TUNE_LUT_PATH, HQ_TUNE_LUT_KSPLIT,
-  HQ_TUNE_NF4_PIPE, HQ_TUNE_AQLM_ROWS, HQ_TUNE_Q8_WGS, HQ_TUNE_Q8_FAST, HQ_TUNE_GEMV_LDS, HQ_TUNE_GEMV_SPLIT, HQ_TUNE_SPLITK_FENCES, HQ_TUNE_COUNT
+  HQ_TUNE_NF4_PIPE, HQ_TUNE_AQLM_ROWS, HQ_TUNE_Q8_WGS, HQ_TUNE_Q8_FAST, HQ_TUNE_GEMV_LDS, HQ_TUNE_GEMV_SPLIT, HQ_TUNE_SPLITK_FENCES, HQ_TUNE_Q3_TILES, HQ_TUNE_COUNT
 };
 int hq_tune(HqTunable id, int dflt);
 

@@ -513,7 +513,7 @@ int hq_q3_block_launch(const void* x, const int32_t* qweight, const float* scale
                        int K, int N, int M, int nsplit, int rpw, int mblocks, float* partial, unsigned* counters,
                        unsigned flags, hipStream_t stream);
 int hq_q3_block_groups_per_round(void);
-int hq_q3_gemm_need(int cus, int K, int N, size_t* floats, size_t* counters);
+int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
 
 namespace {
 // Zeroes n words with a kernel (a memset node inside a captured graph is not an option for callers
@@ -758,7 +758,7 @@ int hq_q3_workspace_need_impl(int cus, int K, int N, int batch_M, size_t* floats
     *counters = b.split.nsplit > 1 ? (size_t)b.split.ntiles : 0;
     return HQ_OK;
   }
-  return hq_q3_gemm_need(cus, K, N, floats, counters);
+  return hq_q3_gemm_need(cus, K, N, batch_M, floats, counters);
 }
 
 extern "C" int hq_q3_workspace_need(int compute_units, int K, int N, int batch_M, int64_t* floats, int64_t* counters) {

@@ -58,8 +58,8 @@ __global__ __launch_bounds__(256) void q3_gemm_prep(const _Float16* __restrict__
   // Eight consecutive rows share the 128-byte lines of Ap; workgroups b, b + 8, b + 16, ... run on the same
   // XCD, so the rows of a line go to workgroups of one XCD and its L2 writes whole lines back instead of
   // eight XCDs writing an eighth of every line each.
-  // (64 workgroups whatever Mpad; those beyond Mpad have nothing to do).
-  const int m = (blockIdx.x & 7) * 8 + (blockIdx.x >> 3);
+  // (a multiple of 64 workgroups whatever Mpad; those beyond Mpad have nothing to do).
+  const int m = ((int)blockIdx.x & ~63) + (blockIdx.x & 7) * 8 + ((blockIdx.x >> 3) & 7);
   if (m >= Mpad) return;
   __shared__ float s_sum[4], s_max[4];
   float sum = 0.f, amax = 0.f;
@@ -369,7 +369,14 @@ GemmPlan gemm_plan(int cus, int K, int N) {
 }
 }  // namespace
 
-int hq_q3_gemm_need(int cus, int K, int N, size_t* floats, size_t* counters) {
+int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad, hipStream_t stream) {
+  hipLaunchKernelGGL(q3_gemm_prep, dim3((Mpad + 63) / 64 * 64), dim3(256), 0, stream, reinterpret_cast<const _Float16*>(A),
+                     reinterpret_cast<_Float16*>(Ap), rowsum, rowinv, M, K, Mpad, Gpad);
+  return hq_launch_status();
+}
+
+int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
+  if (hq_q3_tiles_serve(N, M)) return hq_q3_tiles_need(cus, K, N, M, floats, counters);
   const GemmPlan p = gemm_plan(cus, K, N);
   *floats = p.ap_halves / 2 + 128 + p.partial_floats;
   *counters = 1;
@@ -380,6 +387,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
                       int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
   if (((uintptr_t)x & 15) || (K & 7)) return HQ_ERR_MISALIGNED;
   if (((uintptr_t)scales & 15) || ((uintptr_t)zeros & 15) || ((uintptr_t)y & 15)) return HQ_ERR_MISALIGNED;
+  if (!fixed && hq_q3_tiles_serve(N, M)) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream);
   const HqDevice* dev = nullptr;
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
@@ -409,8 +417,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
     const int MB = Mb > 32 ? 2 : 1;
     const int Mpad = 32 * MB;
     const _Float16* A = reinterpret_cast<const _Float16*>(x) + (size_t)m0 * K;
-    hipLaunchKernelGGL(q3_gemm_prep, dim3(64), dim3(256), 0, stream, A, Ap, rowsum, rowinv, Mb, K, Mpad, Gpad);
-    rc = hq_launch_status();
+    rc = hq_q3_gemm_prep_launch(A, Ap, rowsum, rowinv, Mb, K, Mpad, Gpad, stream);
     if (rc != HQ_OK) return rc;
     GemmArgs a;
     a.w = reinterpret_cast<const uint32_t*>(qweight);

@@ -92,7 +92,7 @@ int hq_shutdown(void);
 
 /* Launch-shape override for tests and sweeps, not part of the stable interface: name is one of
  * HQ_Q3_WAVES, HQ_Q3_STEPS, HQ_Q3_KSPLIT, HQ_Q3_TILE, HQ_Q3_SMALL_BATCH, HQ_Q3_ROW_BLOCKS, HQ_LUT_PATH, HQ_LUT_KSPLIT, HQ_NF4_PIPE,
- * HQ_AQLM_ROWS, HQ_Q8_WGS, HQ_Q8_FAST, HQ_GEMV_LDS, HQ_GEMV_SPLIT, HQ_SPLITK_FENCES (an environment variable of the same name seeds
+ * HQ_AQLM_ROWS, HQ_Q8_WGS, HQ_Q8_FAST, HQ_GEMV_LDS, HQ_GEMV_SPLIT, HQ_SPLITK_FENCES, HQ_Q3_TILES (an environment variable of the same name seeds
  * the knob once per process); clear != 0 returns the knob to the library's own choice.  Results
  * never depend on a knob beyond the documented tolerances. */
 int hq_set_tunable(const char* name, int value, int clear);
@@ -148,7 +148,8 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  *     workgroup unless N / 128 is at least 7/8 of the compute units or K is longer than that;
  *     every activation enters with an error of at most 2^-19 of the largest magnitude
  *     among its 32 neighbours (exactly, if within 2^8 of it);
- *   - everything else: the MFMA GEMM path, which pre-scales every activation row by a
+ *   - everything else: the MFMA GEMM path (64 rows per pass over the weights; more than 96 rows, or more than 64 with
+ *     N > 4096: tiles of 64 or 128 rows, thousands of rows per pass), which pre-scales every activation row by a
  *     power of two, so accuracy does not depend on the magnitude of the activations:
  *     entries within 2^21 of their row's largest magnitude enter the matrix cores
  *     exactly, smaller ones lose low bits (those 2^32 below it vanish).
@@ -168,7 +169,8 @@ int hq_q3_matvec_plan(int K, int N, int batch_M);
 
 /*
  * hq_q3_matvec for callers that cannot allocate (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results, but the
+ * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results (except for the
+ * many rows that hq_q3_matvec takes in tiles: here they go 64 at a time, with results equal to rounding), but the
  * scratch the kernels need (split-K partial sums and arrival counters of batches 1 and 2, the batched
  * path's re-ordered activations, row sums, row scales and K-split sums) is a fixed 10 MiB + 64 KiB array in device
  * memory that each GPU holds from library load to process end, instead of the stream's workspace.

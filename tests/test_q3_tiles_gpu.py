@@ -1,0 +1,75 @@
+"""The tiled kernels of the batched 3-bit GEMM (many rows): every tile kind, undivided and divided along K, at the edges of
+tiles, steps and k-groups, against the oracle row by row."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tests import oracle_api as oa
+from tests.tol import FLOOR_F16, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _t(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+
+
+def _check(y, exact, rows=True):
+    # as for the 64-row kernel: the only error is the matrix cores' fp32 accumulation, about 1e-5 of the RMS - of the row's
+    # own, as every row is a sum of its own magnitude (an outlier's products cancel in single results, not in the row)
+    for m in range(len(y)) if rows else [slice(None)]:
+        if exact[m].any():
+            assert rel_err(y[m], exact[m]) <= 5e-3, m
+            assert rel_err(y[m], exact[m], FLOOR_F16) <= 1e-4, m
+        else:
+            assert not y[m].any(), m
+
+
+@pytest.mark.parametrize("kind,shares", [(0, 1), (0, 2), (0, 5), (1, 1), (1, 2), (1, 3), (2, 1), (2, 2), (2, 8)])
+@pytest.mark.parametrize("M,K,N", [(97, 32, 4), (128, 1024, 256), (129, 2080, 260), (193, 1376, 132), (300, 96, 1028),
+                                   (98, 4128, 516)])
+def test_kinds_and_shares(hq, oracle, tunable, kind, shares, M, K, N):
+    codes, scales, zeros, A = oa.make_q3_problem(M + K + N, K, N, x_dtype=np.float16, batch=M)
+    A[5] *= np.float16(2.0 ** -10)     # rows of other magnitudes, a zero row, an outlier
+    A[7] = 0
+    # An outlier at k = 3 of its k-group.  (At k = 0 the matrix instruction's own sum of sixteen products loses 2^-16 of
+    # the outlier's product: 1.2e-4 of such a row's RMS, here and in the 64-row kernel bit for bit alike.)
+    A[9, K // 64 * 32 + 3] = np.float16(4096.0)
+    mat = oracle.q3_pack(codes)
+    tunable("HQ_Q3_TILES", kind + 10 * shares)
+    y = hq.q3_gemm(_t(A), _t(mat), _t(scales), _t(zeros))
+    again = hq.q3_gemm(_t(A), _t(mat), _t(scales), _t(zeros))
+    assert np.array_equal(y.cpu().numpy(), again.cpu().numpy())  # shares are added in a fixed order
+    exact = oracle.q3_gemm(A, mat, scales, zeros, mode=0)
+    _check(y.cpu().numpy(), exact)
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 4096, 4096), (700, 512, 3000), (1030, 16416, 8), (70, 256, 8200)])
+def test_default_plans(hq, oracle, M, K, N):
+    """The library's own choice: few tiles, several full rounds with a rest, several passes over the rows, 65 ... 96 rows of a
+    wide matrix.  Rows of one magnitude: the RMS of the whole result is the measure, as in the 64-row kernel's tests (a few
+    columns of one row are no sample of it)."""
+    codes, scales, zeros, A = oa.make_q3_problem(M + K, K, N, x_dtype=np.float16, batch=M)
+    mat = oracle.q3_pack(codes)
+    y = hq.q3_gemm(_t(A), _t(mat), _t(scales), _t(zeros)).cpu().numpy()
+    cols = np.unique(np.concatenate([np.arange(0, min(N, 70)), np.arange(max(0, N - 70), N)]))
+    _check(y[:, cols], oracle.q3_gemm(A, np.ascontiguousarray(mat[:, cols]), scales[cols], zeros[cols], mode=0), rows=False)
+
+
+def test_accumulate_and_the_call_that_allocates_nothing(hq, oracle):
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    M, K, N = 200, 1024, 516
+    codes, scales, zeros, A = oa.make_q3_problem(3, K, N, x_dtype=np.float16, batch=M)
+    mat = oracle.q3_pack(codes)
+    exact = oracle.q3_gemm(A, mat, scales, zeros, mode=0)
+    a, w, s, z = _t(A), _t(mat), _t(scales), _t(zeros)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for fn in (lib.hq_q3_matvec, lib.hq_q3_matvec_noalloc):
+        y = torch.full((M, N), 3.0, device="cuda:0")
+        assert fn(a.data_ptr(), 1, w.data_ptr(), s.data_ptr(), z.data_ptr(), y.data_ptr(), K, N, M, 1, stream) == 0
+        torch.cuda.synchronize()
+        _check(y.cpu().numpy() - 3.0, exact)
