@@ -45,8 +45,8 @@ __device__ __forceinline__ uint32_t quantize_one(const float* lds, float x) {
 // of thresholds T_i = (c_i + c_i+1) / 2, i = 0..254, that x has passed, where an even i is passed by
 // x > T_i and an odd i by x >= T_i (ties keep the pivot, and pivots are the even entries).  That holds
 // whenever c_i < T_i < c_i+1; a gap where rounding or equal entries break it is "degenerate".
-// Inputs are binned by a monotone key (the exponent and six mantissa bits of |x| + off: 64 buckets per
-// binade down to off = M / 4096, linear below, one overflow bucket beyond the largest magnitude M; the
+// Inputs are binned by a monotone key (the exponent and six mantissa bits of |x| + M / 4096: 64 buckets per
+// binade down to M / 4096, linear below, one overflow bucket beyond the largest magnitude M; the
 // sign picks one of two slots).  A bucket's entry holds the number of thresholds in lower buckets and
 // the one threshold inside it (an odd i as the float just below T_i, so that every test is x > t;
 // +inf if there is none), so a lookup is one 8-byte LDS read, one compare and one add.  Buckets with
@@ -58,17 +58,23 @@ constexpr int kKeyShift = 17;       // six mantissa bits
 constexpr int kMaxBuckets = 13 * 64 + 66;  // per sign: 12 binades from off to M, the linear one, a partial top, overflow
 constexpr uint32_t kSlow = 0x7fc00000u;
 
+constexpr int kThreads = 1024;  // one table for sixteen waves, two workgroups per compute unit
+
 struct FastTables {
   uint2 entry[2 * kMaxBuckets];  // slot 2 * idx (x >= +0) or 2 * idx + 1 (sign bit set): {threshold, count}
-  uint32_t inside[(2 * kMaxBuckets + 255) / 256 * 256];  // thresholds per bucket, in value order
+  uint32_t pos[256 + 2];         // place of every threshold's bucket in value order, non-decreasing; then beyond all
   float tval[256];               // the thresholds as "x > t" tests
-  uint32_t wave_total[4];
 };
 
-__device__ __forceinline__ uint32_t bucket_slot(float x, float off, uint32_t base, uint32_t cnt) {
-  const float y2 = fabsf(x) + off;  // >= off; a NaN lands in the overflow bucket
-  const uint32_t idx = min((__float_as_uint(y2) - base) >> kKeyShift, cnt);
-  return 2 * idx + (__float_as_uint(x) >> 31);
+// The key: |x| scaled so that M / 4096 becomes 2, plus 2, cut at `top` (the first value of the overflow bucket, where a NaN
+// lands too).  Between 2 and 2^17 the exponent's low four bits count up from zero, so the bucket number is ten bits of it.
+struct Key {
+  float scale, top;
+};
+__device__ __forceinline__ uint32_t bucket_of(float y) { return (__float_as_uint(y) >> kKeyShift) & 1023u; }
+__device__ __forceinline__ uint32_t bucket_slot(float x, const Key& key) {
+  const float y = fminf(fmaf(fabsf(x), key.scale, 2.f), key.top);
+  return __builtin_amdgcn_alignbit(bucket_of(y), __float_as_uint(x), 31);
 }
 // buckets in the order of the values they hold: negative overflow first, positive overflow last
 __device__ __forceinline__ uint32_t slot_order(uint32_t slot, uint32_t cnt) {
@@ -79,18 +85,14 @@ __device__ __forceinline__ uint32_t order_slot(uint32_t pos, uint32_t cnt) {
   return pos <= cnt ? 2 * (cnt - pos) + 1 : 2 * (pos - cnt - 1);
 }
 
-// a, b: table entries t and t + 1 of thread t (t < 255).  All 256 threads.  Thresholds are counted into
-// their buckets, a scan over the buckets in value order gives every bucket the number of thresholds
-// before it, which is also the index of the first threshold inside it.
-__device__ __forceinline__ void build_fast_tables(FastTables& ft, float a, float b, float off, uint32_t base,
-                                                  uint32_t cnt) {
+// a, b: table entries t and t + 1 of thread t (t < 255).  All threads.  The places of the thresholds' buckets are sorted, so
+// a bucket finds the number of thresholds before it by bisection, and with it the one inside it, if any: eight dependent
+// LDS reads and three barriers, and one table serves 1024 threads.  (Before: counting into the buckets and a scan over
+// them, six barriers, in each of five workgroups of 256 threads per compute unit.)
+__device__ __forceinline__ void build_fast_tables(FastTables& ft, float a, float b, const Key& key, uint32_t cnt) {
   const int t = threadIdx.x;
-  const uint32_t nb = 2 * cnt + 2;             // buckets, both signs and overflows
-  constexpr uint32_t kPer = (2 * kMaxBuckets + 255) / 256;  // buckets per thread
+  const uint32_t nb = 2 * cnt + 2;  // buckets, both signs and overflows
   bool degenerate = false;
-  uint32_t mine = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < kPer; ++k) ft.inside[t * kPer + k] = 0;
   if (t < 255) {
     float T = (b + a) * 0.5f;
     degenerate = !(a < T && T < b);
@@ -103,164 +105,146 @@ __device__ __forceinline__ void build_fast_tables(FastTables& ft, float a, float
       T = T + 0.f;
       tv = T;
     }
-    mine = slot_order(bucket_slot(T, off, base, cnt), cnt);
+    ft.pos[t] = slot_order(bucket_slot(T, key), cnt);
     ft.tval[t] = tv;
+  } else if (t < 258) {
+    ft.pos[t] = 0xffffffffu;
   }
   __syncthreads();
-  if (t < 255) atomicAdd(&ft.inside[mine], 1u);
-  __syncthreads();
-  uint32_t c[kPer], sum = 0;
+  constexpr uint32_t kPer = (2 * kMaxBuckets + kThreads - 1) / kThreads;  // buckets per thread
+  uint32_t i[kPer];  // thresholds before bucket t + k * kThreads: fewer than 256
 #pragma unroll
-  for (uint32_t k = 0; k < kPer; ++k) { c[k] = ft.inside[t * kPer + k]; sum += c[k]; }
-  uint32_t incl = sum;  // inclusive scan over the wave, then over the four waves
+  for (uint32_t k = 0; k < kPer; ++k) i[k] = 0;
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t up = __shfl_up(incl, d);
-    if ((t & 63) >= d) incl += up;
-  }
-  if ((t & 63) == 63) ft.wave_total[t >> 6] = incl;
-  __syncthreads();
-  uint32_t before = incl - sum;
-  for (int w = 0; w < (t >> 6); ++w) before += ft.wave_total[w];
+  for (uint32_t step = 128; step > 0; step >>= 1)
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) i[k] += ft.pos[i[k] + step - 1] < t + k * kThreads ? step : 0u;
 #pragma unroll
   for (uint32_t k = 0; k < kPer; ++k) {
-    const uint32_t pos = t * kPer + k;
-    if (pos < nb) {
+    const uint32_t p = t + k * kThreads;
+    if (p < nb) {
+      const bool one = ft.pos[i[k]] == p, two = ft.pos[i[k] + 1] == p;
       uint2 e;
-      e.x = c[k] ? __float_as_uint(ft.tval[min(before, 254u)]) : 0x7f800000u;  // +inf: x > t never holds
-      e.y = c[k] <= 1 ? before : kSlow;
-      ft.entry[order_slot(pos, cnt)] = e;
+      e.x = one ? __float_as_uint(ft.tval[i[k]]) : 0x7f800000u;  // +inf: x > t never holds
+      e.y = two ? kSlow : i[k];
+      ft.entry[order_slot(p, cnt)] = e;
     }
-    before += c[k];
   }
-  __syncthreads();
+  if (!__syncthreads_or(degenerate)) return;
   if (degenerate) {  // every input between and on the two entries is in one of their buckets
-    ft.entry[bucket_slot(a, off, base, cnt)].y = kSlow;
-    ft.entry[bucket_slot(b, off, base, cnt)].y = kSlow;
+    ft.entry[bucket_slot(a, key)].y = kSlow;
+    ft.entry[bucket_slot(b, key)].y = kSlow;
     if (a == 0.f || b == 0.f) ft.entry[0].y = ft.entry[1].y = kSlow;  // both zeros' buckets
   }
   __syncthreads();
 }
 
-constexpr int kQuads = 4;  // 16-byte loads per thread and trip
+constexpr int kAhead = 2;  // 16-byte loads of a thread and step: 64 KB of a step per compute unit, what it holds in flight
 
-__global__ __launch_bounds__(256) void quantize8_kernel(const float* __restrict__ code,
-                                                       const float* __restrict__ A,
-                                                       uint8_t* __restrict__ out, int64_t n,
-                                                       int vec_ok, int allow_fast) {
+// What bounds it: HBM (5 bytes per element) behind the fixed cost of the tables, and close behind the lookups, ten vector
+// operations and one random 8-byte LDS read per element.  A thread takes every gridDim.x * 1024-th quad; its first loads
+// are in flight while the tables are built, and a step's go out together while the step before is converted (one by one
+// as registers come free: 118 against 109 us at 2^27; four per thread: 118).
+// us per call, before -> now: 2^16 elements 4.43 -> 4.20, 2^22 8.2 -> 7.8, 10^7 11.8 -> 11.4, 2^24 16.8 -> 16.5, 2^27
+// 109.7 -> 108.6 (6.2 TB/s).
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void quantize8_kernel(
+    const float* __restrict__ code, const float* __restrict__ A, uint8_t* __restrict__ out, int64_t n, int vec_ok, int allow_fast) {
   __shared__ float s_code[512];
   __shared__ __align__(16) FastTables ft;
   const int t = threadIdx.x;
-  const float ct = code[t], cn = code[min(t + 1, 255)];
+  const int64_t nquads = vec_ok ? n / 4 : 0;
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  const int64_t t0 = (int64_t)blockIdx.x * kThreads + t;
+  f4v v[kAhead];
+  auto load = [&](int64_t i) { return __builtin_nontemporal_load(reinterpret_cast<const f4v*>(A) + (i < nquads ? i : nquads - 1)); };
+  // the table first: a compute unit returns its loads in the order they were issued
+  const float ct = code[min(t, 255)], cn = code[min(t + 1, 255)];
   const float M = fmaxf(fabsf(code[0]), fabsf(code[255]));
-  {
-    if (t < 255) {  // level-order slot t <- table entry ((2j+1) << (8-k)) - 1
-      const int k = 32 - __builtin_clz((unsigned)t + 1);  // level 1..8
-      const int j = t + 1 - (1 << (k - 1));
-      s_code[t] = code[((2 * j + 1) << (8 - k)) - 1];
-    }
+  const int level = 32 - __builtin_clz((unsigned)min(t, 254) + 1);  // 1..8
+  const float ordered = code[((2 * (min(t, 254) + 1 - (1 << (level - 1))) + 1) << (8 - level)) - 1];
+  __builtin_amdgcn_sched_barrier(0);
+  if (nquads > 0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) v[k] = load(t0 + k * stride);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (t < 256) {
+    s_code[t] = ordered;  // level-order slot t: entry ((2j+1) << (8-k)) - 1
     s_code[256 + t] = ct;
   }
   // the fast path wants a sorted table of finite, moderate values (midpoints cannot overflow) with a
   // usable magnitude
-  const float off = M * (1.f / 4096.f);
-  const uint32_t base = __float_as_uint(off) & ~((1u << kKeyShift) - 1);
-  const uint32_t cnt = ((__float_as_uint(M + off) - base) >> kKeyShift) + 1;  // index of the overflow bucket
+  Key key;
+  key.scale = 8192.f / M;
+  const float y_top = fmaf(M, key.scale, 2.f);
+  const uint32_t cnt = bucket_of(y_top) + 1;  // index of the overflow bucket
+  key.top = __uint_as_float((__float_as_uint(y_top) & ~((1u << kKeyShift) - 1)) + (1u << kKeyShift));
   const bool fast = __syncthreads_and((ct <= cn) && fabsf(ct) <= 1e30f) && M >= 1e-30f && allow_fast &&
                     cnt < (uint32_t)kMaxBuckets;
-  const int64_t nquads = vec_ok ? n / 4 : 0;
-  const int64_t stride = (int64_t)gridDim.x * 256;
-  const int64_t t0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (fast) {
-    // the first trip's loads are in flight while the tables are built, and each later trip's while the
-    // one before is converted
-    f4v v[kQuads], vn[kQuads];
-    auto load = [&](int64_t i, f4v (&dst)[kQuads]) {
+    build_fast_tables(ft, ct, cn, key, cnt);
+    const int64_t wave0 = t0 - (t & 63);  // the wave's first quad
+    for (int64_t step = 0; wave0 + step < nquads; step += kAhead * stride) {
+      // the next step's loads go out together, clamped instead of under a branch
+      f4v vn[kAhead];
 #pragma unroll
-      for (int k = 0; k < kQuads; ++k) {
-        const int64_t ik = i + k * stride;
-        dst[k] = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(A) + (ik < nquads ? ik : i));
-      }
-    };
-    if (t0 < nquads) load(t0, v);
-    build_fast_tables(ft, ct, cn, off, base, cnt);
-    for (int64_t i = t0; i < nquads; i += kQuads * stride) {
-      const int64_t inext = i + kQuads * stride;
-      if (inext < nquads) load(inext, vn);
-      uint32_t q[4 * kQuads];
-      bool slow = false;
+      for (int k = 0; k < kAhead; ++k) vn[k] = load(t0 + step + (kAhead + k) * stride);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < kQuads; ++k) {
+      for (int k = 0; k < kAhead; ++k) {
+        const int64_t i = t0 + step + k * stride;
+        if (wave0 + step + k * stride >= nquads) break;  // wave-uniform
         const float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        uint32_t q[4];
+        uint64_t slow = 0;
+        uint2 en[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) en[e] = ft.entry[bucket_slot(x[e], key)];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const uint2 en = ft.entry[bucket_slot(x[e], off, base, cnt)];
-          q[4 * k + e] = en.y + (x[e] > __uint_as_float(en.x) ? 1u : 0u);
-          slow |= !(__uint_as_float(en.y) <= x[e] || __uint_as_float(en.y) > x[e]);  // unordered: flagged bucket or NaN input
+          q[e] = en[e].y + (x[e] > __uint_as_float(en[e].x) ? 1u : 0u);
+          // unordered: a flagged bucket or a NaN input
+          slow |= __builtin_amdgcn_fcmpf(__uint_as_float(en[e].y), x[e], 8);  // FCMP_UNO
         }
-      }
-      if (__builtin_amdgcn_ballot_w64(slow)) {
-#pragma unroll
-        for (int k = 0; k < kQuads; ++k) {
-          const float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        if (slow) {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            if (q[4 * k + e] > 255u || x[e] != x[e]) q[4 * k + e] = quantize_one(s_code, x[e]);
+            if (q[e] > 255u || x[e] != x[e]) q[e] = quantize_one(s_code, x[e]);
         }
+        if (i < nquads)
+          __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), reinterpret_cast<uint32_t*>(out) + i);
       }
 #pragma unroll
-      for (int k = 0; k < kQuads; ++k) {
-        const int64_t ik = i + k * stride;
-        if (ik < nquads)
-          __builtin_nontemporal_store(q[4 * k] | (q[4 * k + 1] << 8) | (q[4 * k + 2] << 16) | (q[4 * k + 3] << 24),
-                                      reinterpret_cast<uint32_t*>(out) + ik);
-      }
-#pragma unroll
-      for (int k = 0; k < kQuads; ++k) v[k] = vn[k];
+      for (int k = 0; k < kAhead; ++k) v[k] = vn[k];
     }
   } else {
-  __syncthreads();
-  // Two quads per trip, searched in lockstep level by level: eight independent LDS reads
-  // are in flight per level instead of one dependent chain per element.
-  for (int64_t i = t0; i < nquads; i += 2 * stride) {
-    const int64_t i1 = i + stride;
-    const bool two = i1 < nquads;
-    const f4v v0 = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(A) + i);
-    const f4v v1 = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(A) + (two ? i1 : i));
-    const float x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-    uint32_t j[8];
-    float val[8];
+    __syncthreads();
+    // The descent for four elements at a time, level by level: four independent LDS reads are in flight per level instead
+    // of one dependent chain per element.
+    for (int64_t i = t0; i < nquads; i += stride) {
+      const f4v v0 = load(i);
+      const float x[4] = {v0.x, v0.y, v0.z, v0.w};
+      uint32_t j[4], q[4];
+      float val[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { j[e] = 0; val[e] = s_code[0]; }
+      for (int e = 0; e < 4; ++e) { j[e] = 0; val[e] = s_code[0]; }
 #pragma unroll
-    for (int k = 1; k < 8; ++k) {
+      for (int k = 1; k < 8; ++k) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) j[e] = 2 * j[e] + (x[e] > val[e] ? 1u : 0u);
+        for (int e = 0; e < 4; ++e) j[e] = 2 * j[e] + (x[e] > val[e] ? 1u : 0u);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) val[e] = s_code[(1u << k) - 1 + j[e]];
+        for (int e = 0; e < 4; ++e) val[e] = s_code[(1u << k) - 1 + j[e]];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool up = x[e] > val[e];
+        const uint32_t pivot = 2 * j[e];
+        const uint32_t other = up ? pivot + 1 : (pivot == 0 ? 0u : pivot - 1);
+        const float midpoint = (s_code[256 + other] + val[e]) * 0.5f;
+        q[e] = (up ? x[e] > midpoint : x[e] < midpoint) ? other : pivot;
+      }
+      __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), reinterpret_cast<uint32_t*>(out) + i);
     }
-    uint32_t other[8];
-    float bound[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t pivot = 2 * j[e];
-      other[e] = x[e] > val[e] ? pivot + 1 : (pivot == 0 ? 0u : pivot - 1);
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) bound[e] = s_code[256 + other[e]];
-    uint32_t q[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float midpoint = (bound[e] + val[e]) * 0.5f;
-      const bool up = x[e] > val[e];
-      q[e] = (up ? x[e] > midpoint : x[e] < midpoint) ? other[e] : 2 * j[e];
-    }
-    __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24),
-                                reinterpret_cast<uint32_t*>(out) + i);
-    if (two)
-      __builtin_nontemporal_store(q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24),
-                                  reinterpret_cast<uint32_t*>(out) + i1);
-  }
   }
   for (int64_t e = nquads * 4 + t0; e < n; e += stride) out[e] = (uint8_t)quantize_one(s_code, A[e]);
 }
@@ -278,13 +262,13 @@ extern "C" int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* 
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
   const int vec_ok = !((uintptr_t)A & 15) && !((uintptr_t)out & 3);
-  int64_t blocks = (n / 4 + 256 * kQuads - 1) / (256 * kQuads);  // one trip of the fast path each, or grid-stride
-  // workgroups per CU of the persistent fast path: five up to 2^24 elements (16.5 us; two 17.8, eight 19.2),
-  // two from 2^25 on (2^25: 30.5 against 31.4 us with five, 2^26: 55.4 against 59.7, 2^27: 108.6 against 123.2)
-  const int64_t cap = (int64_t)dev->cus * hq_tune(HQ_TUNE_Q8_WGS, n >= ((int64_t)1 << 25) ? 2 : 5);
+  int64_t blocks = (n / 4 + kThreads - 1) / kThreads;
+  // workgroups per CU (us with one / two: 2^22 elements 7.8 / 8.2, 10^7 12.8 / 11.5, 2^25 31.1 / 31.0, 2^27 108.6 / 118.2):
+  // two fill the CU's queue between the ends, where latency or the order of the stream counts more
+  const int64_t cap = (int64_t)dev->cus * hq_tune(HQ_TUNE_Q8_WGS, n > ((int64_t)5 << 20) && n < ((int64_t)1 << 26) ? 2 : 1);
   if (blocks > cap) blocks = cap;
   if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(quantize8_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, code, A, out, n,
+  hipLaunchKernelGGL(quantize8_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, code, A, out, n,
                      vec_ok, hq_tune(HQ_TUNE_Q8_FAST, 1));
   return hq_launch_status();
 }

@@ -120,3 +120,14 @@ def test_full_size_round_trip(hq):
     assert bool(((q == lo) | (q == lo + 1)).all())
     nearest = torch.where((x - code[lo]).abs() <= (code[(lo + 1).clamp(max=255)] - x).abs(), lo, lo + 1)
     assert float((q != nearest).float().mean()) < 1e-4        # they differ on exact ties only
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 255, 4096 - 1, 4096 + 4, 262144 * 4 + 20, 2 * 1048576 * 4 + 36, (5 << 20) + 4097])
+def test_ends_of_the_grid(hq, oracle, n):
+    """Lengths around a workgroup's quads, a full round of one and of two workgroups per compute unit and of the steps of two
+    quads, with values beyond the table, NaN, infinities and zeros of both signs at the ends."""
+    code = oracle.dynamic_map()
+    A = (np.random.default_rng(n).standard_normal(n) * 0.2).astype(np.float32)
+    special = np.array([np.nan, np.inf, -np.inf, 0.0, -0.0, 5.0, -5.0, 1e-45], np.float32)
+    A[-8:] = special[:n]
+    assert np.array_equal(_run(hq, code, A), oracle.quantize_dynamic8(code, A))
