@@ -237,3 +237,32 @@ def test_vs_reference_device_kernels(hq, dtype, code):
         assert torch.equal(gs, ws) and torch.equal(got, want), with_azp
         if with_azp:
             assert torch.equal(gz, wz)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_quotients_of_16_bit_rows(hq, oracle, dtype):
+    """Where the three-operation quotient could go wrong: exact ties of either parity and their neighbours, scales with a
+    mantissa of all ones (left to the division) and next to it, zero points at and beyond the bound, overflow on the way."""
+    import torch
+    tdt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    rng = np.random.default_rng(5)
+    k = np.arange(-300, 301, dtype=np.float32)
+    rows = [np.resize(np.concatenate([k * 0.5, k * 0.375, k * 0.25 + 0.125]), 2048),       # ties for 1, 0.75 / 0.03-like, 0.25
+            np.resize(k * 0.0625, 2048) * 3, rng.standard_normal(2048), 1000 + rng.standard_normal(2048),
+            np.clip(rng.standard_normal(2048) * 2e4, -65504, 65504),  # no infinity: undefined with a zero point
+            np.resize(np.array([255.0, 0.0, 127.5, 0.5, 1.5, 2.5], np.float32), 2048)]
+    x = torch.from_numpy(np.stack(rows).astype(np.float32)).to(tdt)
+    x = x if dtype == "bf16" else x.numpy()
+    ones = np.float32(np.uint32(0x3f7fffff).view(np.float32))  # 1 - 2^-24
+    for scale in (1.0, 0.75, 0.5, 0.03, float(ones), float(np.nextafter(ones, np.float32(0))), 1e-20, 3e30, -0.25):
+        for azp in (None, 0, 1, -7, 65536, -65792, 65793, 2 ** 30):
+            if azp and (abs(scale) < 1e-10 or abs(azp) > 2 ** 29 and abs(scale) < 1e-4):
+                continue  # quotient plus zero point beyond int32 is undefined
+            want = oracle.int8_quant_static(x, scale, azp)
+            got = hq.static_scaled_int8_quant(_dev(x), scale, azp).cpu().numpy()
+            assert np.array_equal(got, want), (scale, azp)
+    for with_azp in (False, True):
+        got, gs, gz = hq.dynamic_scaled_int8_quant(_dev(x), with_azp)
+        want, ws, wz = oracle.int8_quant_dynamic(x, with_azp)
+        assert np.array_equal(gs.cpu().numpy(), ws) and np.array_equal(got.cpu().numpy(), want)
+        assert not with_azp or np.array_equal(gz.cpu().numpy(), wz)
