@@ -57,6 +57,19 @@ __device__ __forceinline__ uint32_t deq_pair(const float* tab, uint32_t byte, fl
   return __builtin_bit_cast(uint32_t, h);
 }
 
+// The n % 8 elements behind the last whole word: where there are any, the launch has one workgroup more and that does
+// nothing else.  A launch of its own for them cost every call whose size is no multiple of eight 2.5 us (blocksize 64:
+// 33,223 elements 6.5 us, 4.0 this way; 16,777,221 9.1, 7.1; the same work in a workgroup of the main grid took 7.5, the waits
+// for its loads standing before the others').
+__device__ __forceinline__ void store_tail(const uint32_t* packed, const float* absmax, u4v* out, int64_t nwords, int blocksize,
+                                           int table, int ntail) {
+  if ((int)threadIdx.x >= ntail) return;
+  const int64_t e = nwords * 8 + threadIdx.x;
+  const uint32_t byte = reinterpret_cast<const uint8_t*>(packed)[e >> 1];
+  const uint32_t code = (e & 1) ? (byte & 15u) : (byte >> 4);
+  reinterpret_cast<_Float16*>(out)[e] = (_Float16)mul_rounded_f32((table ? c_fp4 : c_nf4)[code], absmax[e / blocksize]);
+}
+
 // Main path.  A lane turns one packed 32-bit word (8 codes) into one 128-bit store,
 // so every load instruction of a wave reads 256 contiguous bytes and every store
 // instruction writes 1 KB of contiguous, fully covered cache lines (a lane that
@@ -67,11 +80,15 @@ __device__ __forceinline__ uint32_t deq_pair(const float* tab, uint32_t byte, fl
 //   MODE 0: blocksize == 1 << shift and blocksize % 8 == 0 (one absmax per word)
 //   MODE 1: blocksize % 8 == 0, not a power of two (one absmax per word, division)
 //   MODE 2: any even blocksize (absmax looked up per element)
-template <int U, int MODE, int NT>
+template <int U, int MODE, int NT, bool TAIL>
 __global__ __launch_bounds__(256) void dequant4_kernel(const uint32_t* __restrict__ packed,
                                                       const float* __restrict__ absmax,
                                                       u4v* __restrict__ out, int64_t nwords,
-                                                      int blocksize, int shift, int table) {
+                                                      int blocksize, int shift, int table, int ntail) {
+  if (TAIL && blockIdx.x == gridDim.x - 1) {
+    store_tail(packed, absmax, out, nwords, blocksize, table, ntail);
+    return;
+  }
   __shared__ float tab[16];
   if (threadIdx.x < 16) tab[threadIdx.x] = table ? c_fp4[threadIdx.x] : c_nf4[threadIdx.x];
   const int64_t base = (int64_t)blockIdx.x * (256 * U) + threadIdx.x;
@@ -114,11 +131,16 @@ __global__ __launch_bounds__(256) void dequant4_kernel(const uint32_t* __restric
 // words with the next chunk's loads in flight while the current chunk is converted and stored, so the read and
 // the write streams overlap in time.  Index arithmetic is 32-bit; the table offsets of a word's eight codes
 // come from two masked copies of the word (low and high nibble of every byte, times four).
-template <int U>
+template <int U, bool TAIL>
 __global__ __launch_bounds__(256) void dequant4_pipelined_kernel(const uint32_t* __restrict__ packed,
                                                                 const float* __restrict__ absmax,
                                                                 u4v* __restrict__ out, uint32_t nwords, int shift,
-                                                                int table) {
+                                                                int table, int ntail) {
+  const uint32_t grid = TAIL ? gridDim.x - 1 : gridDim.x;
+  if (TAIL && blockIdx.x == grid) {
+    store_tail(packed, absmax, out, nwords, 1 << shift, table, ntail);
+    return;
+  }
   __shared__ float tab[16];
   if (threadIdx.x < 16) tab[threadIdx.x] = table ? c_fp4[threadIdx.x] : c_nf4[threadIdx.x];
   constexpr uint32_t chunk_words = 256 * U;
@@ -139,8 +161,8 @@ __global__ __launch_bounds__(256) void dequant4_pipelined_kernel(const uint32_t*
   if (chunk < nchunks) load(chunk, w, am);
   __syncthreads();
   const char* tb = reinterpret_cast<const char*>(tab);
-  for (; chunk < nchunks; chunk += gridDim.x) {
-    const uint32_t next = chunk + gridDim.x;
+  for (; chunk < nchunks; chunk += grid) {
+    const uint32_t next = chunk + grid;
     if (next < nchunks) load(next, wn, amn);
     const uint32_t base = chunk * chunk_words + threadIdx.x;
 #pragma unroll
@@ -164,12 +186,12 @@ __global__ __launch_bounds__(256) void dequant4_pipelined_kernel(const uint32_t*
   }
 }
 
-// Tail / odd sizes: one element per thread.
-__global__ __launch_bounds__(256) void dequant4_tail_kernel(const uint8_t* __restrict__ packed,
-                                                           const float* __restrict__ absmax,
-                                                           _Float16* __restrict__ out, int64_t e_begin,
-                                                           int64_t n, int blocksize, int table) {
-  const int64_t e = e_begin + (int64_t)blockIdx.x * 256 + threadIdx.x;
+// Buffers without the alignment of words and 128-bit stores, and fewer than eight elements: one element per thread.
+__global__ __launch_bounds__(256) void dequant4_element_kernel(const uint8_t* __restrict__ packed,
+                                                              const float* __restrict__ absmax,
+                                                              _Float16* __restrict__ out, int64_t n, int blocksize,
+                                                              int table) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= n) return;
   const float* tab = table ? c_fp4 : c_nf4;
   const uint32_t byte = packed[e >> 1];
@@ -194,6 +216,7 @@ extern "C" int hq_dequant_nf4(const uint8_t* packed, const float* absmax, void* 
   const bool wide = !((uintptr_t)packed & 3) && !((uintptr_t)out_fp16 & 15);
   const int64_t nwords = wide ? n_elems / 8 : 0;
   if (nwords > 0) {
+    const int ntail = (int)(n_elems - nwords * 8);
     const bool pow2 = (blocksize & (blocksize - 1)) == 0;
     int shift = 0;
     while ((1 << shift) < blocksize) ++shift;
@@ -203,11 +226,14 @@ extern "C" int hq_dequant_nf4(const uint8_t* packed, const float* absmax, void* 
     // fastest combination (7.8 us; plain stores 10-12 us), flat in U from 1 to 8.
     constexpr int U = 8, NT = 2;
     const int64_t blocks = (nwords + 256 * U - 1) / (256 * U);
-    if (blocks > 0x7fffffff) return HQ_ERR_TOO_LARGE;
+    if (blocks >= 0x7fffffff) return HQ_ERR_TOO_LARGE;  // one more for the last elements
 #define HQ_NF4_LAUNCH(MM)                                                                                    \
-  if (mode == MM)                                                                                            \
-    hipLaunchKernelGGL((dequant4_kernel<U, MM, NT>), dim3((unsigned)blocks), dim3(256), 0, stream, pw, absmax, \
-                       (u4v*)out_fp16, nwords, blocksize, shift, table);
+  if (mode == MM && ntail)                                                                                   \
+    hipLaunchKernelGGL((dequant4_kernel<U, MM, NT, true>), dim3((unsigned)blocks + 1), dim3(256), 0, stream, \
+                       pw, absmax, (u4v*)out_fp16, nwords, blocksize, shift, table, ntail);                  \
+  else if (mode == MM)                                                                                       \
+    hipLaunchKernelGGL((dequant4_kernel<U, MM, NT, false>), dim3((unsigned)blocks), dim3(256), 0, stream, pw, \
+                       absmax, (u4v*)out_fp16, nwords, blocksize, shift, table, 0);
     // Pipelined variant, up to eight workgroups per CU, fewer for larger inputs (us per call, one-shot grid /
     // 2 / 4 / 8 workgroups per CU): 2^19 elements 5.17 / 4.11 / 4.13 / 4.11, 2^21 5.23 / 3.97 / 3.94 / 3.96,
     // 2^23 5.87 / 4.86 / 4.74 / 4.70, 2^24 (4096 x 4096) 7.78 / 7.44 / 7.10 / 7.20, 2^25 14.4 / 13.2 / 13.1 / 13.3,
@@ -219,22 +245,20 @@ extern "C" int hq_dequant_nf4(const uint8_t* packed, const float* absmax, void* 
       constexpr int PU = 4;
       const int64_t nch = (nwords + 256 * PU - 1) / (256 * PU);
       const int64_t grid = std::min<int64_t>((int64_t)dev->cus * pipe, nch);
-      hipLaunchKernelGGL((dequant4_pipelined_kernel<PU>), dim3((unsigned)grid), dim3(256), 0, stream, pw, absmax,
-                         (u4v*)out_fp16, (uint32_t)nwords, shift, table);
+      if (ntail)
+        hipLaunchKernelGGL((dequant4_pipelined_kernel<PU, true>), dim3((unsigned)grid + 1), dim3(256), 0, stream, pw, absmax,
+                           (u4v*)out_fp16, (uint32_t)nwords, shift, table, ntail);
+      else
+        hipLaunchKernelGGL((dequant4_pipelined_kernel<PU, false>), dim3((unsigned)grid), dim3(256), 0, stream, pw, absmax,
+                           (u4v*)out_fp16, (uint32_t)nwords, shift, table, 0);
     } else {
     HQ_NF4_LAUNCH(0) HQ_NF4_LAUNCH(1) HQ_NF4_LAUNCH(2)
     }
 #undef HQ_NF4_LAUNCH
-    rc = hq_launch_status();
-    if (rc != HQ_OK) return rc;
+    return hq_launch_status();
   }
-  const int64_t e_begin = nwords * 8;
-  if (e_begin < n_elems) {
-    const int64_t rest = n_elems - e_begin;
-    if ((rest + 255) / 256 > 0x7fffffff) return HQ_ERR_TOO_LARGE;
-    hipLaunchKernelGGL(dequant4_tail_kernel, dim3((unsigned)((rest + 255) / 256)), dim3(256), 0, stream,
-                       packed, absmax, (_Float16*)out_fp16, e_begin, n_elems, blocksize, table);
-    rc = hq_launch_status();
-  }
-  return rc;
+  if ((n_elems + 255) / 256 > 0x7fffffff) return HQ_ERR_TOO_LARGE;
+  hipLaunchKernelGGL(dequant4_element_kernel, dim3((unsigned)((n_elems + 255) / 256)), dim3(256), 0, stream, packed, absmax,
+                     (_Float16*)out_fp16, n_elems, blocksize, table);
+  return hq_launch_status();
 }

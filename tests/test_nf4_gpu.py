@@ -37,6 +37,18 @@ def test_both_launch_variants(hq, oracle, tunable, n, blocksize, pipe):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("pipe", [0, 2])
+@pytest.mark.parametrize("blocksize", [2, 24, 64])
+@pytest.mark.parametrize("n", [7, 9, 15, 8 * 256 * 8 + 1, 8 * 1024 * 3 - 1])
+def test_sizes_beside_whole_words(hq, oracle, tunable, n, blocksize, pipe):
+    """The elements behind the last whole word, which a workgroup of their own writes."""
+    tunable("HQ_NF4_PIPE", pipe)
+    packed, absmax = oa.make_nf4_problem(n + blocksize, n, blocksize)
+    got = _run(hq, packed, absmax, n, blocksize, 1)
+    want = oracle.dequant_4bit(packed, absmax, n, blocksize, 1).view(np.uint16)
+    assert np.array_equal(got, want)
+
+
 def test_all_codes_all_roundings(hq, oracle):
     """Every byte value against absmax values that exercise fp16 rounding,
     fp16 subnormal results and overflow to infinity."""
