@@ -397,10 +397,11 @@ __device__ __forceinline__ void row_max_min(float& a, float& b, float* lds) {
   b = wave_extreme<false>(b);
   if (LANES > 64) {  // the row spans the workgroup
     const int wv = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) { lds[wv] = a; lds[4 + wv] = b; }
+    constexpr int W = LANES / 64;
+    if ((threadIdx.x & 63) == 0) { lds[wv] = a; lds[W + wv] = b; }
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < LANES / 64; ++w) { a = fmaxf(a, lds[w]); b = fminf(b, lds[4 + w]); }
+    for (int w = 0; w < W; ++w) { a = fmaxf(a, lds[w]); b = fminf(b, lds[W + w]); }
   }
 }
 
@@ -411,14 +412,19 @@ __device__ __forceinline__ void row_max_min(float& a, float& b, float* lds) {
 // needed twice the registers for half the waves per CU and measured 18.8 us where this takes 14.0, 4096
 // rows of 5137 fp16: the hardware overlaps one row's stores with another's loads by itself when enough
 // workgroups fit a CU.)
-// VEC: both pointers are aligned and the tensor is a whole number of units, so every unit is loaded whole.
-// 64 registers for the 16-bit types, i.e. eight waves per SIMD (one more register cost bf16 rows of 16384 22.3 -> 26.2 us).
-template <typename T, bool AZP, int LANES, int KEEP, bool VEC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && LANES == 256 ? 8 : 1))) void dynamic_quant_kernel(const T* __restrict__ in, int8_t* __restrict__ out,
+// WHOLE: both pointers are aligned and the tensor is a whole number of units, so every unit is loaded whole; TAIL: aligned,
+// but the tensor's last unit is cut (it alone, in the last row, is loaded element by element); ANY: other pointers.  (With
+// ANY in the place of TAIL 1452 rows of 14519 bf16 took 35.6 us.)
+// 64 registers for the 16-bit types, i.e. eight waves per SIMD, where nothing spills for it (one more register cost bf16 rows of 16384 22.3 -> 26.2 us).
+enum RowMode { WHOLE, TAIL, ANY };
+constexpr int row_threads(int lanes) { return lanes < 256 ? 256 : lanes; }
+
+template <typename T, bool AZP, int LANES, int KEEP, RowMode MODE>
+__global__ __launch_bounds__(row_threads(LANES)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && LANES >= 256 ? (MODE == WHOLE || !AZP ? 8 : 7) : 1))) void dynamic_quant_kernel(const T* __restrict__ in, int8_t* __restrict__ out,
                                                            float* __restrict__ scales, int32_t* __restrict__ azps,
                                                            int64_t tokens, int hidden) {
-  constexpr bool aligned = VEC;
-  __shared__ float lds[8];
+  constexpr bool aligned = MODE != ANY;
+  __shared__ float lds[2 * LANES / 64];
   const int lane = threadIdx.x % LANES;
   const int64_t total = tokens * hidden;
   // uniform over the wave (LANES == 64) or the workgroup
@@ -436,7 +442,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
   const int head = (int)(g0 - u_first * kVec);  // elements of the first unit that belong to the row before
   const T* row_in = in + ubase * kVec;
   int8_t* row_out = out + ubase * kVec;
-  auto fetch = [&](int j) { return VEC ? load_unit(row_in, j) : load_unit_tail(in, ubase + j, total); };
+  // the last unit of the row that lies in the tensor whole (the tensor has one)
+  const int last = MODE == TAIL ? (int)(min(ubase + end, total / kVec) - ubase) - 1 : end - 1;
+  auto fetch = [&](int j) {
+    return MODE == WHOLE || (MODE == TAIL && j <= last) ? load_unit(row_in, j) : load_unit_tail(in, ubase + j, total);
+  };
 
   Raw<T> keep[KEEP];
 #pragma unroll
@@ -444,8 +454,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) =
     const int j = lane + k * LANES;
     // whole units are loaded without a branch, so that the loads stay one straight run the waits can
     // count; a unit outside the row repeats the row's first or last
-    if (VEC) keep[k] = load_unit(row_in, min(max(j, first), end - 1));
+    if (MODE != ANY) keep[k] = load_unit(row_in, min(max(j, first), last));
     else if (j >= first && j < end) keep[k] = fetch(j);
+  }
+  if (MODE == TAIL && last < end - 1) {  // the rows that reach it only
+#pragma unroll
+    for (int k = 0; k < KEEP; ++k)
+      if (lane + k * LANES == end - 1) keep[k] = load_unit_tail(in, ubase + end - 1, total);
   }
 
   // reference initial values: max starts at FLT_MIN (smallest positive normal), min at FLT_MAX
@@ -545,27 +560,34 @@ int launch_static(const T* in, int8_t* out, int64_t tokens, int hidden, float sc
   return hq_launch_status();
 }
 
-template <typename T, bool AZP, bool VEC>
-void launch_dynamic_vec(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
-                        const HqDevice* dev, hipStream_t stream) {
-  // short rows get a wave each, the others the workgroup; the units a thread must keep pick the kernel
+template <typename T, bool AZP, RowMode MODE>
+void launch_dynamic_mode(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
+                         const HqDevice* dev, hipStream_t stream) {
+  // Short rows get a wave each, the others a workgroup of as many threads as keep the whole row in registers with at most
+  // five units each: rows past five units of 256 threads used to be read twice (2048 rows of 16384 bf16 with zero point
+  // 21.4 -> 18.9 us; 3001 of 10241 fp32 69.6 -> 29.2; 1023 of 12289 fp16 22.6 -> 9.2, both of these also cut at the tensor's end).
+  // With no more rows than compute units the latency of one row is all there is, and more threads shorten it (5 rows of 14883
+  // bf16 9.7 -> 4.6 us).
   const bool wave_rows = hidden <= 64 * kVec * 3;
-  const int lanes = wave_rows ? 64 : 256;
   const int span = (hidden + kVec - 1) / kVec + 1 + 63;  // units from the 64-unit boundary before a ragged row to its end
-  const int need = (span + lanes - 1) / lanes;
-  const int64_t groups = wave_rows ? (tokens + 3) / 4 : tokens;
-  const dim3 grid((unsigned)groups), block(256);
-#define HQ_ROWS(LANES, KEEP)                                                                                    \
-  hipLaunchKernelGGL((dynamic_quant_kernel<T, AZP, LANES, KEEP, VEC>), grid, block, 0, stream, in, out, scales, \
-                     azps, tokens, hidden)
+#define HQ_ROWS(LANES, KEEP)                                                                                          \
+  hipLaunchKernelGGL((dynamic_quant_kernel<T, AZP, LANES, KEEP, MODE>),                                               \
+                     dim3((unsigned)(LANES == 64 ? (tokens + 3) / 4 : tokens)), dim3(row_threads(LANES)), 0, stream, in, \
+                     out, scales, azps, tokens, hidden)
   if (wave_rows) {
-    if (need <= 2) HQ_ROWS(64, 2);
-    else if (need <= 3) HQ_ROWS(64, 3);
+    if (span <= 64 * 2) HQ_ROWS(64, 2);
+    else if (span <= 64 * 3) HQ_ROWS(64, 3);
     else HQ_ROWS(64, 5);
+  } else if (tokens <= dev->cus && span > 512) {
+    if (span <= 1024) HQ_ROWS(512, 2);
+    else if (span <= 2048) HQ_ROWS(1024, 2);
+    else HQ_ROWS(1024, 5);
   } else {
-    if (need <= 2) HQ_ROWS(256, 2);
-    else if (need <= 3) HQ_ROWS(256, 3);
-    else HQ_ROWS(256, 5);
+    if (span <= 256 * 2) HQ_ROWS(256, 2);
+    else if (span <= 256 * 3) HQ_ROWS(256, 3);
+    else if (span <= 256 * 5) HQ_ROWS(256, 5);
+    else if (span <= 512 * 5) HQ_ROWS(512, 5);
+    else HQ_ROWS(1024, 5);
   }
 #undef HQ_ROWS
 }
@@ -573,10 +595,13 @@ void launch_dynamic_vec(const T* in, int8_t* out, float* scales, int32_t* azps, 
 template <typename T, bool AZP>
 void launch_dynamic_azp(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
                         const HqDevice* dev, hipStream_t stream) {
-  if (pointers_aligned(in, out) && (tokens * hidden) % kVec == 0)
-    launch_dynamic_vec<T, AZP, true>(in, out, scales, azps, tokens, hidden, dev, stream);
+  const int64_t total = tokens * hidden;
+  if (!pointers_aligned(in, out) || total < kVec)
+    launch_dynamic_mode<T, AZP, ANY>(in, out, scales, azps, tokens, hidden, dev, stream);
+  else if (total % kVec)
+    launch_dynamic_mode<T, AZP, TAIL>(in, out, scales, azps, tokens, hidden, dev, stream);
   else
-    launch_dynamic_vec<T, AZP, false>(in, out, scales, azps, tokens, hidden, dev, stream);
+    launch_dynamic_mode<T, AZP, WHOLE>(in, out, scales, azps, tokens, hidden, dev, stream);
 }
 
 template <typename T>

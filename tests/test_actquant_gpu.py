@@ -56,6 +56,21 @@ def test_ragged_rows_wave_and_group_paths(hq, oracle, dtype, tokens, hidden):
         assert np.array_equal(got.cpu().numpy(), want), with_azp
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("tokens,hidden", [(3, 3587), (3, 4099), (2, 12001), (3, 20483), (8, 8192), (1, 7), (9, 1), (65, 8),
+                                           (300, 10241), (257, 20489), (264, 24000)])
+def test_long_rows_and_a_cut_last_unit(hq, oracle, dtype, tokens, hidden):
+    """Either side of every rule that picks a row's threads: few rows and many, rows of 2 to 5 units per thread and beyond,
+    tensors whose last eight elements are not whole (in one row or shared by several)."""
+    x = _act_inputs(dtype, max(tokens, 2), hidden, tokens * 5 + hidden)[:tokens]
+    dx = _dev(x)
+    for with_azp in (False, True):
+        got, gs, gz = hq.dynamic_scaled_int8_quant(dx, with_azp)
+        want, ws, wz = oracle.int8_quant_dynamic(x, with_azp)
+        assert np.array_equal(gs.cpu().numpy(), ws) and np.array_equal(got.cpu().numpy(), want), with_azp
+        assert not with_azp or np.array_equal(gz.cpu().numpy(), wz)
+
+
 def test_fp16_subnormals_and_special_values(hq, oracle):
     """fp16 rows made of subnormal halves, of the largest halves, and rows that hold -0, infinities (static
     scale only) and isolated NaNs next to ordinary values (NaN is ignored by the reference's max / min and its quantised
