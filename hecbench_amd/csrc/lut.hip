@@ -5,9 +5,8 @@
 //
 //   y[n] = sum_k x[k] * ( q_bias[k/G][n] + sum_b alpha[k/G][b][n] * s(k,b,n) )
 //
-// Shapes with N % 64 == 0 and a group size that is a multiple of 128, 64 or 32 run on the matrix cores
-// (bcq_planes_kernel and bcq_mfma_grouped_kernel below: the packed bits themselves are the operands, no
-// tables).
+// Shapes with K % 128 == 0, N >= 64 and a group size that is a multiple of 128, 64 or 32 run on the matrix cores
+// (bcq_planes_kernel below: the packed bits themselves are the operands, no tables).
 // Every other shape runs the table kernel: for every 8-element sub-vector of x the 256
 // signed sums sum_j (+-x[j]) are tabulated once per workgroup in LDS (fp32 entries), and
 // each byte of a packed bit-plane word becomes one table lookup.  A workgroup owns a tile of columns
@@ -188,7 +187,7 @@ __global__ __launch_bounds__(256) void lut_gemv_kernel(LutArgs a) {
 
 
 // ======================================================================================
-// Matrix-core paths (group size a multiple of 128: bcq_planes_kernel; 64 or 32: bcq_mfma_grouped_kernel).
+// Matrix-core path (group size a multiple of 128, 64 or 32).
 //
 // sum_k s*x = 2*(sum_k bit*x - (sum_k x)/2).  An fp4 (e2m1) nibble with only its lowest bit set
 // is the number 0.5, so `(word >> p) & 0x11111111` (p = 0..3) turns a packed 32-bit word into
@@ -208,11 +207,6 @@ __device__ __forceinline__ v8i unpack_bits_fp4(uint32_t w) {
   const v8i a = {(int)(w & 0x11111111u), (int)((w >> 1) & 0x11111111u), (int)((w >> 2) & 0x11111111u),
                  (int)((w >> 3) & 0x11111111u), 0, 0, 0, 0};
   return a;
-}
-
-__device__ __forceinline__ f4 mfma_fp4_fp8(v8i a, v8i b, f4 c) {
-  // A fp4 e2m1 (cbsz 4), B fp8 e4m3 (blgp 0), both block scales 2^0 (E8M0 code 127)
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 4, 0, 0, 0x7f7f7f7f, 0, 0x7f7f7f7f);
 }
 
 template <int CTRL>
@@ -239,26 +233,9 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
 }
 
-struct Half16 {  // sixteen fp16 values as two 128-bit loads
-  h8 lo, hi;
-  __device__ __forceinline__ float get(int i) const { return (float)(i < 8 ? lo[i] : hi[i - 8]); }
-};
-// The same 128-bit loads for rows that start at any element (N not a multiple of 8 or 4): the types carry
+// 128-bit loads for rows that start at any element (N not a multiple of 8 or 4): the types carry
 // the element's own alignment, the hardware reads unaligned global addresses.
-typedef _Float16 h8_any __attribute__((ext_vector_type(8), aligned(2)));
 typedef uint32_t u4v_any __attribute__((ext_vector_type(4), aligned(4)));
-template <bool RAGGED>
-__device__ __forceinline__ Half16 load_half16(const _Float16* p) {
-  Half16 h;
-  if (RAGGED) {
-    h.lo = reinterpret_cast<const h8_any*>(p)[0];
-    h.hi = reinterpret_cast<const h8_any*>(p)[1];
-  } else {
-    h.lo = reinterpret_cast<const h8*>(p)[0];
-    h.hi = reinterpret_cast<const h8*>(p)[1];
-  }
-  return h;
-}
 template <bool RAGGED>
 __device__ __forceinline__ u4v load_words(const uint32_t* p) {
   if (RAGGED) return *reinterpret_cast<const u4v_any*>(p);
@@ -307,7 +284,15 @@ __device__ __forceinline__ constexpr int dig_piece(int kword, int digit, int hal
 }
 constexpr int planes_of_set(int nb, int s) { return nb - 3 * s < 3 ? nb - 3 * s : 3; }
 
-template <int NB, int QUADS, int WAVES, bool BIAS, bool RAGGED, bool ONE_ROUND>
+// ---- group sizes 64 and 32 (GROUPED) ----------------------------------------------------------------
+// A quad spans two or four groups, so no sum may reach past a k-word of 32.  The weights stream as above with P = NB (block
+// j = 4m + kb is k-word j / NB, plane j % NB); the digit rows of MFMA m are laid by block instead of by plane: row 4r + d
+// holds digit d of block 4m + r's k-word at that block's K positions, zeros elsewhere.  Result quarter kb is then block
+// 4m + kb alone, every MFMA's four digits are combined and take the alpha of their own block, and an MFMA of the same
+// digits against all-ones weights gives the k-word's sum(x).  q_bias: one such sum more, quarter kb for k-word kb.
+// Against weights as first operand with two digit operands per quad and alpha on every digit (four times the multiply-adds, no
+// split of K), K=4096, N=16384, three planes, group 64 / 32: @GROUPED@.
+template <int NB, int QUADS, int WAVES, bool BIAS, bool RAGGED, bool ONE_ROUND, bool GROUPED>
 __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
     const uint32_t* bW_, const _Float16* x_, const _Float16* alpha_, const _Float16* qbias_, int K_, int N_, int nb_,
     int G_, int kslice_, int nsplit_, int strict_, _Float16* y_, float* partial_, unsigned* counters_) {
@@ -316,7 +301,10 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
   LutArgs a;
   a.bW = bW_; a.alpha = alpha_; a.qbias = qbias_; a.x = x_; a.y = y_; a.partial = partial_; a.counters = counters_;
   a.K = K_; a.N = N_; a.nb = nb_; a.G = G_; a.kslice = kslice_; a.nsplit = nsplit_; a.strict = strict_;
-  constexpr int SETS = (NB + 2) / 3;
+  constexpr int SETS = GROUPED ? 1 : (NB + 2) / 3;
+  constexpr int MMAX = GROUPED ? NB : 3;                        // MFMAs of a set per quad and 16 columns, at most
+  constexpr int COEFS = GROUPED ? NB + (BIAS ? 1 : 0) : SETS;   // what a lane multiplies its digits with, per quad
+  auto planes = [](int s) constexpr { return GROUPED ? NB : planes_of_set(NB, s); };
   extern __shared__ float lds[];
   char* xs = reinterpret_cast<char*>(lds);                                   // [waves][QUADS][kDigQuad]
   float* red = reinterpret_cast<float*>(xs + WAVES * QUADS * kDigQuad);      // [waves][4 quarters][64]
@@ -338,19 +326,35 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
   const int st = lane >> 4, sm = lane & 15;
   const int stage_off = dig_piece(sm >> 2, 0, 0) + 2 * (sm & 3);
 
-  // what a lane multiplies its combined digits with, per set: alpha of plane 3s + kb, the bias (quarter 3
-  // of set 0) or nothing (then its sums are zero)
-  const _Float16* cbase[SETS];
-  size_t cstride[SETS];  // elements per group
+  // what a lane multiplies its combined digits with: per set alpha of plane 3s + kb, the bias (quarter 3 of set 0) or
+  // nothing (then its sums are zero); GROUPED: alpha of block 4m + kb, and the bias of k-word kb
+  const int gsub = GROUPED ? 128 / a.G : 1;  // groups per quad (1: a quad lies in one group)
+  const _Float16* cbase[COEFS];
+  size_t cstride[COEFS];  // elements per group, GROUPED: per quad
   float half_sign[SETS];
+  if (GROUPED) {
+    const int gshift = a.G == 64 ? 1 : 0;  // k-words of a group, as a power of two
 #pragma unroll
-  for (int s = 0; s < SETS; ++s) {
-    const int P = planes_of_set(NB, s);
-    const bool is_bias = BIAS && s == 0 && kb == 3;
-    const bool has_plane = kb < P;
-    cbase[s] = (is_bias ? a.qbias : a.alpha + (size_t)(3 * s + min(kb, P - 1)) * a.N) + n0 + col_off;
-    cstride[s] = is_bias ? (size_t)a.N : (size_t)NB * a.N;
-    half_sign[s] = is_bias ? 0.5f : (has_plane ? -0.5f : 0.f);
+    for (int m = 0; m < NB; ++m) {
+      const int j = 4 * m + kb;
+      cbase[m] = a.alpha + (size_t)(((j / NB) >> gshift) * NB + j % NB) * a.N + n0 + col_off;
+      cstride[m] = (size_t)gsub * NB * a.N;
+    }
+    if (BIAS) {
+      cbase[COEFS - 1] = a.qbias + (size_t)(kb >> gshift) * a.N + n0 + col_off;
+      cstride[COEFS - 1] = (size_t)gsub * a.N;
+    }
+    half_sign[0] = -0.5f;
+  } else {
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+      const int P = planes(s);
+      const bool is_bias = BIAS && s == 0 && kb == 3;
+      const bool has_plane = kb < P;
+      cbase[s] = (is_bias ? a.qbias : a.alpha + (size_t)(3 * s + min(kb, P - 1)) * a.N) + n0 + col_off;
+      cstride[s] = is_bias ? (size_t)a.N : (size_t)NB * a.N;
+      half_sign[s] = is_bias ? 0.5f : (has_plane ? -0.5f : 0.f);
+    }
   }
 
   // byte offsets of the lane's weight rows inside a quad's 4*NB rows: block j = 4m + kb of set s is k-word
@@ -358,9 +362,9 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
   uint32_t wbyte[NB];
 #pragma unroll
   for (int s = 0; s < SETS; ++s) {
-    const int P = planes_of_set(NB, s);
+    const int P = planes(s);
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
+    for (int m = 0; m < MMAX; ++m) {
       if (m >= P) continue;
       const int j = 4 * m + kb;
       wbyte[3 * s + m] = (uint32_t)(((size_t)((j / P) * NB + 3 * s + j % P) * a.N + n0 + col_off) * 4);
@@ -374,7 +378,7 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
   struct Round {
     u4v xh;  // eight fp16 activations
     u4v wq[QUADS][NB];
-    h4v cf[QUADS][SETS];
+    h4v cf[QUADS][COEFS];
   };
   auto load_x = [&](int q0, Round& r) {
     const int quad = min(q0 + min(st, QUADS - 1), nquads - 1);
@@ -385,9 +389,9 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
     const char* qb = reinterpret_cast<const char*>(a.bW + ((size_t)(4 * quad) * NB) * a.N);  // scalar
 #pragma unroll
     for (int i = 0; i < NB; ++i) r.wq[t][i] = load_words<RAGGED>(reinterpret_cast<const uint32_t*>(qb + wbyte[i]));
-    const int g = (quad * 128) / a.G;
+    const int g = GROUPED ? quad : (quad * 128) / a.G;
 #pragma unroll
-    for (int s = 0; s < SETS; ++s) {
+    for (int s = 0; s < COEFS; ++s) {
       const _Float16* cp = cbase[s] + (size_t)g * cstride[s];
       if (RAGGED) r.cf[t][s] = *reinterpret_cast<const h4v_any*>(cp);
       else r.cf[t][s] = *reinterpret_cast<const h4v*>(cp);
@@ -412,22 +416,25 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
   // Digit operand reads.  The fp8 operand of lane quarter kb holds MFMA K indices 16kb .. 16kb+15 in its
   // first 16 bytes and 64+16kb .. 64+16kb+15 in its last 16: halves h = 0, 1 lie in block 2h + (kb >> 1),
   // elements 16*(kb & 1) .. +15 of it.  Row c = 4b + d takes digit d there if the block's plane is b.
-  int doff[SETS][3][2];
+  // (GROUPED: row c = 4r + d takes digit d there if the block is the MFMA's r-th.)
+  int doff[SETS][MMAX][2];
 #pragma unroll
   for (int s = 0; s < SETS; ++s) {
-    const int P = planes_of_set(NB, s);
+    const int P = planes(s);
 #pragma unroll
-    for (int m = 0; m < 3; ++m)
+    for (int m = 0; m < MMAX; ++m)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int jj = 4 * m + 2 * h + (kb >> 1);
-        const int b = jj % P, kw = jj / P;
+        const int b = GROUPED ? jj & 3 : jj % P, kw = jj / P;
         doff[s][m][h] = (m < P && (c >> 2) == b) ? dig_piece(kw, c & 3, kb & 1) : kDigZero;
       }
   }
   // plain operand (every row r holds digit r & 3 of all four k-words): one MFMA with all-ones weights
   // gives the digit sums of the quad in every lane
-  const int poff0 = dig_piece(kb >> 1, c & 3, kb & 1), poff1 = dig_piece((kb >> 1) + 2, c & 3, kb & 1);
+  // (GROUPED: row 4r + d holds digit d of k-word r alone, so quarter kb gets the digit sums of k-word kb)
+  const int poff0 = !GROUPED || (c >> 2) == (kb >> 1) ? dig_piece(kb >> 1, c & 3, kb & 1) : kDigZero;
+  const int poff1 = !GROUPED || (c >> 2) == (kb >> 1) + 2 ? dig_piece((kb >> 1) + 2, c & 3, kb & 1) : kDigZero;
   v8i ones;
 #pragma unroll
   for (int r = 0; r < 8; ++r) ones[r] = r < 4 ? 0x11111111 : 0;
@@ -498,18 +505,39 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
         const v8i A = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
         return A;
       };
+      auto whole = [](f4 d, float plus) {  // four digits to a number
+        return fmaf(fmaf(fmaf(d[3], 16.f, d[2]), 16.f, d[1]), 16.f, d[0] + plus);
+      };
+      const f4 none = {0.f, 0.f, 0.f, 0.f};
+      if (GROUPED) {
+#pragma unroll
+        for (int m = 0; m < NB; ++m) {
+          const v8i A = operand(doff[0][m][0], doff[0][m][1]);
+          const float h0 = half_sign[0] * whole(mfma_fp8_fp4(A, ones, none), 0.f);
+          const u4v wv4 = r.wq[t][m];
+          const uint32_t words[4] = {wv4.x, wv4.y, wv4.z, wv4.w};
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            run[q] = fmaf((float)r.cf[t][m][q], whole(mfma_fp8_fp4(A, unpack_bits_fp4(words[q]), none), h0), run[q]);
+        }
+        if (BIAS) {
+          const float xh = 0.5f * whole(mfma_fp8_fp4(operand(poff0, poff1), ones, none), 0.f);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) run[q] = fmaf((float)r.cf[t][COEFS - 1][q], xh, run[q]);
+        }
+        continue;
+      }
       // digit sums of the quad (register i: digit i), in units of 2^-10, identical in all lanes
-      const f4 dsum = mfma_fp8_fp4(operand(poff0, poff1), ones, f4{0.f, 0.f, 0.f, 0.f});
-      const float xsum = fmaf(fmaf(fmaf(dsum[3], 16.f, dsum[2]), 16.f, dsum[1]), 16.f, dsum[0]);  // sum of the quad's x
+      const float xsum = whole(mfma_fp8_fp4(operand(poff0, poff1), ones, none), 0.f);  // sum of the quad's x
 #pragma unroll
       for (int s = 0; s < SETS; ++s) {
-        const int P = planes_of_set(NB, s);
+        const int P = planes(s);
         const float h0 = half_sign[s] * xsum;  // sum s*x = 2 sum bit*x - sum x; +sum x / 2 for the bias quarter
         f4 acc[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int q = 0; q < 4; ++q) acc[q] = none;
 #pragma unroll
-        for (int m = 0; m < 3; ++m) {
+        for (int m = 0; m < MMAX; ++m) {
           if (m >= P) continue;
           const v8i A = operand(doff[s][m][0], doff[s][m][1]);
           const u4v wv4 = r.wq[t][3 * s + m];
@@ -519,10 +547,7 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
         }
         // registers 0..3 are the digits of the lane's plane for weight column 4c + q
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float h = fmaf(fmaf(fmaf(acc[q][3], 16.f, acc[q][2]), 16.f, acc[q][1]), 16.f, acc[q][0] + h0);
-          run[q] = fmaf((float)r.cf[t][s][q], h, run[q]);
-        }
+        for (int q = 0; q < 4; ++q) run[q] = fmaf((float)r.cf[t][s][q], whole(acc[q], h0), run[q]);
       }
     }
     const float descale = __uint_as_float((uint32_t)(127 - E) << 23);
@@ -592,270 +617,9 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
   }
 }
 
-// ---- group sizes 64 and 32 --------------------------------------------------------------------------
-// Here the weights are the first operand (lane quarter kb streams k-word 4*quad + kb of one plane, one MFMA
-// sums a quad of one bit plane for 16 columns) and the digits the second: the activations are biased by
-// 0x8888 before they are cut into nibbles, MFMA column d carries nibble d, and a column of ones counts the
-// set bits, which takes the bias out at the very end.
-// A 128-element quad spans GS = 2 or 4 alpha / bias groups, so one sum per quad is not enough.  The
-// B operand gets a row per (group, digit): row 4g + d holds digit d at the K positions of group g and zeros
-// elsewhere (GS * 4 <= 16 MFMA columns), and a second operand holds a row of ones per group for the bit
-// counts; both are zeroed once, their constant parts written once, and only the digit bytes are rewritten
-// per round.  Every MFMA column then carries one group's sum, is scaled by that group's alpha (lane column
-// c takes the alpha of group c / 4), and the groups are added when the digits are combined at the end.
-// One B operand row is 4 lane quarters x 32 B, rows 128 B apart.  Rows 0, 2, 4 (and 1, 3) then share LDS banks
-// and the bank-conflict counter shows it; rows 144 B apart (an odd multiple of 16 B, no two rows on the same
-// banks) were built and measured slower, so the operand reads are not what bounds the kernel.
-constexpr int kLutRow = 128;
-constexpr int kGroupedQuadBytes = 20 * kLutRow;  // sixteen digit rows and up to four rows of ones
-constexpr int kGroupedRedBytes = 20 * 64 * 4;  // a wave's final sums: twenty columns of 64 outputs
-
-template <int NB, int GS, int QUADS, int WAVES, bool BIAS, bool RAGGED>
-__global__ __launch_bounds__(WAVES * 64) void bcq_mfma_grouped_kernel(
-    const uint32_t* bW_, const _Float16* x_, const _Float16* alpha_, const _Float16* qbias_, int K_, int N_, int nb_,
-    int G_, int kslice_, int nsplit_, int strict_, _Float16* y_, float* partial_, unsigned* counters_) {
-  // leading scalars, not the struct: the first 14 dwords of the arguments (all that the loads need) arrive
-  // preloaded in scalar registers
-  LutArgs a;
-  a.bW = bW_; a.alpha = alpha_; a.qbias = qbias_; a.x = x_; a.y = y_; a.partial = partial_; a.counters = counters_;
-  a.K = K_; a.N = N_; a.nb = nb_; a.G = G_; a.kslice = kslice_; a.nsplit = nsplit_; a.strict = strict_;
-  constexpr int kWaveBytes = QUADS * kGroupedQuadBytes > kGroupedRedBytes ? QUADS * kGroupedQuadBytes : kGroupedRedBytes;
-  extern __shared__ float lds[];
-  char* xs = reinterpret_cast<char*>(lds);  // [waves][kWaveBytes]: operands in the loop, the final sums after it
-  float* poison_w = reinterpret_cast<float*>(xs + WAVES * kWaveBytes);  // [waves]
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int c = lane & 15, kb = lane >> 4;
-  const int tile = blockIdx.x;
-  const int nquads = a.K >> 7;
-  const size_t n0 = RAGGED ? (size_t)min(tile * 64, a.N - 64) : (size_t)tile * 64;
-  const uint32_t col_off = 4u * c;
-  const uint32_t acol = 16u * kb;
-  const int cg = min(c >> 2, GS - 1);  // the group whose sums this lane's MFMA column carries
-  char* xs_w = xs + wv * kWaveBytes;
-  // staging role of a lane, as in bcq_mfma_kernel; its four activations lie in group sg of the quad
-  const int st = lane >> 5, sa = (lane >> 3) & 3, sp = (lane >> 1) & 3, sh = lane & 1;
-  const int e0 = 8 * sp + 4 * sh;
-  const int s_quarter = 2 * (sa & 1) + (e0 >> 4), s_byte = 16 * (sa >> 1) + (e0 & 15);
-  const int sg = (sa * GS) >> 2;
-  constexpr int SP = (QUADS + 1) / 2;
-
-  v8i ones;
-#pragma unroll
-  for (int r = 0; r < 8; ++r) ones[r] = r < 4 ? 0x11111111 : 0;
-  // zero both operands of every quad, then the rows of ones: dword w of a row sits in lane quarter w / 8
-  // at bytes 4 (w % 8), which are MFMA K indices 64 (byte / 16) + 16 quarter + byte % 16
-  {
-    const u4v zero = {0u, 0u, 0u, 0u};
-    for (int i = lane; i < QUADS * kGroupedQuadBytes / 16; i += 64) reinterpret_cast<u4v*>(xs_w)[i] = zero;
-    if (lane < 32) {
-      const int k0 = 64 * ((lane & 7) >> 2) + 16 * (lane >> 3);
-      const int grp = (k0 * GS) >> 7;
-#pragma unroll
-      for (int t = 0; t < QUADS; ++t)
-        *reinterpret_cast<uint32_t*>(xs_w + t * kGroupedQuadBytes + (16 + grp) * kLutRow + lane * 4) = 0x01010101u;
-    }
-  }
-
-  float tot[4][4], totp[4][4];  // digit columns and bit counts, alpha applied
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) tot[q][i] = totp[q][i] = 0.f;
-  float poison = 0.f;
-
-  for (int q0 = wv * QUADS; q0 < nquads; q0 += WAVES * QUADS) {
-    float xv[SP][4];
-    u4v wq[QUADS][NB];
-#pragma unroll
-    for (int sp_ = 0; sp_ < SP; ++sp_) {
-      const int quad = min(q0 + min(2 * sp_ + st, QUADS - 1), nquads - 1);
-      const _Float16* xp = a.x + (size_t)quad * 128 + 32 * sa + 16 * sh + sp;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xv[sp_][j] = (float)xp[4 * j];
-    }
-    // The activations and the first quad's loads go out here, every further quad's just before the
-    // arithmetic of the quad ahead of it (see bcq_planes_kernel: a wave stalls at a load while the compute
-    // unit's queue of outstanding loads is full, and with a round's loads issued at once the later waves
-    // get their data, and do their arithmetic, after the stream has ended).
-    Half16 al[QUADS][NB], bi[QUADS];
-    auto load_quad = [&](int t) {
-      const int quad = min(q0 + t, nquads - 1);
-      const uint32_t* wp = a.bW + ((size_t)(4 * quad + kb) * NB) * a.N + n0 + col_off;
-#pragma unroll
-      for (int b = 0; b < NB; ++b) wq[t][b] = load_words<RAGGED>(wp + (size_t)b * a.N);
-      const int g = quad * GS + cg;
-#pragma unroll
-      for (int b = 0; b < NB; ++b) al[t][b] = load_half16<RAGGED>(a.alpha + ((size_t)g * NB + b) * a.N + n0 + acol);
-      if (BIAS) bi[t] = load_half16<RAGGED>(a.qbias + (size_t)g * a.N + n0 + acol);
-    };
-    load_quad(0);
-    __builtin_amdgcn_sched_barrier(0);
-    float amax = 0.f;
-#pragma unroll
-    for (int sp_ = 0; sp_ < SP; ++sp_) {
-      const int t = 2 * sp_ + st;
-      const bool live = t < QUADS && q0 + t < nquads;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (!live) xv[sp_][j] = 0.f;
-        poison = fmaf(xv[sp_][j], 0.f, poison);
-        amax = fmaxf(amax, fabsf(xv[sp_][j]));
-      }
-    }
-    const float xmax = wave_max(amax);
-    int E = 13 - ((int)((__float_as_uint(xmax) >> 23) & 255u) - 127);
-    E = xmax > 0.f ? max(-120, min(120, E)) : 0;
-    const float scaleE = __uint_as_float((uint32_t)(E + 127) << 23);
-#pragma unroll
-    for (int sp_ = 0; sp_ < SP; ++sp_) {
-      uint32_t ev[4], od[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t u = (uint32_t)((int)rintf(xv[sp_][j] * scaleE) + 0x8888);
-        ev[j] = u & 0x0f0fu;
-        od[j] = (u >> 4) & 0x0f0fu;
-      }
-      const uint32_t pe = __builtin_amdgcn_perm(ev[1], ev[0], 0x05010400u);
-      const uint32_t qe = __builtin_amdgcn_perm(ev[3], ev[2], 0x05010400u);
-      const uint32_t po = __builtin_amdgcn_perm(od[1], od[0], 0x05010400u);
-      const uint32_t qo = __builtin_amdgcn_perm(od[3], od[2], 0x05010400u);
-      const uint32_t dg[4] = {__builtin_amdgcn_perm(qe, pe, 0x05040100u), __builtin_amdgcn_perm(qo, po, 0x05040100u),
-                              __builtin_amdgcn_perm(qe, pe, 0x07060302u), __builtin_amdgcn_perm(qo, po, 0x07060302u)};
-      const int t = 2 * sp_ + st;
-      if (t < QUADS) {
-        char* dst = xs_w + t * kGroupedQuadBytes + (4 * sg) * kLutRow + s_quarter * 32 + s_byte;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) *reinterpret_cast<uint32_t*>(dst + d * kLutRow) = dg[d];
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    float run[4][4], runp[4][4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) run[q][i] = runp[q][i] = 0.f;
-#pragma unroll
-    for (int t = 0; t < QUADS; ++t) {
-      if (q0 + t >= nquads) break;  // wave-uniform
-      if (t + 1 < QUADS) {
-        load_quad(t + 1);
-        __builtin_amdgcn_sched_barrier(0);  // issued here, not where the compiler would like it
-      }
-      // digit rows: MFMA column c reads row c (rows past 4 GS stay zero and are never used);
-      // rows of ones: column c reads its group's
-      const u4v* bp = reinterpret_cast<const u4v*>(xs_w + t * kGroupedQuadBytes + c * kLutRow + kb * 32);
-      const u4v* pp = reinterpret_cast<const u4v*>(xs_w + t * kGroupedQuadBytes + (16 + cg) * kLutRow + kb * 32);
-      const u4v b0 = bp[0], b1 = bp[1], p0 = pp[0], p1 = pp[1];
-      const v8i B = {(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
-      const v8i P = {(int)p0.x, (int)p0.y, (int)p0.z, (int)p0.w, (int)p1.x, (int)p1.y, (int)p1.z, (int)p1.w};
-      const f4 dsum = mfma_fp4_fp8(ones, B, f4{0.f, 0.f, 0.f, 0.f});
-      const f4 psum = mfma_fp4_fp8(ones, P, f4{0.f, 0.f, 0.f, 0.f});
-      const f4 init = {-0.5f * dsum[0], -0.5f * dsum[1], -0.5f * dsum[2], -0.5f * dsum[3]};
-      const f4 initp = {-0.5f * psum[0], -0.5f * psum[1], -0.5f * psum[2], -0.5f * psum[3]};
-      if (BIAS) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            run[q][i] = fmaf(bi[t].get(4 * i + q), 0.5f * dsum[i], run[q][i]);
-            runp[q][i] = fmaf(bi[t].get(4 * i + q), 0.5f * psum[i], runp[q][i]);
-          }
-      }
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const uint32_t words[4] = {wq[t][b].x, wq[t][b].y, wq[t][b].z, wq[t][b].w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const v8i A = unpack_bits_fp4(words[q]);
-          const f4 acc = mfma_fp4_fp8(A, B, init);
-          const f4 accp = mfma_fp4_fp8(A, P, initp);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float al_n = al[t][b].get(4 * i + q);
-            run[q][i] = fmaf(al_n, acc[i], run[q][i]);
-            runp[q][i] = fmaf(al_n, accp[i], runp[q][i]);
-          }
-        }
-      }
-    }
-    const float descale = __uint_as_float((uint32_t)(127 - E) << 23);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        tot[q][i] = fmaf(run[q][i], descale, tot[q][i]);
-        totp[q][i] = fmaf(runp[q][i], descale, totp[q][i]);
-      }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-  }
-  // ---- combine digits, groups and waves: the wave's operand area now takes its sums -----------------
-  {
-    const float wp = wave_sum(poison);
-    if (lane == 0) poison_w[wv] = wp;
-  }
-  float* red_w = reinterpret_cast<float*>(xs_w);  // [20][64]: rows 4g + d digits, rows 16 + g bit counts
-  if (c < 4 * GS) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red_w[c * 64 + 16 * kb + 4 * i + q] = tot[q][i];
-  }
-  if (c < 4 * GS && (c & 3) == 0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red_w[(16 + (c >> 2)) * 64 + 16 * kb + 4 * i + q] = totp[q][i];
-  }
-  __syncthreads();
-  const int n = (int)n0 + tid;
-  if (tid < 64 && n < a.N) {
-    float v = 0.f;
-    for (int w = 0; w < WAVES; ++w) {
-      const float* rw = reinterpret_cast<const float*>(xs + w * kWaveBytes) + tid;
-#pragma unroll
-      for (int g = 0; g < GS; ++g) {
-        const float* rg = rw + 4 * g * 64;
-        v += (((rg[192] * 16.f + rg[128]) * 16.f + rg[64]) * 16.f + rg[0]) - 34952.f * rw[(16 + g) * 64];
-      }
-      v += poison_w[w];
-    }
-    a.y[n] = (_Float16)(v * 2048.f);
-  }
-}
-
-template <int NB, int GS, int QUADS>
-int launch_bcq_grouped(const LutArgs& a, bool ragged, hipStream_t stream) {
-  constexpr int WAVES = 8;
-  constexpr int kWaveBytes = QUADS * kGroupedQuadBytes > kGroupedRedBytes ? QUADS * kGroupedQuadBytes : kGroupedRedBytes;
-  const size_t smem = (size_t)WAVES * kWaveBytes + (size_t)WAVES * 4;
-  const dim3 grid((a.N + 63) / 64), block(WAVES * 64);
-#define HQ_LUT_GO(BIAS, RAG) \
-  hipLaunchKernelGGL((bcq_mfma_grouped_kernel<NB, GS, QUADS, WAVES, BIAS, RAG>), grid, block, smem, stream, a.bW, a.x, a.alpha, a.qbias, a.K, a.N, a.nb, a.G, a.kslice, a.nsplit, a.strict, a.y, a.partial, a.counters)
-  if (a.qbias) { if (ragged) HQ_LUT_GO(true, true); else HQ_LUT_GO(true, false); }
-  else { if (ragged) HQ_LUT_GO(false, true); else HQ_LUT_GO(false, false); }
-#undef HQ_LUT_GO
-  return hq_launch_status();
-}
-template <int GS>
-int launch_bcq_grouped_nb(const LutArgs& a, bool ragged, hipStream_t stream) {
-  switch (a.nb) {  // quads per wave per round, bounded by the register budget
-    case 1: return launch_bcq_grouped<1, GS, 2>(a, ragged, stream);
-    case 2: return launch_bcq_grouped<2, GS, 2>(a, ragged, stream);
-    case 3: return launch_bcq_grouped<3, GS, 2>(a, ragged, stream);
-    case 4: return launch_bcq_grouped<4, GS, 2>(a, ragged, stream);
-    case 5: return launch_bcq_grouped<5, GS, 1>(a, ragged, stream);
-    case 6: return launch_bcq_grouped<6, GS, 1>(a, ragged, stream);
-    case 7: return launch_bcq_grouped<7, GS, 1>(a, ragged, stream);
-    default: return launch_bcq_grouped<8, GS, 1>(a, ragged, stream);
-  }
-}
-
 // Eight waves per workgroup (two per SIMD, up to 256 VGPRs each); QUADS is bounded by the two register
 // sets of a round's loads.
-template <int NB, int QUADS>
+template <int NB, int QUADS, bool GROUPED>
 int launch_bcq_planes(LutArgs a, bool ragged, int cus, hipStream_t stream) {
   constexpr int WAVES = 8;
   // K split: with fewer column tiles than compute units, whole rounds (128 QUADS WAVES elements of K) go to
@@ -884,15 +648,29 @@ int launch_bcq_planes(LutArgs a, bool ragged, int cus, hipStream_t stream) {
   const bool one_round = rpw == 1;
 #define HQ_LUT_GO(BIAS, RAG)                                                                                        \
   do {                                                                                                              \
-    if (one_round) hipLaunchKernelGGL((bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, true>), grid, block, smem, stream, \
+    if (one_round) hipLaunchKernelGGL((bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, true, GROUPED>), grid, block, smem, stream, \
                                        a.bW, a.x, a.alpha, a.qbias, a.K, a.N, a.nb, a.G, a.kslice, a.nsplit, a.strict, a.y, a.partial, a.counters); \
-    else hipLaunchKernelGGL((bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, false>), grid, block, smem, stream, \
+    else hipLaunchKernelGGL((bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, false, GROUPED>), grid, block, smem, stream, \
                             a.bW, a.x, a.alpha, a.qbias, a.K, a.N, a.nb, a.G, a.kslice, a.nsplit, a.strict, a.y, a.partial, a.counters); \
   } while (0)
   if (a.qbias) { if (ragged) HQ_LUT_GO(true, true); else HQ_LUT_GO(true, false); }
   else { if (ragged) HQ_LUT_GO(false, true); else HQ_LUT_GO(false, false); }
 #undef HQ_LUT_GO
   return hq_launch_status();
+}
+
+template <bool GROUPED>
+int launch_bcq_planes_nb(const LutArgs& a, bool ragged, int cus, hipStream_t stream) {
+  switch (a.nb) {  // quads per wave per round, bounded by the register budget
+    case 1: return launch_bcq_planes<1, 4, GROUPED>(a, ragged, cus, stream);
+    case 2: return launch_bcq_planes<2, 4, GROUPED>(a, ragged, cus, stream);
+    case 3: return launch_bcq_planes<3, 4, GROUPED>(a, ragged, cus, stream);
+    case 4: return launch_bcq_planes<4, 2, GROUPED>(a, ragged, cus, stream);
+    case 5: return launch_bcq_planes<5, 2, GROUPED>(a, ragged, cus, stream);
+    case 6: return launch_bcq_planes<6, 2, GROUPED>(a, ragged, cus, stream);
+    case 7: return launch_bcq_planes<7, 1, GROUPED>(a, ragged, cus, stream);
+    default: return launch_bcq_planes<8, 1, GROUPED>(a, ragged, cus, stream);
+  }
 }
 
 // Which kernel a call takes (HQ_LUT_PLAN_* in hq.h).
@@ -929,18 +707,8 @@ extern "C" int hq_lut_gemv(const uint32_t* bW, const void* alpha, const void* q_
     a.bW = bW; a.alpha = (const _Float16*)alpha; a.qbias = (const _Float16*)q_bias;
     a.x = (const _Float16*)x; a.y = (_Float16*)y; a.partial = nullptr; a.counters = nullptr;
     a.K = K; a.N = N; a.nb = nbits; a.G = group_size; a.kslice = K; a.nsplit = 1; a.strict = 0;
-    if ((plan & ~HQ_LUT_PLAN_RAGGED) == HQ_LUT_PLAN_MFMA_GROUPED)
-      return group_size == 64 ? launch_bcq_grouped_nb<2>(a, ragged, stream) : launch_bcq_grouped_nb<4>(a, ragged, stream);
-    switch (nbits) {  // quads per wave per round, bounded by the register budget
-      case 1: return launch_bcq_planes<1, 4>(a, ragged, dev->cus, stream);
-      case 2: return launch_bcq_planes<2, 4>(a, ragged, dev->cus, stream);
-      case 3: return launch_bcq_planes<3, 4>(a, ragged, dev->cus, stream);
-      case 4: return launch_bcq_planes<4, 2>(a, ragged, dev->cus, stream);
-      case 5: return launch_bcq_planes<5, 2>(a, ragged, dev->cus, stream);
-      case 6: return launch_bcq_planes<6, 2>(a, ragged, dev->cus, stream);
-      case 7: return launch_bcq_planes<7, 1>(a, ragged, dev->cus, stream);
-      default: return launch_bcq_planes<8, 1>(a, ragged, dev->cus, stream);
-    }
+    return (plan & ~HQ_LUT_PLAN_RAGGED) == HQ_LUT_PLAN_MFMA_GROUPED ? launch_bcq_planes_nb<true>(a, ragged, dev->cus, stream)
+                                                                    : launch_bcq_planes_nb<false>(a, ragged, dev->cus, stream);
   }
   const bool pair = (N % 2 == 0) && !((uintptr_t)bW & 7);
   const int cpl = pair ? 2 : 1;
