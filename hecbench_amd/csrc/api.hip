@@ -123,6 +123,18 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
   return HQ_OK;
 }
 
+bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    auto it = g_workspaces.find(std::make_pair(dev, stream));
+    if (it != g_workspaces.end() && it->second.partial_floats >= need_floats && it->second.ncounters >= need_counters) return false;
+  }
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
+}
+
 // Upper bound of what any hq_q3_matvec call with K <= max_K, N <= max_N (any batch) and any hq_lut_gemv call
 // of those sizes takes from its stream's workspace on a device of `cus` compute units, with the default launch
 // policy.  Host arithmetic only.  (tests/test_workspace_cpu.py checks it against the per-call need over a

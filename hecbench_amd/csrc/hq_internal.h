@@ -42,13 +42,16 @@ struct HqWorkspace {
 // Allocated on first use, grown geometrically on demand, freed by hq_shutdown().
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
                      HqWorkspace* out);
+// Whether that would allocate while the stream is being captured, where an allocation is an error: a plan that can do
+// without a workspace then does.
+bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters);
 
 // Caller-provided scratch of the GPTQ 3-bit paths (the entry point that allocates nothing passes its
 // fixed device array here; a null pointer means "use the stream's workspace").
 struct HqQ3Scratch {
   float* partial;          // split-K partial sums, also the batched GEMM's re-ordered activations
   size_t partial_floats;
-  float* rows;             // 128 floats: row sums and row scales of the batched GEMM
+  float* rows;             // 256 floats: row sums and row scales of the batched GEMM
   unsigned* counters;      // split-K arrival counters (cleared by the call that uses them)
   size_t ncounters;
   float* sums;             // raw sums of the batched GEMM's K split
@@ -60,11 +63,11 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
 // Batched 3-bit GEMM: the pre-pass (activations [M][K] -> operand-slot order of Mpad rows and Gpad k-groups, row sums and
 // 1 / row scale), and the tiled kernels for many rows.
 int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad, hipStream_t stream);
-bool hq_q3_tiles_serve(int N, int M);
+bool hq_q3_tiles_serve(int cus, int K, int N, int M, bool fixed);
 int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
 void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);
 int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
-                       int M, unsigned flags, hipStream_t stream);
+                       int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
 // Resolves the current device's copy of the fixed scratch array (once per device).
 int hq_noalloc_setup(void);
 

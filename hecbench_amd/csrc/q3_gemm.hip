@@ -376,7 +376,7 @@ int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv
 }
 
 int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
-  if (hq_q3_tiles_serve(N, M)) return hq_q3_tiles_need(cus, K, N, M, floats, counters);
+  if (hq_q3_tiles_serve(cus, K, N, M, false)) return hq_q3_tiles_need(cus, K, N, M, floats, counters);
   const GemmPlan p = gemm_plan(cus, K, N);
   *floats = p.ap_halves / 2 + 128 + p.partial_floats;
   *counters = 1;
@@ -387,10 +387,11 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
                       int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
   if (((uintptr_t)x & 15) || (K & 7)) return HQ_ERR_MISALIGNED;
   if (((uintptr_t)scales & 15) || ((uintptr_t)zeros & 15) || ((uintptr_t)y & 15)) return HQ_ERR_MISALIGNED;
-  if (!fixed && hq_q3_tiles_serve(N, M)) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream);
   const HqDevice* dev = nullptr;
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
+  if (hq_q3_tiles_serve(dev->cus, K, N, M, fixed != nullptr))
+    return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   const GemmPlan plan = gemm_plan(dev->cus, K, N);
   const int Gpad = plan.Gpad, nsplit = plan.nsplit, spp = plan.spp;
   const size_t ap_halves = plan.ap_halves, partial_floats = plan.partial_floats;
@@ -441,7 +442,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
 // workspace.  Every GPU holds its own copy of the array at its own address, resolved once per device.
 namespace {
 constexpr size_t kScratchPartialBytes = (size_t)2 << 20;  // 2 MiB: K <= 16384 batched, 8192 partial rows of 64 floats
-constexpr size_t kScratchRowBytes = 1024;                 // 128 floats used
+constexpr size_t kScratchRowBytes = 1024;                 // 256 floats
 constexpr size_t kScratchCounterBytes = 64 * 1024 - kScratchRowBytes;
 constexpr size_t kScratchSumBytes = (size_t)kMaxSplitGroups * 64 * kTileN * sizeof(float);  // 8 MiB: the GEMM's K split
 constexpr size_t kScratchBytes = kScratchPartialBytes + kScratchRowBytes + kScratchCounterBytes + kScratchSumBytes;

@@ -148,8 +148,8 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  *     workgroup unless N / 128 is at least 7/8 of the compute units or K is longer than that;
  *     every activation enters with an error of at most 2^-19 of the largest magnitude
  *     among its 32 neighbours (exactly, if within 2^8 of it);
- *   - everything else: the MFMA GEMM path (64 rows per pass over the weights; more than 96 rows, or more than 64 with
- *     N > 4096: tiles of 64 or 128 rows, thousands of rows per pass), which pre-scales every activation row by a
+ *   - everything else: the MFMA GEMM path (64 rows per pass over the weights; more than 96 rows, or more than 64 unless
+ *     N <= 4096 and K * N >= 2^25: tiles of 64 or 128 rows, thousands of rows per pass), which pre-scales every activation row by a
  *     power of two, so accuracy does not depend on the magnitude of the activations:
  *     entries within 2^21 of their row's largest magnitude enter the matrix cores
  *     exactly, smaller ones lose low bits (those 2^32 below it vanish).
