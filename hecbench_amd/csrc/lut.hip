@@ -291,7 +291,7 @@ constexpr int planes_of_set(int nb, int s) { return nb - 3 * s < 3 ? nb - 3 * s 
 // 4m + kb alone, every MFMA's four digits are combined and take the alpha of their own block, and an MFMA of the same
 // digits against all-ones weights gives the k-word's sum(x).  q_bias: one such sum more, quarter kb for k-word kb.
 // Against weights as first operand with two digit operands per quad and alpha on every digit (four times the multiply-adds, no
-// split of K), K=4096, N=16384, three planes, group 64 / 32: @GROUPED@.
+// split of K), K=4096, N=16384, three planes, group 64 / 32: 11.4 / 12.6 -> 8.2 / 9.6 us.
 template <int NB, int QUADS, int WAVES, bool BIAS, bool RAGGED, bool ONE_ROUND, bool GROUPED>
 __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
     const uint32_t* bW_, const _Float16* x_, const _Float16* alpha_, const _Float16* qbias_, int K_, int N_, int nb_,
@@ -620,17 +620,10 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
 // Eight waves per workgroup (two per SIMD, up to 256 VGPRs each); QUADS is bounded by the two register
 // sets of a round's loads.
 template <int NB, int QUADS, bool GROUPED>
-int launch_bcq_planes(LutArgs a, bool ragged, int cus, hipStream_t stream) {
+int launch_bcq_planes(LutArgs a, bool ragged, int nsplit, hipStream_t stream) {
   constexpr int WAVES = 8;
-  // K split: with fewer column tiles than compute units, whole rounds (128 QUADS WAVES elements of K) go to
-  // workgroups of their own, as many as there are compute units to take them (K=11008, N=4096, three planes:
-  // 64 tiles x 3 rounds)
   const int ntiles = (a.N + 63) / 64;
-  const int nquads = a.K >> 7;
-  const int rounds = (nquads + WAVES * QUADS - 1) / (WAVES * QUADS);
-  int nsplit = cus / ntiles;
-  if (nsplit > rounds) nsplit = rounds;
-  if (nsplit < 1) nsplit = 1;
+  const int rounds = ((a.K >> 7) + WAVES * QUADS - 1) / (WAVES * QUADS);
   const int rpw = (rounds + nsplit - 1) / nsplit;
   nsplit = (rounds + rpw - 1) / rpw;
   a.kslice = rpw * WAVES * QUADS * 128;
@@ -659,17 +652,49 @@ int launch_bcq_planes(LutArgs a, bool ragged, int cus, hipStream_t stream) {
   return hq_launch_status();
 }
 
+// Split of K over workgroups.  Ordinary: rounds of QUADS quads (128 elements of K) per wave, and as many workgroups as there
+// are compute units to take them (K=11008, N=4096, three planes: 64 tiles x 3 rounds).  Fine: one quad per wave, one round per
+// workgroup, all rounds side by side.  From measurements of both over thirty shapes (MI355X): a quad takes a wave 0.11 us per
+// plane (0.23 with groups of 64 or 32), the exchange of a split 1.4 us and 0.16 more for every part.  Fine splits are taken
+// where they save more than they cost and all workgroups are on the device at once, two per compute unit (us, ordinary / fine:
+// 4224 x 5562 four planes 9.1 / 7.9; 4352 x 622 two planes 5.9 / 4.9; 7552 x 2166 group 64 8.5 / 7.3; 1024 x 1024 group 32 5.8 /
+// 4.6; not 11008 x 4096 7.9 / 8.7, 13184 x 1025 7.2 / 7.7, 4096 x 4096 5.7 / 6.1), and where several rounds of few more tiles than
+// compute units would leave most of those idle behind the first tile (2432 x 20485 four planes group 32 18.7 / 13.7; 5120 x 20480
+// 14.2 / 13.0; not 4096 x 28672 four planes 15.6 / 16.6).
+template <int NB, bool GROUPED>
+int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t stream) {
+  constexpr int QUADS = NB <= 3 ? 4 : (NB <= 6 ? 2 : 1);  // bounded by the register budget
+  const int ntiles = (a.N + 63) / 64, nquads = a.K >> 7;
+  auto rounds_of = [&](int quads) { return (nquads + 8 * quads - 1) / (8 * quads); };
+  const int rounds = rounds_of(QUADS), parts = rounds_of(1);
+  int nsplit = cus / ntiles;
+  nsplit = nsplit < 1 ? 1 : (nsplit > rounds ? rounds : nsplit);
+  const int rpw = (rounds + nsplit - 1) / nsplit;
+  bool fine = false;
+  if (QUADS > 1) {
+    const float saves = (GROUPED ? 0.23f : 0.11f) * NB * (rpw * QUADS - 1);
+    const float costs = parts == 1 ? 0.f : (nsplit == 1 ? 1.4f : 0.f) + 0.16f * (parts - nsplit);
+    fine = (int64_t)ntiles * parts <= 2 * cus && saves > costs;
+    if (ntiles > cus && ntiles * 8 <= cus * 11 && rpw > 1 && parts <= 5) fine = true;
+    const int force = hq_tune(HQ_TUNE_LUT_KSPLIT, 0);  // tests: 1 ordinary, 2 fine
+    if (force > 0) fine = force == 2;
+  }
+  if (fine) nsplit = parts;
+  if (nsplit > 1 && hq_workspace_out_of_reach(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles)) nsplit = 1;
+  return fine ? launch_bcq_planes<NB, 1, GROUPED>(a, ragged, nsplit, stream)
+              : launch_bcq_planes<NB, QUADS, GROUPED>(a, ragged, nsplit, stream);
+}
 template <bool GROUPED>
 int launch_bcq_planes_nb(const LutArgs& a, bool ragged, int cus, hipStream_t stream) {
-  switch (a.nb) {  // quads per wave per round, bounded by the register budget
-    case 1: return launch_bcq_planes<1, 4, GROUPED>(a, ragged, cus, stream);
-    case 2: return launch_bcq_planes<2, 4, GROUPED>(a, ragged, cus, stream);
-    case 3: return launch_bcq_planes<3, 4, GROUPED>(a, ragged, cus, stream);
-    case 4: return launch_bcq_planes<4, 2, GROUPED>(a, ragged, cus, stream);
-    case 5: return launch_bcq_planes<5, 2, GROUPED>(a, ragged, cus, stream);
-    case 6: return launch_bcq_planes<6, 2, GROUPED>(a, ragged, cus, stream);
-    case 7: return launch_bcq_planes<7, 1, GROUPED>(a, ragged, cus, stream);
-    default: return launch_bcq_planes<8, 1, GROUPED>(a, ragged, cus, stream);
+  switch (a.nb) {
+    case 1: return launch_bcq_planes_of<1, GROUPED>(a, ragged, cus, stream);
+    case 2: return launch_bcq_planes_of<2, GROUPED>(a, ragged, cus, stream);
+    case 3: return launch_bcq_planes_of<3, GROUPED>(a, ragged, cus, stream);
+    case 4: return launch_bcq_planes_of<4, GROUPED>(a, ragged, cus, stream);
+    case 5: return launch_bcq_planes_of<5, GROUPED>(a, ragged, cus, stream);
+    case 6: return launch_bcq_planes_of<6, GROUPED>(a, ragged, cus, stream);
+    case 7: return launch_bcq_planes_of<7, GROUPED>(a, ragged, cus, stream);
+    default: return launch_bcq_planes_of<8, GROUPED>(a, ragged, cus, stream);
   }
 }
 

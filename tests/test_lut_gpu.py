@@ -63,6 +63,41 @@ def test_k_split_of_the_plane_kernel(hq, oracle, tunable, K, N, nb):
     assert np.array_equal(y, _run(hq, bW, alpha, qbias, x, 128))
 
 
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("K,N,nb,group", [(128, 64, 1, 32), (1024, 100, 3, 64), (1152, 130, 3, 32), (2304, 200, 4, 64),
+                                          (3200, 64, 6, 32), (4224, 321, 2, 128), (8192, 65, 5, 64), (1280, 192, 8, 64)])
+def test_ordinary_and_fine_splits(hq, oracle, tunable, split, K, N, nb, group):
+    """One quad per wave with a workgroup per round, and several quads per wave: every plane count's kind, either group size,
+    K of less than a round, of one and of several with a rest."""
+    tunable("HQ_LUT_KSPLIT", split)
+    bW, alpha, qbias, x = oa.make_lut_problem(K + N + nb, K, N, nb, group, False)
+    y = _run(hq, bW, alpha, qbias, x, group)
+    ref = oracle.lut_gemv_f64(bW, alpha, qbias, x, group)
+    assert rel_err(y, ref, FLOOR_F16) <= 2e-3
+    assert np.array_equal(y, _run(hq, bW, alpha, qbias, x, group))
+    assert rel_err(_run(hq, bW, alpha, None, x, group), oracle.lut_gemv_f64(bW, alpha, None, x, group), FLOOR_F16) <= 2e-3
+
+
+def test_capture_without_a_workspace(hq, oracle):
+    """A split of K needs the stream's workspace; under capture, where none can be allocated, the call runs unsplit."""
+    import torch
+    K, N, nb, group = 8192, 128, 3, 64
+    bW, alpha, qbias, x = oa.make_lut_problem(5, K, N, nb, group, False)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    args = [t(x), t(bW.view(np.int32)), t(alpha), t(qbias)]
+    out = torch.zeros(N, dtype=torch.float16, device="cuda:0")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        hq.lut_matmul(*args, group, out=out)
+    ref = oracle.lut_gemv_f64(bW, alpha, qbias, x, group)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_err(out.cpu().numpy(), ref, FLOOR_F16) <= 2e-3
+
+
 def test_plans(hq):
     """Which kernel a shape takes, asked of the library itself: ragged shapes stay on the matrix cores."""
     from hecbench_amd import _lib
