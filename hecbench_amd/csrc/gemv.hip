@@ -12,7 +12,7 @@
 // zp sum v ), which leaves a sign-extending conversion and one fused multiply-add per int8 weight and
 // 9 instructions per 8 int4 weights.
 //
-// A wave owns R consecutive rows and walks the columns in steps of 64 lanes x 16 bytes of
+// In the general kernel a wave owns R consecutive rows and walks the columns in steps of 64 lanes x 16 bytes of
 // matrix per row (1 KB contiguous per wave and row); the matching piece of the vector is
 // loaded once and used for the R rows.  A 4-bit code left in place in the low bits of
 // a 16-bit half is the fp16 subnormal code * 2^-24, so `word >> 4i & 0x000f000f` is a pair
@@ -248,6 +248,81 @@ __global__ __launch_bounds__(SPLIT * 64) void gemv_split_kernel(const char* mat_
   }
 }
 
+// Lanes' sums of R rows at once: half-wave swaps and row swaps turn R values per lane into R / 4, each summed over the four
+// rows of sixteen lanes, which the data path's own lane exchanges finish: R = 8 takes 20 instructions (one row after the other
+// 88).  Value i of lane group g (sixteen lanes) is the sum of row i + R / 4 * g, in all lanes of the group.
+__device__ __forceinline__ float swap_add_32(float a, float b) {  // low half: a over both halves, high half: b
+  const auto p = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  return __builtin_bit_cast(float, (uint32_t)p[0]) + __builtin_bit_cast(float, (uint32_t)p[1]);
+}
+__device__ __forceinline__ float swap_add_16(float a, float b) {  // even rows of 16: a over the pair of rows, odd rows: b
+  const auto p = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  return __builtin_bit_cast(float, (uint32_t)p[0]) + __builtin_bit_cast(float, (uint32_t)p[1]);
+}
+template <int R>
+__device__ __forceinline__ void row_sums(const float (&s)[R], float (&w)[R / 4]) {
+#pragma unroll
+  for (int i = 0; i < R / 4; ++i) {
+    float v = swap_add_16(swap_add_32(s[i], s[i + R / 2]), swap_add_32(s[i + R / 4], s[i + R / 2 + R / 4]));
+    v += dpp_f<0xB1>(v);
+    v += dpp_f<0x4E>(v);
+    v += dpp_f<0x141>(v);
+    v += dpp_f<0x140>(v);
+    w[i] = v;
+  }
+}
+
+// A column slice per wave: the waves of a workgroup cover a row once, one 16-byte unit per lane, and every wave multiplies
+// its piece of the vector, which it loads and prepares once, by R rows: R loads and it ends (see below why that streams
+// best).  Memory-bound: 28672 x 16384 int4 runs at 6.6 TB/s, 5.6 with the vector in LDS.  Eight waves per SIMD need 64 registers.
+template <int MODE, int R>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void gemv_columns_kernel(const char* mat_, const u4v* vec_, _Float16* res_, int rows_, int n_,
+                                                            float scale_, float zp_) {
+  using G = Geom<MODE>;
+  __shared__ float part[16][R + 1];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = blockIdx.x * R;
+  const int units = n_ / G::kPerUnit;
+  const int u = wv * 64 + lane, uc = min(u, units - 1);
+  const size_t row_bytes = (size_t)units * 16;
+  u4v m[R], v[G::kVecUnits];
+#pragma unroll
+  for (int i = 0; i < G::kVecUnits; ++i) v[i] = vec_[(size_t)uc * G::kVecUnits + i];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    m[r] = __builtin_nontemporal_load(reinterpret_cast<const u4v*>(mat_ + (size_t)min(row0 + r, rows_ - 1) * row_bytes) + uc);
+  float acc[R], acc16[R], vsum = 0.f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = acc16[r] = 0.f;
+  if (u < units) gemv_step<MODE, R, true>(m, v, acc, acc16, vsum);  // lanes past the row add nothing, whatever they read
+  if (MODE == kI4) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = fmaf(acc16[r], 0.0625f, acc[r]);
+  }
+  float w[R / 4];
+  row_sums<R>(acc, w);
+#pragma unroll
+  for (int i = 0; i < R / 4; ++i)
+    if ((lane & 15) == i) part[wv][i + R / 4 * (lane >> 4)] = w[i];
+  if (MODE != kF16) {
+    const float vs = wave_sum(vsum);
+    if (lane == 0) part[wv][R] = vs;
+  }
+  __syncthreads();
+  if (threadIdx.x < R && row0 + (int)threadIdx.x < rows_) {
+    const int waves = blockDim.x >> 6;
+    float s = 0.f, vs = 0.f;
+    for (int k = 0; k < waves; ++k) {
+      s += part[k][threadIdx.x];
+      if (MODE != kF16) vs += part[k][R];
+    }
+    if (MODE == kI8) s = scale_ * (s - zp_ * vs);
+    if (MODE == kI4) s = scale_ * (s * 16777216.f - zp_ * vs);  // codes were fp16 subnormals code * 2^-24
+    res_[row0 + threadIdx.x] = (_Float16)s;
+  }
+}
+
 // The vector in LDS, the workgroups persistent.  A CU returns its loads in issue order and holds about
 // 64 KB of them, whichever cache serves them: every piece of the vector a wave loads next to its matrix
 // rows (as many bytes as the rows themselves for int8 with two rows per wave and int4 with four) takes a
@@ -356,21 +431,37 @@ int launch_gemv(const void* mat, const void* vec, void* res, int rows, int n, fl
   // (int4 reads four times as many bytes of the vector per byte of the matrix as fp16: rows per wave pay
   // there even when they leave only eight waves per compute unit - 8192 x 28672: 33.1 us with one row per
   // wave, 25.0 with two, 20.6 with four; fp16 at 4096 x 16384: 23.7 us with one row, 28.0 with two)
-  // The LDS kernel pays where a wave loads as many bytes of the vector as of the matrix and walks over several
-  // row groups: int4 with four rows per wave (32768 x 8192 29.0 -> 24.2 us, 28672 x 8192 25.7 -> 22.5,
-  // 16384 x 28672 41.7 -> 38.8, 16384 x 16384 25.8 -> 25.5); fp16 and int8 gain on some shapes and lose on
-  // others (fp16 16384 x 16384 88.7 -> 83.0 us but 28672 x 8192 70.6 -> 79.0), fewer rows lose throughout.
-  // HQ_GEMV_LDS: 0 never, 1 wherever the vector fits, unset: the rule above.
+  // Up to 1024 units of 16 bytes a row (int4 32768 elements, with many rows 16384; int8 16384; fp16 below 8192) a wave takes a
+  // column slice and several rows, eight once that leaves 24 waves per compute unit, else four (fp16 always four), us with whole rows per wave or the
+  // vector in LDS / eight / four: int4 16384 x 16384 25.3 / 21.2 / 24.8, 28672 x 8192 21.3 / 18.3 / 20.8, 18432 x 16384 37.6 / 25.2
+  // / 27.6, 1218 x 15392 6.8 / 4.3 / 4.5, 16384 x 4096 9.0 / 7.2 / 6.9, 8192 x 28672 20.2 / 22.8 / 24.5; int8 16384 x 16384 42.0 / 37.8
+  // / 40.2, 8192 x 8192 13.9 / 11.7 / 11.9, 1000 x 16000 10.4 / 6.4 / 5.4; fp16 16384 x 4096 22.8 / 21.2 / 19.8, 932 x 5568 7.1 / 4.9 /
+  // 4.7.  (Sixteen rows: 22.7 at the first shape, 37.8 against 35.9 at 28672 x 16384.)  Few short rows keep a wave each, which
+  // meets no barrier (fp16 2000 x 1024 4.6 against 4.9).
   // Rows cut across the waves of a workgroup: fp16 rows of 8192 elements or more, two steps of two rows per
-  // wave (16384 x 16384: 88.7 -> 75.7 us = 7.1 TB/s; 28672 x 8192 70.5 -> 64.3; 8192 x 28672 73.8 -> 66.8;
-  // 4096 x 16384 23.0 -> 21.0).  Other step counts per wave are worse, some much (four steps, i.e. waves that
-  // start 4 KB apart: 97.5 us at 16384 x 16384), and int8 / int4 rows gain little or lose: they keep whole
-  // rows per wave.  HQ_GEMV_SPLIT: 0 never, 4 / 8 / 16 that many waves per pair of rows, unset: this rule.
+  // wave (16384 x 16384: 88.7 -> 75.7 us = 7.1 TB/s; 28672 x 8192 70.5 -> 64.3, a column slice per wave 68.7; 8192 x 28672
+  // 73.8 -> 66.8; 4096 x 16384 23.0 -> 21.0).  Other step counts per wave are worse, some much (four steps, i.e. waves that
+  // start 4 KB apart: 97.5 us at 16384 x 16384).  HQ_GEMV_SPLIT: 0 never, 1 / 2 a column slice and eight / four rows per wave,
+  // 4 / 8 / 16 that many waves per pair of rows, unset: these rules.
+  // Longer rows: the LDS kernel pays where a wave loads as many bytes of the vector as of the matrix and walks over several
+  // row groups, int4 with four rows per wave; fp16 and int8 gain on some shapes and lose on others (fp16 16384 x 16384 88.7 -> 83.0
+  // us but 28672 x 8192 70.6 -> 79.0), fewer rows lose throughout.  HQ_GEMV_LDS: 0 never, 1 wherever the vector fits, unset: this rule.
   {
     int split = hq_tune(HQ_TUNE_GEMV_SPLIT, -1);
     const int units = n / Geom<MODE>::kPerUnit;
-    if (split < 0)  // (a forced choice between the two whole-row kernels below stands)
-      split = (MODE == kF16 && units >= 1024 && hq_tune(HQ_TUNE_GEMV_LDS, -1) < 0) ? (units >= 2048 ? 16 : 8) : 0;
+    const int waves = (units + 63) / 64;
+    if (split < 0 && hq_tune(HQ_TUNE_GEMV_LDS, -1) < 0) {  // (a forced choice between the two whole-row kernels stands)
+      if (MODE == kF16 && units >= 1024) split = units >= 2048 ? 16 : 8;
+      else if (units <= (MODE == kI4 && rows >= dev->cus * 16 ? 512 : 1024) &&
+               !((units <= 256 && rows <= dev->cus * 16) || (units <= 128 && rows <= dev->cus * 32)))
+        split = MODE != kF16 && (int64_t)rows * waves >= (int64_t)dev->cus * 192 ? 1 : 2;
+    }
+    if ((split == 1 || split == 2) && units <= 1024) {
+      const dim3 block(waves * 64);
+      if (split == 1) hipLaunchKernelGGL((gemv_columns_kernel<MODE, 8>), dim3((rows + 7) / 8), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
+      else hipLaunchKernelGGL((gemv_columns_kernel<MODE, 4>), dim3((rows + 3) / 4), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
+      return hq_launch_status();
+    }
     const int groups = (rows + 1) / 2;
 #define HQ_GEMV_SPLIT_CASE(S) \
     if (split == S) { \

@@ -78,6 +78,29 @@ def test_rows_cut_across_waves(hq, oracle, tunable, rows, n, mode, split):
     _check(got, r64)
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("rows,n", [(1, 32), (7, 512), (9, 544), (33, 2016), (8, 2080), (131, 8192), (5, 11008), (17, 16384),
+                                    (3, 32768)])
+def test_a_column_slice_per_wave(hq, oracle, tunable, rows, n, mode, split):
+    """Eight and four rows per workgroup of waves that cover a row once: row counts beside multiples of either, rows of one
+    unit, beside whole waves and of the most waves (longer ones take the general path)."""
+    mat, vec = gemv_problem(rows * 5 + n + mode + split, rows, n, mode)
+    _, r64 = oracle.gemv(mat, mode, vec, SCALE, ZP)
+    tunable("HQ_GEMV_SPLIT", split)
+    got, _, _ = _run(hq, mat, vec, mode)
+    _check(got, r64)
+
+
+@pytest.mark.parametrize("mode,rows,n", [(0, 4100, 1056), (0, 700, 7936), (1, 513, 8224), (1, 4099, 16384), (2, 1027, 16416),
+                                         (2, 4097, 16384), (2, 4096, 16416)])
+def test_column_slices_by_default(hq, oracle, mode, rows, n):
+    mat, vec = gemv_problem(rows + n + mode, rows, n, mode)
+    _, r64 = oracle.gemv(mat, mode, vec, SCALE, ZP)
+    got, _, _ = _run(hq, mat, vec, mode)
+    _check(got, r64)
+
+
 @pytest.mark.parametrize("rows,n", [(130, 8192), (33, 16384), (66, 28672), (5, 32768)])
 def test_long_fp16_rows_default_rule(hq, oracle, rows, n):
     """fp16 rows of 8192 elements or more take the split kernel by default."""
