@@ -99,6 +99,23 @@ __device__ __forceinline__ float hq_sum_partials(const float* p, size_t stride, 
   return sum;
 }
 
+// Raw sums of a share of K, write-through to the memory side, and back past the caches of this XCD.
+typedef float hq_f4v __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void hq_store_share(hq_f4v* p, hq_f4v v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+__device__ __forceinline__ hq_f4v hq_load_share(const hq_f4v* p) {  // hq_wait_shares() before the value is used
+  hq_f4v v;
+  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=&v"(v) : "v"(p) : "memory");
+  return v;
+}
+template <int N>
+__device__ __forceinline__ void hq_wait_shares(hq_f4v (&v)[N]) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));  // no use moves in front of the wait
+}
+
 // Streaming stores: write-through (sc1) and nontemporal (nt), i.e. the data is on its way to memory at once
 // and is not kept in the L2.  For a 33.5 MB write stream on MI355X: 5.80 us against 6.46 us with nt alone
 // and 7.04 us with plain stores.  The compiler cannot see that the assembly is a store, so the wait states it

@@ -150,6 +150,7 @@ struct GemmArgs {
   const float* zeros;
   float* out;           // [M][N]
   float* partial;       // K split: [tile][split][Mpad][128] raw sums of a workgroup
+  unsigned* counters;   // and the workgroups of each tile that have left theirs; null: q3_gemm_reduce adds them
   int M, K, N, Gpad;
   int nsplit, spp;      // workgroups per column tile, steps per workgroup (a multiple of kBufs)
   unsigned flags;
@@ -167,18 +168,18 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
                                                              int Gpad_, int nsplit_, int spp_, unsigned flags_,
                                                              const float* scales_, const float* zeros_,
                                                              const float* rowsum_, const float* rowinv_, float* out_,
-                                                             float* partial_) {
+                                                             float* partial_, unsigned* counters_) {
   // leading scalars, not the struct: the first 14 dwords of the arguments arrive preloaded in scalar registers
   GemmArgs a;
   a.w = w_; a.Ap = Ap_; a.rowsum = rowsum_; a.rowinv = rowinv_; a.scales = scales_; a.zeros = zeros_; a.out = out_;
-  a.partial = partial_; a.M = M_; a.K = K_; a.N = N_; a.Gpad = Gpad_; a.nsplit = nsplit_; a.spp = spp_; a.flags = flags_;
+  a.partial = partial_; a.counters = counters_; a.M = M_; a.K = K_; a.N = N_; a.Gpad = Gpad_; a.nsplit = nsplit_; a.spp = spp_; a.flags = flags_;
   constexpr int Mpad = 32 * MB;
   extern __shared__ u4v lds[];  // used by the final reduction only
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int nl = lane & 31, kb = lane >> 5;
   const int G = a.K >> 5;
   // K split: workgroup (tile, split) takes steps t_begin .. t_begin + nsteps - 1 (both multiples of kBufs:
-  // Gpad is a multiple of 32 k-groups) and leaves its raw sums to hq_q3_gemm_reduce
+  // Gpad is a multiple of 32 k-groups) and the last of the tile to arrive, or q3_gemm_reduce, adds them up
   const int t_begin = blockIdx.y * a.spp;
   const int nsteps = min(a.spp, a.Gpad / kStepGroups - t_begin);
   const int col0 = blockIdx.x * kTileN;
@@ -258,6 +259,19 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
 
   float* red = reinterpret_cast<float*>(lds);
   constexpr int REGION = 32 * kTileN;
+  auto share = [&](int split, int m) {  // this lane's raw sums of row m
+    return reinterpret_cast<f4v*>(a.partial + (((size_t)blockIdx.x * a.nsplit + split) * Mpad + m) * kTileN) + nl;
+  };
+  auto finish = [&](f4v v, int mb, int j) {
+    const int m = mb * 32 + 8 * wv + 4 * kb + j;
+    if (m >= a.M || n_out >= a.N) return;
+    f4v o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = sc[e] * (v[e] * ri[mb][j]) - zr[e] * rs[mb][j];
+    f4v* dst = reinterpret_cast<f4v*>(a.out + (size_t)m * a.N + n_out);
+    if (a.flags & HQ_FLAG_ACCUMULATE) { const f4v old = *dst; o += old; }
+    *dst = o;
+  };
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     if (mb) __syncthreads();
@@ -277,18 +291,49 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
       for (int w = 1; w < kWaves; ++w)
         v += *reinterpret_cast<const f4v*>(red + (size_t)w * REGION + r * kTileN + 4 * nl);
       if (a.nsplit > 1) {
-        f4v* dst = reinterpret_cast<f4v*>(a.partial + (((size_t)blockIdx.x * a.nsplit + blockIdx.y) * Mpad + m) * kTileN) + nl;
-        __builtin_nontemporal_store(v, dst);
-      } else if (m < a.M && n_out < a.N) {
-        f4v o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = sc[e] * (v[e] * ri[mb][j]) - zr[e] * rs[mb][j];
-        f4v* dst = reinterpret_cast<f4v*>(a.out + (size_t)m * a.N + n_out);
-        if (a.flags & HQ_FLAG_ACCUMULATE) { const f4v old = *dst; o += old; }
-        *dst = o;
+        hq_store_share(share(blockIdx.y, m), v);
+      } else {
+        finish(v, mb, j);
       }
     }
   }
+  if (a.nsplit == 1 || !a.counters) return;
+  // Every wave waits for the acknowledgement of its write-through stores, the workgroup counts itself at the memory side,
+  // and the last of the tile adds the raw sums in split order, four splits' loads in flight.  (As a kernel of its own this took
+  // 3.4 to 5.1 us and a launch: 23 rows, K=1952, N=12980 13.7 -> 11.7 us, 64 rows, K=4096, N=11008 19.9 -> 18.5; with eight splits of 64
+  // rows, 256 KB for one workgroup, the kernel of its own stays ahead, 24.4 against 25.4 at K=16384, N=4096.)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();  // also: nobody reads the waves' sums in LDS any more
+  unsigned* flag = reinterpret_cast<unsigned*>(lds);
+  if (tid == 0) {
+    const unsigned old = __hip_atomic_fetch_add(&a.counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = old == (unsigned)(a.nsplit - 1);
+    if (old == (unsigned)(a.nsplit - 1))  // ready for the next call
+      __hip_atomic_store(&a.counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!*flag) return;
+  constexpr int F = 4 * MB, AT_ONCE = 4;
+  f4v sum[F];
+#pragma unroll
+  for (int i = 0; i < F; ++i) sum[i] = f4v{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < a.nsplit; s0 += AT_ONCE) {
+    f4v x[AT_ONCE * F];
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k)
+#pragma unroll
+      for (int i = 0; i < F; ++i)
+        x[k * F + i] = hq_load_share(share(min(s0 + k, a.nsplit - 1), (i >> 2) * 32 + 8 * wv + 4 * kb + (i & 3)));
+    hq_wait_shares(x);
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k)
+      if (s0 + k < a.nsplit) {
+#pragma unroll
+        for (int i = 0; i < F; ++i) sum[i] += x[k * F + i];
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < F; ++i) finish(sum[i], i >> 2, i & 3);
 }
 
 // K split: sums the workgroups' raw sums of a tile in split order and applies scale, zero and the row's power
@@ -332,9 +377,10 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
   if (attr != hipSuccess) return (int)attr;
   const int ntiles = (a.N + kTileN - 1) / kTileN;
   hipLaunchKernelGGL((q3_gemm_kernel<MB>), dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K,
-                     a.N, a.Gpad, a.nsplit, a.spp, a.flags, a.scales, a.zeros, a.rowsum, a.rowinv, a.out, a.partial);
+                     a.N, a.Gpad, a.nsplit, a.spp, a.flags, a.scales, a.zeros, a.rowsum, a.rowinv, a.out, a.partial,
+                     a.counters);
   int rc = hq_launch_status();
-  if (rc != HQ_OK || a.nsplit == 1) return rc;
+  if (rc != HQ_OK || a.nsplit == 1 || a.counters) return rc;
   hipLaunchKernelGGL(q3_gemm_reduce, dim3(ntiles, (a.M + 7) / 8 < 8 ? (a.M + 7) / 8 : 8), dim3(256), 0, stream, a, 32 * MB);
   return hq_launch_status();
 }
@@ -345,11 +391,11 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
 // query share it).  K split: column tiles alone leave most CUs idle when N is small (N = 4096: 32 tiles), so K
 // is cut into as many ranges as give every CU a workgroup (at most kMaxSplitGroups of them, which is what the
 // fixed scratch of the entry point that allocates nothing holds), each range a multiple of kBufs steps; the
-// workgroups leave raw sums in the workspace and a second kernel adds them in split order (deterministic).
+// workgroups leave raw sums in the workspace and the last one, or a second kernel, adds them in split order (deterministic).
 namespace {
 struct GemmPlan {
   int Gpad, nsplit, spp;
-  size_t ap_halves, partial_floats;
+  size_t ap_halves, partial_floats, counters;
 };
 GemmPlan gemm_plan(int cus, int K, int N) {
   GemmPlan p;
@@ -365,6 +411,7 @@ GemmPlan gemm_plan(int cus, int K, int N) {
   p.spp = (p.spp + kBufs - 1) / kBufs * kBufs;
   p.nsplit = (nsteps + p.spp - 1) / p.spp;
   p.partial_floats = p.nsplit > 1 ? (size_t)ntiles * p.nsplit * 64 * kTileN : 0;
+  p.counters = p.nsplit > 1 ? (size_t)ntiles : 1;
   return p;
 }
 }  // namespace
@@ -379,7 +426,7 @@ int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counte
   if (hq_q3_tiles_serve(cus, K, N, M, false)) return hq_q3_tiles_need(cus, K, N, M, floats, counters);
   const GemmPlan p = gemm_plan(cus, K, N);
   *floats = p.ap_halves / 2 + 128 + p.partial_floats;
-  *counters = 1;
+  *counters = p.counters;
   return HQ_OK;
 }
 
@@ -397,20 +444,23 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   const size_t ap_halves = plan.ap_halves, partial_floats = plan.partial_floats;
   _Float16* Ap;
   float *rowsum, *rowinv, *partial = nullptr;
+  unsigned* counters;
   if (fixed) {
-    if (ap_halves / 2 > fixed->partial_floats || partial_floats > fixed->sums_floats) return HQ_ERR_TOO_LARGE;
+    if (ap_halves / 2 > fixed->partial_floats || partial_floats > fixed->sums_floats || plan.counters > fixed->ncounters) return HQ_ERR_TOO_LARGE;
     Ap = reinterpret_cast<_Float16*>(fixed->partial);
     rowsum = fixed->rows;
     rowinv = fixed->rows + 64;
     partial = fixed->sums;
+    counters = fixed->counters;
   } else {
     HqWorkspace ws;
-    rc = hq_get_workspace(stream, ap_halves / 2 + 128 + partial_floats, 1, &ws);
+    rc = hq_get_workspace(stream, ap_halves / 2 + 128 + partial_floats, plan.counters, &ws);
     if (rc != HQ_OK) return rc;
     Ap = reinterpret_cast<_Float16*>(ws.partial);
     rowsum = ws.partial + ap_halves / 2;
     rowinv = rowsum + 64;
     partial = rowsum + 128;
+    counters = ws.counters;
   }
   // up to 64 rows per pass over the weights
   for (int m0 = 0; m0 < M; m0 += 64) {
@@ -429,7 +479,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
     a.zeros = zeros;
     a.out = y + (size_t)m0 * N;
     a.M = Mb; a.K = K; a.N = N; a.Gpad = Gpad; a.flags = flags;
-    a.partial = partial; a.nsplit = nsplit; a.spp = spp;
+    a.partial = partial; a.counters = MB == 2 && nsplit > 4 ? nullptr : counters; a.nsplit = nsplit; a.spp = spp;
     rc = MB == 2 ? launch_gemm<2>(a, stream) : launch_gemm<1>(a, stream);
     if (rc != HQ_OK) return rc;
   }

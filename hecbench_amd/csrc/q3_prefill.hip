@@ -99,22 +99,6 @@ struct TileArgs {
   unsigned flags;
 };
 
-// Raw sums of a share, write-through to the memory side, and back past the caches of this XCD.
-__device__ __forceinline__ void store_share(f4v* p, f4v v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
-}
-__device__ __forceinline__ f4v load_share(const f4v* p) {  // wait_shares() before the value is used
-  f4v v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=&v"(v) : "v"(p) : "memory");
-  return v;
-}
-template <int N>
-__device__ __forceinline__ void wait_shares(f4v (&v)[N]) {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));  // no use moves in front of the wait
-}
-
 template <int MB, int KS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void q3_tile_kernel(TileArgs a) {
   using S = Shape<MB, KS>;
@@ -325,7 +309,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       };
       f4v* dst = slot(share);
 #pragma unroll
-      for (int i = 0; i < F * 2; ++i) store_share(dst + i * kThreads, fin[i / 2][i % 2]);
+      for (int i = 0; i < F * 2; ++i) hq_store_share(dst + i * kThreads, fin[i / 2][i % 2]);
       unsigned* last = reinterpret_cast<unsigned*>(lds + S::kStages * S::kStageBytes);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
@@ -345,8 +329,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
           const f4v* src = slot(c);
           f4v x[F * 2];
 #pragma unroll
-          for (int i = 0; i < F * 2; ++i) x[i] = load_share(src + i * kThreads);
-          wait_shares(x);
+          for (int i = 0; i < F * 2; ++i) x[i] = hq_load_share(src + i * kThreads);
+          hq_wait_shares(x);
 #pragma unroll
           for (int i = 0; i < F * 2; ++i) fin[i / 2][i % 2] = !two && c == 0 ? x[i] : fin[i / 2][i % 2] + x[i];
         }

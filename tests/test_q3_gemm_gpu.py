@@ -56,6 +56,22 @@ def test_small_n_splits_k(hq, oracle, M, K, N, seed):
     assert rel_err(y[:, cols], exact, FLOOR_F16) <= 1e-4
 
 
+@pytest.mark.parametrize("M,K,N", [(23, 1952, 12980), (24, 16384, 4096), (33, 12288, 5000), (64, 4096, 11008), (20, 16384, 6148)])
+def test_split_sums_by_the_last_workgroup(hq, oracle, M, K, N):
+    """Two to eight shares per tile, one and two row blocks, a last tile of any width."""
+    import torch
+    codes, scales, zeros, A = oa.make_q3_problem(M + N, K, N, x_dtype=np.float16, batch=M)
+    mat = oracle.q3_pack(codes)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    args = t(A), t(mat), t(scales), t(zeros)
+    y = hq.q3_gemm(*args)
+    for _ in range(3):
+        assert torch.equal(y, hq.q3_gemm(*args))
+    cols = np.unique(np.concatenate([np.arange(0, 130), np.arange(N - 130, N)]))
+    exact = oracle.q3_gemm(A, np.ascontiguousarray(mat[:, cols]), scales[cols], zeros[cols], mode=0)
+    assert rel_err(y.cpu().numpy()[:, cols], exact, FLOOR_F16) <= 1e-4
+
+
 @pytest.mark.parametrize("scale_exp", [-16, -12, -8, 0, 4])
 def test_dynamic_range(hq, oracle, scale_exp):
     """Accuracy must not depend on the magnitude of the activations: whole problem scaled by a power of
