@@ -170,7 +170,8 @@ int hq_q3_matvec_plan(int K, int N, int batch_M);
 /*
  * hq_q3_matvec for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results (except for the
- * many rows that hq_q3_matvec takes in tiles: here they go 64 at a time, with results equal to rounding), but the
+ * many rows that hq_q3_matvec takes in tiles, but for up to 96 rows with N <= 4096: here they go 64 at a time, with results
+ * equal to rounding), but the
  * scratch the kernels need (split-K partial sums and arrival counters of batches 1 and 2, the batched
  * path's re-ordered activations, row sums, row scales and K-split sums) is a fixed 10 MiB + 64 KiB array in device
  * memory that each GPU holds from library load to process end, instead of the stream's workspace.
