@@ -5,7 +5,7 @@
 //
 //   y[m] = fp16_rn( scale[m] * sum_g dot8(codebook[cb(m)][u16(codes[m][g])], x[8g..8g+7]) )
 //
-// One wave owns ROWS consecutive output rows.  Lane l always works on the same
+// One wave owns ROWS consecutive output rows, or the four waves of a workgroup share them (SPLIT).  Lane l always works on the same
 // 64 activations (codes 8l..8l+7 of a 512-code chunk), so the activations live
 // in registers for every row of the wave.  A row chunk is
 // one 128-bit code load per lane (1 KB contiguous per wave); each code gathers a
@@ -50,11 +50,11 @@ __device__ __forceinline__ float dot8(u4v e, u4v xv, float acc) {
 // copies x into LDS in whole lines, behind the loads of the first codes, piece i of unit u at [i][u] (the pieces an odd
 // number of units apart: neither the copy's stores nor the reads meet in a bank); the next chunk's codes are loaded under
 // a chunk's gathers.  4096 x 4096 12.5 -> 12.1 us, 2123 x 6272 13.8 -> 11.7, 16234 x 10496 96.7 -> 90.7 (235 G gathers/s of the
-// 257-262 that the L2 takes), 28672 x 4096 with three code books 68.2 -> 62.6; 1000 x 16384, one row per wave, 13.6 and 13.8.
+// 257-262 that the L2 takes), 28672 x 4096 with three code books 68.2 -> 62.6.
 constexpr int kMaxLdsK = 24576;  // 48 KB
 __host__ __device__ constexpr int aqlm_x_stride(int units) { return (units + 7) / 8 * 8 + 1; }
 
-template <int ROWS, bool XLDS>
+template <int ROWS, bool XLDS, bool SPLIT>
 __global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, const u4v* codebooks_, const u4v* x_, int M_, int K_, int cb_stride_,
                                                          int cb0_, int cb1_, int cb2_, int cb3_,
                                                          const _Float16* scales_, _Float16* y_) {
@@ -69,9 +69,10 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, con
   // writes the line back whole instead of eight XCDs writing 16 bytes of it each).
   const int b = blockIdx.x;
   const int blk = b < (int)(gridDim.x & ~63u) ? ((b & ~63) | ((b & 7) << 3) | ((b >> 3) & 7)) : b;
-  const int wave = (blk * 256 + threadIdx.x) >> 6;
-  const int row0 = wave * ROWS;
-  if (!XLDS && row0 >= a.M) return;  // wave-uniform
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = (SPLIT ? blk : blk * 4 + wv) * ROWS;
+  const int chunk0 = SPLIT ? wv * 64 : 0, step = SPLIT ? 256 : 64;  // units: this wave's first chunk, and to its next
+  if (!XLDS && !SPLIT && row0 >= a.M) return;  // wave-uniform (SPLIT: never)
   const int units_per_row = a.K >> 6;         // 16-byte code units (8 codes) per row; K % 64 == 0
   extern __shared__ u4v xl[];
   const int xstride = aqlm_x_stride(units_per_row);
@@ -83,11 +84,11 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, con
     }
   };
   u4v cw[ROWS];
-  load_codes(lane, cw);
+  load_codes(chunk0 + lane, cw);
   if (XLDS) {
     for (int t = threadIdx.x; t < units_per_row * 8; t += 256) xl[(t & 7) * xstride + (t >> 3)] = a.x[t];
     __syncthreads();
-    if (row0 >= a.M) return;
+    if (!SPLIT && row0 >= a.M) return;
   }
   const u4v* cb[ROWS];
   float acc[ROWS];
@@ -99,10 +100,10 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, con
     cb[r] = p;
     acc[r] = 0.f;
   }
-  for (int u0 = 0; u0 < units_per_row; u0 += 64) {
+  for (int u0 = chunk0; u0 < units_per_row; u0 += step) {
     const int u = u0 + lane;
     u4v next[ROWS];
-    if (u0 + 64 < units_per_row) load_codes(u + 64, next);  // under this chunk's gathers
+    if (u0 + step < units_per_row) load_codes(u + step, next);  // under this chunk's gathers
     if (u < units_per_row) {
       u4v xv[8];
 #pragma unroll
@@ -123,14 +124,26 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, con
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) cw[r] = next[r];
   }
+  __shared__ float part[4][ROWS];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
     float v = acc[r];
 #pragma unroll
     for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m);
-    if (lane == 0 && row0 + r < a.M) {
+    if (SPLIT) {
+      if (lane == 0) part[wv][r] = v;
+    } else if (lane == 0 && row0 + r < a.M) {
       if (a.scales) v *= (float)a.scales[row0 + r];
       a.y[row0 + r] = (_Float16)v;
+    }
+  }
+  if (SPLIT) {
+    __syncthreads();
+    const int row = row0 + (int)threadIdx.x;
+    if (threadIdx.x < ROWS && row < a.M) {
+      float v = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
+      if (a.scales) v *= (float)a.scales[row];
+      a.y[row] = (_Float16)v;
     }
   }
 }
@@ -154,24 +167,37 @@ extern "C" int hq_aqlm_matvec(const int16_t* codes, const void* codebooks, const
   a.codes = (const u4v*)codes; a.codebooks = (const u4v*)codebooks; a.scales = (const _Float16*)scales;
   a.x = (const u4v*)x; a.y = (_Float16*)y; a.M = M; a.K = K; a.cb_stride = cb_stride_int4;
   for (int j = 0; j < 4; ++j) a.cb_sizes[j] = cb_a_sizes[j];
-  // Rows per wave: keep at least ~8 waves per CU in flight (mirrors the CU-count
-  // based sizing of the reference launcher, src/quantAQLM-hip/main.cu:108-121).
+  // Rows per wave, and whether the four waves of a workgroup share its rows, each with every fourth chunk of 512 codes (split).
+  // What counts is gathers in flight and evenly over the compute units.  Measured (us, one / two / four rows per wave; one / two
+  // split): 4096 x 4096 11.7 12.4 12.8; 13.3 12.9 - 9788 x 5440 31.3 30.9 33.1; 34.2 33.0 - 28672 x 4096 three code books 62.0 61.1
+  // 62.9; 71.9 68.2 - 28672 x 16384 291 239 237; 271 248 - 1228 x 16192 25.1 23.2 39.6; 17.1 16.6 - 2472 x 11968 24.9 27.1 27.2;
+  // 21.9 20.2 - 512 x 16384 12.3 17.3 28.7; 9.4 9.4 - 689 x 5184 6.8 9.1 15; 6.3 6.5.  HQ_AQLM_ROWS: 1, 2, 4; 11, 12 split.
   int rows = hq_tune(HQ_TUNE_AQLM_ROWS, 0);
+  bool split = rows == 11 || rows == 12;
+  if (split) rows -= 10;
   if (rows != 1 && rows != 2 && rows != 4) {
     const long waves_wanted = (long)dev->cus * 8;
-    rows = (M >= 4 * waves_wanted) ? 4 : (M >= 2 * waves_wanted ? 2 : 1);
+    if (K > kMaxLdsK) rows = M >= 4 * waves_wanted ? 4 : (M >= 2 * waves_wanted ? 2 : 1);
+    else if (K > 8192) rows = M >= 8 * waves_wanted ? 4 : 2;
+    else rows = M >= 4 * waves_wanted ? 2 : 1;
+    split = K <= kMaxLdsK && (K > 8192 ? M < 2 * waves_wanted : (K >= 4096 && M <= waves_wanted));
   }
-  const int nwaves = (M + rows - 1) / rows;
-  const int blocks = (nwaves + 3) / 4;
+  const int per_block = split ? rows : 4 * rows;
+  const int blocks = (M + per_block - 1) / per_block;
   // one row per wave: four rows share what the workgroup copies, and beyond 8192 elements that takes as long as it saves
-  const bool lds = K <= (rows > 1 ? kMaxLdsK : 8192);
+  const bool lds = K <= (rows > 1 || split ? kMaxLdsK : 8192);
   const size_t smem = lds ? (size_t)aqlm_x_stride(K >> 6) * 8 * 16 : 0;
-#define HQ_AQLM_GO(R, L)                                                                                                \
-  hipLaunchKernelGGL((aqlm_matvec_kernel<R, L>), dim3(blocks), dim3(256), smem, stream, a.codes, a.codebooks, a.x, a.M, \
+#define HQ_AQLM_GO(R, L, S)                                                                                                \
+  hipLaunchKernelGGL((aqlm_matvec_kernel<R, L, S>), dim3(blocks), dim3(256), smem, stream, a.codes, a.codebooks, a.x, a.M, \
                      a.K, a.cb_stride, a.cb_sizes[0], a.cb_sizes[1], a.cb_sizes[2], a.cb_sizes[3], a.scales, a.y)
-  if (rows == 4) { if (lds) HQ_AQLM_GO(4, true); else HQ_AQLM_GO(4, false); }
-  else if (rows == 2) { if (lds) HQ_AQLM_GO(2, true); else HQ_AQLM_GO(2, false); }
-  else { if (lds) HQ_AQLM_GO(1, true); else HQ_AQLM_GO(1, false); }
+#define HQ_AQLM_ROWS_GO(R, S) \
+  { if (lds) HQ_AQLM_GO(R, true, S); else HQ_AQLM_GO(R, false, S); }
+  if (rows == 4) HQ_AQLM_ROWS_GO(4, false)
+  else if (rows == 2 && split) HQ_AQLM_ROWS_GO(2, true)
+  else if (rows == 2) HQ_AQLM_ROWS_GO(2, false)
+  else if (split) HQ_AQLM_ROWS_GO(1, true)
+  else HQ_AQLM_ROWS_GO(1, false)
+#undef HQ_AQLM_ROWS_GO
 #undef HQ_AQLM_GO
   return hq_launch_status();
 }

@@ -30,12 +30,21 @@ def test_vs_oracle(hq, oracle, M, K, seed):
     assert rel_err(y, ref16.astype(np.float64), FLOOR_F16) <= TOL_F16_ACC
 
 
-@pytest.mark.parametrize("M,K,rows", [(5, 8192, 1), (5, 8256, 1), (9, 24576, 2), (9, 24640, 4), (11, 4160, 4), (4, 4096, 2), (6, 8128, 4), (2049, 64, 1)])
+@pytest.mark.parametrize("M,K,rows", [(5, 8192, 1), (5, 8256, 1), (9, 24576, 2), (9, 24640, 4), (11, 4160, 4), (4, 4096, 2), (6, 8128, 4), (2049, 64, 1),
+                                      (1, 64, 11), (3, 512, 12), (5, 1600, 11), (7, 2112, 12), (9, 24576, 12), (4, 24640, 11)])
 def test_activations_in_lds_and_not(hq, oracle, tunable, M, K, rows):
     """Either side of the longest row whose activations go through LDS, chunks of 512 codes whole and cut, the last workgroup
-    with waves that have no row."""
+    with waves that have no row; waves that share rows (11, 12), some without a chunk."""
     tunable("HQ_AQLM_ROWS", rows)
     codes, cb, scales, x = oa.make_aqlm_problem(M + K, M, K)
+    y = _run(hq, codes, cb, scales, x, (M, 0, 0, 0))
+    _, ref64 = oracle.aqlm_matvec(codes, cb, scales, x, (M, 0, 0, 0), 65536, mode=0)
+    assert rel_err(y, ref64, FLOOR_F16) <= 2e-3
+
+
+@pytest.mark.parametrize("M,K", [(2049, 4096), (2048, 4160), (1001, 8256), (4097, 8320), (8193, 576)])
+def test_default_rules(hq, oracle, M, K):
+    codes, cb, scales, x = oa.make_aqlm_problem(M + 2 * K, M, K)
     y = _run(hq, codes, cb, scales, x, (M, 0, 0, 0))
     _, ref64 = oracle.aqlm_matvec(codes, cb, scales, x, (M, 0, 0, 0), 65536, mode=0)
     assert rel_err(y, ref64, FLOOR_F16) <= 2e-3
