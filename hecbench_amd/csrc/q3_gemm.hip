@@ -451,8 +451,14 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   const HqDevice* dev = nullptr;
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
-  if (hq_q3_tiles_serve(dev->cus, K, N, M, fixed != nullptr))
-    return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
+  bool tiles = hq_q3_tiles_serve(dev->cus, K, N, M, fixed != nullptr);
+  if (tiles && !fixed) {
+    // under capture without room for all rows' activations: 64 rows at a time need less
+    size_t floats, counters;
+    hq_q3_tiles_need(dev->cus, K, N, M, &floats, &counters);
+    tiles = !hq_workspace_out_of_reach(stream, floats, counters);
+  }
+  if (tiles) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   const GemmPlan plan = gemm_plan(dev->cus, K, N);
   const int Gpad = plan.Gpad, nsplit = plan.nsplit, spp = plan.spp;
   const size_t ap_halves = plan.ap_halves, partial_floats = plan.partial_floats;

@@ -73,3 +73,29 @@ def test_accumulate_and_the_call_that_allocates_nothing(hq, oracle):
         assert fn(a.data_ptr(), 1, w.data_ptr(), s.data_ptr(), z.data_ptr(), y.data_ptr(), K, N, M, 1, stream) == 0
         torch.cuda.synchronize()
         _check(y.cpu().numpy() - 3.0, exact)
+
+
+def test_capture_with_the_workspace_of_a_smaller_call(hq, oracle):
+    """Under capture nothing can be allocated: where the stream's workspace holds what 64 rows need and not what all do, the
+    call goes 64 rows at a time."""
+    import torch
+    M, K, N = 1000, 4096, 16512
+    codes, scales, zeros, A = oa.make_q3_problem(11, K, N, x_dtype=np.float16, batch=M)
+    mat = oracle.q3_pack(codes)
+    a, w, s, z = _t(A), _t(mat), _t(scales), _t(zeros)
+    out = torch.zeros((M, N), device="cuda:0")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        hq.q3_gemm(a[:32].contiguous(), w, s, z)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream):
+        hq.q3_gemm(a, w, s, z, out=out)
+    cols = np.concatenate([np.arange(0, 40), np.arange(N - 40, N)])
+    exact = oracle.q3_gemm(A, np.ascontiguousarray(mat[:, cols]), scales[cols], zeros[cols], mode=0)
+    for _ in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _check(out.cpu().numpy()[:, cols], exact, rows=False)
