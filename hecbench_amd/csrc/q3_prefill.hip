@@ -294,8 +294,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int i = 0; i < F * 2; ++i) {
       f4v x = group(0, i / 2, i % 2);
 #pragma unroll
-      for (int p = 1; p < KS; ++p) x += at(kp, p - 1)[i * 64];
-      fin[i / 2][i % 2] = x;
+      for (int p = 1; p < KS; ++p) {
+        const f4v other = at(kp, p - 1)[i * 64];
+        x = p & 1 ? x - other : x + other;  // odd parts' k-groups are the negated ones (see the pre-pass)
+      }
+      fin[i / 2][i % 2] = x;  // negated itself where kp is odd
     }
     __syncthreads();  // before the next tile's loads
 
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if (m0 + e < a.M && n < a.N) {
-            const float unit = ri[e] * 16777216.f;  // 2^24: the unit of the code operands
+            const float unit = ri[e] * (kp & 1 ? -16777216.f : 16777216.f);  // 2^24: the unit of the code operands
             f2v o = {sc.x * (fin[i][0][e] * unit) - zr.x * rs[e], sc.y * (fin[i][1][e] * unit) - zr.y * rs[e]};
             f2v* p = reinterpret_cast<f2v*>(a.out + (size_t)(m0 + e) * a.N + n);
             if (a.flags & HQ_FLAG_ACCUMULATE) o += *p;

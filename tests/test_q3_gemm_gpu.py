@@ -72,6 +72,20 @@ def test_split_sums_by_the_last_workgroup(hq, oracle, M, K, N):
     assert rel_err(y.cpu().numpy()[:, cols], exact, FLOOR_F16) <= 1e-4
 
 
+@pytest.mark.parametrize("M,K,N", [(40, 8192, 1000), (64, 4096, 132), (70, 4096, 2048), (128, 8192, 516), (300, 4096, 260)])
+def test_error_has_no_offset(hq, oracle, M, K, N):
+    """The matrix instruction cuts its sums towards minus infinity.  With every product entering with its own sign that was an
+    offset of all results, 9e-6 (K=4096) and 1.3e-5 (K=8192) of them in 2-norm, and grew with K; with the cuts of two halves of
+    opposite sign cancelling, what is left is their scatter, 1.8e-6 whatever K.  64-row kernel and tiles, K whole and split."""
+    codes, scales, zeros, A = oa.make_q3_problem(M + N, K, N, x_dtype=np.float16, batch=M)
+    mat = oracle.q3_pack(codes)
+    y = _run(hq, A, mat, scales, zeros).astype(np.float64)
+    exact = oracle.q3_gemm(A, mat, scales, zeros, mode=0)
+    err = (y - exact) / scales           # in units of the raw sums, as the offset is
+    assert np.linalg.norm(y - exact) <= 4e-6 * np.linalg.norm(exact)
+    assert abs(err.mean()) <= 0.25 * np.sqrt(np.mean(err ** 2))
+
+
 @pytest.mark.parametrize("scale_exp", [-16, -12, -8, 0, 4])
 def test_dynamic_range(hq, oracle, scale_exp):
     """Accuracy must not depend on the magnitude of the activations: whole problem scaled by a power of
