@@ -61,8 +61,9 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
                       float* y, int K, int N, int batch_M, unsigned flags, hipStream_t stream,
                       const HqQ3Scratch* fixed);
 // Batched 3-bit GEMM: the pre-pass (activations [M][K] -> operand-slot order of Mpad rows and Gpad k-groups, row sums and
-// 1 / row scale), and the tiled kernels for many rows.
-int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad, hipStream_t stream);
+// 1 / row scale; the product's arrival counters cleared), and the tiled kernels for many rows.
+int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad,
+                           unsigned* counters, size_t ncounters, hipStream_t stream);
 bool hq_q3_tiles_serve(int cus, int K, int N, int M, bool fixed);
 int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
 void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);

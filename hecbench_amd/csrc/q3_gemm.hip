@@ -67,6 +67,8 @@ __device__ __forceinline__ float prep_wave(float v) {
 // of an operand slot (pos <= 7) then leaves every entry within 2^21 of its row's largest an fp16 normal
 // number, i.e. exactly the input's mantissa; the main kernel's epilogue divides by P[m] again.  (Without
 // P[m] the slot factor alone pushed activations below 2^-7 into the fp16 subnormals.)
+// It also clears the arrival counters of the product behind it: they come back to zero by themselves, but a call that was cut
+// short leaves some behind, with which no later call would finish those tiles.
 // Every second pair of k-groups enters negated.  The matrix instruction cuts its sum towards minus infinity, a little for
 // every sixteen products: with all sums of one sign that was an offset of the whole result, 95 % of its error and growing
 // with K.  The kernels keep the negated pairs in accumulators of their own (odd waves, odd parts of K) and subtract those at
@@ -74,7 +76,8 @@ __device__ __forceinline__ float prep_wave(float v) {
 // 9.1e-6 -> 1.8e-6; 128 rows, K=8192, N=2048 1.28e-5 -> 1.8e-6; 295 rows, K=1376, N=11252 5.5e-6 -> 1.8e-6; same time.
 __global__ __launch_bounds__(256) void q3_gemm_prep(const _Float16* __restrict__ A, _Float16* __restrict__ Ap,
                                                    float* __restrict__ rowsum, float* __restrict__ rowinv,
-                                                   int M, int K, int Mpad, int Gpad) {
+                                                   int M, int K, int Mpad, int Gpad, unsigned* __restrict__ counters,
+                                                   int ncounters) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int G = K >> 5;
   // Eight consecutive rows share the 128-byte lines of Ap; workgroups b, b + 8, b + 16, ... run on the same
@@ -144,6 +147,7 @@ __global__ __launch_bounds__(256) void q3_gemm_prep(const _Float16* __restrict__
       *dst = *reinterpret_cast<const u4v*>(out + 8 * j);
     }
   }
+  for (int i = m * 256 + (int)threadIdx.x; i < ncounters; i += Mpad * 256) counters[i] = 0u;
 }
 
 // Sixteen two-field registers of one column's k-group (see q3_recipe.h).
@@ -437,9 +441,10 @@ GemmPlan gemm_plan(int cus, int K, int N) {
 }
 }  // namespace
 
-int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad, hipStream_t stream) {
+int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad,
+                           unsigned* counters, size_t ncounters, hipStream_t stream) {
   hipLaunchKernelGGL(q3_gemm_prep, dim3((Mpad + 63) / 64 * 64), dim3(256), 0, stream, reinterpret_cast<const _Float16*>(A),
-                     reinterpret_cast<_Float16*>(Ap), rowsum, rowinv, M, K, Mpad, Gpad);
+                     reinterpret_cast<_Float16*>(Ap), rowsum, rowinv, M, K, Mpad, Gpad, counters, (int)ncounters);
   return hq_launch_status();
 }
 
@@ -495,7 +500,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
     const int MB = Mb > 32 ? 2 : 1;
     const int Mpad = 32 * MB;
     const _Float16* A = reinterpret_cast<const _Float16*>(x) + (size_t)m0 * K;
-    rc = hq_q3_gemm_prep_launch(A, Ap, rowsum, rowinv, Mb, K, Mpad, Gpad, stream);
+    rc = hq_q3_gemm_prep_launch(A, Ap, rowsum, rowinv, Mb, K, Mpad, Gpad, counters, nsplit > 1 ? plan.counters : 0, stream);
     if (rc != HQ_OK) return rc;
     GemmArgs a;
     a.w = reinterpret_cast<const uint32_t*>(qweight);

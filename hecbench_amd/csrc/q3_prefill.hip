@@ -505,14 +505,15 @@ int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scale
       return HQ_ERR_TOO_LARGE;
     float* ap = fixed ? fixed->partial : ws.partial;
     float* rowsum = fixed ? fixed->rows : ws.partial + p.ap_floats;
+    unsigned* counters = fixed ? fixed->counters : ws.counters;
     rc = hq_q3_gemm_prep_launch(reinterpret_cast<const _Float16*>(x) + (size_t)m0 * K, ap, rowsum, rowsum + p.Mpad, Mb, K,
-                                p.Mpad, 2 * p.ks * p.T, stream);
+                                p.Mpad, 2 * p.ks * p.T, counters, p.nshare > 1 ? p.counters : 0, stream);
     if (rc != HQ_OK) return rc;
     TileArgs a;
     a.w = reinterpret_cast<const uint32_t*>(qweight);
     a.Ap = reinterpret_cast<const unsigned char*>(ap);
     a.rowsum = rowsum; a.rowinv = rowsum + p.Mpad; a.partial = fixed ? fixed->sums : rowsum + p.row_floats;
-    a.counters = fixed ? fixed->counters : ws.counters;
+    a.counters = counters;
     a.scales = scales; a.zeros = zeros; a.out = y + (size_t)m0 * N;
     a.M = Mb; a.N = N; a.G = K / 32; a.Mpad = p.Mpad; a.nmt = p.nmt; a.T = p.T; a.rounds = p.rounds; a.rest = p.rest;
     a.nshare = p.nshare; a.L = p.L; a.flags = flags;

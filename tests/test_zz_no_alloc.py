@@ -59,6 +59,38 @@ def test_noalloc_matches_workspace_path(hq, oracle):
         assert np.array_equal(_call(lib.hq_q3_matvec_noalloc, p, 1), _call(lib.hq_q3_matvec, p, 1))
 
 
+class _Scratch(ctypes.Structure):  # HqQ3Scratch of csrc/hq_internal.h
+    _fields_ = [("partial", ctypes.c_void_p), ("partial_floats", ctypes.c_size_t), ("rows", ctypes.c_void_p),
+                ("counters", ctypes.c_void_p), ("ncounters", ctypes.c_size_t), ("sums", ctypes.c_void_p),
+                ("sums_floats", ctypes.c_size_t)]
+
+
+@pytest.mark.parametrize("K,N,M", [(4096, 516, 40), (8192, 516, 20), (8192, 2048, 64), (4096, 4096, 70), (8192, 512, 66)])
+def test_batched_call_after_one_that_was_cut_short(hq, oracle, K, N, M):
+    """A call that does not finish leaves its arrival counters part of the way up.  The next call must not count on from
+    there: the library's own launch function with a scratch of the test's, counters as such a call leaves them; 64-row kernel
+    (K split, sums by the last workgroup and, eight splits of 64 rows, by the second kernel) and tiles."""
+    import torch
+    from hecbench_amd import _lib
+    launch = getattr(_lib.load(), "_Z17hq_q3_gemm_launchPKvPKiPKfS4_PfiiijP12ihipStream_tPK11HqQ3Scratch")
+    p = _problem(oracle, 303, K, N, M)
+    dev = "cuda:0"
+    partial = torch.zeros(1 << 19, device=dev)
+    rows = torch.zeros(256, device=dev)
+    sums = torch.zeros(1 << 21, device=dev)
+    counters = torch.full((4096,), 100, dtype=torch.int32, device=dev)  # of a call with more parts
+    vp = lambda t: ctypes.c_void_p(t.data_ptr())
+    s = _Scratch(partial.data_ptr(), partial.numel(), rows.data_ptr(), counters.data_ptr(), counters.numel(), sums.data_ptr(),
+                 sums.numel())
+    want = oracle.q3_gemm(p["host"][4], *p["host"][1:4], mode=0)
+    for _ in range(2):
+        y = torch.full((M, N), float("nan"), device=dev)
+        stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        assert launch(vp(p["A"]), vp(p["mat"]), vp(p["s"]), vp(p["z"]), vp(y), K, N, M, 0, stream, ctypes.byref(s)) == 0
+        torch.cuda.synchronize()
+        assert rel_err(y.cpu().numpy(), want) <= 5e-3
+
+
 def test_noalloc_rejects_beyond_its_limits(hq):
     import torch
     from hecbench_amd import _lib
