@@ -42,6 +42,7 @@ constexpr int kBufs = kDeep + 1;
 constexpr int kChunk = kStepGroups * kBufs;  // the pre-pass pads K to a multiple of this many k-groups
 constexpr int kTileN = 128;     // output columns per workgroup
 constexpr int kMaxSplitGroups = 256;  // workgroups of a K-split launch (tiles times splits)
+constexpr int kFixedMaxK = 16384;     // longest K of a batched call in the fixed scratch
 
 
 // Sum or maximum over the 64 lanes on the data path's own lane exchanges (two times six rounds of shuffles through the LDS
@@ -449,7 +450,7 @@ int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv
 }
 
 int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
-  if (hq_q3_tiles_serve(cus, K, N, M, false)) return hq_q3_tiles_need(cus, K, N, M, floats, counters);
+  if (hq_q3_tiles_serve(cus, K, N, M)) return hq_q3_tiles_need(cus, K, N, M, floats, counters);
   const GemmPlan p = gemm_plan(cus, K, N);
   *floats = p.ap_halves / 2 + 128 + p.partial_floats;
   *counters = p.counters;
@@ -463,12 +464,13 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   const HqDevice* dev = nullptr;
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
-  bool tiles = hq_q3_tiles_serve(dev->cus, K, N, M, fixed != nullptr);
-  if (tiles && !fixed) {
-    // under capture without room for all rows' activations: 64 rows at a time need less
+  bool tiles = hq_q3_tiles_serve(dev->cus, K, N, M);
+  if (tiles) {
+    // 64 rows at a time need less: under capture without room for all rows' activations, and where the fixed array cannot hold
+    // the tiles' plan (a device of more compute units than it was sized for; K beyond its limit, which is refused below)
     size_t floats, counters;
     hq_q3_tiles_need(dev->cus, K, N, M, &floats, &counters);
-    tiles = !hq_workspace_out_of_reach(stream, floats, counters);
+    tiles = fixed ? K <= kFixedMaxK && floats <= fixed->tiles_floats : !hq_workspace_out_of_reach(stream, floats, counters);
   }
   if (tiles) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   const GemmPlan plan = gemm_plan(dev->cus, K, N);
@@ -521,13 +523,19 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
 // ---- the entry point that allocates nothing ----------------------------------------------------
 // Its scratch (split-K partial sums and arrival counters of the matvec, re-ordered activations, row
 // sums, row scales and K-split sums of the batched GEMM) lives in a fixed device array instead of the stream's
-// workspace.  Every GPU holds its own copy of the array at its own address, resolved once per device.
+// workspace.  Every GPU holds its own copy of the array at its own address, resolved once per device.  It holds what the
+// tiled kernels take at most (hq_q3_tiles_need, 256 compute units), so that every batch takes the kernels and the plan of
+// hq_q3_matvec and returns its bits; the other paths use the front of it, within the limits they had before there were tiles.
 namespace {
-constexpr size_t kScratchPartialBytes = (size_t)2 << 20;  // 2 MiB: K <= 16384 batched, 8192 partial rows of 64 floats
 constexpr size_t kScratchRowBytes = 1024;                 // 256 floats
 constexpr size_t kScratchCounterBytes = 64 * 1024 - kScratchRowBytes;
+constexpr size_t kScratchPartialBytes = (size_t)2 << 20;  // 2 MiB: K <= 16384 batched, 8192 partial rows of 64 floats
 constexpr size_t kScratchSumBytes = (size_t)kMaxSplitGroups * 64 * kTileN * sizeof(float);  // 8 MiB: the GEMM's K split
-constexpr size_t kScratchBytes = kScratchPartialBytes + kScratchRowBytes + kScratchCounterBytes + kScratchSumBytes;
+static_assert(kScratchPartialBytes == (size_t)kFixedMaxK * 64 * sizeof(_Float16), "64 rows of the longest K");
+// tiles: 36 MiB of re-ordered activations, sums and scales of 8192 rows, 256 shares of 128 x 256 sums
+constexpr size_t kScratchTileBytes = ((size_t)36 << 20) + 2 * 8192 * sizeof(float) + (size_t)256 * 128 * 256 * sizeof(float);
+static_assert(kScratchTileBytes >= kScratchPartialBytes + kScratchSumBytes, "the other paths use the tiles' space");
+constexpr size_t kScratchBytes = kScratchRowBytes + kScratchCounterBytes + kScratchTileBytes;  // 68 MiB + 128 KiB
 }  // namespace
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -565,12 +573,15 @@ extern "C" int hq_q3_matvec_noalloc(const void* x, int x_dtype, const int32_t* q
   if (rc != HQ_OK) return rc;
   unsigned char* b = static_cast<unsigned char*>(base);
   HqQ3Scratch s;
+  s.rows = reinterpret_cast<float*>(b);
+  s.counters = reinterpret_cast<unsigned*>(b + kScratchRowBytes);
+  s.ncounters = kScratchCounterBytes / sizeof(unsigned);
+  b += kScratchRowBytes + kScratchCounterBytes;
   s.partial = reinterpret_cast<float*>(b);
   s.partial_floats = kScratchPartialBytes / sizeof(float);
-  s.rows = reinterpret_cast<float*>(b + kScratchPartialBytes);
-  s.counters = reinterpret_cast<unsigned*>(b + kScratchPartialBytes + kScratchRowBytes);
-  s.ncounters = kScratchCounterBytes / sizeof(unsigned);
-  s.sums = reinterpret_cast<float*>(b + kScratchPartialBytes + kScratchRowBytes + kScratchCounterBytes);
+  s.sums = reinterpret_cast<float*>(b + kScratchPartialBytes);
   s.sums_floats = kScratchSumBytes / sizeof(float);
+  s.tiles = reinterpret_cast<float*>(b);
+  s.tiles_floats = kScratchTileBytes / sizeof(float);
   return hq_q3_matvec_impl(x, x_dtype, qweight, scales, zeros, y, K, N, batch_M, flags, (hipStream_t)stream, &s);
 }

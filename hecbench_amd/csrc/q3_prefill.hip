@@ -413,11 +413,10 @@ TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int wa
   return p;
 }
 
-// 65 to 96 rows of a matrix of less than 2^25 weights: served here as well, with the smallest tile, as far as the fixed array
-// of hq_q3_matvec_noalloc holds the plan (whose results are then those of hq_q3_matvec): 2 MiB of activations, two sums of 128
-// rows, 8 MiB of shares.  The 64-row kernel reads the weights twice and launches six times: 70 rows, K=4096, N=4096 27.2 -> 17.6
-// us; 90 rows, K=512, N=2048 18.4 -> 10.5; 66 rows, K=8192, N=512 26.0 -> 20.3.  (Larger matrices would gain as much, 96 rows,
-// K=8192, N=4096 33.1 -> 22.5, but their callers have reserved what the 64-row kernel needs.)
+// 65 to 96 rows of a narrow matrix of less than 2^25 weights are served here as well, with the smallest tile.  The 64-row kernel
+// reads the weights twice and launches six times: 70 rows, K=4096, N=4096 27.2 -> 17.6 us; 90 rows, K=512, N=2048 18.4 -> 10.5; 66
+// rows, K=8192, N=512 26.0 -> 20.3.  The line at 2^25 weights and K=8192 is where the workspace of such a call was once agreed on
+// and not where the times cross: beyond it as much would be gained (96 rows, K=8192, N=4096 33.1 -> 22.5).
 bool few_rows(int cus, int K, int N, int M) {
   return M > 64 && M <= 96 && N <= 4096 && K <= 8192 && (int64_t)K * N < (1 << 25) && cus <= 256;
 }
@@ -453,11 +452,10 @@ int launch_tiles(const TileArgs& a, int nwg, hipStream_t stream) {
 
 }  // namespace
 
-// Batches the tiled kernels serve, and those they serve in the fixed array of hq_q3_matvec_noalloc.  Up to 64 rows go
-// through the 64-row kernel of q3_gemm.hip (64 rows, K=8192, N=28672: 36.8 us there, 40.2 here; 32 rows 26.5 and 35.4; 58 rows,
-// K=6464, N=13924 28.7 and 25.9).
-bool hq_q3_tiles_serve(int cus, int K, int N, int M, bool fixed) {
-  return few_rows(cus, K, N, M) || (!fixed && (M > 96 || (M > 64 && N > 4096)));
+// Batches the tiled kernels serve.  Up to 64 rows go through the 64-row kernel of q3_gemm.hip (64 rows, K=8192, N=28672: 36.8 us
+// there, 40.2 here; 32 rows 26.5 and 35.4; 58 rows, K=6464, N=13924 28.7 and 25.9).
+bool hq_q3_tiles_serve(int cus, int K, int N, int M) {
+  return few_rows(cus, K, N, M) || M > 96 || (M > 64 && N > 4096);
 }
 
 int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
@@ -489,30 +487,33 @@ int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scale
   const HqDevice* dev = nullptr;
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
-  HqWorkspace ws;
-  if (!fixed) {
-    size_t floats, counters;
-    hq_q3_tiles_need(dev->cus, K, N, M, &floats, &counters);
-    rc = hq_get_workspace(stream, floats, counters, &ws);
+  size_t floats, ncounters;
+  hq_q3_tiles_need(dev->cus, K, N, M, &floats, &ncounters);
+  float* ap;
+  unsigned* counters;
+  if (fixed) {
+    if (floats > fixed->tiles_floats || ncounters > fixed->ncounters) return HQ_ERR_TOO_LARGE;
+    ap = fixed->tiles;
+    counters = fixed->counters;
+  } else {
+    HqWorkspace ws;
+    rc = hq_get_workspace(stream, floats, ncounters, &ws);
     if (rc != HQ_OK) return rc;
+    ap = ws.partial;
+    counters = ws.counters;
   }
   const int rows = rows_per_pass(K, M);
   for (int m0 = 0; m0 < M; m0 += rows) {
     const int Mb = M - m0 < rows ? M - m0 : rows;
     const TilePlan p = tile_plan(dev->cus, K, N, Mb);
-    if (fixed && (p.ap_floats > fixed->partial_floats || p.row_floats > 256 || p.partial_floats > fixed->sums_floats ||
-                  p.counters > fixed->ncounters))
-      return HQ_ERR_TOO_LARGE;
-    float* ap = fixed ? fixed->partial : ws.partial;
-    float* rowsum = fixed ? fixed->rows : ws.partial + p.ap_floats;
-    unsigned* counters = fixed ? fixed->counters : ws.counters;
+    float* rowsum = ap + p.ap_floats;
     rc = hq_q3_gemm_prep_launch(reinterpret_cast<const _Float16*>(x) + (size_t)m0 * K, ap, rowsum, rowsum + p.Mpad, Mb, K,
                                 p.Mpad, 2 * p.ks * p.T, counters, p.nshare > 1 ? p.counters : 0, stream);
     if (rc != HQ_OK) return rc;
     TileArgs a;
     a.w = reinterpret_cast<const uint32_t*>(qweight);
     a.Ap = reinterpret_cast<const unsigned char*>(ap);
-    a.rowsum = rowsum; a.rowinv = rowsum + p.Mpad; a.partial = fixed ? fixed->sums : rowsum + p.row_floats;
+    a.rowsum = rowsum; a.rowinv = rowsum + p.Mpad; a.partial = rowsum + p.row_floats;
     a.counters = counters;
     a.scales = scales; a.zeros = zeros; a.out = y + (size_t)m0 * N;
     a.M = Mb; a.N = N; a.G = K / 32; a.Mpad = p.Mpad; a.nmt = p.nmt; a.T = p.T; a.rounds = p.rounds; a.rest = p.rest;

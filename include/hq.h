@@ -148,8 +148,12 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  *     workgroup unless N / 128 is at least 7/8 of the compute units or K is longer than that;
  *     every activation enters with an error of at most 2^-19 of the largest magnitude
  *     among its 32 neighbours (exactly, if within 2^8 of it);
- *   - everything else: the MFMA GEMM path (64 rows per pass over the weights; more than 96 rows, or more than 64 unless
- *     N <= 4096 and K * N >= 2^25: tiles of 64 or 128 rows, thousands of rows per pass), which pre-scales every activation row by a
+ *   - everything else: the MFMA GEMM path.  Up to 64 rows go in one pass over the weights; more than 96 rows, and 65 to 96
+ *     rows where N > 4096 or where K <= 8192 and K * N < 2^25, in tiles of 64 or 128 rows, up to thousands of rows per pass;
+ *     the remaining 65 to 96 rows in two passes of up to 64.  Under stream capture, where the stream's workspace is too small
+ *     for the tiles' scratch and cannot grow, the call still succeeds with the workspace of a call of 64 rows: it goes 64 rows at a
+ *     time, with results equal to rounding (not bit for bit) and slower, 1.3 to 5 times at hundreds of rows;
+ *     hq_reserve_workspace keeps calls off that path.  Every activation row is pre-scaled by a
  *     power of two, so accuracy does not depend on the magnitude of the activations:
  *     entries within 2^21 of their row's largest magnitude enter the matrix cores
  *     exactly, smaller ones lose low bits (those 2^32 below it vanish).
@@ -169,11 +173,9 @@ int hq_q3_matvec_plan(int K, int N, int batch_M);
 
 /*
  * hq_q3_matvec for callers that cannot allocate (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results (except for the
- * many rows that hq_q3_matvec takes in tiles, but for up to 96 rows with N <= 4096: here they go 64 at a time, with results
- * equal to rounding), but the
+ * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results, but the
  * scratch the kernels need (split-K partial sums and arrival counters of batches 1 and 2, the batched
- * path's re-ordered activations, row sums, row scales and K-split sums) is a fixed 10 MiB + 64 KiB array in device
+ * path's re-ordered activations, row sums, row scales and K-split sums) is a fixed 68 MiB + 128 KiB array in device
  * memory that each GPU holds from library load to process end, instead of the stream's workspace.
  * The call runs no hipMalloc, hipFree or allocating library routine.  Limits: a batch that the MFMA
  * GEMM serves (hq_q3_matvec_plan) needs K <= 16384; a split-K matvec needs tiles * splits * batch_M <= 8192 (the one-per-round split falls

@@ -59,10 +59,30 @@ def test_noalloc_matches_workspace_path(hq, oracle):
         assert np.array_equal(_call(lib.hq_q3_matvec_noalloc, p, 1), _call(lib.hq_q3_matvec, p, 1))
 
 
+@pytest.mark.parametrize("K,N,M", [(4096, 11008, 65), (8192, 4096, 72), (1024, 2048, 97), (4096, 4096, 128), (8192, 28672, 200),
+                                   (16384, 6148, 300), (512, 260, 9000), (2080, 1028, 1100), (4160, 28672, 1030)])
+def test_many_rows_give_the_bits_of_the_workspace_path(hq, oracle, K, N, M):
+    """Batches that hq_q3_matvec takes in tiles (and one that it takes 64 rows at a time): whole rounds, divided rests, several
+    passes over the rows, the longest K."""
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    dev = "cuda:0"
+    A = torch.empty((M, K), dtype=torch.float16, device=dev).normal_(generator=g)
+    w = torch.randint(-2 ** 31, 2 ** 31, (3 * K // 32, N), dtype=torch.int32, device=dev, generator=g)
+    s = torch.rand(N, device=dev, generator=g).mul_(0.01).add_(0.002)
+    p = dict(K=K, N=N, M=M, x=None, mat=w, s=s, z=s * 3, A=A)
+    want = _call(lib.hq_q3_matvec, p, M)
+    assert np.isfinite(want).all()
+    for _ in range(2):
+        assert np.array_equal(_call(lib.hq_q3_matvec_noalloc, p, M), want)
+
+
 class _Scratch(ctypes.Structure):  # HqQ3Scratch of csrc/hq_internal.h
     _fields_ = [("partial", ctypes.c_void_p), ("partial_floats", ctypes.c_size_t), ("rows", ctypes.c_void_p),
                 ("counters", ctypes.c_void_p), ("ncounters", ctypes.c_size_t), ("sums", ctypes.c_void_p),
-                ("sums_floats", ctypes.c_size_t)]
+                ("sums_floats", ctypes.c_size_t), ("tiles", ctypes.c_void_p), ("tiles_floats", ctypes.c_size_t)]
 
 
 @pytest.mark.parametrize("K,N,M", [(4096, 516, 40), (8192, 516, 20), (8192, 2048, 64), (4096, 4096, 70), (8192, 512, 66)])
@@ -78,10 +98,11 @@ def test_batched_call_after_one_that_was_cut_short(hq, oracle, K, N, M):
     partial = torch.zeros(1 << 19, device=dev)
     rows = torch.zeros(256, device=dev)
     sums = torch.zeros(1 << 21, device=dev)
+    tiles = torch.zeros(1 << 22, device=dev)
     counters = torch.full((4096,), 100, dtype=torch.int32, device=dev)  # of a call with more parts
     vp = lambda t: ctypes.c_void_p(t.data_ptr())
     s = _Scratch(partial.data_ptr(), partial.numel(), rows.data_ptr(), counters.data_ptr(), counters.numel(), sums.data_ptr(),
-                 sums.numel())
+                 sums.numel(), tiles.data_ptr(), tiles.numel())
     want = oracle.q3_gemm(p["host"][4], *p["host"][1:4], mode=0)
     for _ in range(2):
         y = torch.full((M, N), float("nan"), device=dev)
