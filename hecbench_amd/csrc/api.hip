@@ -93,15 +93,16 @@ int hq_current_device(const HqDevice** out) {
 }
 
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
-                     HqWorkspace* out) {
+                     HqWorkspace* out, bool reserve) {
   int dev = 0;
   HQ_HIP_TRY(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_mu);
   HqWorkspace& ws = g_workspaces[std::make_pair(dev, stream)];
   if (ws.partial_floats < need_floats) {
-    // grow geometrically: a stream that sees larger and larger problems allocates O(log) times
+    // grow geometrically: a stream that sees larger and larger problems allocates O(log) times; a reservation names the largest
     size_t n = ws.partial_floats ? ws.partial_floats * 2 : (size_t)1 << 20;
     while (n < need_floats) n *= 2;
+    if (reserve) n = need_floats;
     float* p = nullptr;
     HQ_HIP_TRY(hipMalloc((void**)&p, n * sizeof(float)));
     // kernels in flight may still read the previous buffer: it is kept until hq_shutdown()
@@ -185,7 +186,7 @@ extern "C" int hq_reserve_workspace(void* stream, int max_K, int max_N) {
   size_t floats = 0, counters = 0;
   reserve_bound(d->cus, max_K, max_N, &floats, &counters);
   HqWorkspace ws;
-  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws);
+  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, true);
 }
 
 extern "C" int hq_shutdown(void) {

@@ -39,9 +39,9 @@ struct HqWorkspace {
 };
 
 // Workspace of (current device, stream) holding at least the requested sizes.
-// Allocated on first use, grown geometrically on demand, freed by hq_shutdown().
+// Allocated on first use, grown geometrically on demand (reserve: to no more than the request), freed by hq_shutdown().
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
-                     HqWorkspace* out);
+                     HqWorkspace* out, bool reserve = false);
 // Whether that would allocate while the stream is being captured, where an allocation is an error: a plan that can do
 // without a workspace then does.
 bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters);

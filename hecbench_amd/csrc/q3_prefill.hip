@@ -384,6 +384,11 @@ constexpr TileKind kKinds[3] = {{128, 256, 2, 1.4f, 4.0f, 3.2f}, {64, 256, 2, 0.
 constexpr int kMaxShares = 8;
 constexpr int kMaxWorkgroups = 512;  // bounds the workspace on larger devices
 
+// What T steps of a tile take in c shares.
+float tile_us(const TileKind& kind, int T, int c) {
+  return 3.f + (T + c - 1) / c * kind.step_us + (c > 1 ? kind.share_us + c * kind.per_share_us : 0.f);
+}
+
 TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int want_shares) {
   TilePlan p;
   const int G = K / 32;
@@ -399,7 +404,7 @@ TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int wa
   p.nshare = 1;
   float best = 0.f;
   for (int c = 1; p.rest && c <= kMaxShares && c * p.rest <= p.nwg && c <= p.T; ++c) {
-    const float t = 3.f + (p.T + c - 1) / c * kind.step_us + (c > 1 ? kind.share_us + c * kind.per_share_us : 0.f);
+    const float t = tile_us(kind, p.T, c);
     if (c == 1 || (want_shares ? c <= want_shares : t < best)) { best = t; p.nshare = c; }
   }
   p.us = p.rounds * (3.f + p.T * kind.step_us) + best;
@@ -473,12 +478,21 @@ int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* count
 // Upper bound of hq_q3_tiles_need over every K <= max_K, any N and any M.
 void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters) {
   const size_t wgs = cus < kMaxWorkgroups ? cus : kMaxWorkgroups;
+  // re-ordered activations, K padded to whole steps: 8192 rows of a short K, 32 MB of rows of a longer one, 1024 rows at least
   const size_t kpad = ((size_t)max_K + 255) / 256 * 256;
-  // re-ordered activations: 1024 rows of max_K, or 32 MB of a shorter K, padded to whole row tiles and steps
-  size_t ap = (size_t)1024 * kpad / 2;
-  const size_t ap32 = ((size_t)16 << 20) / 2 + (size_t)8192 * 256 / 2;
-  if (ap < ap32) ap = ap32;
-  *floats = ap + 2 * 8192 + wgs * 128 * 256;
+  const size_t of_32mb = ((size_t)16 << 20) / 2 + (size_t)8192 * 256 / 2;
+  size_t ap = (size_t)8192 * kpad / 2 < of_32mb ? (size_t)8192 * kpad / 2 : of_32mb;
+  if (ap < (size_t)1024 * kpad / 2) ap = (size_t)1024 * kpad / 2;
+  // shares of divided tiles: one per workgroup, of the largest tile that is ever divided (a K of few steps is not)
+  size_t tile = 0;
+  for (const TileKind& kind : kKinds) {
+    const int T = (max_K / 32 + 2 * kind.ks - 1) / (2 * kind.ks);
+    bool divided = false;
+    for (int t = 2; t <= T && !divided; ++t)
+      for (int c = 2; c <= kMaxShares && c <= t; ++c) divided = divided || tile_us(kind, t, c) < tile_us(kind, t, 1);
+    if (divided && (size_t)kind.tm * kind.tn > tile) tile = (size_t)kind.tm * kind.tn;
+  }
+  *floats = ap + 2 * 8192 + wgs * tile;
   *counters = wgs;
 }
 

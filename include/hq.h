@@ -17,11 +17,11 @@
  *   - nothing is printed; hq_strerror() turns a code into text;
  *   - a NaN or an infinity among the activations makes the affected outputs non-finite (the
  *     fixed-point matrix-core paths give NaN where the reference arithmetic would give +-Inf);
- *   - the library keeps one small workspace per (device, stream) pair (split-K
+ *   - the library keeps one workspace per (device, stream) pair (split-K
  *     partial sums, arrival counters, re-ordered GEMM activations), allocated by
  *     hq_init() / hq_reserve_workspace() or by the first call that needs more than
  *     is there (that call then runs hipMalloc, which fails under stream capture:
- *     reserve first).  A workspace grows geometrically, lives until hq_shutdown()
+ *     reserve first).  A workspace grows geometrically (a reservation to what it names), lives until hq_shutdown()
  *     and is used by every call on its stream: calls on different streams may
  *     overlap, two host threads must not issue calls on the SAME stream at the
  *     same time (the calls of one stream share the workspace in stream order).
@@ -73,7 +73,11 @@ int hq_init(void);
 
 /* Sizes the workspace of (current device, stream) for split-K matvecs up to max_N columns and
  * batched GEMMs up to max_K input features, so that later calls on that stream never allocate
- * (needed before stream capture).  No counterpart in the reference. */
+ * (needed before stream capture).  It allocates what hq_reserve_need tells: room for batches of any size, thousands of
+ * re-ordered rows and the shares of divided tiles among them - on 256 compute units 8 MiB for max_K = 512, 16 MiB for
+ * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152.  A stream that only ever sees smaller calls takes less without a
+ * reservation: a workspace grows with the calls (hq_q3_workspace_need; batch 1 at most a few MiB, up to 64 rows 16 MiB).
+ * No counterpart in the reference. */
 int hq_reserve_workspace(void* stream, int max_K, int max_N);
 
 /* Host-only size queries behind hq_reserve_workspace (plain arithmetic: no device is touched, so they also

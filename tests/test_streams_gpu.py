@@ -1,5 +1,7 @@
 """Calls on different streams use different workspaces and may overlap: interleaved split-K
 matvecs and batched GEMMs on two streams give the results of the same calls on one stream."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -39,3 +41,20 @@ def test_two_streams_interleaved(hq, oracle, tunable):
         for y, g in outs[i]:
             assert torch.equal(y, want[i][0])
             assert torch.equal(g, want[i][1])
+
+
+def test_a_reservation_allocates_what_it_names(hq):
+    """Memory of a stream's reservation: what hq_reserve_need tells, rounded to the allocator's units and not to a power of two."""
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    cus = hq.device_info()["compute_units"]
+    stream = torch.cuda.Stream()
+    for K, N in ((512, 512), (4096, 11008)):     # the second one replaces the first one's buffer, which stays
+        f, c = ctypes.c_int64(), ctypes.c_int64()
+        assert lib.hq_reserve_need(cus, K, N, ctypes.byref(f), ctypes.byref(c)) == 0
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        assert lib.hq_reserve_workspace(ctypes.c_void_p(stream.cuda_stream), K, N) == 0
+        taken = free - torch.cuda.mem_get_info()[0]
+        assert taken <= f.value * 4 + c.value * 4 + (6 << 20), (K, N, taken, f.value * 4)

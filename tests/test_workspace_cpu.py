@@ -47,6 +47,25 @@ def test_reserve_covers_every_smaller_call(cus, max_K, max_N):
     assert worst[0] > 0 or max_K < 2048
 
 
+@pytest.mark.parametrize("cus", [256, 304, 64])
+@pytest.mark.parametrize("max_K,max_N", [(512, 512), (1024, 4096), (1920, 4096), (4096, 11008), (16384, 16384), (49152, 12288)])
+def test_reserve_is_close_to_the_largest_need(cus, max_K, max_N):
+    """Batches of any size are covered, and no more is reserved than a quarter beyond what the largest of them takes (a layer of
+    512 x 512 once reserved 68 MiB for a need of 8)."""
+    lib = _lib.load()
+    bf, bc = _bound(lib, cus, max_K, max_N)
+    rng = random.Random(max_K + cus)
+    worst = 0
+    for i in range(6000):
+        K = max_K if i % 2 else rng.randrange(1, max_K // 32 + 1) * 32
+        N = max_N if i % 3 else rng.randrange(1, max_N // 4 + 1) * 4
+        M = int(2 ** rng.uniform(6, 15))
+        f, c = _need(lib, cus, K, N, M)
+        assert f <= bf and c <= bc, (cus, K, N, M, f, bf, c, bc)
+        worst = max(worst, f)
+    assert bf <= 1.25 * worst
+
+
 def test_the_case_that_used_to_fall_short():
     # 256 compute units: a reservation for (8192, 28672) must hold M=72, K=8192, N=4096, whose 32 column tiles
     # split K eight ways (re-ordered activations 262,144 floats + 128 + 32 x 8 x 64 x 128 raw sums)
