@@ -216,12 +216,15 @@ __device__ __forceinline__ float dpp_f(float v) {
 __device__ __forceinline__ float lane_f(float v, int l) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
-// Maximum over the 64 lanes: four DPP butterfly steps per 16-lane row, then the row results.
-__device__ __forceinline__ float wave_max(float v) {
+// Maximum over 16 lanes (four DPP butterfly steps), and over all 64: then the row results.
+__device__ __forceinline__ float row_max(float v) {
   v = fmaxf(v, dpp_f<0xB1>(v));   // quad_perm [1,0,3,2]
   v = fmaxf(v, dpp_f<0x4E>(v));   // quad_perm [2,3,0,1]
   v = fmaxf(v, dpp_f<0x141>(v));  // row_half_mirror
-  v = fmaxf(v, dpp_f<0x140>(v));  // row_mirror
+  return fmaxf(v, dpp_f<0x140>(v));  // row_mirror
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = row_max(v);
   return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
 }
 
@@ -290,6 +293,8 @@ constexpr int planes_of_set(int nb, int s) { return nb - 3 * s < 3 ? nb - 3 * s 
 // holds digit d of block 4m + r's k-word at that block's K positions, zeros elsewhere.  Result quarter kb is then block
 // 4m + kb alone, every MFMA's four digits are combined and take the alpha of their own block, and an MFMA of the same
 // digits against all-ones weights gives the k-word's sum(x).  q_bias: one such sum more, quarter kb for k-word kb.
+// The fixed-point scale is a quad's own: with one for the wave's round, up to four quads, an outlier took low bits from
+// activations as far as 511 elements away.
 // Against weights as first operand with two digit operands per quad and alpha on every digit (four times the multiply-adds, no
 // split of K), K=4096, N=16384, three planes, group 64 / 32: 11.4 / 12.6 -> 8.2 / 9.6 us.
 template <int NB, int QUADS, int WAVES, bool BIAS, bool RAGGED, bool ONE_ROUND, bool GROUPED>
@@ -455,11 +460,13 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
         amax = fmaxf(amax, fabsf(xv[j]));
       }
     }
-    const float xmax = wave_max(amax);
+    // GROUPED: a quad's scale is its own (its sixteen lanes are one DPP row), otherwise the round's
+    const float xmax = GROUPED ? row_max(amax) : wave_max(amax);
     // 2^E * max|x| lies in [2^14, 2^15): u = rint(|x| * 2^E) <= 2^15 stays inside 16 bits
     int E = 14 - ((int)((__float_as_uint(xmax) >> 23) & 255u) - 127);
     E = xmax > 0.f ? max(-120, min(120, E)) : 0;
     const float scaleE = __uint_as_float((uint32_t)(E + 127) << 23);
+    const float descale_lane = __uint_as_float((uint32_t)(127 - E) << 23);
     {
       uint32_t ev[8], od[8];
 #pragma unroll
@@ -525,6 +532,9 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
 #pragma unroll
           for (int q = 0; q < 4; ++q) run[q] = fmaf((float)r.cf[t][COEFS - 1][q], xh, run[q]);
         }
+        const float descale = lane_f(descale_lane, 16 * t);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { tot[q] = fmaf(run[q], descale, tot[q]); run[q] = 0.f; }
         continue;
       }
       // digit sums of the quad (register i: digit i), in units of 2^-10, identical in all lanes
@@ -550,9 +560,10 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
         for (int q = 0; q < 4; ++q) run[q] = fmaf((float)r.cf[t][s][q], whole(acc[q], h0), run[q]);
       }
     }
-    const float descale = __uint_as_float((uint32_t)(127 - E) << 23);
+    if (!GROUPED) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) tot[q] = fmaf(run[q], descale, tot[q]);
+      for (int q = 0; q < 4; ++q) tot[q] = fmaf(run[q], descale_lane, tot[q]);
+    }
     // the digits of this round are consumed before the next round overwrites them
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();

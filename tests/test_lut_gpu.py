@@ -78,6 +78,27 @@ def test_ordinary_and_fine_splits(hq, oracle, tunable, split, K, N, nb, group):
     assert rel_err(_run(hq, bW, alpha, None, x, group), oracle.lut_gemv_f64(bW, alpha, None, x, group), FLOOR_F16) <= 2e-3
 
 
+@pytest.mark.parametrize("split", [1, 2])
+@pytest.mark.parametrize("nb,group", [(1, 32), (3, 64), (4, 32), (5, 64), (6, 32), (8, 64)])
+def test_outlier_in_another_quad(hq, oracle, tunable, split, nb, group):
+    """Groups of 64 and 32: an outlier of 4096 sigma takes low bits from the 128 activations of its own quad, whose weights count
+    nothing here, and from no others (with one scale for a wave's four quads it left two bits of them).  The bound is the one
+    the problems without an outlier meet."""
+    tunable("HQ_LUT_KSPLIT", split)
+    K, N = 4096, 130
+    bW, alpha, qbias, x = oa.make_lut_problem(300 + nb, K, N, nb, group, False)
+    alpha, qbias, x = alpha.copy(), qbias.copy(), x.copy()
+    per_quad = 128 // group
+    for q in range(0, K // 128, 8):                 # one of every eight quads, at another place of a wave's round each time
+        at = q + (q // 8) % 4
+        x[128 * at + 17] = np.float16(4096.0)
+        alpha[at * per_quad:(at + 1) * per_quad] = 0
+        qbias[at * per_quad:(at + 1) * per_quad] = 0
+    y = _run(hq, bW, alpha, qbias, x, group)
+    ref = oracle.lut_gemv_f64(bW, alpha, qbias, x, group)
+    assert rel_err(y, ref, FLOOR_F16) <= 2e-3
+
+
 def test_capture_without_a_workspace(hq, oracle):
     """A split of K needs the stream's workspace; under capture, where none can be allocated, the call runs unsplit."""
     import torch
