@@ -20,24 +20,31 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 //    ((2j+1) << (8-k)) - 1), the nodes one level touches are contiguous in LDS, so lanes on
 //    different nodes hit different banks instead of a few banks 2^(8-k) entries apart;
 //  * the bounds the reference tracks on the way down are, at the leaf p, always the
-//    neighbours p+1 (the nearest ancestor above; entry 255 when p = 254) and max(p-1, 0)
-//    (the nearest ancestor below), so they need not be tracked, only looked up at the end.
-// lds: [0..254] level order, [256..511] the table in index order.
+//    neighbours p+1 (the nearest ancestor above; entry 255 when p = 254) and p-1
+//    (the nearest ancestor below; none when p = 0), so they need not be tracked: the leaf's two midpoints
+//    lie next to each other.
+// lds: [0..254] level order, [256] minus infinity, [257 + i] midpoint of entries i and i + 1.
+// j4: four times the node's number in its level, the byte offset of its entry.
+__device__ __forceinline__ float level_entry(const float* lds, int k, uint32_t j4) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(lds + (1u << k) - 1) + j4);
+}
+__device__ __forceinline__ uint32_t next_node(uint32_t j4, float x, float val) { return (j4 << 1) | (x > val ? 4u : 0u); }
+// The leaf's decision, by selects: with branches on the side of x the lanes of a wave took all of them in turn.
+__device__ __forceinline__ uint32_t leaf_code(const float* lds, uint32_t j4, float val, float x) {
+  const float2 mid = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(lds + 256) + 2 * j4);
+  const bool up = x > val;
+  // ties keep the pivot (strict comparisons, src/quantBnB-hip/main.cu:47-65)
+  return (j4 >> 1) + ((up & (x > mid.y)) ? 1u : 0u) - ((!up & (x < mid.x)) ? 1u : 0u);
+}
 __device__ __forceinline__ uint32_t quantize_one(const float* lds, float x) {
-  uint32_t j = 0;
+  uint32_t j4 = 0;
   float val = lds[0];
 #pragma unroll
   for (int k = 1; k < 8; ++k) {
-    j = 2 * j + (x > val ? 1u : 0u);
-    val = lds[(1u << k) - 1 + j];
+    j4 = next_node(j4, x, val);
+    val = level_entry(lds, k, j4);
   }
-  const uint32_t pivot = 2 * j;  // leaf index = table index
-  const bool up = x > val;
-  const uint32_t other = up ? pivot + 1 : (pivot == 0 ? 0u : pivot - 1);
-  const float bound = lds[256 + other];
-  const float midpoint = (bound + val) * 0.5f;
-  // ties keep the pivot (strict comparisons, src/quantBnB-hip/main.cu:47-65)
-  return (up ? x > midpoint : x < midpoint) ? other : pivot;
+  return leaf_code(lds, j4, val, x);
 }
 
 // ---- fast path for a sorted table ---------------------------------------------------------------
@@ -145,11 +152,11 @@ constexpr int kAhead = 2;  // 16-byte loads of a thread and step: 64 KB of a ste
 // operations and one random 8-byte LDS read per element.  A thread takes every gridDim.x * 1024-th quad; its first loads
 // are in flight while the tables are built, and a step's go out together while the step before is converted (one by one
 // as registers come free: 118 against 109 us at 2^27; four per thread: 118).
-// us per call, before -> now: 2^16 elements 4.43 -> 4.20, 2^22 8.2 -> 7.8, 10^7 11.8 -> 11.4, 2^24 16.8 -> 16.5, 2^27
+// us per call, before -> now: 2^16 elements 4.43 -> 4.20, 2^22 8.2 -> 7.8, 10^7 11.8 -> 10.9, 2^24 16.8 -> 16.5, 2^27
 // 109.7 -> 108.6 (6.2 TB/s).
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void quantize8_kernel(
     const float* __restrict__ code, const float* __restrict__ A, uint8_t* __restrict__ out, int64_t n, int vec_ok, int allow_fast) {
-  __shared__ float s_code[512];
+  __shared__ __align__(16) float s_code[512];
   __shared__ __align__(16) FastTables ft;
   const int t = threadIdx.x;
   const int64_t nquads = vec_ok ? n / 4 : 0;
@@ -170,7 +177,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))
   __builtin_amdgcn_sched_barrier(0);
   if (t < 256) {
     s_code[t] = ordered;  // level-order slot t: entry ((2j+1) << (8-k)) - 1
-    s_code[256 + t] = ct;
+    s_code[t < 255 ? 257 + t : 256] = t < 255 ? (cn + ct) * 0.5f : -__builtin_inff();
   }
   // the fast path wants a sorted table of finite, moderate values (midpoints cannot overflow) with a
   // usable magnitude
@@ -218,32 +225,44 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))
       for (int k = 0; k < kAhead; ++k) v[k] = vn[k];
     }
   } else {
-    __syncthreads();
-    // The descent for four elements at a time, level by level: four independent LDS reads are in flight per level instead
-    // of one dependent chain per element.
-    for (int64_t i = t0; i < nquads; i += stride) {
-      const f4v v0 = load(i);
-      const float x[4] = {v0.x, v0.y, v0.z, v0.w};
-      uint32_t j[4], q[4];
-      float val[4];
+    // The descent for a quad's four elements at a time, level by level: four independent LDS reads are in flight per level
+    // instead of one dependent chain per element, the next step's loads run under them.  Vector instructions bound it,
+    // three per level, and close behind the LDS reads.  Unsorted table, us per call, five workgroups of 256 threads with
+    // eight elements in lockstep / 1024 threads, four elements and a branch on the leaf's side / this: 2^22 elements
+    // 8.8 / 10.9 / 8.6, 10^7 16.9 / 18.9 / 14.8, 2^24 25.4 / 26.8 / 20.8, 2^27 275 / 214 / 152 (eight elements spill here:
+    // 10^7 20.2).
+    const int64_t wave0 = t0 - (t & 63);
+    for (int64_t step = 0; wave0 + step < nquads; step += kAhead * stride) {
+      f4v vn[kAhead];
+      if (wave0 + step + kAhead * stride < nquads) {  // wave-uniform
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { j[e] = 0; val[e] = s_code[0]; }
+        for (int k = 0; k < kAhead; ++k) vn[k] = load(t0 + step + (kAhead + k) * stride);
+      }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 1; k < 8; ++k) {
+      for (int k = 0; k < kAhead; ++k) {
+        const int64_t i = t0 + step + k * stride;
+        if (wave0 + step + k * stride >= nquads) break;  // wave-uniform
+        const float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+        uint32_t j4[4], q[4];
+        float val[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) j[e] = 2 * j[e] + (x[e] > val[e] ? 1u : 0u);
+        for (int e = 0; e < 4; ++e) { j4[e] = 0; val[e] = s_code[0]; }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) val[e] = s_code[(1u << k) - 1 + j[e]];
+        for (int l = 1; l < 8; ++l) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) j4[e] = next_node(j4[e], x[e], val[e]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) val[e] = level_entry(s_code, l, j4[e]);
+          __builtin_amdgcn_sched_barrier(0);  // the compiler would descend one element after the other to save registers
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = leaf_code(s_code, j4[e], val[e], x[e]);
+        if (i < nquads)
+          __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), reinterpret_cast<uint32_t*>(out) + i);
       }
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool up = x[e] > val[e];
-        const uint32_t pivot = 2 * j[e];
-        const uint32_t other = up ? pivot + 1 : (pivot == 0 ? 0u : pivot - 1);
-        const float midpoint = (s_code[256 + other] + val[e]) * 0.5f;
-        q[e] = (up ? x[e] > midpoint : x[e] < midpoint) ? other : pivot;
-      }
-      __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), reinterpret_cast<uint32_t*>(out) + i);
+      for (int k = 0; k < kAhead; ++k) v[k] = vn[k];
     }
   }
   for (int64_t e = nquads * 4 + t0; e < n; e += stride) out[e] = (uint8_t)quantize_one(s_code, A[e]);

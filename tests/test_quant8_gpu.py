@@ -131,3 +131,15 @@ def test_ends_of_the_grid(hq, oracle, n):
     special = np.array([np.nan, np.inf, -np.inf, 0.0, -0.0, 5.0, -5.0, 1e-45], np.float32)
     A[-8:] = special[:n]
     assert np.array_equal(_run(hq, code, A), oracle.quantize_dynamic8(code, A))
+
+
+@pytest.mark.parametrize("n", [1, 5, 4096 + 4, 262144 * 4 + 260, 2 * 1048576 * 4 + 36, (5 << 20) + 4097])
+def test_ends_of_the_grid_of_an_unsorted_table(hq, oracle, n):
+    """The tree descent at the same lengths: a step of one quad and of two, the next step's loads under one and none behind
+    the last, special values at the ends."""
+    rng = np.random.default_rng(n)
+    code = rng.permutation(oracle.dynamic_map())
+    A = (rng.standard_normal(n) * 0.2).astype(np.float32)
+    special = np.array([np.nan, np.inf, -np.inf, 0.0, -0.0, code[0], code[255], 1e-45], np.float32)
+    A[-8:] = special[:n]
+    assert np.array_equal(_run(hq, code, A), oracle.quantize_dynamic8(code, A))
