@@ -59,7 +59,7 @@ struct Shape {
 // for every load in flight before the first LDS read behind one; the waits are the loop's own.
 __device__ __forceinline__ void load_lds(uint32_t lds, uint32_t voff, const void* base) {
   lds = __builtin_amdgcn_readfirstlane(lds);  // wave-uniform, whatever registers the compiler computed it in
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_loads_and_meet() {
