@@ -104,13 +104,30 @@ void same_device(const at::Tensor* first, T... rest) {
 }
 
 int64_t integer(PyObject* o) {
-  const long long v = PyLong_AsLongLong(o);
+  int overflow = 0;
+  const long long v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  if (overflow) value_error("an integer argument is out of range");
   if (v == -1 && PyErr_Occurred()) throw python_error();
   return v;
 }
 int small_integer(PyObject* o, const char* name) {
   const int64_t v = integer(o);
   if (v < INT_MIN || v > INT_MAX) value_error(std::string(name) + " is out of range");
+  return (int)v;
+}
+// A 32-bit value by its low bits, as a C cast takes it: any integer is accepted.
+int low_bits(PyObject* o) {
+  const unsigned long long v = PyLong_AsUnsignedLongLongMask(o);
+  if (v == (unsigned long long)-1 && PyErr_Occurred()) throw python_error();
+  return (int)(unsigned)v;
+}
+// A bound that is compared with 32-bit numbers: beyond their range the nearest of them compares alike.
+int bound(PyObject* o) {
+  int overflow = 0;
+  const long long v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  if (v == -1 && !overflow && PyErr_Occurred()) throw python_error();
+  if (overflow > 0 || v > INT_MAX) return INT_MAX;
+  if (overflow < 0 || v < INT_MIN) return INT_MIN;
   return (int)v;
 }
 // problem sizes are C ints at the boundary
@@ -206,7 +223,7 @@ PyObject* q3_gemm(PyObject* const* a) {  // A, qweight, scales, zeros, out
 
 PyObject* dequant_4bit(PyObject* const* a) {  // packed, absmax, n_elems, blocksize, table, out
   const int64_t n = integer(a[2]);
-  const int bs = small_integer(a[3], "blocksize"), table = small_integer(a[4], "table");
+  const int bs = small_integer(a[3], "blocksize"), table = low_bits(a[4]);
   if (n < 0 || bs <= 0) value_error("n_elems must be >= 0 and blocksize > 0");
   const at::Tensor* p = tensor(a[0], "packed", kU8, n / 2 + (n & 1));
   const at::Tensor* am = tensor(a[1], "absmax", kF32, n / bs + (n % bs != 0));
@@ -220,7 +237,7 @@ PyObject* dequant_4bit(PyObject* const* a) {  // packed, absmax, n_elems, blocks
 
 PyObject* quantize_4bit(PyObject* const* a) {  // x, blocksize, table
   const at::Tensor* x = tensor(a[0], "x", kF32 | kF16);
-  const int bs = small_integer(a[1], "blocksize"), table = small_integer(a[2], "table");
+  const int bs = small_integer(a[1], "blocksize"), table = low_bits(a[2]);
   if (bs <= 0) value_error("blocksize must be > 0");
   same_device(x);
   const int64_t n = x->numel();
@@ -274,11 +291,12 @@ PyObject* code1x16_matvec(PyObject* const* a) {  // codes, x, codebooks, codeboo
   if (!bounds) throw python_error();
   if (PySequence_Fast_GET_SIZE(bounds.get()) != 4) value_error("codebook_a_sizes must hold four row bounds");
   int sizes[4];
-  for (int j = 0; j < 4; ++j) sizes[j] = small_integer(PySequence_Fast_GET_ITEM(bounds.get(), j), "codebook_a_sizes");
-  const int stride = small_integer(a[4], "codebook_stride_int4");
+  for (int j = 0; j < 4; ++j) sizes[j] = bound(PySequence_Fast_GET_ITEM(bounds.get(), j));
   int ncb = 0;  // code book of the last row: the first j with M-1 < codebook_a_sizes[j]
   while (ncb < 3 && M - 1 >= sizes[ncb]) ++ncb;
   ++ncb;
+  // one code book: no row goes by the stride
+  const int stride = ncb == 1 ? low_bits(a[4]) : small_integer(a[4], "codebook_stride_int4");
   const at::Tensor* cb = tensor(a[2], "codebooks", kF16);
   if (cb->numel() < (int64_t)(ncb - 1) * stride * 8 + 65536 * 8)
     value_error("codebooks too small for " + std::to_string(ncb) + " code book(s) of 65536 x 8 halves at the given stride");
@@ -325,7 +343,7 @@ PyObject* int8_quant_static(PyObject* const* a) {  // x, scale, azp, out
   same_device(x, o);
   const float scale = real(a[1]);
   const bool has_azp = a[2] != Py_None;
-  const int azp = has_azp ? small_integer(a[2], "azp") : 0;
+  const int azp = has_azp ? low_bits(a[2]) : 0;
   const int64_t tokens = x->size(0), hidden = x->size(1);
   Result r(a[3], o, *x, {tokens, hidden}, ScalarType::Char);
   const int h = size_of(hidden);

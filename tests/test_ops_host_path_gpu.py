@@ -51,3 +51,17 @@ def test_current_stream(hq):
         y = hq.q3_matvec(late, w, s, z)
     side.synchronize()
     assert torch.equal(y, want)
+
+
+def test_integers_beyond_32_bits(hq):
+    """A zero point counts by its low 32 bits; a code book's row bound beyond them holds for every row."""
+    dev = torch.device("cuda:0")
+    x = torch.randn(4, 64, device=dev)
+    assert torch.equal(hq.static_scaled_int8_quant(x, 0.05, 2 ** 32 + 7), hq.static_scaled_int8_quant(x, 0.05, 7))
+    assert torch.equal(hq.static_scaled_int8_quant(x, 0.05, -2 ** 63 - 3), hq.static_scaled_int8_quant(x, 0.05, -3))
+    codes = torch.randint(-2 ** 15, 2 ** 15, (16, 8), dtype=torch.int16, device=dev)
+    v, cb = torch.randn(64, device=dev).half(), torch.randn(2, 65536, 8, device=dev).half()
+    assert torch.equal(hq.code1x16_matvec(codes, v, cb, (2 ** 32 + 5, 0, 0, 0), 65536),
+                       hq.code1x16_matvec(codes, v, cb, (16, 0, 0, 0), 65536))
+    assert torch.equal(hq.code1x16_matvec(codes, v, cb, (5, 2 ** 40, 0, 0), 65536),
+                       hq.code1x16_matvec(codes, v, cb, (5, 16, 0, 0), 65536))

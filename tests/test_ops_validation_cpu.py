@@ -116,3 +116,20 @@ def test_gemv_and_int8_checks():
         hq.mxfp4_qdq(torch.zeros(64))
     with pytest.raises(ValueError, match="device tensors only"):
         hq.mxfp4_qdq(torch.zeros(64, dtype=torch.float16))
+
+
+def test_integers_beyond_32_bits_are_taken_as_before():
+    """Row bounds beyond 32 bits mean what they say; table numbers, and the stride where there is one code book, count by their
+    low 32 bits, as a C call takes them.  All of it ends at the device check; sizes that no tensor has are a ValueError."""
+    codes, x = torch.zeros((16, 8), dtype=torch.int16), torch.zeros(64, dtype=torch.float16)
+    cb = torch.zeros((2, 65536, 8), dtype=torch.float16)
+    for bounds, stride in (((2 ** 32 + 5, 0, 0, 0), 65536), ((2 ** 70, 0, 0, 0), 65536), ((-2 ** 40, 2 ** 40, 0, 0), 65536),
+                           ((16, 0, 0, 0), 2 ** 33 + 65536)):
+        with pytest.raises(ValueError, match="device tensors only"):
+            hq.code1x16_matvec(codes, x, cb, bounds, stride)
+    with pytest.raises(ValueError, match="device tensors only"):
+        hq.dequant_4bit(torch.zeros(32, dtype=torch.uint8), torch.zeros(1), 64, 64, 2 ** 32)
+    with pytest.raises(ValueError, match="device tensors only"):
+        hq.quantize_4bit(torch.zeros(64), 64, 2 ** 32 + 1)
+    with pytest.raises(ValueError):
+        hq.dequant_4bit(torch.zeros(32, dtype=torch.uint8), torch.zeros(1), 2 ** 64, 64)
