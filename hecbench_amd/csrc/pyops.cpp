@@ -292,8 +292,8 @@ PyObject* code1x16_matvec(PyObject* const* a) {  // codes, x, codebooks, codeboo
   if (PySequence_Fast_GET_SIZE(bounds.get()) != 4) value_error("codebook_a_sizes must hold four row bounds");
   int sizes[4];
   for (int j = 0; j < 4; ++j) sizes[j] = bound(PySequence_Fast_GET_ITEM(bounds.get(), j));
-  int ncb = 0;  // code book of the last row: the first j with M-1 < codebook_a_sizes[j]
-  while (ncb < 3 && M - 1 >= sizes[ncb]) ++ncb;
+  int ncb = 0;  // code book of the last row: the first j with M-1 < codebook_a_sizes[j], the fifth where there is none
+  while (ncb < 4 && M - 1 >= sizes[ncb]) ++ncb;
   ++ncb;
   // one code book: no row goes by the stride
   const int stride = ncb == 1 ? low_bits(a[4]) : small_integer(a[4], "codebook_stride_int4");

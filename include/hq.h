@@ -225,7 +225,7 @@ int hq_lut_gemv_plan(const uint32_t* bW, const void* alpha_fp16, const void* q_b
  *   y[m] = fp16_rn( scale[m] * sum_g dot8(codebook[cb(m)][u16(codes[m][g])], x[8g..8g+7]) )
  * codes int16[M][K/8] (read as unsigned), codebooks fp16[..][65536][8] with
  * consecutive code books codebook_stride_int4*16 bytes apart, cb(m) = first j
- * with m < codebook_a_sizes[j].  scales_fp16 may be NULL (the reference kernel
+ * with m < codebook_a_sizes[j] (4 where there is none).  scales_fp16 may be NULL (the reference kernel
  * applies no scale).  K % 64 == 0 (as in the reference).  fp32 accumulation, one rounding.  Replaces
  * code1x16_matvec, src/quantAQLM-hip/main.cu:103-139 (without its internal
  * synchronisation, timing and printing).

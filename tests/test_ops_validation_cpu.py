@@ -133,3 +133,13 @@ def test_integers_beyond_32_bits_are_taken_as_before():
         hq.quantize_4bit(torch.zeros(64), 64, 2 ** 32 + 1)
     with pytest.raises(ValueError):
         hq.dequant_4bit(torch.zeros(32, dtype=torch.uint8), torch.zeros(1), 2 ** 64, 64)
+
+
+def test_rows_beyond_every_bound_need_a_fifth_code_book():
+    """As in the reference kernel, a row beyond all four bounds reads the code book behind the fourth."""
+    codes, x = torch.zeros((16, 8), dtype=torch.int16), torch.zeros(64, dtype=torch.float16)
+    with pytest.raises(ValueError, match="codebooks too small for 5"):
+        hq.code1x16_matvec(codes, x, torch.zeros((4, 65536, 8), dtype=torch.float16), (4, 8, 12, 14), 65536)
+    for books, bounds in ((5, (4, 8, 12, 14)), (4, (4, 8, 12, 16))):
+        with pytest.raises(ValueError, match="device tensors only"):
+            hq.code1x16_matvec(codes, x, torch.zeros((books, 65536, 8), dtype=torch.float16), bounds, 65536)
