@@ -82,22 +82,28 @@ def load():
 
 
 def native_ops():
-    """The module of the operators' host path (csrc/pyops.cpp, linked against libhq.so).  Where it is not built, an
-    object that raises at the first operator call, as load() does: importing the package needs no build."""
+    """The module of the operators' host path (csrc/pyops.cpp, linked against libhq.so).  Where it is not built, or cannot be
+    loaded (built against another torch), an object that raises at the first operator call, as load() does: importing the
+    package needs no build."""
+    reason = f"{OPS_PATH} is not built"
+    cause = None
     if os.path.exists(OPS_PATH):
         import importlib.util
 
         import torch  # noqa: F401  (its libraries are what the module is linked against)
         spec = importlib.util.spec_from_file_location("hecbench_amd._ops", OPS_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        return module
+        try:
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            return module
+        except ImportError as e:
+            reason, cause = f"{OPS_PATH} cannot be loaded ({e})", e
 
-    class NotBuilt:
+    class NotThere:
         def __getattr__(self, name):
-            raise ImportError(f"{OPS_PATH} is not built; run `python -m hecbench_amd.build` (needs hipcc)")
+            raise ImportError(f"{reason}; run `python -m hecbench_amd.build` (needs hipcc)") from cause
 
-    return NotBuilt()
+    return NotThere()
 
 
 class HqError(RuntimeError):

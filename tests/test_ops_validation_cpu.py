@@ -143,3 +143,16 @@ def test_rows_beyond_every_bound_need_a_fifth_code_book():
     for books, bounds in ((5, (4, 8, 12, 14)), (4, (4, 8, 12, 16))):
         with pytest.raises(ValueError, match="device tensors only"):
             hq.code1x16_matvec(codes, x, torch.zeros((books, 65536, 8), dtype=torch.float16), bounds, 65536)
+
+
+@pytest.mark.parametrize("content", [None, b"not a library", b"\x7fELF" + bytes(60)])
+def test_a_host_path_that_cannot_be_loaded_raises_at_the_first_call(tmp_path, monkeypatch, content):
+    """Missing, or built for something else (the loader refuses the file): the package imports, an operator call says why."""
+    from hecbench_amd import _lib
+    path = tmp_path / "_ops.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_lib, "OPS_PATH", str(path))
+    native = _lib.native_ops()
+    with pytest.raises(ImportError, match="not built" if content is None else "cannot be loaded"):
+        native.q3_matvec(None, None, None, None, None, False)
