@@ -72,7 +72,8 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, con
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = (SPLIT ? blk : blk * 4 + wv) * ROWS;
   const int chunk0 = SPLIT ? wv * 64 : 0, step = SPLIT ? 256 : 64;  // units: this wave's first chunk, and to its next
-  if (!XLDS && !SPLIT && row0 >= a.M) return;  // wave-uniform (SPLIT: never)
+  static_assert(XLDS || !SPLIT, "shared rows take their activations from LDS");
+  if (!XLDS && row0 >= a.M) return;  // wave-uniform
   const int units_per_row = a.K >> 6;         // 16-byte code units (8 codes) per row; K % 64 == 0
   extern __shared__ u4v xl[];
   const int xstride = aqlm_x_stride(units_per_row);
@@ -171,10 +172,12 @@ extern "C" int hq_aqlm_matvec(const int16_t* codes, const void* codebooks, const
   // What counts is gathers in flight and evenly over the compute units.  Measured (us, one / two / four rows per wave; one / two
   // split): 4096 x 4096 11.7 12.4 12.8; 13.3 12.9 - 9788 x 5440 31.3 30.9 33.1; 34.2 33.0 - 28672 x 4096 three code books 62.0 61.1
   // 62.9; 71.9 68.2 - 28672 x 16384 291 239 237; 271 248 - 1228 x 16192 25.1 23.2 39.6; 17.1 16.6 - 2472 x 11968 24.9 27.1 27.2;
-  // 21.9 20.2 - 512 x 16384 12.3 17.3 28.7; 9.4 9.4 - 689 x 5184 6.8 9.1 15; 6.3 6.5.  HQ_AQLM_ROWS: 1, 2, 4; 11, 12 split.
+  // 21.9 20.2 - 512 x 16384 12.3 17.3 28.7; 9.4 9.4 - 689 x 5184 6.8 9.1 15; 6.3 6.5.  HQ_AQLM_ROWS: 1, 2, 4; 11, 12 split
+  // (rows that go through LDS only: sharing longer ones was never the choice).
   int rows = hq_tune(HQ_TUNE_AQLM_ROWS, 0);
   bool split = rows == 11 || rows == 12;
   if (split) rows -= 10;
+  split = split && K <= kMaxLdsK;
   if (rows != 1 && rows != 2 && rows != 4) {
     const long waves_wanted = (long)dev->cus * 8;
     if (K > kMaxLdsK) rows = M >= 4 * waves_wanted ? 4 : (M >= 2 * waves_wanted ? 2 : 1);
@@ -190,13 +193,13 @@ extern "C" int hq_aqlm_matvec(const int16_t* codes, const void* codebooks, const
 #define HQ_AQLM_GO(R, L, S)                                                                                                \
   hipLaunchKernelGGL((aqlm_matvec_kernel<R, L, S>), dim3(blocks), dim3(256), smem, stream, a.codes, a.codebooks, a.x, a.M, \
                      a.K, a.cb_stride, a.cb_sizes[0], a.cb_sizes[1], a.cb_sizes[2], a.cb_sizes[3], a.scales, a.y)
-#define HQ_AQLM_ROWS_GO(R, S) \
-  { if (lds) HQ_AQLM_GO(R, true, S); else HQ_AQLM_GO(R, false, S); }
-  if (rows == 4) HQ_AQLM_ROWS_GO(4, false)
-  else if (rows == 2 && split) HQ_AQLM_ROWS_GO(2, true)
-  else if (rows == 2) HQ_AQLM_ROWS_GO(2, false)
-  else if (split) HQ_AQLM_ROWS_GO(1, true)
-  else HQ_AQLM_ROWS_GO(1, false)
+#define HQ_AQLM_ROWS_GO(R) \
+  { if (lds) HQ_AQLM_GO(R, true, false); else HQ_AQLM_GO(R, false, false); }
+  if (rows == 4) HQ_AQLM_ROWS_GO(4)
+  else if (rows == 2 && split) HQ_AQLM_GO(2, true, true);
+  else if (rows == 2) HQ_AQLM_ROWS_GO(2)
+  else if (split) HQ_AQLM_GO(1, true, true);
+  else HQ_AQLM_ROWS_GO(1)
 #undef HQ_AQLM_ROWS_GO
 #undef HQ_AQLM_GO
   return hq_launch_status();

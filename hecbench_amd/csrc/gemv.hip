@@ -441,7 +441,7 @@ int launch_gemv(const void* mat, const void* vec, void* res, int rows, int n, fl
   // Rows cut across the waves of a workgroup: fp16 rows of 8192 elements or more, two steps of two rows per
   // wave (16384 x 16384: 88.7 -> 75.7 us = 7.1 TB/s; 28672 x 8192 70.5 -> 64.3, a column slice per wave 68.7; 8192 x 28672
   // 73.8 -> 66.8; 4096 x 16384 23.0 -> 21.0).  Other step counts per wave are worse, some much (four steps, i.e. waves that
-  // start 4 KB apart: 97.5 us at 16384 x 16384).  HQ_GEMV_SPLIT: 0 never, 1 / 2 a column slice and eight / four rows per wave,
+  // start 4 KB apart: 97.5 us at 16384 x 16384).  HQ_GEMV_SPLIT: 0 never, 1 / 2 a column slice and eight (fp16 four) / four rows per wave,
   // 4 / 8 / 16 that many waves per pair of rows, unset: these rules.
   // Longer rows: the LDS kernel pays where a wave loads as many bytes of the vector as of the matrix and walks over several
   // row groups, int4 with four rows per wave; fp16 and int8 gain on some shapes and lose on others (fp16 16384 x 16384 88.7 -> 83.0
@@ -458,7 +458,8 @@ int launch_gemv(const void* mat, const void* vec, void* res, int rows, int n, fl
     }
     if ((split == 1 || split == 2) && units <= 1024) {
       const dim3 block(waves * 64);
-      if (split == 1) hipLaunchKernelGGL((gemv_columns_kernel<MODE, 8>), dim3((rows + 7) / 8), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
+      constexpr int kMost = MODE == kF16 ? 4 : 8;
+      if (split == 1) hipLaunchKernelGGL((gemv_columns_kernel<MODE, kMost>), dim3((rows + kMost - 1) / kMost), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
       else hipLaunchKernelGGL((gemv_columns_kernel<MODE, 4>), dim3((rows + 3) / 4), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
       return hq_launch_status();
     }
