@@ -57,10 +57,13 @@ struct Shape {
 
 // 64 lanes x 16 bytes from base + voff (per lane) to LDS bytes lds .. lds + 1023.  Assembly, as the compiler would wait
 // for every load in flight before the first LDS read behind one; the waits are the loop's own.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // that m0 is the compiler's own is why it is listed
 __device__ __forceinline__ void load_lds(uint32_t lds, uint32_t voff, const void* base) {
   lds = __builtin_amdgcn_readfirstlane(lds);  // wave-uniform, whatever registers the compiler computed it in
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 template <int N>
 __device__ __forceinline__ void wait_loads_and_meet() {
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
