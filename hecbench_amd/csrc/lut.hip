@@ -687,8 +687,7 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
     const float costs = parts == 1 ? 0.f : (nsplit == 1 ? 1.4f : 0.f) + 0.16f * (parts - nsplit);
     fine = (int64_t)ntiles * parts <= 2 * cus && saves > costs;
     if (ntiles > cus && ntiles * 8 <= cus * 11 && rpw > 1 && parts <= 5) fine = true;
-    const int force = hq_tune(HQ_TUNE_LUT_KSPLIT, 0);  // tests: 1 ordinary, 2 fine
-    if (force > 0) fine = force == 2;
+    fine = hq_tune(HQ_TUNE_LUT_FINE, fine) != 0;
   }
   if (fine) nsplit = parts;
   if (nsplit > 1 && hq_workspace_out_of_reach(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles)) nsplit = 1;

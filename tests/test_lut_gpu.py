@@ -69,7 +69,7 @@ def test_k_split_of_the_plane_kernel(hq, oracle, tunable, K, N, nb):
 def test_ordinary_and_fine_splits(hq, oracle, tunable, split, K, N, nb, group):
     """One quad per wave with a workgroup per round, and several quads per wave: every plane count's kind, either group size,
     K of less than a round, of one and of several with a rest."""
-    tunable("HQ_LUT_KSPLIT", split)
+    tunable("HQ_LUT_FINE", split - 1)
     bW, alpha, qbias, x = oa.make_lut_problem(K + N + nb, K, N, nb, group, False)
     y = _run(hq, bW, alpha, qbias, x, group)
     ref = oracle.lut_gemv_f64(bW, alpha, qbias, x, group)
@@ -84,7 +84,7 @@ def test_outlier_in_another_quad(hq, oracle, tunable, split, nb, group):
     """Groups of 64 and 32: an outlier of 4096 sigma takes low bits from the 128 activations of its own quad, whose weights count
     nothing here, and from no others (with one scale for a wave's four quads it left two bits of them).  The bound is the one
     the problems without an outlier meet."""
-    tunable("HQ_LUT_KSPLIT", split)
+    tunable("HQ_LUT_FINE", split - 1)
     K, N = 4096, 130
     bW, alpha, qbias, x = oa.make_lut_problem(300 + nb, K, N, nb, group, False)
     alpha, qbias, x = alpha.copy(), qbias.copy(), x.copy()
