@@ -34,8 +34,9 @@ def test_kinds_and_shares(hq, oracle, tunable, kind, shares, M, K, N):
     codes, scales, zeros, A = oa.make_q3_problem(M + K + N, K, N, x_dtype=np.float16, batch=M)
     A[5] *= np.float16(2.0 ** -10)     # rows of other magnitudes, a zero row, an outlier
     A[7] = 0
-    # An outlier at k = 3 of its k-group.  (At k = 0 the matrix instruction's own sum of sixteen products loses 2^-16 of
-    # the outlier's product: 1.2e-4 of such a row's RMS, here and in the 64-row kernel bit for bit alike.)
+    # An outlier at k = 3 of its k-group, whose code lies at bit 5 of its operand: what the matrix instruction cuts off the
+    # products next to it is 2^-5 of what it cuts at k = 0, where 1e-4 of such a row's RMS does not hold (the bound that holds
+    # at every k, here and in the 64-row kernel: test_outlier_at_any_code).
     A[9, K // 64 * 32 + 3] = np.float16(4096.0)
     mat = oracle.q3_pack(codes)
     tunable("HQ_Q3_TILES", kind + 10 * shares)
@@ -44,6 +45,24 @@ def test_kinds_and_shares(hq, oracle, tunable, kind, shares, M, K, N):
     assert np.array_equal(y.cpu().numpy(), again.cpu().numpy())  # shares are added in a fixed order
     exact = oracle.q3_gemm(A, mat, scales, zeros, mode=0)
     _check(y.cpu().numpy(), exact)
+
+
+@pytest.mark.parametrize("M,K,N", [(40, 2080, 516), (64, 8192, 132), (129, 2080, 260), (300, 1024, 1028)])
+@pytest.mark.parametrize("k,pos", [(0, 0), (19, 0), (29, 0), (14, 1), (3, 5)])
+@pytest.mark.parametrize("amp", [64.0, 4096.0, -60000.0])
+def test_outlier_at_any_code(hq, oracle, tunable, M, K, N, k, pos, amp):
+    """What an outlier costs its row, in the 64-row kernel and in the tiles.  A code at bit pos of its operand is a subnormal
+    number: the matrix instruction aligns its product as if the code were 2^(10 - pos), and cuts the other fifteen products and
+    the sum so far below the 24th bit of that: 17 cuts of at most 2^(10 - pos) * 2^-24 of the outlier's power of two, times the
+    column's scale (seen: a quarter of that).  The rest of the row: 1e-5 of its RMS."""
+    tunable("HQ_Q3_SMALL_BATCH", 0)
+    codes, scales, zeros, A = oa.make_q3_problem(M + K + N, K, N, x_dtype=np.float16, batch=M)
+    A[9, K // 64 * 32 + k] = np.float16(amp)
+    mat = oracle.q3_pack(codes)
+    y = hq.q3_gemm(_t(A), _t(mat), _t(scales), _t(zeros)).cpu().numpy()[9].astype(np.float64)
+    exact = oracle.q3_gemm(A[9:10], mat, scales, zeros, mode=0)[0]
+    cut = 2.0 ** (np.floor(np.log2(abs(amp))) + 10 - pos - 24)
+    assert np.all(np.abs(y - exact) <= 17 * cut * scales + 1e-5 * np.sqrt(np.mean(exact ** 2)))
 
 
 @pytest.mark.parametrize("M,K,N", [(100, 4096, 4096), (700, 512, 3000), (1030, 16416, 8), (70, 256, 8200)])
