@@ -180,7 +180,8 @@ int hq_q3_matvec_plan(int K, int N, int batch_M);
  * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results, but the
  * scratch the kernels need (split-K partial sums and arrival counters of batches 1 and 2, the batched
  * path's re-ordered activations, row sums, row scales and K-split sums) is a fixed 68 MiB + 128 KiB array in device
- * memory that each GPU holds from library load to process end, instead of the stream's workspace.
+ * memory that each GPU holds from library load to process end, instead of the stream's workspace (the runtime clears it
+ * when it loads the library onto a GPU: about 25 ms of the first hq_init).
  * The call runs no hipMalloc, hipFree or allocating library routine.  Limits: a batch that the MFMA
  * GEMM serves (hq_q3_matvec_plan) needs K <= 16384; a split-K matvec needs tiles * splits * batch_M <= 8192 (the one-per-round split falls
  * back to one workgroup per compute unit where it would not fit) and N <= 1032192; beyond them

@@ -66,6 +66,18 @@ def test_reserve_is_close_to_the_largest_need(cus, max_K, max_N):
     assert bf <= 1.25 * worst
 
 
+def test_the_array_of_the_call_that_allocates_nothing_holds_every_batch():
+    """hq_q3_matvec_noalloc takes the tiles' plan at every batch as long as its fixed array holds it (68 MiB + 64 KiB, 16128
+    arrival counters; 256 compute units, K <= 16384): there is no batch beyond 64 rows that it does not hold."""
+    lib = _lib.load()
+    rng = random.Random(17)
+    for i in range(20000):
+        K = (16384, 2080, rng.randrange(1, 513) * 32)[i % 3]   # the longest, one that pads much, any
+        N = rng.randrange(1, 16385) * 4
+        f, c = _need(lib, 256, K, N, int(2 ** rng.uniform(6.03, 15)))
+        assert f * 4 <= (68 << 20) + (64 << 10) and c <= 16128, (K, N, f, c)
+
+
 def test_the_case_that_used_to_fall_short():
     # 256 compute units: a reservation for (8192, 28672) must hold M=72, K=8192, N=4096, whose 32 column tiles
     # split K eight ways (re-ordered activations 262,144 floats + 128 + 32 x 8 x 64 x 128 raw sums)
