@@ -71,6 +71,14 @@ int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* count
 void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);
 int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
+float hq_q3_tiles_us(int cus, int K, int N, int M);  // estimate of a call, pre-pass included
+// The same product in one launch (small and medium problems): estimate of a call, a test's override, scratch, launch.  Always able
+// to do without scratch.
+float hq_q3_direct_us(int cus, int K, int N, int M);
+bool hq_q3_direct_forced();
+void hq_q3_direct_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
+int hq_q3_direct_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
+                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
 // Resolves the current device's copy of the fixed scratch array (once per device).
 int hq_noalloc_setup(void);
 

@@ -575,6 +575,18 @@ int q3_block_row_blocks(int cus, int K, int N, int batch_M, int nsplit, int rpw)
   return batch_M <= 12 ? 1 : 0;
 }
 
+// Small launches of more than four rows: row blocks while every workgroup has a compute unit of its own (then 5 to 7 us, ahead of
+// anything else by a quarter), beyond that the one-launch matrix-core kernel of q3_direct.hip.  Workgroups per compute unit that
+// row blocks would need, and both (us): 0.86: 5.3 / 7.3 (26 rows, K=2528, N=1960); 1.04: 6.9 / 6.7 (11 rows, K=1824, N=5640); 1.5: 9.6 /
+// 8.3 (16 rows, K=5120, N=3068); 2.5: 9.9 / 6.8 (12 rows, K=1696, N=13684); 3.7: 14.6 / 8.9 (45 rows, K=3648, N=5028).
+bool q3_block_yields(int cus, int K, int N, int batch_M) {
+  if (hq_q3_direct_forced()) return true;
+  if (batch_M <= 4 || hq_tune(HQ_TUNE_Q3_ROW_BLOCKS, -1) >= 0 || hq_q3_direct_us(cus, K, N, batch_M) > 1e29f) return false;
+  int nsplit, rpw;
+  q3_block_split(cus, K, N, batch_M, &nsplit, &rpw);
+  return (int64_t)((N + 63) / 64) * nsplit * ((batch_M + 3) / 4) > cus;
+}
+
 int q3_plan(int cus, int K, int N, int batch_M) {
   if (batch_M == 1) return HQ_Q3_PLAN_MATVEC;
   const int limit = hq_tune(HQ_TUNE_Q3_SMALL_BATCH, kRowBlockBatchMax);  // 0: every batch takes the GEMM
@@ -756,6 +768,12 @@ int hq_q3_workspace_need_impl(int cus, int K, int N, int batch_M, size_t* floats
     const Q3BlockPlan b = q3_block_shape(cus, K, N, batch_M, nullptr);
     *floats = b.split.floats;
     *counters = b.split.nsplit > 1 ? (size_t)b.split.ntiles : 0;
+    if (q3_block_yields(cus, K, N, batch_M)) {
+      size_t f, c;
+      hq_q3_direct_need(cus, K, N, batch_M, &f, &c);
+      if (f > *floats) *floats = f;
+      if (c > *counters) *counters = c;
+    }
     return HQ_OK;
   }
   return hq_q3_gemm_need(cus, K, N, batch_M, floats, counters);
@@ -807,6 +825,8 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
     if (q3_plan(dev->cus, K, N, batch_M) == HQ_Q3_PLAN_BLOCK) {
       const Q3BlockPlan b = q3_block_shape(dev->cus, K, N, batch_M, lim);
       if (b.split.nsplit != b.nsplit) return HQ_ERR_BAD_SHAPE;
+      if (!b.split.too_large && q3_block_yields(dev->cus, K, N, batch_M))
+        return hq_q3_direct_launch(x, qweight, scales, zeros, y, K, N, batch_M, flags, stream, fixed);
       rc = q3_split_acquire(b.split, fixed, stream, &sp);
       if (rc != HQ_OK) return rc;
       return hq_q3_block_launch(x, qweight, scales, zeros, y, K, N, batch_M, b.nsplit, b.rpw, b.mblocks, sp.partial,

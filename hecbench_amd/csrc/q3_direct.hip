@@ -1,0 +1,514 @@
+// Batched GPTQ 3-bit product in one launch, without a pre-pass, for the small and medium problems between the few rows of
+// q3_block.hip and the many of q3_prefill.hip (fp16 activations, fp32 output):
+//
+//   out[m][n] = s[n] * sum_k A[m][k]*q[k][n]  -  z[n] * sum_k A[m][k]
+//
+// What bounds such a problem is latency: launches, the first data, and how fast one compute unit can pull its operands (64 KB in
+// flight, 50 GB/s where HBM is among their sources).  The pre-pass of the other kernels was 3 to 5 us of 12 to 25, and their
+// tiles, dividing K eight ways among workgroups, spent as long on adding up the shares.  So here
+//   - activations are read as they lie, straight into LDS, and put in order on the way from LDS into the operand registers
+//     (one byte permutation per register); nothing is scaled: the codes themselves become fp16 numbers, by one AND/OR per word
+//     and v_cvt_scalef32_pk32_f16_fp6, which makes 32 of them at once (64 cycles; 3-bit fields as subnormals in place, as the
+//     other kernels have them, need the activations scaled, and a multiplication for each to be rid of that: 0.38 -> 0.33 us for
+//     256 elements of K);
+//   - a tile is small, 32 rows by 64 or 128 columns, and its K is divided among the WAVES of a workgroup, each of which streams
+//     its own operands through a ring of its own in LDS without ever meeting the others before the end (with operands shared
+//     between waves and a barrier per step 13.4 instead of 10.3 us at 341 rows, K=4096+320, N=644);
+//   - the rows' sums for the zero term come out of the operand registers (v_dot2_f32_f16).
+// Measured, before -> now: 70 x 4096 x 4096 17 -> 9 us; 341 x 4416 x 644 21.6 -> 10.4; 39 x 4160 x 3176 16.6 -> 9.5; 128 x 4096 x
+// 4096 17.8 -> 9.4; 64 x 4096 x 11008 18.5 -> 12.3; 210 x 6976 x 4592 28 -> 19; 23 x 1952 x 12980 11.7 -> 7.4.
+// Codes that are normal numbers also lose less in the matrix instruction, which aligns the products of a sum by their
+// exponents: error against 64 bits 2e-7 of the result (2-norm) instead of 1.8e-6.
+#include <type_traits>
+
+#include "hq_internal.h"
+#include "q3_tile.h"
+
+namespace {
+
+using namespace hq_q3;
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u6v __attribute__((ext_vector_type(6)));
+typedef uint32_t u16v __attribute__((ext_vector_type(16)));
+typedef _Float16 h32 __attribute__((ext_vector_type(32)));
+
+// Read six bits at a time the 96-bit string of a k-group and column is sixteen fp6 (e2m3) numbers: bits 0 to 2 of field f are
+// code 2f, with the three above cleared the number code / 8; three bits further on, code 2f + 1.  Word w of the string: bits
+// `first` and up of its fields, n of them.
+constexpr uint32_t field_bits(int w, int first, int n) {
+  uint32_t m = 0;
+  for (int b = 0; b < 32; ++b)
+    if ((32 * w + b) % 6 >= first && (32 * w + b) % 6 < first + n) m |= 1u << b;
+  return m;
+}
+
+// A wave multiplies MB 32-row blocks by CB times 32 columns over its own part of every step of K (64 elements of 64 KS); the KS
+// waves of a workgroup share a tile of 32 MB x 32 CB results and meet once, at its end.  Nothing a wave loads is read by another:
+// each streams its operands through ST stages of LDS of its own, without a barrier.
+template <int MB, int CB, int KS, int SA, int SW>
+struct Form {
+  static constexpr int kThreads = 64 * KS;
+  static constexpr int kTileM = 32 * MB, kTileN = 32 * CB;
+  static constexpr int kABytes = kTileM * 128, kWBytes = 6 * kTileN * 4;  // a wave's stage: 128 bytes of every row, six packed rows
+  static constexpr int kALoads = kABytes / 1024;           // LDS loads of a stage: activations,
+  static constexpr int kWLoads = (kWBytes + 1023) / 1024;  // and packed rows, the last load by half of the lanes if CB is 2
+  static constexpr int kLoads = kALoads + kWLoads;
+  static constexpr int kCols = CB < 4 ? CB : 4, kHalves = CB / kCols;  // a lane's columns: kCols adjacent ones of every 32 kCols
+  static constexpr int kUnits = 4 * MB * CB;               // groups of eight rows, every kCols-th column (of a half)
+  static constexpr int kMeetUnits = kUnits * KS > 128 ? 128 / KS : kUnits;  // of which so many meet at a time,
+  static constexpr int kRounds = kUnits / kMeetUnits, kFinal = kMeetUnits / KS;  // and a wave finishes some of them
+  static constexpr int kWaveBytes = SA * kABytes + SW * kWBytes, kRing = KS * kWaveBytes, kMeet = KS * kMeetUnits * 1024;
+  static constexpr int kBulk = kRing > kMeet ? kRing : kMeet;
+  static constexpr int kSums = 2 * KS * kTileM;            // floats: parts of the row sums
+  static constexpr int kSmem = kBulk + (kSums + kTileM) * 4 + 16;
+  static constexpr int kPerSimd = MB * CB > 8 ? 1 : 2;    // waves
+  static_assert(KS % 2 == 0, "odd parts of K enter negated");
+  static constexpr int kInFlight = (SA - 1) * kLoads + (SW > SA ? kWLoads : 0);  // loads behind the next step's operands
+  static_assert(SW >= SA && kInFlight < 64, "the wait counts them");
+  static_assert(kSmem <= 160 * 1024, "LDS");
+};
+
+struct DirectArgs {
+  const uint32_t* w;
+  const _Float16* x;
+  const float* scales;
+  const float* zeros;
+  float* out;
+  float* partial;      // [tile][nshare][kTileM * kTileN]
+  unsigned* counters;  // [tile], zero between calls
+  int M, N, K, nmt, T, nshare, L;  // row tiles; steps of K, shares of L steps each
+  unsigned flags;
+};
+
+template <int MB, int CB, int KS, int SA, int SW>
+__global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void q3_direct_kernel(DirectArgs a) {
+  using S = Form<MB, CB, KS, SA, SW>;
+  constexpr int C = S::kCols, H = S::kHalves;
+  typedef uint32_t wv_t __attribute__((ext_vector_type(C)));
+  extern __shared__ unsigned char lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int kp = __builtin_amdgcn_readfirstlane(tid >> 6);  // part of K
+  const int nl = lane & 31, kb = lane >> 5;
+  const int G = a.K >> 5, nwg = gridDim.x;
+  // workgroup b runs on XCD b mod 8: an XCD takes consecutive tiles (row tiles of one column tile first), which share
+  // weights and activations in its L2
+  const int xcd = blockIdx.x & 7;
+  const int v = xcd * (nwg >> 3) + min(xcd, nwg & 7) + (int)(blockIdx.x >> 3);
+  const int tile = v / a.nshare, share = v - tile * a.nshare;
+  const int ct = __builtin_amdgcn_readfirstlane(tile / a.nmt), mt = __builtin_amdgcn_readfirstlane(tile - ct * a.nmt);
+  const int t0 = share * a.L, len = min(a.L, a.T - t0);
+
+  // ---- loader ----
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)lds + kp * S::kWaveBytes;
+  const unsigned char* const abase = reinterpret_cast<const unsigned char*>(a.x + (size_t)mt * S::kTileM * a.K);
+  // Activations keep their order: 16-byte piece c of a row's 128 bytes stands in column c ^ (row / 2 mod 8): the sixteen lanes
+  // of a 128-bit LDS read pass, which are sixteen rows, then meet sixteen different bank groups.
+  // Offsets of a step's pieces from its first.  In the last step of K a wave may have one k-group or none: it loads the last
+  // k-group in place of those that are not there (and takes its codes as zero).
+  constexpr int L0 = S::kALoads;
+  uint32_t off[S::kLoads];
+#pragma unroll
+  for (int i = 0; i < L0; ++i) {
+    const int row = i * 8 + (lane >> 3);
+    off[i] = (uint32_t)(min(mt * S::kTileM + row, a.M - 1) - mt * S::kTileM) * (uint32_t)a.K * 2u +
+             (uint32_t)((lane & 7) ^ ((row >> 1) & 7)) * 16u + (uint32_t)kp * 128u;
+  }
+#pragma unroll
+  for (int i = 0; i < S::kWLoads; ++i) {
+    const int o = i * 1024 + (CB == 2 && i ? lane & 31 : lane) * 16, row = 6 * kp + o / (S::kTileN * 4), col = o % (S::kTileN * 4) / 4;
+    off[L0 + i] = (uint32_t)row * (uint32_t)a.N * 4u + (uint32_t)min(ct * S::kTileN + col, a.N - 4) * 4u;
+  }
+  const int t_last = a.T - 1;
+  const int missing = max(0, 2 * KS * t_last + 2 * kp + 2 - G);  // k-groups of this wave's last step, 2 and more: all
+  auto back = [&](int l) {  // how far the last step's offset lies in front of off[l]
+    const int shift = max(missing - 2, 0) + (missing > 1 ? 1 : 0);  // whole k-groups: the wave's first becomes the last of K
+    bool second;                                                     // does the lane load for the wave's second k-group?
+    if (l < L0) second = ((lane >> 2) ^ l) & 1;
+    else second = ((l - L0) * 1024 + (CB == 2 && l > L0 ? lane & 31 : lane) * 16) / (S::kTileN * 4) >= 3;
+    const int groups = shift + (second && missing > 0 ? 1 : 0);
+    return (uint32_t)groups * (l < L0 ? 64u : 12u * (uint32_t)a.N);
+  };
+  // activations of step ta and packed rows of step tw (negative: none) into their rings' slots
+  auto dma = [&](int sa, int ta, int sw, int tw, bool may_be_last) {
+    const unsigned char* const ax = abase + (size_t)ta * (128 * KS);
+    const unsigned char* const wx = reinterpret_cast<const unsigned char*>(a.w) + (size_t)(6 * KS * tw) * a.N * 4u;
+#pragma unroll
+    for (int l = 0; l < S::kLoads; ++l) {
+      uint32_t o = off[l];
+      if (may_be_last && (l < L0 ? ta : tw) == t_last) o -= back(l);
+      if (l < L0) {
+        if (ta >= 0) load_lds(lds0 + sa * S::kABytes + l * 1024, o, ax);
+      } else if (tw >= 0) {
+        if (CB != 2 || l == L0 || lane < 32) load_lds(lds0 + SA * S::kABytes + sw * S::kWBytes + (l - L0) * 1024, o, wx);
+      }
+    }
+  };
+  // waits until at most n of this wave's loads are in flight
+  auto wait = [&](auto n) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
+  };
+
+  f16v acc[MB][CB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int q = 0; q < CB; ++q)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mb][q][i] = 0.f;
+  float rs[MB];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) rs[mb] = 0.f;
+
+  const unsigned char* const ring = lds + kp * S::kWaveBytes;
+  const unsigned char* const a_lane = ring + nl * 128;
+  const unsigned char* const w_lane = ring + SA * S::kABytes + (3 * kb * S::kTileN + C * nl) * 4;
+  u4v P[MB][2];
+  auto read_pieces = [&](int slot, int i0) {  // two of the four of the lane's k-group
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        P[mb][i] = *reinterpret_cast<const u4v*>(a_lane + slot * S::kABytes + mb * 4096 + (((4 * kb + i0 + i) ^ ((nl >> 1) & 7)) * 16));
+  };
+  struct Words { wv_t v[3][H]; };
+  auto read_w = [&](int slot, int t, bool may_be_last, Words& dst) {
+    const bool real = !may_be_last || 2 * KS * t + 2 * kp + kb < G;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        const wv_t x = *reinterpret_cast<const wv_t*>(w_lane + slot * S::kWBytes + (j * S::kTileN + h * 128) * 4);
+#pragma unroll
+        for (int c = 0; c < C; ++c) dst.v[j][h][c] = real ? x[c] : 0u;
+      }
+  };
+  // Column q's 32 codes as fp16 numbers code / 8: elements 0..15 the even codes, 16..31 the odd ones (odd parts of K negative).
+  const uint32_t neg = kp & 1 ? 0xffffffffu : 0u;
+  const uint32_t sign[3] = {neg & field_bits(0, 5, 1), neg & field_bits(1, 5, 1), neg & field_bits(2, 5, 1)};
+  uint32_t keep[3] = {field_bits(0, 0, 3), field_bits(1, 0, 3), field_bits(2, 0, 3)};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) asm("" : "+v"(keep[i]));  // in registers, so that the AND and the OR are one instruction
+  auto codes = [&](const Words& words, int q) {
+    uint32_t w[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) w[j] = words.v[j][q / C][q % C];
+    u6v f;
+    f[0] = (w[0] & keep[0]) | sign[0];
+    f[1] = (w[1] & keep[1]) | sign[1];
+    f[2] = (w[2] & keep[2]) | sign[2];
+    f[3] = (__builtin_amdgcn_alignbit(w[1], w[0], 3) & keep[0]) | sign[0];
+    f[4] = (__builtin_amdgcn_alignbit(w[2], w[1], 3) & keep[1]) | sign[1];
+    f[5] = (w[2] >> 3 & keep[2]) | sign[2];
+    return __builtin_bit_cast(u16v, __builtin_amdgcn_cvt_scalef32_pk32_f16_fp6(f, 1.f));
+  };
+  // and the activations in that order: operand j of a lane's 32, out of pieces 2 (j & 1) and the next
+  auto rows_operand = [&](int j, u4v (&dst)[MB]) {
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const u4v& p = P[mb][i >> 1];
+        dst[mb][i] = __builtin_amdgcn_perm(p[2 * (i & 1) + 1], p[2 * (i & 1)], j < 2 ? 0x05040100u : 0x07060302u);
+      }
+  };
+
+  u4v A[4][MB];
+  u16v B;
+  Words w;
+  auto dma_step = [&](int sa, int sw, int s, bool may_be_last) {  // step s's activations and step s + SW - SA's packed rows
+    dma(sa, s < len ? t0 + s : -1, sw, s + SW - SA < len ? t0 + s + SW - SA : -1, may_be_last);
+  };
+#pragma unroll
+  for (int i = 0; i < SW - SA; ++i) dma(0, -1, i, i < len ? t0 + i : -1, true);
+#pragma unroll
+  for (int i = 0; i < SA; ++i) dma_step(i, (i + SW - SA) % SW, i, true);
+  if (len > SW) wait(std::integral_constant<int, S::kInFlight>());
+  else wait(std::integral_constant<int, 0>());
+  read_w(0, t0, true, w);
+  read_pieces(0, 0);
+  rows_operand(0, A[0]);
+  rows_operand(2, A[2]);
+  read_pieces(0, 2);
+  rows_operand(1, A[1]);
+  rows_operand(3, A[3]);
+  int sa = 0, sw = 0, s = 0;
+  // A step: column by column of a lane's CB the codes and the products; under the last column the next step's operands come out
+  // of LDS and are made.  MODE 2: loads another stage, 1: perhaps the last of K, 0: none.
+  auto step = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    const int sa1 = sa + 1 == SA ? 0 : sa + 1, sw1 = sw + 1 == SW ? 0 : sw + 1;
+    // this step's operands are in registers, its places in the rings are free
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (MODE == 2) dma(sa, t0 + s + SA, sw, t0 + s + SW, false);
+    else if (MODE) dma_step(sa, sw, s + SA, true);
+    __builtin_amdgcn_sched_barrier(0);
+    const h2 one = MODE == 2 || 2 * KS * (t0 + s) + 2 * kp + kb < G ? h2{(_Float16)1.f, (_Float16)1.f} : h2{(_Float16)0.f, (_Float16)0.f};
+#pragma unroll
+    for (int q = 0; q < CB; ++q) {
+      B = codes(w, q);
+      if (q == CB - 1) {
+        // the next step's operands have to be in LDS (MODE 1 may have left out packed rows)
+        wait(std::integral_constant<int, MODE == 2 ? S::kInFlight : (MODE == 1 ? (SA - 1) * S::kALoads : 0)>());
+        read_pieces(sa1, 0);
+        read_w(sw1, t0 + s + 1, MODE < 2, w);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        constexpr int kOrder[4] = {0, 2, 1, 3};  // operands 0 and 2 are made of the same pieces
+        const int j = kOrder[jj];
+        const u4v b = {B[4 * j], B[4 * j + 1], B[4 * j + 2], B[4 * j + 3]};
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb)
+          acc[mb][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, A[j][mb]), __builtin_bit_cast(h8, b), acc[mb][q], 0, 0, 0);
+        if (q == (CB == 2 ? 0 : j & 1))
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)  // the sums of the rows
+              rs[mb] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, (uint32_t)A[j][mb][i]), one, rs[mb], false);
+        if (q == CB - 1) {
+          rows_operand(j, A[j]);
+          if (jj == 1) read_pieces(sa1, 2);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    sa = sa1;
+    sw = sw1;
+    ++s;
+  };
+  while (s < len - SW - 1) step(std::integral_constant<int, 2>());
+  while (s < len - SA) step(std::integral_constant<int, 1>());
+  while (s < len) step(std::integral_constant<int, 0>());
+
+  // ---- the parts of K meet: wave p finishes units p * kFinal and up (no load is in flight into LDS any more: the last steps
+  // waited for theirs) ----
+  constexpr int F = S::kFinal, R = S::kRounds;
+  constexpr int V = F < C ? F : C;  // adjacent columns of a wave's units
+  typedef float fv_t __attribute__((ext_vector_type(V)));
+  float* const sums = reinterpret_cast<float*>(lds + S::kBulk);  // [2 KS][kTileM], then the rows' sums
+  float* const total = sums + S::kSums;
+  f4v* const meet = reinterpret_cast<f4v*>(lds) + lane;
+  auto first_row = [&](int r, int i) { return (r * S::kMeetUnits + kp * F + i) / C % (4 * MB) * 8 + 4 * kb; };  // of unit i of round r
+  auto first_col = [&](int r) { return ct * S::kTileN + r * S::kMeetUnits / (4 * MB * C) * 128 + C * nl + kp * F % C; };
+  f4v fin[R][F];
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) sums[(2 * kp + kb) * S::kTileM + mb * 32 + nl] = rs[mb];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    __syncthreads();  // every wave is done with its stages, and with the round before
+#pragma unroll
+    for (int v = 0; v < S::kMeetUnits; ++v) {
+      const int u = r * S::kMeetUnits + v, h = u / (4 * MB * C), mb = u / (4 * C) % MB;
+      f4v x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = acc[mb][h * C + u % C][4 * (u / C % 4) + e];
+      meet[(v * KS + kp) * 64] = x;
+    }
+    if (r == 0 && tid < S::kTileM) {  // (the sums' parts were written ahead of the barrier)
+      float t = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2 * KS; ++i) t += sums[i * S::kTileM + tid];
+      total[tid] = t;
+    }
+    __syncthreads();
+    const int nc = min(first_col(r), a.N - V);
+    const fv_t sc = *reinterpret_cast<const fv_t*>(a.scales + nc), zr = *reinterpret_cast<const fv_t*>(a.zeros + nc);
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+      f4v x = meet[((kp * F + i) * KS) * 64];
+#pragma unroll
+      for (int p = 1; p < KS; ++p) {
+        const f4v other = meet[((kp * F + i) * KS + p) * 64];
+        x = p & 1 ? x - other : x + other;  // odd parts are the negated ones
+      }
+      const f4v t = *reinterpret_cast<const f4v*>(total + first_row(r, i));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) fin[r][i][e] = sc[i % V] * (x[e] * 8.f) - zr[i % V] * t[e];  // codes enter as eighths
+    }
+  }
+
+  if (a.nshare > 1) {
+    // A share of a divided tile: its results go out, every wave waits for their acknowledgement, the workgroup counts
+    // itself at the memory side, and the last to arrive adds the shares in order of k.
+    auto slot_of_share = [&](int c) {
+      return reinterpret_cast<f4v*>(a.partial) + (size_t)(tile * a.nshare + c) * (S::kTileM * S::kTileN / 4) + tid;
+    };
+    f4v* dst = slot_of_share(share);
+#pragma unroll
+    for (int i = 0; i < R * F; ++i) hq_store_share(dst + i * S::kThreads, fin[i / F][i % F]);
+    unsigned* last = reinterpret_cast<unsigned*>(total + S::kTileM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      const unsigned old = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *last = old == (unsigned)(a.nshare - 1);
+      if (old == (unsigned)(a.nshare - 1))  // ready for the next call
+        __hip_atomic_store(&a.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*last) return;
+    constexpr int kAtOnce = R * F >= 16 ? 1 : (F >= 8 ? 2 : (F >= 4 ? 4 : 8));
+    for (int c0 = 0; c0 < a.nshare; c0 += kAtOnce) {
+      f4v x[kAtOnce * R * F];
+#pragma unroll
+      for (int k = 0; k < kAtOnce; ++k)
+#pragma unroll
+        for (int i = 0; i < R * F; ++i)
+          x[k * R * F + i] = hq_load_share(slot_of_share(min(c0 + k, a.nshare - 1)) + i * S::kThreads);
+      hq_wait_shares(x);
+#pragma unroll
+      for (int k = 0; k < kAtOnce; ++k)
+        if (c0 + k < a.nshare) {
+#pragma unroll
+          for (int i = 0; i < R * F; ++i)
+            fin[i / F][i % F] = c0 + k == 0 ? x[k * R * F + i] : fin[i / F][i % F] + x[k * R * F + i];
+        }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int i = 0; i < F; i += V) {
+      const int m0 = mt * S::kTileM + first_row(r, i), n = first_col(r);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (m0 + e < a.M && n < a.N) {
+          fv_t* p = reinterpret_cast<fv_t*>(a.out + (size_t)(m0 + e) * a.N + n);
+          fv_t o;
+#pragma unroll
+          for (int c = 0; c < V; ++c) o[c] = fin[r][i + c][e];
+          if (a.flags & HQ_FLAG_ACCUMULATE) o += *p;
+          __builtin_nontemporal_store(o, p);
+        }
+      }
+    }
+}
+
+__global__ __launch_bounds__(256) void clear_counters(unsigned* p, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
+// Host arithmetic of a launch (the launch, the choice between the kernels and the size query share it).
+struct DirectPlan {
+  int kind, tm, tn, ks, nmt, ntiles, T, nshare, L;
+  float us;
+  size_t partial_floats, counters;
+};
+
+// The workgroups and what they cost, fitted to 5700 timings of 520 problems on MI355X (spread about the fit: 7 %): a workgroup
+// takes base_us and step_us for every step of 64 ks elements; workgroups that share a compute unit take their steps one after
+// the other (their operands come through one queue), beyond per_cu of them in rounds; dividing a tile's K among c workgroups costs
+// share_us + c * per_share_us.  Eight waves per workgroup where every compute unit has but one, four otherwise; 128 columns load
+// fewer activations per weight, 64 divide smaller problems.
+struct DirectKind {
+  int tm, tn, ks, per_cu;
+  float base_us, step_us, share_us, per_share_us;
+};
+constexpr DirectKind kKinds[4] = {{32, 64, 4, 3, 3.83f, 0.385f, 1.36f, 0.17f}, {32, 64, 8, 1, 4.2f, 0.575f, 1.54f, 0.12f},
+                                  {32, 128, 4, 2, 4.06f, 0.574f, 1.2f, 0.35f}, {32, 128, 8, 1, 4.9f, 0.904f, 1.9f, 0.15f}};
+constexpr int kMaxShares = 8;
+
+DirectPlan direct_plan_of(int cus, int K, int N, int M, int kind, int nshare) {
+  const DirectKind& kd = kKinds[kind];
+  DirectPlan p;
+  p.kind = kind;
+  p.tm = kd.tm; p.tn = kd.tn; p.ks = kd.ks;
+  p.nmt = (M + p.tm - 1) / p.tm;
+  p.ntiles = p.nmt * ((N + p.tn - 1) / p.tn);
+  p.T = (K / 32 + 2 * p.ks - 1) / (2 * p.ks);
+  p.nshare = nshare < p.T ? nshare : p.T;
+  p.L = (p.T + p.nshare - 1) / p.nshare;
+  p.nshare = (p.T + p.L - 1) / p.L;
+  const int wgs = p.ntiles * p.nshare, per_cu = (wgs + cus - 1) / cus;
+  const float side = per_cu <= kd.per_cu ? (float)per_cu : (float)wgs / cus + 1.1f;
+  p.us = kd.base_us + p.L * side * kd.step_us + (p.nshare > 1 ? kd.share_us + p.nshare * kd.per_share_us : 0.f);
+  p.partial_floats = p.nshare > 1 ? (size_t)wgs * p.tm * p.tn : 0;
+  p.counters = p.nshare > 1 ? p.ntiles : 0;
+  return p;
+}
+
+DirectPlan direct_plan(int cus, int K, int N, int M, bool undivided) {
+  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: 3 + kind + 10 * shares
+  if (force >= 0 && force % 10 >= 3 && force % 10 < 7)
+    return direct_plan_of(cus, K, N, M, force % 10 - 3, undivided || force < 10 ? 1 : force / 10);
+  DirectPlan best = direct_plan_of(cus, K, N, M, 0, 1);
+  for (int kind = 0; kind < 4; ++kind)
+    for (int c = 1; c <= (undivided ? 1 : kMaxShares); ++c) {
+      const DirectPlan p = direct_plan_of(cus, K, N, M, kind, c);
+      if (p.nshare != c) continue;
+      const int64_t wgs = (int64_t)p.ntiles * c;
+      if (c > 1 && wgs > 2 * cus) break;                       // bounds the workspace: 2 * cus * 32 * 128 floats
+      if (kKinds[kind].per_cu == 1 && wgs > cus) continue;
+      if (p.us < best.us) best = p;
+    }
+  return best;
+}
+
+template <int MB, int CB, int KS, int SA, int SW>
+int launch(const DirectArgs& a, int nwg, hipStream_t stream) {
+  using S = Form<MB, CB, KS, SA, SW>;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_direct_kernel<MB, CB, KS, SA, SW>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, S::kSmem);
+  if (attr != hipSuccess) return (int)attr;
+  hipLaunchKernelGGL((q3_direct_kernel<MB, CB, KS, SA, SW>), dim3(nwg), dim3(S::kThreads), S::kSmem, stream, a);
+  return hq_launch_status();
+}
+
+}  // namespace
+
+// Estimate of one call (us), and whether the kernel can take it at all: offsets inside a step are 32-bit.
+float hq_q3_direct_us(int cus, int K, int N, int M) {
+  return K > (1 << 24) || N > (1 << 22) ? 1e30f : direct_plan(cus, K, N, M, false).us;
+}
+bool hq_q3_direct_forced() {
+  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);
+  return force >= 0 && force % 10 >= 3 && force % 10 < 7;
+}
+
+void hq_q3_direct_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
+  const DirectPlan p = direct_plan(cus, K, N, M, false);
+  *floats = p.partial_floats;
+  *counters = p.counters;
+}
+
+int hq_q3_direct_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
+                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
+  const HqDevice* dev = nullptr;
+  int rc = hq_current_device(&dev);
+  if (rc != HQ_OK) return rc;
+  DirectPlan p = direct_plan(dev->cus, K, N, M, false);
+  // without room for the shares' sums no tile is divided
+  if (p.nshare > 1 && (fixed ? p.partial_floats > fixed->tiles_floats || p.counters > fixed->ncounters
+                             : hq_workspace_out_of_reach(stream, p.partial_floats, p.counters)))
+    p = direct_plan(dev->cus, K, N, M, true);
+  DirectArgs a;
+  a.partial = nullptr; a.counters = nullptr;
+  if (p.nshare > 1 && fixed) {
+    a.partial = fixed->tiles;
+    a.counters = fixed->counters;
+    // shared by every call on this device: a call that was cut short may have left counts behind
+    hipLaunchKernelGGL(clear_counters, dim3((p.ntiles + 255) / 256), dim3(256), 0, stream, a.counters, p.ntiles);
+    rc = hq_launch_status();
+    if (rc != HQ_OK) return rc;
+  } else if (p.nshare > 1) {
+    HqWorkspace ws;
+    rc = hq_get_workspace(stream, p.partial_floats, p.counters, &ws);
+    if (rc != HQ_OK) return rc;
+    a.partial = ws.partial;
+    a.counters = ws.counters;
+  }
+  a.w = reinterpret_cast<const uint32_t*>(qweight);
+  a.x = reinterpret_cast<const _Float16*>(x);
+  a.scales = scales; a.zeros = zeros; a.out = y;
+  a.M = M; a.N = N; a.K = K; a.nmt = p.nmt; a.T = p.T; a.nshare = p.nshare; a.L = p.L; a.flags = flags;
+  const int nwg = p.ntiles * p.nshare;
+  switch (p.kind) {
+    case 0: return launch<1, 2, 4, 2, 2>(a, nwg, stream);
+    case 1: return launch<1, 2, 8, 2, 2>(a, nwg, stream);
+    case 2: return launch<1, 4, 4, 2, 2>(a, nwg, stream);
+    default: return launch<1, 4, 8, 2, 2>(a, nwg, stream);
+  }
+}

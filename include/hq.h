@@ -172,7 +172,8 @@ int hq_q3_matvec(const void* x, int x_dtype, const int32_t* qweight, const float
  */
 #define HQ_Q3_PLAN_MATVEC 0 /* batch_M == 1 */
 #define HQ_Q3_PLAN_GEMM 2   /* batched MFMA GEMM */
-#define HQ_Q3_PLAN_BLOCK 3  /* batch_M 2 ... 64: the matvec's kernel, four rows per pass or workgroup */
+#define HQ_Q3_PLAN_BLOCK 3  /* batch_M 2 ... 64, a small launch: the matvec's kernel, four rows per pass or workgroup, or,
+                             * with more workgroups than compute units, matrix-core tiles in one launch */
 int hq_q3_matvec_plan(int K, int N, int batch_M);
 
 /*
