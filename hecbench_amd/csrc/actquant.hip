@@ -343,8 +343,8 @@ __device__ __forceinline__ bool fast8(const Raw<T>& raw, const FastRow<MODE>& ro
 constexpr int kStaticUnroll = 2;
 
 template <typename T, bool AZP>
-__global__ __launch_bounds__(256) void static_quant_kernel(const T* __restrict__ in, int8_t* __restrict__ out,
-                                                          float scale, int azp, int64_t total, int aligned) {
+__device__ __forceinline__ void static_quant_body(const T* __restrict__ in, int8_t* __restrict__ out, float scale, int azp,
+                                                  int64_t total, int aligned) {
   const Divisor d(scale);
   const FastRow<AZP ? kQuotientAzp : kQuotient> row(0.f, d, azp);
   const int64_t units = (total + kVec - 1) / kVec;
@@ -368,6 +368,17 @@ __global__ __launch_bounds__(256) void static_quant_kernel(const T* __restrict__
       if (u < units) store_unit<true>(out, u, q, 0, (int)min((int64_t)kVec, total - u * kVec), aligned);
     }
   }
+}
+template <typename T, bool AZP>
+__global__ __launch_bounds__(256) void static_quant_kernel(HQ_ARGS12) {
+  HqReader r(HQ_PASS12);
+  const T* const in = r;
+  int8_t* const out = r;
+  const float scale = r;
+  const int azp = r;
+  const int64_t total = r;
+  const int aligned = r;
+  static_quant_body<T, AZP>(in, out, scale, azp, total, aligned);
 }
 
 // ---- dynamic scale: LANES threads per row --------------------------------------------------------
@@ -420,9 +431,8 @@ enum RowMode { WHOLE, TAIL, ANY };
 constexpr int row_threads(int lanes) { return lanes < 256 ? 256 : lanes; }
 
 template <typename T, bool AZP, int LANES, int KEEP, RowMode MODE>
-__global__ __launch_bounds__(row_threads(LANES)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && LANES >= 256 ? (MODE == WHOLE || !AZP ? 8 : 7) : 1))) void dynamic_quant_kernel(const T* __restrict__ in, int8_t* __restrict__ out,
-                                                           float* __restrict__ scales, int32_t* __restrict__ azps,
-                                                           int64_t tokens, int hidden) {
+__device__ __forceinline__ void dynamic_quant_body(const T* __restrict__ in, int8_t* __restrict__ out, float* __restrict__ scales,
+                                                   int32_t* __restrict__ azps, int64_t tokens, int hidden) {
   constexpr bool aligned = MODE != ANY;
   __shared__ float lds[2 * LANES / 64];
   const int lane = threadIdx.x % LANES;
@@ -532,6 +542,18 @@ __global__ __launch_bounds__(row_threads(LANES)) __attribute__((amdgpu_waves_per
   }
   for (int j = lane + KEEP * LANES; j < end; j += LANES) emit(fetch(j), j);
 }
+template <typename T, bool AZP, int LANES, int KEEP, RowMode MODE>
+__global__ __launch_bounds__(row_threads(LANES)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && LANES >= 256 ? (MODE == WHOLE || !AZP ? 8 : 7) : 1)))
+void dynamic_quant_kernel(HQ_ARGS12) {
+  HqReader r(HQ_PASS12);
+  const T* const in = r;
+  int8_t* const out = r;
+  float* const scales = r;
+  int32_t* const azps = r;
+  const int64_t tokens = r;
+  const int hidden = r;
+  dynamic_quant_body<T, AZP, LANES, KEEP, MODE>(in, out, scales, azps, tokens, hidden);
+}
 
 // The 128-bit loads and 64-bit stores need both base pointers on their grid; other pointers are served
 // element by element.
@@ -552,16 +574,12 @@ int launch_static(const T* in, int8_t* out, int64_t tokens, int hidden, float sc
   const int64_t cap = (int64_t)dev->cus * 6;
   if (blocks > cap) blocks = cap;
   if (has_azp)
-    hipLaunchKernelGGL((static_quant_kernel<T, true>), dim3((unsigned)blocks), dim3(256), 0, stream, in, out, scale, azp,
-                       total, aligned);
-  else
-    hipLaunchKernelGGL((static_quant_kernel<T, false>), dim3((unsigned)blocks), dim3(256), 0, stream, in, out, scale, azp,
-                       total, aligned);
-  return hq_launch_status();
+    return hq_launch(static_quant_kernel<T, true>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, scale, azp, total, aligned);
+  return hq_launch(static_quant_kernel<T, false>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, scale, azp, total, aligned);
 }
 
 template <typename T, bool AZP, RowMode MODE>
-void launch_dynamic_mode(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
+int launch_dynamic_mode(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
                          const HqDevice* dev, hipStream_t stream) {
   // Short rows get a wave each, the others a workgroup of as many threads as keep the whole row in registers with at most
   // five units each: rows past five units of 256 threads used to be read twice (2048 rows of 16384 bf16 with zero point
@@ -571,9 +589,8 @@ void launch_dynamic_mode(const T* in, int8_t* out, float* scales, int32_t* azps,
   const bool wave_rows = hidden <= 64 * kVec * 3;
   const int span = (hidden + kVec - 1) / kVec + 1 + 63;  // units from the 64-unit boundary before a ragged row to its end
 #define HQ_ROWS(LANES, KEEP)                                                                                          \
-  hipLaunchKernelGGL((dynamic_quant_kernel<T, AZP, LANES, KEEP, MODE>),                                               \
-                     dim3((unsigned)(LANES == 64 ? (tokens + 3) / 4 : tokens)), dim3(row_threads(LANES)), 0, stream, in, \
-                     out, scales, azps, tokens, hidden)
+  return hq_launch(dynamic_quant_kernel<T, AZP, LANES, KEEP, MODE>, dim3((unsigned)(LANES == 64 ? (tokens + 3) / 4 : tokens)), \
+                   dim3(row_threads(LANES)), 0, stream, in, out, scales, azps, tokens, hidden)
   if (wave_rows) {
     if (span <= 64 * 2) HQ_ROWS(64, 2);
     else if (span <= 64 * 3) HQ_ROWS(64, 3);
@@ -593,23 +610,21 @@ void launch_dynamic_mode(const T* in, int8_t* out, float* scales, int32_t* azps,
 }
 
 template <typename T, bool AZP>
-void launch_dynamic_azp(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
+int launch_dynamic_azp(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
                         const HqDevice* dev, hipStream_t stream) {
   const int64_t total = tokens * hidden;
   if (!pointers_aligned(in, out) || total < kVec)
-    launch_dynamic_mode<T, AZP, ANY>(in, out, scales, azps, tokens, hidden, dev, stream);
-  else if (total % kVec)
-    launch_dynamic_mode<T, AZP, TAIL>(in, out, scales, azps, tokens, hidden, dev, stream);
-  else
-    launch_dynamic_mode<T, AZP, WHOLE>(in, out, scales, azps, tokens, hidden, dev, stream);
+    return launch_dynamic_mode<T, AZP, ANY>(in, out, scales, azps, tokens, hidden, dev, stream);
+  if (total % kVec)
+    return launch_dynamic_mode<T, AZP, TAIL>(in, out, scales, azps, tokens, hidden, dev, stream);
+  return launch_dynamic_mode<T, AZP, WHOLE>(in, out, scales, azps, tokens, hidden, dev, stream);
 }
 
 template <typename T>
 int launch_dynamic(const T* in, int8_t* out, float* scales, int32_t* azps, int64_t tokens, int hidden,
                    const HqDevice* dev, hipStream_t stream) {
-  if (azps) launch_dynamic_azp<T, true>(in, out, scales, azps, tokens, hidden, dev, stream);
-  else launch_dynamic_azp<T, false>(in, out, scales, azps, tokens, hidden, dev, stream);
-  return hq_launch_status();
+  if (azps) return launch_dynamic_azp<T, true>(in, out, scales, azps, tokens, hidden, dev, stream);
+  return launch_dynamic_azp<T, false>(in, out, scales, azps, tokens, hidden, dev, stream);
 }
 
 int check_common(const void* x, int x_dtype, const int8_t* out, int64_t tokens, int hidden) {

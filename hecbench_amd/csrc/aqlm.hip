@@ -55,14 +55,13 @@ constexpr int kMaxLdsK = 24576;  // 48 KB
 __host__ __device__ constexpr int aqlm_x_stride(int units) { return (units + 7) / 8 * 8 + 1; }
 
 template <int ROWS, bool XLDS, bool SPLIT>
-__global__ __launch_bounds__(256) void aqlm_matvec_kernel(const u4v* codes_, const u4v* codebooks_, const u4v* x_, int M_, int K_, int cb_stride_,
-                                                         int cb0_, int cb1_, int cb2_, int cb3_,
-                                                         const _Float16* scales_, _Float16* y_) {
-  // leading scalars, not the struct: the first 14 dwords of the arguments arrive preloaded in scalar registers
+__global__ __launch_bounds__(256) void aqlm_matvec_kernel(HQ_ARGS24) {
+  // the first 14 dwords of the arguments arrive preloaded in scalar registers: all but scales and y
+  HqReader r(HQ_PASS24);
   AqlmArgs a;
-  a.codes = codes_; a.codebooks = codebooks_; a.scales = scales_; a.x = x_; a.y = y_;
-  a.M = M_; a.K = K_; a.cb_stride = cb_stride_;
-  a.cb_sizes[0] = cb0_; a.cb_sizes[1] = cb1_; a.cb_sizes[2] = cb2_; a.cb_sizes[3] = cb3_;
+  a.codes = r; a.codebooks = r; a.x = r; a.M = r; a.K = r; a.cb_stride = r;
+  for (int i = 0; i < 4; ++i) a.cb_sizes[i] = r;
+  a.scales = r; a.y = r;
   const int lane = threadIdx.x & 63;
   // Workgroups b, b + 8, b + 16, ... run on the same XCD; inside every 64 of them the row blocks are dealt
   // out so that the eight workgroups whose results share a 128-byte line of y are on one XCD (its L2 then
@@ -191,8 +190,8 @@ extern "C" int hq_aqlm_matvec(const int16_t* codes, const void* codebooks, const
   const bool lds = K <= (rows > 1 || split ? kMaxLdsK : 8192);
   const size_t smem = lds ? (size_t)aqlm_x_stride(K >> 6) * 8 * 16 : 0;
 #define HQ_AQLM_GO(R, L, S)                                                                                                \
-  hipLaunchKernelGGL((aqlm_matvec_kernel<R, L, S>), dim3(blocks), dim3(256), smem, stream, a.codes, a.codebooks, a.x, a.M, \
-                     a.K, a.cb_stride, a.cb_sizes[0], a.cb_sizes[1], a.cb_sizes[2], a.cb_sizes[3], a.scales, a.y)
+  return hq_launch(aqlm_matvec_kernel<R, L, S>, dim3(blocks), dim3(256), smem, stream, a.codes, a.codebooks, a.x, a.M, a.K, \
+                   a.cb_stride, a.cb_sizes[0], a.cb_sizes[1], a.cb_sizes[2], a.cb_sizes[3], a.scales, a.y)
 #define HQ_AQLM_ROWS_GO(R) \
   { if (lds) HQ_AQLM_GO(R, true, false); else HQ_AQLM_GO(R, false, false); }
   if (rows == 4) HQ_AQLM_ROWS_GO(4)
@@ -202,5 +201,4 @@ extern "C" int hq_aqlm_matvec(const int16_t* codes, const void* codebooks, const
   else HQ_AQLM_ROWS_GO(1)
 #undef HQ_AQLM_ROWS_GO
 #undef HQ_AQLM_GO
-  return hq_launch_status();
 }

@@ -51,6 +51,11 @@ struct GemvArgs {
   int rows, n;
   float scale, zp;  // already rounded to fp16 precision
 };
+__device__ __forceinline__ GemvArgs gemv_args(HqReader& r) {
+  GemvArgs a;
+  a.mat = r; a.vec = r; a.res = r; a.rows = r; a.n = r; a.scale = r; a.zp = r;
+  return a;
+}
 
 template <int MODE> struct Geom;
 template <> struct Geom<kF16> { static constexpr int kPerUnit = 8, kVecUnits = 1; };   // weights per 16-byte unit
@@ -149,11 +154,9 @@ __device__ __forceinline__ void gemv_finish(const GemvArgs& a, int row0, const f
 }
 
 template <int MODE, int R>
-__global__ __launch_bounds__(256) void gemv_kernel(const char* mat_, const u4v* vec_, _Float16* res_, int rows_, int n_, float scale_,
-                                                  float zp_) {
-  // leading scalars, not the struct: the arguments arrive preloaded in scalar registers
-  GemvArgs a;
-  a.mat = mat_; a.vec = vec_; a.res = res_; a.rows = rows_; a.n = n_; a.scale = scale_; a.zp = zp_;
+__global__ __launch_bounds__(256) void gemv_kernel(HQ_ARGS12) {
+  HqReader args(HQ_PASS12);
+  const GemvArgs a = gemv_args(args);
   using G = Geom<MODE>;
   const int lane = threadIdx.x & 63;
   const int wave = (blockIdx.x * 256 + threadIdx.x) >> 6;
@@ -189,10 +192,9 @@ __global__ __launch_bounds__(256) void gemv_kernel(const char* mat_, const u4v* 
 // workgroup of SPLIT waves shares R rows, every wave takes every SPLIT-th two-step piece of the columns,
 // and the waves' sums meet in LDS in wave order (deterministic).
 template <int MODE, int R, int SPLIT>
-__global__ __launch_bounds__(SPLIT * 64) void gemv_split_kernel(const char* mat_, const u4v* vec_, _Float16* res_, int rows_,
-                                                                int n_, float scale_, float zp_) {
-  GemvArgs a;
-  a.mat = mat_; a.vec = vec_; a.res = res_; a.rows = rows_; a.n = n_; a.scale = scale_; a.zp = zp_;
+__global__ __launch_bounds__(SPLIT * 64) void gemv_split_kernel(HQ_ARGS12) {
+  HqReader args(HQ_PASS12);
+  const GemvArgs a = gemv_args(args);
   using G = Geom<MODE>;
   __shared__ float part[SPLIT][R + 1];
   const int lane = threadIdx.x & 63;
@@ -276,22 +278,23 @@ __device__ __forceinline__ void row_sums(const float (&s)[R], float (&w)[R / 4])
 // its piece of the vector, which it loads and prepares once, by R rows: R loads and it ends (see below why that streams
 // best).  Memory-bound: 28672 x 16384 int4 runs at 6.6 TB/s, 5.6 with the vector in LDS.  Eight waves per SIMD need 64 registers.
 template <int MODE, int R>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void gemv_columns_kernel(const char* mat_, const u4v* vec_, _Float16* res_, int rows_, int n_,
-                                                            float scale_, float zp_) {
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void gemv_columns_kernel(HQ_ARGS12) {
+  HqReader args(HQ_PASS12);
+  const GemvArgs a = gemv_args(args);
   using G = Geom<MODE>;
   __shared__ float part[16][R + 1];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = blockIdx.x * R;
-  const int units = n_ / G::kPerUnit;
+  const int units = a.n / G::kPerUnit;
   const int u = wv * 64 + lane, uc = min(u, units - 1);
   const size_t row_bytes = (size_t)units * 16;
   u4v m[R], v[G::kVecUnits];
 #pragma unroll
-  for (int i = 0; i < G::kVecUnits; ++i) v[i] = vec_[(size_t)uc * G::kVecUnits + i];
+  for (int i = 0; i < G::kVecUnits; ++i) v[i] = a.vec[(size_t)uc * G::kVecUnits + i];
 #pragma unroll
   for (int r = 0; r < R; ++r)
-    m[r] = __builtin_nontemporal_load(reinterpret_cast<const u4v*>(mat_ + (size_t)min(row0 + r, rows_ - 1) * row_bytes) + uc);
+    m[r] = __builtin_nontemporal_load(reinterpret_cast<const u4v*>(a.mat + (size_t)min(row0 + r, a.rows - 1) * row_bytes) + uc);
   float acc[R], acc16[R], vsum = 0.f;
 #pragma unroll
   for (int r = 0; r < R; ++r) acc[r] = acc16[r] = 0.f;
@@ -310,16 +313,16 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
     if (lane == 0) part[wv][R] = vs;
   }
   __syncthreads();
-  if (threadIdx.x < R && row0 + (int)threadIdx.x < rows_) {
+  if (threadIdx.x < R && row0 + (int)threadIdx.x < a.rows) {
     const int waves = blockDim.x >> 6;
     float s = 0.f, vs = 0.f;
     for (int k = 0; k < waves; ++k) {
       s += part[k][threadIdx.x];
       if (MODE != kF16) vs += part[k][R];
     }
-    if (MODE == kI8) s = scale_ * (s - zp_ * vs);
-    if (MODE == kI4) s = scale_ * (s * 16777216.f - zp_ * vs);  // codes were fp16 subnormals code * 2^-24
-    res_[row0 + threadIdx.x] = (_Float16)s;
+    if (MODE == kI8) s = a.scale * (s - a.zp * vs);
+    if (MODE == kI4) s = a.scale * (s * 16777216.f - a.zp * vs);  // codes were fp16 subnormals code * 2^-24
+    a.res[row0 + threadIdx.x] = (_Float16)s;
   }
 }
 
@@ -339,12 +342,11 @@ __host__ __device__ constexpr int gemv_lds_stride(int units) {
 }
 
 template <int MODE, int R>
-__global__ __launch_bounds__(1024) void gemv_lds_kernel(const char* mat_, const u4v* vec_, _Float16* res_, int rows_, int n_, float scale_,
-                                                       float zp_, int groups) {
-  // leading scalars, not the struct: the arguments arrive preloaded in scalar registers
-  GemvArgs a;
-  a.mat = mat_; a.vec = vec_; a.res = res_; a.rows = rows_; a.n = n_; a.scale = scale_; a.zp = zp_;
+__global__ __launch_bounds__(1024) void gemv_lds_kernel(HQ_ARGS12) {
+  HqReader args(HQ_PASS12);
+  const GemvArgs a = gemv_args(args);
   using G = Geom<MODE>;
+  const int groups = args;
   extern __shared__ u4v vl[];
   const int lane = threadIdx.x & 63;
   const int units = a.n / G::kPerUnit;  // 16-byte units per matrix row
@@ -406,8 +408,8 @@ int launch_gemv_lds(const GemvArgs& a, int cus, hipStream_t stream) {
   if (attr != hipSuccess) return (int)attr;
   const int groups = (a.rows + R - 1) / R;
   const int wgs = (groups + 15) / 16;
-  hipLaunchKernelGGL((gemv_lds_kernel<MODE, R>), dim3(wgs < cus ? wgs : cus), dim3(1024), smem, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp, groups);
-  return hq_launch_status();
+  return hq_launch(gemv_lds_kernel<MODE, R>, dim3(wgs < cus ? wgs : cus), dim3(1024), smem, stream, a.mat, a.vec, a.res, a.rows, a.n,
+                   a.scale, a.zp, groups);
 }
 
 template <int MODE>
@@ -426,6 +428,9 @@ int launch_gemv(const void* mat, const void* vec, void* res, int rows, int n, fl
   a.rows = rows; a.n = n;
   a.scale = (float)(_Float16)scale;  // the reference rounds both to fp16 (src/gemv-hip/gemv.cu:18-19)
   a.zp = (float)(_Float16)zp;
+  auto go = [&](auto kernel, int wgs, dim3 block) {
+    return hq_launch(kernel, dim3(wgs), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
+  };
   // several rows per wave (the vector piece is loaded and prepared once for them) once there are
   // enough rows to fill the chip with such waves
   // (int4 reads four times as many bytes of the vector per byte of the matrix as fp16: rows per wave pay
@@ -459,16 +464,12 @@ int launch_gemv(const void* mat, const void* vec, void* res, int rows, int n, fl
     if ((split == 1 || split == 2) && units <= 1024) {
       const dim3 block(waves * 64);
       constexpr int kMost = MODE == kF16 ? 4 : 8;
-      if (split == 1) hipLaunchKernelGGL((gemv_columns_kernel<MODE, kMost>), dim3((rows + kMost - 1) / kMost), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
-      else hipLaunchKernelGGL((gemv_columns_kernel<MODE, 4>), dim3((rows + 3) / 4), block, 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
-      return hq_launch_status();
+      if (split == 1) return go(gemv_columns_kernel<MODE, kMost>, (rows + kMost - 1) / kMost, block);
+      return go(gemv_columns_kernel<MODE, 4>, (rows + 3) / 4, block);
     }
     const int groups = (rows + 1) / 2;
 #define HQ_GEMV_SPLIT_CASE(S) \
-    if (split == S) { \
-      hipLaunchKernelGGL((gemv_split_kernel<MODE, 2, S>), dim3(groups), dim3(S * 64), 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp); \
-      return hq_launch_status(); \
-    }
+    if (split == S) return go(gemv_split_kernel<MODE, 2, S>, groups, dim3(S * 64));
     HQ_GEMV_SPLIT_CASE(4) HQ_GEMV_SPLIT_CASE(8) HQ_GEMV_SPLIT_CASE(16)
 #undef HQ_GEMV_SPLIT_CASE
   }
@@ -483,14 +484,13 @@ int launch_gemv(const void* mat, const void* vec, void* res, int rows, int n, fl
   constexpr int kMinWaves = MODE == kI4 ? 8 : 16;  // per compute unit
   if (rows >= dev->cus * kMinWaves * RMAX) {
     const int waves = (rows + RMAX - 1) / RMAX;
-    hipLaunchKernelGGL((gemv_kernel<MODE, RMAX>), dim3((waves + 3) / 4), dim3(256), 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
-  } else if (RMAX > 2 && rows >= dev->cus * kMinWaves * 2) {
-    const int waves = (rows + 1) / 2;
-    hipLaunchKernelGGL((gemv_kernel<MODE, 2>), dim3((waves + 3) / 4), dim3(256), 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
-  } else {
-    hipLaunchKernelGGL((gemv_kernel<MODE, 1>), dim3((rows + 3) / 4), dim3(256), 0, stream, a.mat, a.vec, a.res, a.rows, a.n, a.scale, a.zp);
+    return go(gemv_kernel<MODE, RMAX>, (waves + 3) / 4, dim3(256));
   }
-  return hq_launch_status();
+  if (RMAX > 2 && rows >= dev->cus * kMinWaves * 2) {
+    const int waves = (rows + 1) / 2;
+    return go(gemv_kernel<MODE, 2>, (waves + 3) / 4, dim3(256));
+  }
+  return go(gemv_kernel<MODE, 1>, (rows + 3) / 4, dim3(256));
 }
 
 }  // namespace

@@ -298,14 +298,12 @@ constexpr int planes_of_set(int nb, int s) { return nb - 3 * s < 3 ? nb - 3 * s 
 // Against weights as first operand with two digit operands per quad and alpha on every digit (four times the multiply-adds, no
 // split of K), K=4096, N=16384, three planes, group 64 / 32: 11.4 / 12.6 -> 8.2 / 9.6 us.
 template <int NB, int QUADS, int WAVES, bool BIAS, bool RAGGED, bool ONE_ROUND, bool GROUPED>
-__global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(
-    const uint32_t* bW_, const _Float16* x_, const _Float16* alpha_, const _Float16* qbias_, int K_, int N_, int nb_,
-    int G_, int kslice_, int nsplit_, int strict_, _Float16* y_, float* partial_, unsigned* counters_) {
-  // leading scalars, not the struct: the first 14 dwords of the arguments (all that the loads need) arrive
-  // preloaded in scalar registers
+__global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(HQ_ARGS24) {
+  // the first 14 dwords of the arguments (all that the loads need) arrive preloaded in scalar registers
+  HqReader r(HQ_PASS24);
   LutArgs a;
-  a.bW = bW_; a.alpha = alpha_; a.qbias = qbias_; a.x = x_; a.y = y_; a.partial = partial_; a.counters = counters_;
-  a.K = K_; a.N = N_; a.nb = nb_; a.G = G_; a.kslice = kslice_; a.nsplit = nsplit_; a.strict = strict_;
+  a.bW = r; a.x = r; a.alpha = r; a.qbias = r; a.K = r; a.N = r; a.nb = r; a.G = r; a.kslice = r; a.nsplit = r; a.strict = r;
+  a.y = r; a.partial = r; a.counters = r;
   constexpr int SETS = GROUPED ? 1 : (NB + 2) / 3;
   constexpr int MMAX = GROUPED ? NB : 3;                        // MFMAs of a set per quad and 16 columns, at most
   constexpr int COEFS = GROUPED ? NB + (BIAS ? 1 : 0) : SETS;   // what a lane multiplies its digits with, per quad
@@ -652,15 +650,14 @@ int launch_bcq_planes(LutArgs a, bool ragged, int nsplit, hipStream_t stream) {
   const bool one_round = rpw == 1;
 #define HQ_LUT_GO(BIAS, RAG)                                                                                        \
   do {                                                                                                              \
-    if (one_round) hipLaunchKernelGGL((bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, true, GROUPED>), grid, block, smem, stream, \
-                                       a.bW, a.x, a.alpha, a.qbias, a.K, a.N, a.nb, a.G, a.kslice, a.nsplit, a.strict, a.y, a.partial, a.counters); \
-    else hipLaunchKernelGGL((bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, false, GROUPED>), grid, block, smem, stream, \
-                            a.bW, a.x, a.alpha, a.qbias, a.K, a.N, a.nb, a.G, a.kslice, a.nsplit, a.strict, a.y, a.partial, a.counters); \
+    const auto kernel = one_round ? bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, true, GROUPED>                   \
+                                  : bcq_planes_kernel<NB, QUADS, WAVES, BIAS, RAG, false, GROUPED>;                 \
+    return hq_launch(kernel, grid, block, smem, stream, a.bW, a.x, a.alpha, a.qbias, a.K, a.N, a.nb, a.G, a.kslice, a.nsplit, \
+                     a.strict, a.y, a.partial, a.counters);                                                         \
   } while (0)
   if (a.qbias) { if (ragged) HQ_LUT_GO(true, true); else HQ_LUT_GO(true, false); }
   else { if (ragged) HQ_LUT_GO(false, true); else HQ_LUT_GO(false, false); }
 #undef HQ_LUT_GO
-  return hq_launch_status();
 }
 
 // Split of K over workgroups.  Ordinary: rounds of QUADS quads (128 elements of K) per wave, and as many workgroups as there
@@ -777,9 +774,7 @@ extern "C" int hq_lut_gemv(const uint32_t* bW, const void* alpha, const void* q_
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
   if (attr1 != hipSuccess) return (int)attr1;
   if (attr2 != hipSuccess) return (int)attr2;
-  if (pair) hipLaunchKernelGGL(lut_gemv_kernel<2>, dim3(ntiles * nsplit), dim3(256), smem, stream, a);
-  else hipLaunchKernelGGL(lut_gemv_kernel<1>, dim3(ntiles * nsplit), dim3(256), smem, stream, a);
-  return hq_launch_status();
+  return hq_launch_as_is(pair ? lut_gemv_kernel<2> : lut_gemv_kernel<1>, dim3(ntiles * nsplit), dim3(256), smem, stream, a);
 }
 
 extern "C" int hq_lut_gemv_plan(const uint32_t* bW, const void* alpha, const void* q_bias, int K, int N, int nbits,

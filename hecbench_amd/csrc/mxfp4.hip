@@ -93,8 +93,11 @@ __device__ __forceinline__ u4v qdq_unit(const u4v raw) {
 // 13.1 us with nontemporal, 13.8 with plain stores).  units is a multiple of 4, so the four lanes of a group are
 // in range or out of range together and the quad permutes never read an idle lane's data.
 template <bool BF16>
-__global__ __launch_bounds__(256) void mxfp4_qdq_kernel(const u4v* __restrict__ in, u4v* __restrict__ out,
-                                                       int64_t units) {
+__global__ __launch_bounds__(256) void mxfp4_qdq_kernel(HQ_ARGS8) {
+  HqReader r(HQ_PASS8);
+  const u4v* const in = r;
+  u4v* const out = r;
+  const int64_t units = r;
   const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (u >= units) return;
   const u4v res = qdq_unit<BF16>(__builtin_nontemporal_load(in + u));
@@ -117,10 +120,6 @@ extern "C" int hq_mxfp4_qdq(const void* in, void* out, int64_t n_elems, int dtyp
   const int64_t blocks = (units + 255) / 256;
   if (blocks > 0x7fffffffLL) return HQ_ERR_TOO_LARGE;
   if (dtype == HQ_DTYPE_BF16)
-    hipLaunchKernelGGL(mxfp4_qdq_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       reinterpret_cast<const u4v*>(in), reinterpret_cast<u4v*>(out), units);
-  else
-    hipLaunchKernelGGL(mxfp4_qdq_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                       reinterpret_cast<const u4v*>(in), reinterpret_cast<u4v*>(out), units);
-  return hq_launch_status();
+    return hq_launch(mxfp4_qdq_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, units);
+  return hq_launch(mxfp4_qdq_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, units);
 }

@@ -81,10 +81,9 @@ __device__ __forceinline__ void store_tail(const uint32_t* packed, const float* 
 //   MODE 1: blocksize % 8 == 0, not a power of two (one absmax per word, division)
 //   MODE 2: any even blocksize (absmax looked up per element)
 template <int U, int MODE, int NT, bool TAIL>
-__global__ __launch_bounds__(256) void dequant4_kernel(const uint32_t* __restrict__ packed,
-                                                      const float* __restrict__ absmax,
-                                                      u4v* __restrict__ out, int64_t nwords,
-                                                      int blocksize, int shift, int table, int ntail) {
+__device__ __forceinline__ void dequant4_body(const uint32_t* __restrict__ packed, const float* __restrict__ absmax,
+                                              u4v* __restrict__ out, int64_t nwords, int blocksize, int shift, int table,
+                                              int ntail) {
   if (TAIL && blockIdx.x == gridDim.x - 1) {
     store_tail(packed, absmax, out, nwords, blocksize, table, ntail);
     return;
@@ -127,15 +126,24 @@ __global__ __launch_bounds__(256) void dequant4_kernel(const uint32_t* __restric
   }
 }
 
+template <int U, int MODE, int NT, bool TAIL>
+__global__ __launch_bounds__(256) void dequant4_kernel(HQ_ARGS16) {
+  HqReader r(HQ_PASS16);
+  const uint32_t* const packed = r;
+  const float* const absmax = r;
+  u4v* const out = r;
+  const int64_t nwords = r;
+  const int blocksize = r, shift = r, table = r, ntail = r;
+  dequant4_body<U, MODE, NT, TAIL>(packed, absmax, out, nwords, blocksize, shift, table, ntail);
+}
+
 // Persistent variant of the main path (MODE 0 only, fewer than 2^31 words): a workgroup walks chunks of 256*U
 // words with the next chunk's loads in flight while the current chunk is converted and stored, so the read and
 // the write streams overlap in time.  Index arithmetic is 32-bit; the table offsets of a word's eight codes
 // come from two masked copies of the word (low and high nibble of every byte, times four).
 template <int U, bool TAIL>
-__global__ __launch_bounds__(256) void dequant4_pipelined_kernel(const uint32_t* __restrict__ packed,
-                                                                const float* __restrict__ absmax,
-                                                                u4v* __restrict__ out, uint32_t nwords, int shift,
-                                                                int table, int ntail) {
+__device__ __forceinline__ void dequant4_pipelined_body(const uint32_t* __restrict__ packed, const float* __restrict__ absmax,
+                                                        u4v* __restrict__ out, uint32_t nwords, int shift, int table, int ntail) {
   const uint32_t grid = TAIL ? gridDim.x - 1 : gridDim.x;
   if (TAIL && blockIdx.x == grid) {
     store_tail(packed, absmax, out, nwords, 1 << shift, table, ntail);
@@ -186,11 +194,25 @@ __global__ __launch_bounds__(256) void dequant4_pipelined_kernel(const uint32_t*
   }
 }
 
+template <int U, bool TAIL>
+__global__ __launch_bounds__(256) void dequant4_pipelined_kernel(HQ_ARGS12) {
+  HqReader r(HQ_PASS12);
+  const uint32_t* const packed = r;
+  const float* const absmax = r;
+  u4v* const out = r;
+  const uint32_t nwords = r;
+  const int shift = r, table = r, ntail = r;
+  dequant4_pipelined_body<U, TAIL>(packed, absmax, out, nwords, shift, table, ntail);
+}
+
 // Buffers without the alignment of words and 128-bit stores, and fewer than eight elements: one element per thread.
-__global__ __launch_bounds__(256) void dequant4_element_kernel(const uint8_t* __restrict__ packed,
-                                                              const float* __restrict__ absmax,
-                                                              _Float16* __restrict__ out, int64_t n, int blocksize,
-                                                              int table) {
+__global__ __launch_bounds__(256) void dequant4_element_kernel(HQ_ARGS12) {
+  HqReader r(HQ_PASS12);
+  const uint8_t* const packed = r;
+  const float* const absmax = r;
+  _Float16* const out = r;
+  const int64_t n = r;
+  const int blocksize = r, table = r;
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= n) return;
   const float* tab = table ? c_fp4 : c_nf4;
@@ -229,11 +251,11 @@ extern "C" int hq_dequant_nf4(const uint8_t* packed, const float* absmax, void* 
     if (blocks >= 0x7fffffff) return HQ_ERR_TOO_LARGE;  // one more for the last elements
 #define HQ_NF4_LAUNCH(MM)                                                                                    \
   if (mode == MM && ntail)                                                                                   \
-    hipLaunchKernelGGL((dequant4_kernel<U, MM, NT, true>), dim3((unsigned)blocks + 1), dim3(256), 0, stream, \
-                       pw, absmax, (u4v*)out_fp16, nwords, blocksize, shift, table, ntail);                  \
+    return hq_launch(dequant4_kernel<U, MM, NT, true>, dim3((unsigned)blocks + 1), dim3(256), 0, stream, pw, \
+                     absmax, out_fp16, nwords, blocksize, shift, table, ntail);                              \
   else if (mode == MM)                                                                                       \
-    hipLaunchKernelGGL((dequant4_kernel<U, MM, NT, false>), dim3((unsigned)blocks), dim3(256), 0, stream, pw, \
-                       absmax, (u4v*)out_fp16, nwords, blocksize, shift, table, 0);
+    return hq_launch(dequant4_kernel<U, MM, NT, false>, dim3((unsigned)blocks), dim3(256), 0, stream, pw,    \
+                     absmax, out_fp16, nwords, blocksize, shift, table, 0);
     // Pipelined variant, up to eight workgroups per CU, fewer for larger inputs (us per call, one-shot grid /
     // 2 / 4 / 8 workgroups per CU): 2^19 elements 5.17 / 4.11 / 4.13 / 4.11, 2^21 5.23 / 3.97 / 3.94 / 3.96,
     // 2^23 5.87 / 4.86 / 4.74 / 4.70, 2^24 (4096 x 4096) 7.78 / 7.44 / 7.10 / 7.20, 2^25 14.4 / 13.2 / 13.1 / 13.3,
@@ -246,19 +268,16 @@ extern "C" int hq_dequant_nf4(const uint8_t* packed, const float* absmax, void* 
       const int64_t nch = (nwords + 256 * PU - 1) / (256 * PU);
       const int64_t grid = std::min<int64_t>((int64_t)dev->cus * pipe, nch);
       if (ntail)
-        hipLaunchKernelGGL((dequant4_pipelined_kernel<PU, true>), dim3((unsigned)grid + 1), dim3(256), 0, stream, pw, absmax,
-                           (u4v*)out_fp16, (uint32_t)nwords, shift, table, ntail);
-      else
-        hipLaunchKernelGGL((dequant4_pipelined_kernel<PU, false>), dim3((unsigned)grid), dim3(256), 0, stream, pw, absmax,
-                           (u4v*)out_fp16, (uint32_t)nwords, shift, table, 0);
-    } else {
-    HQ_NF4_LAUNCH(0) HQ_NF4_LAUNCH(1) HQ_NF4_LAUNCH(2)
+        return hq_launch(dequant4_pipelined_kernel<PU, true>, dim3((unsigned)grid + 1), dim3(256), 0, stream, pw, absmax,
+                         out_fp16, (uint32_t)nwords, shift, table, ntail);
+      return hq_launch(dequant4_pipelined_kernel<PU, false>, dim3((unsigned)grid), dim3(256), 0, stream, pw, absmax,
+                       out_fp16, (uint32_t)nwords, shift, table, 0);
     }
+    HQ_NF4_LAUNCH(0) HQ_NF4_LAUNCH(1) HQ_NF4_LAUNCH(2)
 #undef HQ_NF4_LAUNCH
-    return hq_launch_status();
+    return HQ_ERR_BAD_ENUM;
   }
   if ((n_elems + 255) / 256 > 0x7fffffff) return HQ_ERR_TOO_LARGE;
-  hipLaunchKernelGGL(dequant4_element_kernel, dim3((unsigned)((n_elems + 255) / 256)), dim3(256), 0, stream, packed, absmax,
-                     (_Float16*)out_fp16, n_elems, blocksize, table);
-  return hq_launch_status();
+  return hq_launch(dequant4_element_kernel, dim3((unsigned)((n_elems + 255) / 256)), dim3(256), 0, stream, packed, absmax, out_fp16,
+                   n_elems, blocksize, table);
 }

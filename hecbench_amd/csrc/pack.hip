@@ -300,8 +300,7 @@ int launch_quantize4_units(const T* x, uint8_t* packed, float* absmax, int64_t n
   const int shift = __builtin_ctz((unsigned)blocksize);
   const int lanes = SPAN ? 64 : blocksize / 8;
   const auto kernel = table == HQ_TABLE_NF4 ? &quantize4_units_kernel<T, true, UNITS, SPAN> : &quantize4_units_kernel<T, false, UNITS, SPAN>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(256), 0, stream, x, packed, absmax, n, shift, lanes);
-  return hq_launch_status();
+  return hq_launch_as_is(kernel, dim3((unsigned)groups), dim3(256), 0, stream, x, packed, absmax, n, shift, lanes);
 }
 
 // Units per lane.  Blocks up to 512 elements: one, as the wave launcher is the better load scheduler (2^23 fp16 elements
@@ -371,10 +370,6 @@ extern "C" int hq_quantize_4bit(const void* x, int x_dtype, uint8_t* packed, flo
   if ((nblocks + 3) / 4 > 0x7fffffff) return HQ_ERR_TOO_LARGE;
   const dim3 grid((unsigned)((nblocks + 3) / 4));
   if (x_dtype == HQ_DTYPE_F16)
-    hipLaunchKernelGGL(quantize4_kernel<_Float16>, grid, dim3(256), 0, stream, (const _Float16*)x, packed, absmax,
-                       n_elems, blocksize, table);
-  else
-    hipLaunchKernelGGL(quantize4_kernel<float>, grid, dim3(256), 0, stream, (const float*)x, packed, absmax, n_elems,
-                       blocksize, table);
-  return hq_launch_status();
+    return hq_launch_as_is(quantize4_kernel<_Float16>, grid, dim3(256), 0, stream, (const _Float16*)x, packed, absmax, n_elems, blocksize, table);
+  return hq_launch_as_is(quantize4_kernel<float>, grid, dim3(256), 0, stream, (const float*)x, packed, absmax, n_elems, blocksize, table);
 }

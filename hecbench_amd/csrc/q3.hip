@@ -129,15 +129,13 @@ __device__ __forceinline__ constexpr int step_off(int s) { return s * kStepBytes
 // with only the first step's loads at the top of a round and step s + 1 of the next round before the
 // arithmetic of step s.
 template <int WAVES, int STEPS, bool XF16, int ROUNDS, int CPL = 4>
-__global__ __launch_bounds__(WAVES * 64) void q3_matvec_kernel(const uint32_t* w_, const void* x_, int K_, int N_, int gpw_,
-                                                              int nsplit_, int x_f16_, unsigned flags_,
-                                                              const float* scales_, const float* zeros_, float* y_,
-                                                              float* partial_, unsigned* counters_) {
-  // leading scalars rather than the struct: those are preloaded into scalar registers (the first 14 dwords,
-  // i.e. everything the loads and the staging need; y, partial and counters are fetched for the tail)
+__global__ __launch_bounds__(WAVES * 64) void q3_matvec_kernel(HQ_ARGS24) {
+  // the first 14 dwords of the arguments arrive preloaded in scalar registers: everything the loads and the staging need; y,
+  // partial and counters are fetched for the tail
+  HqReader r(HQ_PASS24);
   Q3Args a;
-  a.x = x_; a.w = w_; a.scales = scales_; a.zeros = zeros_; a.y = y_; a.partial = partial_; a.counters = counters_;
-  a.K = K_; a.N = N_; a.gpw = gpw_; a.nsplit = nsplit_; a.x_f16 = x_f16_; a.flags = flags_;
+  a.w = r; a.x = r; a.K = r; a.N = r; a.gpw = r; a.nsplit = r; a.x_f16 = r; a.flags = r; a.scales = r; a.zeros = r; a.y = r;
+  a.partial = r; a.counters = r;
   // LDS: dig[WAVES][STEPS * kStepBytes] | red[WAVES][8][kRedStride] | part[WAVES][64] | xsum[WAVES]
   extern __shared__ uint4 smem[];
   char* dig = reinterpret_cast<char*>(smem);
@@ -476,10 +474,8 @@ int launch_matvec_t(const Q3Args& a, int ntiles, hipStream_t stream) {
   if (attr != hipSuccess) return (int)attr;
   // narrow tiles: whole groups of eight 64-column tiles (the workgroups beyond N leave at once)
   const int gx = CPL == 4 ? ntiles : ((a.N + 63) / 64 + 7) / 8 * 8 * (4 / CPL);
-  hipLaunchKernelGGL((q3_matvec_kernel<WAVES, STEPS, XF16, ROUNDS, CPL>), dim3(gx, a.nsplit), dim3(WAVES * 64), smem,
-                     stream, a.w, a.x, a.K, a.N, a.gpw, a.nsplit, a.x_f16, a.flags, a.scales, a.zeros, a.y, a.partial,
-                     a.counters);
-  return hq_launch_status();
+  return hq_launch(q3_matvec_kernel<WAVES, STEPS, XF16, ROUNDS, CPL>, dim3(gx, a.nsplit), dim3(WAVES * 64), smem, stream, a.w,
+                   a.x, a.K, a.N, a.gpw, a.nsplit, a.x_f16, a.flags, a.scales, a.zeros, a.y, a.partial, a.counters);
 }
 template <int WAVES, int STEPS>
 int launch_matvec(const Q3Args& a, int ntiles, int cus, int cpl, hipStream_t stream) {
@@ -578,12 +574,14 @@ int q3_block_row_blocks(int cus, int K, int N, int batch_M, int nsplit, int rpw)
 // Small launches of more than four rows: row blocks while every workgroup has a compute unit of its own (then 5 to 7 us, ahead of
 // anything else by a quarter), beyond that the one-launch matrix-core kernel of q3_direct.hip.  Workgroups per compute unit that
 // row blocks would need, and both (us): 0.86: 5.3 / 7.3 (26 rows, K=2528, N=1960); 1.04: 6.9 / 6.7 (11 rows, K=1824, N=5640); 1.5: 9.6 /
-// 8.3 (16 rows, K=5120, N=3068); 2.5: 9.9 / 6.8 (12 rows, K=1696, N=13684); 3.7: 14.6 / 8.9 (45 rows, K=3648, N=5028).
+// 8.3 (16 rows, K=5120, N=3068); 2.5: 9.9 / 6.8 (12 rows, K=1696, N=13684); 3.7: 14.6 / 8.9 (45 rows, K=3648, N=5028).  Up to eight rows of
+// a large matrix are as fast either way (7e7 weights and more: 14.3 / 14.4, 19.2 / 19.6, 25.2 / 25.0) and stay where they were.
 bool q3_block_yields(int cus, int K, int N, int batch_M) {
   if (hq_q3_direct_forced()) return true;
   if (batch_M <= 4 || hq_tune(HQ_TUNE_Q3_ROW_BLOCKS, -1) >= 0 || hq_q3_direct_us(cus, K, N, batch_M) > 1e29f) return false;
   int nsplit, rpw;
   q3_block_split(cus, K, N, batch_M, &nsplit, &rpw);
+  if (batch_M <= 8 && (int64_t)K * N >= 70000000) return false;
   return (int64_t)((N + 63) / 64) * nsplit * ((batch_M + 3) / 4) > cus;
 }
 

@@ -366,15 +366,20 @@ __device__ __forceinline__ void q3_block_body(const BlockArgs& a, const int tile
   }
 }
 
+// The arguments in the order of the launches; the first 14 dwords arrive preloaded in scalar registers.
+__device__ __forceinline__ BlockArgs block_args(HqReader& r) {
+  BlockArgs a;
+  a.w = r; a.x = r; a.K = r; a.N = r; a.M = r; a.nsplit = r; a.rpw = r; a.flags = r; a.scales = r; a.zeros = r; a.y = r;
+  a.partial = r; a.counters = r;
+  a.prow = a.M;
+  return a;
+}
+
 // One and two passes: at most 128 registers, so that two workgroups share a compute unit.
 template <int PASSES, bool MULTI>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void q3_block_kernel(
-                   const uint32_t* w_, const _Float16* x_, int K_, int N_, int M_, int nsplit_, int rpw_, unsigned flags_,
-                   const float* scales_, const float* zeros_, float* y_, float* partial_, unsigned* counters_) {
-  // leading scalars, not the struct: the first 14 dwords of the arguments arrive preloaded in scalar registers
-  BlockArgs a;
-  a.x = x_; a.w = w_; a.scales = scales_; a.zeros = zeros_; a.y = y_; a.partial = partial_; a.counters = counters_;
-  a.K = K_; a.N = N_; a.M = M_; a.nsplit = nsplit_; a.rpw = rpw_; a.flags = flags_; a.prow = M_;
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void q3_block_kernel(HQ_ARGS24) {
+  HqReader r(HQ_PASS24);
+  const BlockArgs a = block_args(r);
   q3_block_body<PASSES, MULTI>(a, blockIdx.x, blockIdx.x);
 }
 // More than four rows as several workgroups per column tile, each with up to four rows of its own (one pass):
@@ -382,30 +387,24 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 
 // workgroups of a tile run on one XCD, close in time (workgroup b runs on XCD b mod 8: slot b / 8 of an XCD
 // is row block slot % mblocks of tile (slot / mblocks) * 8 + b mod 8), so the tile's weights come out of
 // that XCD's L2 for all but the first of them.
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void q3_block_rows_kernel(
-                   const uint32_t* w_, const _Float16* x_, int K_, int N_, int M_, int nsplit_, int mblocks_, unsigned flags_,
-                   const float* scales_, const float* zeros_, float* y_, float* partial_, unsigned* counters_) {
-  const int slot = blockIdx.x >> 3;
-  const int tile = (slot / mblocks_) * 8 + (blockIdx.x & 7), mb = slot % mblocks_;
-  if (tile * 64 >= N_) return;  // the last group of eight tiles may be short
-  BlockArgs a;
-  a.x = x_ + (size_t)mb * kPassRows * K_;
-  a.y = y_ + (size_t)mb * kPassRows * N_;
-  a.w = w_; a.scales = scales_; a.zeros = zeros_; a.partial = partial_; a.counters = counters_;
-  a.K = K_; a.N = N_; a.M = min(kPassRows, M_ - mb * kPassRows); a.nsplit = nsplit_; a.rpw = 1; a.flags = flags_; a.prow = kPassRows;
-  q3_block_body<1, false>(a, tile, tile * mblocks_ + mb);
+__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void q3_block_rows_kernel(HQ_ARGS24) {
+  HqReader r(HQ_PASS24);
+  BlockArgs a = block_args(r);
+  const int mblocks = a.rpw, slot = blockIdx.x >> 3;
+  const int tile = (slot / mblocks) * 8 + (blockIdx.x & 7), mb = slot % mblocks;
+  if (tile * 64 >= a.N) return;  // the last group of eight tiles may be short
+  a.x += (size_t)mb * kPassRows * a.K;
+  a.y += (size_t)mb * kPassRows * a.N;
+  a.M = min(kPassRows, a.M - mb * kPassRows); a.rpw = 1; a.prow = kPassRows;
+  q3_block_body<1, false>(a, tile, tile * mblocks + mb);
 }
 // Three passes (9 ... 12 rows) take 127 registers and more time than two workgroups per compute unit leave
 // room for; they run where the launch has at most one workgroup per compute unit and is a matter of latency
 // (K=4096, N=11008: 11.2-12.7 us against the batched GEMM's 14.7; four passes: 16.1 against 14.9 at 16 rows).
 template <int PASSES>
-__global__ __launch_bounds__(kWaves * 64) void q3_block_kernel_many(
-                   const uint32_t* w_, const _Float16* x_, int K_, int N_, int M_, int nsplit_, int rpw_, unsigned flags_,
-                   const float* scales_, const float* zeros_, float* y_, float* partial_, unsigned* counters_) {
-  // leading scalars, not the struct: the first 14 dwords of the arguments arrive preloaded in scalar registers
-  BlockArgs a;
-  a.x = x_; a.w = w_; a.scales = scales_; a.zeros = zeros_; a.y = y_; a.partial = partial_; a.counters = counters_;
-  a.K = K_; a.N = N_; a.M = M_; a.nsplit = nsplit_; a.rpw = rpw_; a.flags = flags_; a.prow = M_;
+__global__ __launch_bounds__(kWaves * 64) void q3_block_kernel_many(HQ_ARGS24) {
+  HqReader r(HQ_PASS24);
+  const BlockArgs a = block_args(r);
   q3_block_body<PASSES, false>(a, blockIdx.x, blockIdx.x);
 }
 
@@ -415,9 +414,8 @@ int launch_block(const BlockArgs& a, hipStream_t stream) {
   static const hipError_t attr =
       hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (attr != hipSuccess) return (int)attr;
-  hipLaunchKernelGGL(KERNEL, dim3((a.N + 63) / 64, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.x, a.K, a.N, a.M,
-                     a.nsplit, a.rpw, a.flags, a.scales, a.zeros, a.y, a.partial, a.counters);
-  return hq_launch_status();
+  return hq_launch(KERNEL, dim3((a.N + 63) / 64, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.x, a.K, a.N, a.M, a.nsplit,
+                   a.rpw, a.flags, a.scales, a.zeros, a.y, a.partial, a.counters);
 }
 
 }  // namespace
@@ -445,9 +443,8 @@ int hq_q3_block_launch(const void* x, const int32_t* qweight, const float* scale
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (attr != hipSuccess) return (int)attr;
     const int groups8 = ((N + 63) / 64 + 7) / 8;
-    hipLaunchKernelGGL(q3_block_rows_kernel, dim3(groups8 * mblocks * 8, nsplit), dim3(kWaves * 64), smem, stream, a.w, a.x,
-                       a.K, a.N, a.M, a.nsplit, mblocks, a.flags, a.scales, a.zeros, a.y, a.partial, a.counters);
-    return hq_launch_status();
+    return hq_launch(q3_block_rows_kernel, dim3(groups8 * mblocks * 8, nsplit), dim3(kWaves * 64), smem, stream, a.w, a.x, a.K, a.N,
+                     a.M, a.nsplit, mblocks, a.flags, a.scales, a.zeros, a.y, a.partial, a.counters);
   }
   if (rpw > 1) return M <= kPassRows ? launch_block<&q3_block_kernel<1, true>>(a, stream) : HQ_ERR_BAD_SHAPE;
   if (M <= kPassRows) return launch_block<&q3_block_kernel<1, false>>(a, stream);

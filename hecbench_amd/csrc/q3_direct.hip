@@ -13,7 +13,7 @@
 //     256 elements of K);
 //   - a tile is small, 32 rows by 64 or 128 columns, and its K is divided among the WAVES of a workgroup, each of which streams
 //     its own operands through a ring of its own in LDS without ever meeting the others before the end (with operands shared
-//     between waves and a barrier per step 13.4 instead of 10.3 us at 341 rows, K=4096+320, N=644);
+//     between waves and a barrier per step 13.4 instead of 10.3 us at 341 rows, K=4416, N=644);
 //   - the rows' sums for the zero term come out of the operand registers (v_dot2_f32_f16).
 // Measured, before -> now: 70 x 4096 x 4096 17 -> 9 us; 341 x 4416 x 644 21.6 -> 10.4; 39 x 4160 x 3176 16.6 -> 9.5; 128 x 4096 x
 // 4096 17.8 -> 9.4; 64 x 4096 x 11008 18.5 -> 12.3; 210 x 6976 x 4592 28 -> 19; 23 x 1952 x 12980 11.7 -> 7.4.
@@ -453,8 +453,7 @@ int launch(const DirectArgs& a, int nwg, hipStream_t stream) {
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_direct_kernel<MB, CB, KS, SA, SW>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, S::kSmem);
   if (attr != hipSuccess) return (int)attr;
-  hipLaunchKernelGGL((q3_direct_kernel<MB, CB, KS, SA, SW>), dim3(nwg), dim3(S::kThreads), S::kSmem, stream, a);
-  return hq_launch_status();
+  return hq_launch_as_is(q3_direct_kernel<MB, CB, KS, SA, SW>, dim3(nwg), dim3(S::kThreads), S::kSmem, stream, a);
 }
 
 }  // namespace

@@ -419,8 +419,7 @@ int launch_tiles(const TileArgs& a, int nwg, hipStream_t stream) {
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_tile_kernel<MB, KS>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, Shape<MB, KS>::kSmem);
   if (attr != hipSuccess) return (int)attr;
-  hipLaunchKernelGGL((q3_tile_kernel<MB, KS>), dim3(nwg), dim3(kThreads), (Shape<MB, KS>::kSmem), stream, a);
-  return hq_launch_status();
+  return hq_launch_as_is(q3_tile_kernel<MB, KS>, dim3(nwg), dim3(kThreads), Shape<MB, KS>::kSmem, stream, a);
 }
 
 }  // namespace

@@ -287,7 +287,6 @@ extern "C" int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* 
   const int64_t cap = (int64_t)dev->cus * hq_tune(HQ_TUNE_Q8_WGS, n > ((int64_t)5 << 20) && n < ((int64_t)1 << 26) ? 2 : 1);
   if (blocks > cap) blocks = cap;
   if (blocks < 1) blocks = 1;
-  hipLaunchKernelGGL(quantize8_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, code, A, out, n,
-                     vec_ok, hq_tune(HQ_TUNE_Q8_FAST, 1));
-  return hq_launch_status();
+  return hq_launch_as_is(quantize8_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, code, A, out, n, vec_ok,
+                   hq_tune(HQ_TUNE_Q8_FAST, 1));
 }
