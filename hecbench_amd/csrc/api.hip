@@ -155,6 +155,9 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   const size_t full_split = tiles * rounds;
   const size_t per_cu = tiles + 2 * (size_t)cus;
   size_t split_floats = (full_split > per_cu ? full_split : per_cu) * 64 * 2;
+  // and a row of 64 per tile and 1024 elements of K where those cut K finest
+  const size_t finest = tiles * (((size_t)max_K + 1023) / 1024) * 64;
+  if (finest > split_floats) split_floats = finest;
   // batches 2 ... 64 on the matvec-like kernel: one partial row per tile, range of K and activation row, at most
   // 8192 of them whatever the shape
   if ((size_t)8192 * 64 > split_floats) split_floats = (size_t)8192 * 64;

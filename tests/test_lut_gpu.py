@@ -78,6 +78,19 @@ def test_ordinary_and_fine_splits(hq, oracle, tunable, split, K, N, nb, group):
     assert rel_err(_run(hq, bW, alpha, None, x, group), oracle.lut_gemv_f64(bW, alpha, None, x, group), FLOOR_F16) <= 2e-3
 
 
+@pytest.mark.parametrize("K,N,nb,group", [(8448, 6401, 2, 256), (10880, 16500, 3, 128), (6528, 16450, 3, 32), (4224, 8127, 4, 64)])
+def test_rounds_apart(hq, oracle, K, N, nb, group):
+    """The default split where workgroups would walk several rounds: few tiles divided already, and a last wave of tiles that
+    leaves the device idle; every round a workgroup, or every quad of a wave."""
+    bW, alpha, qbias, x = oa.make_lut_problem(K + N, K, N, nb, group, False)
+    y = _run(hq, bW, alpha, qbias, x, group)
+    assert np.array_equal(y, _run(hq, bW, alpha, qbias, x, group))
+    cols = np.unique(np.concatenate([np.arange(0, 130), np.arange(N - 130, N)]))
+    ref = oracle.lut_gemv_f64(np.ascontiguousarray(bW[:, :, cols]), np.ascontiguousarray(alpha[:, :, cols]),
+                              np.ascontiguousarray(qbias[:, cols]), x, group)
+    assert rel_err(y[cols], ref, FLOOR_F16) <= 2e-3
+
+
 @pytest.mark.parametrize("split", [1, 2])
 @pytest.mark.parametrize("nb,group", [(1, 32), (3, 64), (4, 32), (5, 64), (6, 32), (8, 64)])
 def test_outlier_in_another_quad(hq, oracle, tunable, split, nb, group):
