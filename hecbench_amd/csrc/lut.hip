@@ -315,7 +315,7 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(HQ_ARGS24) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: addresses of a round stay scalar
   const int c = lane & 15, kb = lane >> 4;
-  const int tile = blockIdx.x;
+  const int tile = RAGGED ? hq_column_tile(blockIdx.x, (a.N + 63) / 64, hq_tiles_share_lines(a.bW, a.N)) : (int)blockIdx.x;
   // K split: workgroup (tile, split) takes the quads of its slice; nquads is where the slice ends
   const int q_begin = blockIdx.y * (a.kslice >> 7);
   const int nquads = min(a.K >> 7, q_begin + (a.kslice >> 7));

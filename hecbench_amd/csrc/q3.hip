@@ -150,9 +150,12 @@ __global__ __launch_bounds__(WAVES * 64) void q3_matvec_kernel(HQ_ARGS24) {
   // neighbouring slots: workgroup b runs on XCD b mod 8.
   constexpr int TW = 16 * CPL, SUB = 4 / CPL;
   const int slot = blockIdx.x >> 3;
-  const int tile = CPL == 4 ? (int)blockIdx.x : ((slot / SUB) * 8 + (int)(blockIdx.x & 7)) * SUB + slot % SUB;
+  const bool share_lines = hq_tiles_share_lines(a.w, a.N);
+  const int ntiles = (a.N + TW - 1) / TW;
+  const int place = CPL == 4 || share_lines ? (int)blockIdx.x : ((slot / SUB) * 8 + (int)(blockIdx.x & 7)) * SUB + slot % SUB;
   const int split = blockIdx.y;
-  if (CPL < 4 && tile * TW >= a.N) return;  // the last group of eight may be short
+  if (CPL < 4 && place >= ntiles) return;  // the last group of eight may be short
+  const int tile = hq_column_tile(place, ntiles, share_lines);
   const int G = a.K >> 5;
   const int g_begin = split * a.gpw;
   const int g_count = min(a.gpw, G - g_begin);

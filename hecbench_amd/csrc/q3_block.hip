@@ -380,7 +380,8 @@ template <int PASSES, bool MULTI>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void q3_block_kernel(HQ_ARGS24) {
   HqReader r(HQ_PASS24);
   const BlockArgs a = block_args(r);
-  q3_block_body<PASSES, MULTI>(a, blockIdx.x, blockIdx.x);
+  const int tile = hq_column_tile(blockIdx.x, (a.N + 63) / 64, hq_tiles_share_lines(a.w, a.N));
+  q3_block_body<PASSES, MULTI>(a, tile, tile);
 }
 // More than four rows as several workgroups per column tile, each with up to four rows of its own (one pass):
 // the rows need no exchange, a launch that leaves compute units idle has room for the workgroups, and the
@@ -391,8 +392,10 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4, 
   HqReader r(HQ_PASS24);
   BlockArgs a = block_args(r);
   const int mblocks = a.rpw, slot = blockIdx.x >> 3;
-  const int tile = (slot / mblocks) * 8 + (blockIdx.x & 7), mb = slot % mblocks;
-  if (tile * 64 >= a.N) return;  // the last group of eight tiles may be short
+  const int place = (slot / mblocks) * 8 + (blockIdx.x & 7), mb = slot % mblocks;
+  const int ntiles = (a.N + 63) / 64;
+  if (place >= ntiles) return;  // the last group of eight tiles may be short
+  const int tile = hq_column_tile(place, ntiles, hq_tiles_share_lines(a.w, a.N));
   a.x += (size_t)mb * kPassRows * a.K;
   a.y += (size_t)mb * kPassRows * a.N;
   a.M = min(kPassRows, a.M - mb * kPassRows); a.rpw = 1; a.prow = kPassRows;
@@ -405,7 +408,8 @@ template <int PASSES>
 __global__ __launch_bounds__(kWaves * 64) void q3_block_kernel_many(HQ_ARGS24) {
   HqReader r(HQ_PASS24);
   const BlockArgs a = block_args(r);
-  q3_block_body<PASSES, false>(a, blockIdx.x, blockIdx.x);
+  const int tile = hq_column_tile(blockIdx.x, (a.N + 63) / 64, hq_tiles_share_lines(a.w, a.N));
+  q3_block_body<PASSES, false>(a, tile, tile);
 }
 
 template <auto KERNEL>

@@ -212,7 +212,8 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(HQ_ARGS28) {
   // Gpad is a multiple of 32 k-groups) and the last of the tile to arrive, or q3_gemm_reduce, adds them up
   const int t_begin = blockIdx.y * a.spp;
   const int nsteps = min(a.spp, a.Gpad / kStepGroups - t_begin);
-  const int col0 = blockIdx.x * kTileN;
+  const int tile = hq_column_tile(blockIdx.x, (a.N + kTileN - 1) / kTileN, hq_tiles_share_lines(a.w, a.N));
+  const int col0 = tile * kTileN;
   const int col = min(col0 + 4 * nl, a.N - 4);
   const size_t row_stride = (size_t)a.N;
   const int n_out = col0 + 4 * nl;
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(HQ_ARGS28) {
   float* red = reinterpret_cast<float*>(lds);
   constexpr int REGION = 32 * kTileN;
   auto share = [&](int split, int m) {  // this lane's raw sums of row m
-    return reinterpret_cast<f4v*>(a.partial + (((size_t)blockIdx.x * a.nsplit + split) * Mpad + m) * kTileN) + nl;
+    return reinterpret_cast<f4v*>(a.partial + (((size_t)tile * a.nsplit + split) * Mpad + m) * kTileN) + nl;
   };
   auto finish = [&](f4v v, int mb, int j) {
     const int m = mb * 32 + 8 * wv + 4 * kb + j;
@@ -338,10 +339,10 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(HQ_ARGS28) {
   __syncthreads();  // also: nobody reads the waves' sums in LDS any more
   unsigned* flag = reinterpret_cast<unsigned*>(lds);
   if (tid == 0) {
-    const unsigned old = __hip_atomic_fetch_add(&a.counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned old = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     *flag = old == (unsigned)(a.nsplit - 1);
     if (old == (unsigned)(a.nsplit - 1))  // ready for the next call
-      __hip_atomic_store(&a.counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&a.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!*flag) return;

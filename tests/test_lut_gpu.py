@@ -91,6 +91,16 @@ def test_rounds_apart(hq, oracle, K, N, nb, group):
     assert rel_err(y[cols], ref, FLOOR_F16) <= 2e-3
 
 
+@pytest.mark.parametrize("K,N,nb,group", [(1024, 97, 3, 128), (4096, 577, 2, 64), (2944, 16810, 3, 64), (8448, 1100, 4, 128)])
+def test_tiles_in_any_order(hq, oracle, K, N, nb, group):
+    """Where column tiles share 128-byte lines they are dealt out in another order; every column is computed as in the matrix
+    with whole tiles, to the bit."""
+    full = (N + 63) // 64 * 64
+    bW, alpha, qbias, x = oa.make_lut_problem(K + N, K, full, nb, group, False)
+    cut = lambda a: np.ascontiguousarray(a[..., :N])
+    assert np.array_equal(_run(hq, cut(bW), cut(alpha), cut(qbias), x, group), _run(hq, bW, alpha, qbias, x, group)[:N])
+
+
 @pytest.mark.parametrize("split", [1, 2])
 @pytest.mark.parametrize("nb,group", [(1, 32), (3, 64), (4, 32), (5, 64), (6, 32), (8, 64)])
 def test_outlier_in_another_quad(hq, oracle, tunable, split, nb, group):

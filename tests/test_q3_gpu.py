@@ -250,3 +250,31 @@ def test_vs_reference_kernels(hq, oracle):
     # and the oracle's restatement of the fp16 kernel agrees with the real one
     o16 = oracle.q3_matvec_f16(x.astype(np.float16), mat, scales, zeros)
     assert rel_err(o16, mul16.cpu().numpy(), FLOOR_F16) <= 2e-3
+
+
+def _cut(t, n, lead=0):
+    """The first n columns, packed, from element `lead` of an allocation."""
+    import torch
+    flat = torch.empty(t.shape[0] * n + lead, dtype=t.dtype, device=t.device)
+    out = flat[lead:].view(t.shape[0], n)
+    out.copy_(t[:, :n])
+    return out
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 512, 68), (1, 1024, 580), (1, 8192, 516), (1, 5760, 2020), (1, 11008, 4100), (2, 4096, 1028),
+                                   (4, 36864, 260), (8, 2048, 2052), (12, 2048, 516), (40, 12288, 8196)])
+def test_tiles_in_any_order(hq, M, K, N):
+    """Where column tiles share 128-byte lines (rows, or the matrix, off a line's start) they are dealt out in another order;
+    every column is computed as in the matrix with whole tiles, to the bit."""
+    import torch
+    full = (N + 63) // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(N)
+    qw = torch.randint(-2**31, 2**31 - 1, (3 * K // 32, full), dtype=torch.int32, device="cuda", generator=g)
+    s = torch.rand(full, device="cuda", generator=g)
+    z = torch.rand(full, device="cuda", generator=g)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    run = (lambda w, n: hq.q3_matvec(x[0], w, s[:n].clone(), z[:n].clone())[None]) if M == 1 else \
+          (lambda w, n: hq.q3_gemm(x, w, s[:n].clone(), z[:n].clone()))
+    want = run(qw, full)
+    assert torch.equal(run(_cut(qw, N), N), want[:, :N])
+    assert torch.equal(run(_cut(qw, full, 4), full), want)
