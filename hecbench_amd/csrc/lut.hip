@@ -685,13 +685,16 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
     fine = (int64_t)ntiles * parts <= 2 * cus && saves > costs;
     if (ntiles > cus && ntiles * 8 <= cus * 11 && rpw > 1 && parts <= 5) fine = true;
     // Several rounds per workgroup, and the exchange paid for anyway (nsplit > 1) or a last wave of tiles that would leave more
-    // than a fifth of the device idle: every round is a workgroup of its own, which has half the registers, so that two share
+    // than a fifth of the device idle (three eighths, where the last round is not half full: a workgroup for little work; 4352 x 25600,
+    // 34 quads, 12.2 / 13.1): every round is a workgroup of its own, which has half the registers, so that two share
     // a compute unit and the work is even whatever the tiles (us, walked / apart: 10880 x 17510 three planes 29.0 / 22.8; 14208 x 16512
     // 28.5 / 21.5; 8448 x 7943 two planes 9.3 / 7.9; 10624 x 25368 group 64 37.8 / 33.2; not 4864 x 26591 one plane, 416 tiles, 7.6 / 9.2;
     // not 4224 x 12997, 204 tiles, 8.7 / 9.8), with three or more planes in small groups one quad per wave (6656 x 18823 group 32 30.9,
     // 25.0, fine 22.3; 13568 x 4444 group 64 14.3, 13.5, 12.1).
     const int waves_of_tiles = (ntiles + cus - 1) / cus;
-    apart = !fine && rpw > 1 && (nsplit > 1 || (ntiles > cus && (int64_t)ntiles * 32 <= (int64_t)waves_of_tiles * cus * 25));
+    const bool full_end = 2 * nquads >= (2 * rounds - 1) * 8 * QUADS;
+    apart = !fine && rpw > 1 &&
+            (nsplit > 1 || (ntiles > cus && (int64_t)ntiles * 32 <= (int64_t)waves_of_tiles * cus * (full_end ? 25 : 20)));
     fine = fine || (apart && GROUPED && NB >= 3);
     fine = hq_tune(HQ_TUNE_LUT_FINE, fine) != 0;
   }
