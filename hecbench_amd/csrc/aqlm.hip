@@ -67,7 +67,9 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(HQ_ARGS24) {
   // out so that the eight workgroups whose results share a 128-byte line of y are on one XCD (its L2 then
   // writes the line back whole instead of eight XCDs writing 16 bytes of it each).
   const int b = blockIdx.x;
-  const int blk = b < (int)(gridDim.x & ~63u) ? ((b & ~63) | ((b & 7) << 3) | ((b >> 3) & 7)) : b;
+  constexpr int kPerBlock = SPLIT ? ROWS : 4 * ROWS;
+  const int blocks = (a.M + kPerBlock - 1) / kPerBlock;  // (as the host: gridDim is a load of its own, ahead of every address)
+  const int blk = b < (blocks & ~63) ? ((b & ~63) | ((b & 7) << 3) | ((b >> 3) & 7)) : b;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = (SPLIT ? blk : blk * 4 + wv) * ROWS;
   const int chunk0 = SPLIT ? wv * 64 : 0, step = SPLIT ? 256 : 64;  // units: this wave's first chunk, and to its next

@@ -84,7 +84,7 @@ template <int U, int MODE, int NT, bool TAIL>
 __device__ __forceinline__ void dequant4_body(const uint32_t* __restrict__ packed, const float* __restrict__ absmax,
                                               u4v* __restrict__ out, int64_t nwords, int blocksize, int shift, int table,
                                               int ntail) {
-  if (TAIL && blockIdx.x == gridDim.x - 1) {
+  if (TAIL && (int64_t)blockIdx.x * (256 * U) >= nwords) {  // (the last workgroup; gridDim is a load of its own)
     store_tail(packed, absmax, out, nwords, blocksize, table, ntail);
     return;
   }

@@ -42,29 +42,26 @@ constexpr uint32_t field_bits(int w, int first, int n) {
   return m;
 }
 
-// A wave multiplies MB 32-row blocks by CB times 32 columns over its own part of every step of K (64 elements of 64 KS); the KS
-// waves of a workgroup share a tile of 32 MB x 32 CB results and meet once, at its end.  Nothing a wave loads is read by another:
-// each streams its operands through ST stages of LDS of its own, without a barrier.
-template <int MB, int CB, int KS, int SA, int SW>
+// A wave multiplies 32 rows by CB times 32 columns over its own part of every step of K (64 elements of 64 KS); the KS waves of a
+// workgroup share a tile of 32 x 32 CB results and meet once, at its end.  Nothing a wave loads is read by another: each streams
+// its operands through two stages of LDS of its own, without a barrier.
+template <int CB, int KS>
 struct Form {
   static constexpr int kThreads = 64 * KS;
-  static constexpr int kTileM = 32 * MB, kTileN = 32 * CB;
+  static constexpr int kTileM = 32, kTileN = 32 * CB;
   static constexpr int kABytes = kTileM * 128, kWBytes = 6 * kTileN * 4;  // a wave's stage: 128 bytes of every row, six packed rows
   static constexpr int kALoads = kABytes / 1024;           // LDS loads of a stage: activations,
   static constexpr int kWLoads = (kWBytes + 1023) / 1024;  // and packed rows, the last load by half of the lanes if CB is 2
-  static constexpr int kLoads = kALoads + kWLoads;
-  static constexpr int kCols = CB < 4 ? CB : 4, kHalves = CB / kCols;  // a lane's columns: kCols adjacent ones of every 32 kCols
-  static constexpr int kUnits = 4 * MB * CB;               // groups of eight rows, every kCols-th column (of a half)
+  static constexpr int kLoads = kALoads + kWLoads, kStageBytes = kABytes + kWBytes;
+  static constexpr int kUnits = 4 * CB;                    // groups of eight rows, every CB-th column
   static constexpr int kMeetUnits = kUnits * KS > 128 ? 128 / KS : kUnits;  // of which so many meet at a time,
   static constexpr int kRounds = kUnits / kMeetUnits, kFinal = kMeetUnits / KS;  // and a wave finishes some of them
-  static constexpr int kWaveBytes = SA * kABytes + SW * kWBytes, kRing = KS * kWaveBytes, kMeet = KS * kMeetUnits * 1024;
+  static constexpr int kWaveBytes = 2 * kStageBytes, kRing = KS * kWaveBytes, kMeet = KS * kMeetUnits * 1024;
   static constexpr int kBulk = kRing > kMeet ? kRing : kMeet;
   static constexpr int kSums = 2 * KS * kTileM;            // floats: parts of the row sums
   static constexpr int kSmem = kBulk + (kSums + kTileM) * 4 + 16;
-  static constexpr int kPerSimd = MB * CB > 8 ? 1 : 2;    // waves
   static_assert(KS % 2 == 0, "odd parts of K enter negated");
-  static constexpr int kInFlight = (SA - 1) * kLoads + (SW > SA ? kWLoads : 0);  // loads behind the next step's operands
-  static_assert(SW >= SA && kInFlight < 64, "the wait counts them");
+  static_assert(CB == 2 || CB == 4, "a lane's columns are one LDS read");
   static_assert(kSmem <= 160 * 1024, "LDS");
 };
 
@@ -76,24 +73,28 @@ struct DirectArgs {
   float* out;
   float* partial;      // [tile][nshare][kTileM * kTileN]
   unsigned* counters;  // [tile], zero between calls
-  int M, N, K, nmt, T, nshare, L;  // row tiles; steps of K, shares of L steps each
+  int M, N, K, nmt, T, nshare, L, nwg;  // row tiles; steps of K, shares of L steps each; workgroups
   unsigned flags;
 };
 
-template <int MB, int CB, int KS, int SA, int SW>
-__global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void q3_direct_kernel(DirectArgs a) {
-  using S = Form<MB, CB, KS, SA, SW>;
-  constexpr int C = S::kCols, H = S::kHalves;
-  typedef uint32_t wv_t __attribute__((ext_vector_type(C)));
+template <int CB, int KS>
+__global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
+  // the first 14 dwords of the arguments (all that the loads need) arrive preloaded in scalar registers
+  HqReader r(HQ_PASS24);
+  DirectArgs a;
+  a.w = r; a.x = r; a.M = r; a.N = r; a.K = r; a.nmt = r; a.T = r; a.nshare = r; a.L = r; a.nwg = r; a.scales = r; a.zeros = r;
+  a.out = r; a.partial = r; a.counters = r; a.flags = r;
+  using S = Form<CB, KS>;
+  typedef uint32_t wv_t __attribute__((ext_vector_type(CB)));
   extern __shared__ unsigned char lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int kp = __builtin_amdgcn_readfirstlane(tid >> 6);  // part of K
   const int nl = lane & 31, kb = lane >> 5;
-  const int G = a.K >> 5, nwg = gridDim.x;
+  const int G = a.K >> 5;
   // workgroup b runs on XCD b mod 8: an XCD takes consecutive tiles (row tiles of one column tile first), which share
   // weights and activations in its L2
   const int xcd = blockIdx.x & 7;
-  const int v = xcd * (nwg >> 3) + min(xcd, nwg & 7) + (int)(blockIdx.x >> 3);
+  const int v = xcd * (a.nwg >> 3) + min(xcd, a.nwg & 7) + (int)(blockIdx.x >> 3);
   const int tile = v / a.nshare, share = v - tile * a.nshare;
   const int ct = __builtin_amdgcn_readfirstlane(tile / a.nmt), mt = __builtin_amdgcn_readfirstlane(tile - ct * a.nmt);
   const int t0 = share * a.L, len = min(a.L, a.T - t0);
@@ -128,19 +129,17 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
     const int groups = shift + (second && missing > 0 ? 1 : 0);
     return (uint32_t)groups * (l < L0 ? 64u : 12u * (uint32_t)a.N);
   };
-  // activations of step ta and packed rows of step tw (negative: none) into their rings' slots
-  auto dma = [&](int sa, int ta, int sw, int tw, bool may_be_last) {
-    const unsigned char* const ax = abase + (size_t)ta * (128 * KS);
-    const unsigned char* const wx = reinterpret_cast<const unsigned char*>(a.w) + (size_t)(6 * KS * tw) * a.N * 4u;
+  // operands of step t into a stage
+  auto dma = [&](int stage, int t, bool may_be_last) {
+    const unsigned char* const ax = abase + (size_t)t * (128 * KS);
+    const unsigned char* const wx = reinterpret_cast<const unsigned char*>(a.w) + (size_t)(6 * KS * t) * a.N * 4u;
 #pragma unroll
     for (int l = 0; l < S::kLoads; ++l) {
       uint32_t o = off[l];
-      if (may_be_last && (l < L0 ? ta : tw) == t_last) o -= back(l);
-      if (l < L0) {
-        if (ta >= 0) load_lds(lds0 + sa * S::kABytes + l * 1024, o, ax);
-      } else if (tw >= 0) {
-        if (CB != 2 || l == L0 || lane < 32) load_lds(lds0 + SA * S::kABytes + sw * S::kWBytes + (l - L0) * 1024, o, wx);
-      }
+      if (may_be_last && t == t_last) o -= back(l);
+      const uint32_t at = lds0 + stage * S::kStageBytes + l * 1024;
+      if (l < L0) load_lds(at, o, ax);
+      else if (CB != 2 || l == L0 || lane < 32) load_lds(at, o, wx);
     }
   };
   // waits until at most n of this wave's loads are in flight
@@ -148,39 +147,31 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
   };
 
-  f16v acc[MB][CB];
+  f16v acc[CB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb)
+  for (int q = 0; q < CB; ++q)
 #pragma unroll
-    for (int q = 0; q < CB; ++q)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mb][q][i] = 0.f;
-  float rs[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) rs[mb] = 0.f;
+    for (int i = 0; i < 16; ++i) acc[q][i] = 0.f;
+  float rs = 0.f;
 
   const unsigned char* const ring = lds + kp * S::kWaveBytes;
   const unsigned char* const a_lane = ring + nl * 128;
-  const unsigned char* const w_lane = ring + SA * S::kABytes + (3 * kb * S::kTileN + C * nl) * 4;
-  u4v P[MB][2];
-  auto read_pieces = [&](int slot, int i0) {  // two of the four of the lane's k-group
+  const unsigned char* const w_lane = ring + S::kABytes + (3 * kb * S::kTileN + CB * nl) * 4;
+  u4v P[2];
+  auto read_pieces = [&](int stage, int i0) {  // two of the four of the lane's k-group
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        P[mb][i] = *reinterpret_cast<const u4v*>(a_lane + slot * S::kABytes + mb * 4096 + (((4 * kb + i0 + i) ^ ((nl >> 1) & 7)) * 16));
+      P[i] = *reinterpret_cast<const u4v*>(a_lane + stage * S::kStageBytes + (((4 * kb + i0 + i) ^ ((nl >> 1) & 7)) * 16));
   };
-  struct Words { wv_t v[3][H]; };
-  auto read_w = [&](int slot, int t, bool may_be_last, Words& dst) {
+  struct Words { wv_t v[3]; };
+  auto read_w = [&](int stage, int t, bool may_be_last, Words& dst) {
     const bool real = !may_be_last || 2 * KS * t + 2 * kp + kb < G;
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
+    for (int j = 0; j < 3; ++j) {
+      const wv_t x = *reinterpret_cast<const wv_t*>(w_lane + stage * S::kStageBytes + j * S::kTileN * 4);
 #pragma unroll
-      for (int h = 0; h < H; ++h) {
-        const wv_t x = *reinterpret_cast<const wv_t*>(w_lane + slot * S::kWBytes + (j * S::kTileN + h * 128) * 4);
-#pragma unroll
-        for (int c = 0; c < C; ++c) dst.v[j][h][c] = real ? x[c] : 0u;
-      }
+      for (int c = 0; c < CB; ++c) dst.v[j][c] = real ? x[c] : 0u;
+    }
   };
   // Column q's 32 codes as fp16 numbers code / 8: elements 0..15 the even codes, 16..31 the odd ones (odd parts of K negative).
   const uint32_t neg = kp & 1 ? 0xffffffffu : 0u;
@@ -191,7 +182,7 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
   auto codes = [&](const Words& words, int q) {
     uint32_t w[3];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) w[j] = words.v[j][q / C][q % C];
+    for (int j = 0; j < 3; ++j) w[j] = words.v[j][q];
     u6v f;
     f[0] = (w[0] & keep[0]) | sign[0];
     f[1] = (w[1] & keep[1]) | sign[1];
@@ -202,27 +193,20 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
     return __builtin_bit_cast(u16v, __builtin_amdgcn_cvt_scalef32_pk32_f16_fp6(f, 1.f));
   };
   // and the activations in that order: operand j of a lane's 32, out of pieces 2 (j & 1) and the next
-  auto rows_operand = [&](int j, u4v (&dst)[MB]) {
+  auto rows_operand = [&](int j, u4v& dst) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const u4v& p = P[mb][i >> 1];
-        dst[mb][i] = __builtin_amdgcn_perm(p[2 * (i & 1) + 1], p[2 * (i & 1)], j < 2 ? 0x05040100u : 0x07060302u);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const u4v& p = P[i >> 1];
+      dst[i] = __builtin_amdgcn_perm(p[2 * (i & 1) + 1], p[2 * (i & 1)], j < 2 ? 0x05040100u : 0x07060302u);
+    }
   };
 
-  u4v A[4][MB];
+  u4v A[4];
   u16v B;
   Words w;
-  auto dma_step = [&](int sa, int sw, int s, bool may_be_last) {  // step s's activations and step s + SW - SA's packed rows
-    dma(sa, s < len ? t0 + s : -1, sw, s + SW - SA < len ? t0 + s + SW - SA : -1, may_be_last);
-  };
-#pragma unroll
-  for (int i = 0; i < SW - SA; ++i) dma(0, -1, i, i < len ? t0 + i : -1, true);
-#pragma unroll
-  for (int i = 0; i < SA; ++i) dma_step(i, (i + SW - SA) % SW, i, true);
-  if (len > SW) wait(std::integral_constant<int, S::kInFlight>());
+  dma(0, t0, true);
+  if (len > 1) dma(1, t0 + 1, true);
+  if (len > 1) wait(std::integral_constant<int, S::kLoads>());
   else wait(std::integral_constant<int, 0>());
   read_w(0, t0, true, w);
   read_pieces(0, 0);
@@ -231,26 +215,24 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
   read_pieces(0, 2);
   rows_operand(1, A[1]);
   rows_operand(3, A[3]);
-  int sa = 0, sw = 0, s = 0;
+  int stage = 0, s = 0;
   // A step: column by column of a lane's CB the codes and the products; under the last column the next step's operands come out
-  // of LDS and are made.  MODE 2: loads another stage, 1: perhaps the last of K, 0: none.
+  // of LDS and are made.  MODE 2: loads the step after the next, 1: which may be the last of K, 0: none.
   auto step = [&](auto mode) {
     constexpr int MODE = decltype(mode)::value;
-    const int sa1 = sa + 1 == SA ? 0 : sa + 1, sw1 = sw + 1 == SW ? 0 : sw + 1;
-    // this step's operands are in registers, its places in the rings are free
+    // this step's operands are in registers, its stage is free
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (MODE == 2) dma(sa, t0 + s + SA, sw, t0 + s + SW, false);
-    else if (MODE) dma_step(sa, sw, s + SA, true);
+    if (MODE) dma(stage, t0 + s + 2, MODE == 1);
     __builtin_amdgcn_sched_barrier(0);
+    stage ^= 1;
     const h2 one = MODE == 2 || 2 * KS * (t0 + s) + 2 * kp + kb < G ? h2{(_Float16)1.f, (_Float16)1.f} : h2{(_Float16)0.f, (_Float16)0.f};
 #pragma unroll
     for (int q = 0; q < CB; ++q) {
       B = codes(w, q);
       if (q == CB - 1) {
-        // the next step's operands have to be in LDS (MODE 1 may have left out packed rows)
-        wait(std::integral_constant<int, MODE == 2 ? S::kInFlight : (MODE == 1 ? (SA - 1) * S::kALoads : 0)>());
-        read_pieces(sa1, 0);
-        read_w(sw1, t0 + s + 1, MODE < 2, w);
+        wait(std::integral_constant<int, MODE ? S::kLoads : 0>());  // the next step's operands have to be in LDS
+        read_pieces(stage, 0);
+        read_w(stage, t0 + s + 1, MODE < 2, w);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -258,52 +240,45 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
         constexpr int kOrder[4] = {0, 2, 1, 3};  // operands 0 and 2 are made of the same pieces
         const int j = kOrder[jj];
         const u4v b = {B[4 * j], B[4 * j + 1], B[4 * j + 2], B[4 * j + 3]};
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-          acc[mb][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, A[j][mb]), __builtin_bit_cast(h8, b), acc[mb][q], 0, 0, 0);
+        acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, A[j]), __builtin_bit_cast(h8, b), acc[q], 0, 0, 0);
         if (q == (CB == 2 ? 0 : j & 1))
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)  // the sums of the rows
-              rs[mb] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, (uint32_t)A[j][mb][i]), one, rs[mb], false);
+          for (int i = 0; i < 4; ++i)  // the sums of the rows
+            rs = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, (uint32_t)A[j][i]), one, rs, false);
         if (q == CB - 1) {
           rows_operand(j, A[j]);
-          if (jj == 1) read_pieces(sa1, 2);
+          if (jj == 1) read_pieces(stage, 2);
         }
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    sa = sa1;
-    sw = sw1;
     ++s;
   };
-  while (s < len - SW - 1) step(std::integral_constant<int, 2>());
-  while (s < len - SA) step(std::integral_constant<int, 1>());
+  while (s < len - 3) step(std::integral_constant<int, 2>());
+  while (s < len - 2) step(std::integral_constant<int, 1>());
   while (s < len) step(std::integral_constant<int, 0>());
 
   // ---- the parts of K meet: wave p finishes units p * kFinal and up (no load is in flight into LDS any more: the last steps
   // waited for theirs) ----
   constexpr int F = S::kFinal, R = S::kRounds;
-  constexpr int V = F < C ? F : C;  // adjacent columns of a wave's units
+  constexpr int V = F < CB ? F : CB;  // adjacent columns of a wave's units
   typedef float fv_t __attribute__((ext_vector_type(V)));
   float* const sums = reinterpret_cast<float*>(lds + S::kBulk);  // [2 KS][kTileM], then the rows' sums
   float* const total = sums + S::kSums;
   f4v* const meet = reinterpret_cast<f4v*>(lds) + lane;
-  auto first_row = [&](int r, int i) { return (r * S::kMeetUnits + kp * F + i) / C % (4 * MB) * 8 + 4 * kb; };  // of unit i of round r
-  auto first_col = [&](int r) { return ct * S::kTileN + r * S::kMeetUnits / (4 * MB * C) * 128 + C * nl + kp * F % C; };
+  auto first_row = [&](int r, int i) { return (r * S::kMeetUnits + kp * F + i) / CB * 8 + 4 * kb; };  // of unit i of round r
+  const int first_col = ct * S::kTileN + CB * nl + kp * F % CB;
   f4v fin[R][F];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) sums[(2 * kp + kb) * S::kTileM + mb * 32 + nl] = rs[mb];
+  sums[(2 * kp + kb) * S::kTileM + nl] = rs;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     __syncthreads();  // every wave is done with its stages, and with the round before
 #pragma unroll
     for (int v = 0; v < S::kMeetUnits; ++v) {
-      const int u = r * S::kMeetUnits + v, h = u / (4 * MB * C), mb = u / (4 * C) % MB;
+      const int u = r * S::kMeetUnits + v;
       f4v x;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = acc[mb][h * C + u % C][4 * (u / C % 4) + e];
+      for (int e = 0; e < 4; ++e) x[e] = acc[u % CB][4 * (u / CB) + e];
       meet[(v * KS + kp) * 64] = x;
     }
     if (r == 0 && tid < S::kTileM) {  // (the sums' parts were written ahead of the barrier)
@@ -313,7 +288,7 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
       total[tid] = t;
     }
     __syncthreads();
-    const int nc = min(first_col(r), a.N - V);
+    const int nc = min(first_col, a.N - V);
     const fv_t sc = *reinterpret_cast<const fv_t*>(a.scales + nc), zr = *reinterpret_cast<const fv_t*>(a.zeros + nc);
 #pragma unroll
     for (int i = 0; i < F; ++i) {
@@ -371,7 +346,7 @@ __global__ __launch_bounds__(64 * KS, (Form<MB, CB, KS, SA, SW>::kPerSimd)) void
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int i = 0; i < F; i += V) {
-      const int m0 = mt * S::kTileM + first_row(r, i), n = first_col(r);
+      const int m0 = mt * S::kTileM + first_row(r, i), n = first_col;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if (m0 + e < a.M && n < a.N) {
@@ -407,8 +382,8 @@ struct DirectKind {
   int tm, tn, ks, per_cu;
   float base_us, step_us, share_us, per_share_us;
 };
-constexpr DirectKind kKinds[4] = {{32, 64, 4, 3, 3.83f, 0.385f, 1.36f, 0.17f}, {32, 64, 8, 1, 4.2f, 0.575f, 1.54f, 0.12f},
-                                  {32, 128, 4, 2, 4.06f, 0.574f, 1.2f, 0.35f}, {32, 128, 8, 1, 4.9f, 0.904f, 1.9f, 0.15f}};
+constexpr DirectKind kKinds[4] = {{32, 64, 4, 3, 3.58f, 0.385f, 1.36f, 0.17f}, {32, 64, 8, 1, 3.95f, 0.575f, 1.54f, 0.12f},
+                                  {32, 128, 4, 2, 3.81f, 0.574f, 1.2f, 0.35f}, {32, 128, 8, 1, 4.65f, 0.904f, 1.9f, 0.15f}};
 constexpr int kMaxShares = 8;
 
 DirectPlan direct_plan_of(int cus, int K, int N, int M, int kind, int nshare) {
@@ -447,13 +422,14 @@ DirectPlan direct_plan(int cus, int K, int N, int M, bool undivided) {
   return best;
 }
 
-template <int MB, int CB, int KS, int SA, int SW>
-int launch(const DirectArgs& a, int nwg, hipStream_t stream) {
-  using S = Form<MB, CB, KS, SA, SW>;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_direct_kernel<MB, CB, KS, SA, SW>),
+template <int CB, int KS>
+int launch(const DirectArgs& a, hipStream_t stream) {
+  using S = Form<CB, KS>;
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_direct_kernel<CB, KS>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, S::kSmem);
   if (attr != hipSuccess) return (int)attr;
-  return hq_launch_as_is(q3_direct_kernel<MB, CB, KS, SA, SW>, dim3(nwg), dim3(S::kThreads), S::kSmem, stream, a);
+  return hq_launch(q3_direct_kernel<CB, KS>, dim3(a.nwg), dim3(S::kThreads), S::kSmem, stream, a.w, a.x, a.M, a.N, a.K, a.nmt, a.T,
+                   a.nshare, a.L, a.nwg, a.scales, a.zeros, a.out, a.partial, a.counters, a.flags);
 }
 
 }  // namespace
@@ -502,12 +478,12 @@ int hq_q3_direct_launch(const void* x, const int32_t* qweight, const float* scal
   a.w = reinterpret_cast<const uint32_t*>(qweight);
   a.x = reinterpret_cast<const _Float16*>(x);
   a.scales = scales; a.zeros = zeros; a.out = y;
-  a.M = M; a.N = N; a.K = K; a.nmt = p.nmt; a.T = p.T; a.nshare = p.nshare; a.L = p.L; a.flags = flags;
-  const int nwg = p.ntiles * p.nshare;
+  a.M = M; a.N = N; a.K = K; a.nmt = p.nmt; a.T = p.T; a.nshare = p.nshare; a.L = p.L; a.nwg = p.ntiles * p.nshare;
+  a.flags = flags;
   switch (p.kind) {
-    case 0: return launch<1, 2, 4, 2, 2>(a, nwg, stream);
-    case 1: return launch<1, 2, 8, 2, 2>(a, nwg, stream);
-    case 2: return launch<1, 4, 4, 2, 2>(a, nwg, stream);
-    default: return launch<1, 4, 8, 2, 2>(a, nwg, stream);
+    case 0: return launch<2, 4>(a, stream);
+    case 1: return launch<2, 8>(a, stream);
+    case 2: return launch<4, 4>(a, stream);
+    default: return launch<4, 8>(a, stream);
   }
 }
