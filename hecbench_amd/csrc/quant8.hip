@@ -5,9 +5,9 @@
 // table followed by a midpoint comparison against the neighbour on the side of x
 // (ties keep the pivot).  Bit-exact with the reference for every input.
 // A lane converts four consecutive floats (one 128-bit load) into one packed 32-bit store.  A sorted
-// table (the normal case, checked in the kernel) is served by a bucket table of thresholds built in LDS
+// table (the normal case, checked in the kernel) is served, in large calls, by a bucket table of thresholds built in LDS
 // by every workgroup: one LDS read and about ten vector instructions per element instead of nine reads
-// and over forty; any other table by the descent itself, read from LDS in level order.
+// and over forty; any other table, and every table in small calls, by the descent itself, read from LDS in level order.
 #include "hq_internal.h"
 
 namespace {
@@ -66,6 +66,7 @@ constexpr int kMaxBuckets = 13 * 64 + 66;  // per sign: 12 binades from off to M
 constexpr uint32_t kSlow = 0x7fc00000u;
 
 constexpr int kThreads = 1024;  // one table for sixteen waves, two workgroups per compute unit
+constexpr int kDescentThreads = 512;  // of a workgroup that only descends
 
 struct FastTables {
   uint2 entry[2 * kMaxBuckets];  // slot 2 * idx (x >= +0) or 2 * idx + 1 (sign bit set): {threshold, count}
@@ -152,21 +153,21 @@ constexpr int kAhead = 2;  // 16-byte loads of a thread and step: 64 KB of a ste
 // operations and one random 8-byte LDS read per element.  A thread takes every gridDim.x * 1024-th quad; its first loads
 // are in flight while the tables are built, and a step's go out together while the step before is converted (one by one
 // as registers come free: 118 against 109 us at 2^27; four per thread: 118).
-// us per call, before -> now: 2^16 elements 4.43 -> 4.20, 2^22 8.2 -> 7.8, 10^7 11.8 -> 10.9, 2^24 16.8 -> 16.5, 2^27
-// 109.7 -> 108.6 (6.2 TB/s).
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void quantize8_kernel(
-    const float* __restrict__ code, const float* __restrict__ A, uint8_t* __restrict__ out, int64_t n, int vec_ok, int allow_fast) {
+// us per call, before -> now: 10^7 11.8 -> 10.9, 2^24 16.8 -> 16.5, 2^27 109.7 -> 108.6 (6.2 TB/s).
+// FAST: the bucket table, if the code table is sorted; otherwise every call descends.
+template <bool FAST, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8, 8))) void quantize8_kernel(
+    const float* __restrict__ code, const float* __restrict__ A, uint8_t* __restrict__ out, int64_t n, int vec_ok) {
   __shared__ __align__(16) float s_code[512];
-  __shared__ __align__(16) FastTables ft;
   const int t = threadIdx.x;
   const int64_t nquads = vec_ok ? n / 4 : 0;
-  const int64_t stride = (int64_t)gridDim.x * kThreads;
-  const int64_t t0 = (int64_t)blockIdx.x * kThreads + t;
+  const int64_t stride = (int64_t)gridDim.x * THREADS;
+  const int64_t t0 = (int64_t)blockIdx.x * THREADS + t;
   f4v v[kAhead];
   auto load = [&](int64_t i) { return __builtin_nontemporal_load(reinterpret_cast<const f4v*>(A) + (i < nquads ? i : nquads - 1)); };
   // the table first: a compute unit returns its loads in the order they were issued
   const float ct = code[min(t, 255)], cn = code[min(t + 1, 255)];
-  const float M = fmaxf(fabsf(code[0]), fabsf(code[255]));
+  const float M = FAST ? fmaxf(fabsf(code[0]), fabsf(code[255])) : 0.f;
   const int level = 32 - __builtin_clz((unsigned)min(t, 254) + 1);  // 1..8
   const float ordered = code[((2 * (min(t, 254) + 1 - (1 << (level - 1))) + 1) << (8 - level)) - 1];
   __builtin_amdgcn_sched_barrier(0);
@@ -179,52 +180,59 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(8, 8))
     s_code[t] = ordered;  // level-order slot t: entry ((2j+1) << (8-k)) - 1
     s_code[t < 255 ? 257 + t : 256] = t < 255 ? (cn + ct) * 0.5f : -__builtin_inff();
   }
-  // the fast path wants a sorted table of finite, moderate values (midpoints cannot overflow) with a
-  // usable magnitude
-  Key key;
-  key.scale = 8192.f / M;
-  const float y_top = fmaf(M, key.scale, 2.f);
-  const uint32_t cnt = bucket_of(y_top) + 1;  // index of the overflow bucket
-  key.top = __uint_as_float((__float_as_uint(y_top) & ~((1u << kKeyShift) - 1)) + (1u << kKeyShift));
-  const bool fast = __syncthreads_and((ct <= cn) && fabsf(ct) <= 1e30f) && M >= 1e-30f && allow_fast &&
-                    cnt < (uint32_t)kMaxBuckets;
-  if (fast) {
-    build_fast_tables(ft, ct, cn, key, cnt);
-    const int64_t wave0 = t0 - (t & 63);  // the wave's first quad
-    for (int64_t step = 0; wave0 + step < nquads; step += kAhead * stride) {
-      // the next step's loads go out together, clamped instead of under a branch
-      f4v vn[kAhead];
+  bool fast = false;
+  if constexpr (FAST) {
+    __shared__ __align__(16) FastTables ft;
+    // the fast path wants a sorted table of finite, moderate values (midpoints cannot overflow) with a
+    // usable magnitude
+    Key key;
+    key.scale = 8192.f / M;
+    const float y_top = fmaf(M, key.scale, 2.f);
+    const uint32_t cnt = bucket_of(y_top) + 1;  // index of the overflow bucket
+    key.top = __uint_as_float((__float_as_uint(y_top) & ~((1u << kKeyShift) - 1)) + (1u << kKeyShift));
+    fast = __syncthreads_and((ct <= cn) && fabsf(ct) <= 1e30f) && M >= 1e-30f &&
+                      cnt < (uint32_t)kMaxBuckets;
+    if (fast) {
+      build_fast_tables(ft, ct, cn, key, cnt);
+      const int64_t wave0 = t0 - (t & 63);  // the wave's first quad
+      for (int64_t step = 0; wave0 + step < nquads; step += kAhead * stride) {
+        // the next step's loads go out together, clamped instead of under a branch
+        f4v vn[kAhead];
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) vn[k] = load(t0 + step + (kAhead + k) * stride);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int k = 0; k < kAhead; ++k) vn[k] = load(t0 + step + (kAhead + k) * stride);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) {
-        const int64_t i = t0 + step + k * stride;
-        if (wave0 + step + k * stride >= nquads) break;  // wave-uniform
-        const float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-        uint32_t q[4];
-        uint64_t slow = 0;
-        uint2 en[4];
+        for (int k = 0; k < kAhead; ++k) {
+          const int64_t i = t0 + step + k * stride;
+          if (wave0 + step + k * stride >= nquads) break;  // wave-uniform
+          const float x[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+          uint32_t q[4];
+          uint64_t slow = 0;
+          uint2 en[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) en[e] = ft.entry[bucket_slot(x[e], key)];
+          for (int e = 0; e < 4; ++e) en[e] = ft.entry[bucket_slot(x[e], key)];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          q[e] = en[e].y + (x[e] > __uint_as_float(en[e].x) ? 1u : 0u);
-          // unordered: a flagged bucket or a NaN input
-          slow |= __builtin_amdgcn_fcmpf(__uint_as_float(en[e].y), x[e], 8);  // FCMP_UNO
+          for (int e = 0; e < 4; ++e) {
+            q[e] = en[e].y + (x[e] > __uint_as_float(en[e].x) ? 1u : 0u);
+            // unordered: a flagged bucket or a NaN input
+            slow |= __builtin_amdgcn_fcmpf(__uint_as_float(en[e].y), x[e], 8);  // FCMP_UNO
+          }
+          if (slow) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (q[e] > 255u || x[e] != x[e]) q[e] = quantize_one(s_code, x[e]);
+          }
+          if (i < nquads)
+            __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), reinterpret_cast<uint32_t*>(out) + i);
         }
-        if (slow) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (q[e] > 255u || x[e] != x[e]) q[e] = quantize_one(s_code, x[e]);
-        }
-        if (i < nquads)
-          __builtin_nontemporal_store(q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), reinterpret_cast<uint32_t*>(out) + i);
+        for (int k = 0; k < kAhead; ++k) v[k] = vn[k];
       }
-#pragma unroll
-      for (int k = 0; k < kAhead; ++k) v[k] = vn[k];
     }
   } else {
+    __syncthreads();
+  }
+  if (!fast) {
     // The descent for a quad's four elements at a time, level by level: four independent LDS reads are in flight per level
     // instead of one dependent chain per element, the next step's loads run under them.  Vector instructions bound it,
     // three per level, and close behind the LDS reads.  Unsorted table, us per call, five workgroups of 256 threads with
@@ -281,12 +289,23 @@ extern "C" int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* 
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
   const int vec_ok = !((uintptr_t)A & 15) && !((uintptr_t)out & 3);
-  int64_t blocks = (n / 4 + kThreads - 1) / kThreads;
-  // workgroups per CU (us with one / two: 2^22 elements 7.8 / 8.2, 10^7 12.8 / 11.5, 2^25 31.1 / 31.0, 2^27 108.6 / 118.2):
-  // two fill the CU's queue between the ends, where latency or the order of the stream counts more
-  const int64_t cap = (int64_t)dev->cus * hq_tune(HQ_TUNE_Q8_WGS, n > ((int64_t)5 << 20) && n < ((int64_t)1 << 26) ? 2 : 1);
+  // Building the bucket table takes a workgroup as long as descending for some 24 elements a thread: up to 5 M elements every call
+  // descends, in smaller workgroups, whatever the table (us, bucket table / descent: 2^14 elements 4.9 / 4.2, 2^18 5.75 / 4.2,
+  // 2^20 5.9 / 4.6, 2^21 6.8 / 5.5, 2^22 8.2 / 7.25, 2^23 11.1 / 11.9; workgroups of 256, 512, 1024 threads: 2^20 5.0, 4.6, 4.6; 2^22
+  // 7.4, 7.25, 7.8).  HQ_Q8_FAST: 1 the bucket table, 0 the descent, unset: this rule.
+  constexpr int64_t kDescend = (int64_t)5 << 20;
+  const int mode = hq_tune(HQ_TUNE_Q8_FAST, -1);
+  const bool fast = mode < 0 ? n > kDescend : mode != 0;
+  const int threads = fast ? kThreads : kDescentThreads;
+  int64_t blocks = (n / 4 + threads - 1) / threads;
+  // workgroups per CU (bucket table, us with one / two: 10^7 12.8 / 11.5, 2^25 31.1 / 31.0, 2^27 108.6 / 118.2): two fill the CU's queue
+  // between the ends, where latency or the order of the stream counts more; the descent as many as fit
+  const int per_cu = fast ? (n > kDescend && n < ((int64_t)1 << 26) ? 2 : 1) : 2048 / kDescentThreads;
+  const int64_t cap = (int64_t)dev->cus * hq_tune(HQ_TUNE_Q8_WGS, per_cu);
   if (blocks > cap) blocks = cap;
   if (blocks < 1) blocks = 1;
-  return hq_launch_as_is(quantize8_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, code, A, out, n, vec_ok,
-                   hq_tune(HQ_TUNE_Q8_FAST, 1));
+  if (!fast)
+    return hq_launch_as_is(quantize8_kernel<false, kDescentThreads>, dim3((unsigned)blocks), dim3(threads), 0, stream, code, A, out, n,
+                           vec_ok);
+  return hq_launch_as_is(quantize8_kernel<true, kThreads>, dim3((unsigned)blocks), dim3(threads), 0, stream, code, A, out, n, vec_ok);
 }

@@ -83,6 +83,18 @@ def test_bit_exact_over_tables(hq, oracle, name):
     assert bad.size == 0, (name, A[bad[:8]], got[bad[:8]], want[bad[:8]])
 
 
+@pytest.mark.parametrize("bucket_table", [0, 1])
+@pytest.mark.parametrize("name", ["dynamic", "linear", "duplicates", "tiny", "one_bucket", "minus_zero_entry", "unsorted", "huge", "nan_entry"])
+def test_either_way_at_any_size(hq, oracle, tunable, name, bucket_table):
+    """The descent alone (what small calls take) and the bucket table (what large ones do) at a size where neither is the rule's
+    choice for both, and at lengths around a workgroup's."""
+    tunable("HQ_Q8_FAST", bucket_table)
+    code = _tables(oracle)[name]
+    A = _probe_inputs(code, np.random.default_rng(len(name) + 50))
+    for n in (A.size, 3, 2047, 2048, 2049, 4 * 1024 + 1):
+        assert np.array_equal(_run(hq, code, A[:n]), oracle.quantize_dynamic8(code, A[:n])), n
+
+
 def test_vs_reference_kernel(hq, oracle):
     import torch
     ref = oa.load_ref_hip()
