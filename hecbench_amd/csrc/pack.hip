@@ -112,9 +112,9 @@ __global__ __launch_bounds__(256) void quantize4_kernel(const T* __restrict__ x,
 
 // ---- the 4-bit quantiser's main path ---------------------------------------------------------------------------------
 // Power-of-two blocks of 8 to 4096 elements.  A lane owns units of eight consecutive elements (one or two 128-bit
-// loads, one packed dword out), a wave owns UNITS of them 512 elements apart, so a block lies within one wave: blocks
-// up to 512 elements are blocksize / 8 lanes of one unit, longer ones all lanes of blocksize / 512 units.  The input
-// is read once and stays in registers between the maximum and the codes.
+// loads, one packed dword out), a wave owns UNITS of them 512 elements apart, so a block lies within one workgroup: blocks
+// up to 512 elements are blocksize / 8 lanes of one unit, longer ones all lanes of blocksize / 512 units of one to four waves.  The
+// input is read once and stays in registers between the maximum and the codes.
 //
 // What bounds it: HBM, if the code search stays under 14 lane operations per fp16 element (45 M elements in the 17 us
 // their bytes take).  The search is one LDS read: 32 equal cells over the table's range are narrower than the distance
@@ -122,8 +122,7 @@ __global__ __launch_bounds__(256) void quantize4_kernel(const T* __restrict__ x,
 // The cell of a threshold is computed with the very operations that find the cell of a value, and both are monotone,
 // so every value gets the code the thresholds define, whatever the rounding.  32 cells of 8 bytes are one entry per
 // bank pair: no LDS conflicts beyond equal addresses, which broadcast.
-// Measured, 4096 x 11008, blocksize 64, NF4: fp16 203 -> 18.9 us (6.1 TB/s), fp32 33.9 us (6.1 TB/s); blocksize 4096
-// 20.1 / 36.3 us.  Before: a wave per block, one or two elements per lane, a four-step search in LDS per element.
+// Measured, 4096 x 11008, blocksize 64, NF4: fp16 203 -> 18.9 us (6.1 TB/s), fp32 33.9 us (6.1 TB/s).  Before: a wave per block, one or two elements per lane, a four-step search in LDS per element.
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 
@@ -228,9 +227,9 @@ struct Unit8<float> {
   __device__ float operator[](int i) const { return v[i]; }
 };
 
-// UNITS units per lane; SPAN: one block covers all of them (blocksize = 512 * UNITS), otherwise `lanes` =
-// blocksize / 8 lanes of each unit.
-template <typename T, bool NF4, int UNITS, bool SPAN>
+// UNITS units per lane.  SPAN: the waves that share a block (blocksize = 512 * UNITS * SPAN), one, two or all four; 0: a block is
+// `lanes` = blocksize / 8 lanes of a unit.
+template <typename T, bool NF4, int UNITS, int SPAN>
 __global__ __launch_bounds__(256) void quantize4_units_kernel(const T* __restrict__ x, uint8_t* __restrict__ packed,
                                                              float* __restrict__ absmax, int64_t n, int shift, int lanes) {
   // fp16: 1 / amax is finite and quotients are infinite or NaN only where an input is, which zeroes 1 / amax
@@ -238,8 +237,8 @@ __global__ __launch_bounds__(256) void quantize4_units_kernel(const T* __restric
   constexpr bool SAFE = sizeof(T) == 4;
   __shared__ Cell cells[kCells];
   const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t e0 = wave * (512 * UNITS) + lane * 8;
+  const int wv = threadIdx.x >> 6;
+  const int64_t e0 = ((int64_t)blockIdx.x * 4 + wv) * (512 * UNITS) + lane * 8;
   Unit8<T> u[UNITS];
 #pragma unroll
   for (int i = 0; i < UNITS; ++i) {
@@ -248,7 +247,7 @@ __global__ __launch_bounds__(256) void quantize4_units_kernel(const T* __restric
     else u[i].load_part(x + e, (int)(n - e > 0 ? n - e : 0));
   }
   build_cells<NF4, SAFE>(cells);
-  __syncthreads();
+  if (SPAN <= 1) __syncthreads();
   float am[UNITS];
 #pragma unroll
   for (int i = 0; i < UNITS; ++i) am[i] = u[i].amax();
@@ -256,6 +255,13 @@ __global__ __launch_bounds__(256) void quantize4_units_kernel(const T* __restric
 #pragma unroll
     for (int i = 1; i < UNITS; ++i) am[0] = fmaxf(am[0], am[i]);
     am[0] = group_max(am[0], 64);
+    if (SPAN > 1) {
+      __shared__ float wave_max[4];
+      if (lane == 0) wave_max[wv] = am[0];
+      __syncthreads();
+#pragma unroll
+      for (int w = 1; w < SPAN; ++w) am[0] = fmaxf(am[0], wave_max[wv ^ w]);
+    }
 #pragma unroll
     for (int i = 1; i < UNITS; ++i) am[i] = am[0];
   } else {
@@ -267,7 +273,7 @@ __global__ __launch_bounds__(256) void quantize4_units_kernel(const T* __restric
   for (int i = 0; i < UNITS; ++i) {
     const int64_t e = e0 + 512 * i;
     if (e >= n) continue;
-    if ((lane & (lanes - 1)) == 0 && (!SPAN || i == 0)) absmax[e >> shift] = am[i];
+    if ((lane & (lanes - 1)) == 0 && (!SPAN || i == 0) && (SPAN <= 1 || wv % SPAN == 0)) absmax[e >> shift] = am[i];
     const float inv = am[i] > 0.f ? 1.0f / am[i] : 0.f;
     uint32_t word = 0, sign = 0;
 #pragma unroll
@@ -293,7 +299,7 @@ __global__ __launch_bounds__(256) void quantize4_units_kernel(const T* __restric
   }
 }
 
-template <typename T, int UNITS, bool SPAN>
+template <typename T, int UNITS, int SPAN>
 int launch_quantize4_units(const T* x, uint8_t* packed, float* absmax, int64_t n, int blocksize, int table, hipStream_t stream) {
   const int64_t groups = (n + 2048 * UNITS - 1) / (2048 * UNITS);
   if (groups > 0x7fffffff) return HQ_ERR_TOO_LARGE;
@@ -305,15 +311,21 @@ int launch_quantize4_units(const T* x, uint8_t* packed, float* absmax, int64_t n
 
 // Units per lane.  Blocks up to 512 elements: one, as the wave launcher is the better load scheduler (2^23 fp16 elements
 // 5.2 / 5.5 / 6.5 us with 1 / 2 / 4; fp32 4096 x 11008 33.9 / 36.2 / 37.9), except for large fp16 inputs, where a
-// workgroup's table and barrier weigh more (4096 x 11008: 20.2 / 18.9 / 19.6).
+// workgroup's table and barrier weigh more (4096 x 11008: 20.2 / 18.9 / 19.6).  Longer blocks keep to one (fp32) or two (fp16) units
+// and are shared by the waves of a workgroup, which exchange their maxima at the barrier that the cells need anyway (us with one
+// wave per block, of 2, 4, 8 units a lane / this: blocksize 4096 of 5521 fp16 elements 5.4 / 2.9, 1 M 4.9 / 3.0, 8.4 M 6.9 / 5.7, 45 M
+// 22.5 / 20.3, fp32 38.6 / 35.2; 2048 of 45 M fp16 21.9 / 20.35, fp32 37.4 / 33.4; 1024 fp32 35.2 / 33.7.  One unit of fp16: 2048 22.4,
+// 1024 22.3 instead of 20.3).
 template <typename T>
 int quantize4_units(const T* x, uint8_t* packed, float* absmax, int64_t n, int blocksize, int table, hipStream_t stream) {
-  if (blocksize == 1024) return launch_quantize4_units<T, 2, true>(x, packed, absmax, n, blocksize, table, stream);
-  if (blocksize == 2048) return launch_quantize4_units<T, 4, true>(x, packed, absmax, n, blocksize, table, stream);
-  if (blocksize == 4096) return launch_quantize4_units<T, 8, true>(x, packed, absmax, n, blocksize, table, stream);
+  constexpr bool kHalf = sizeof(T) == 2;
+  constexpr int kUnits = kHalf ? 2 : 1;
+  if (blocksize == 1024) return launch_quantize4_units<T, kUnits, 2 / kUnits>(x, packed, absmax, n, blocksize, table, stream);
+  if (blocksize == 2048) return launch_quantize4_units<T, kUnits, 4 / kUnits>(x, packed, absmax, n, blocksize, table, stream);
+  if (blocksize == 4096) return launch_quantize4_units<T, 2, 4>(x, packed, absmax, n, blocksize, table, stream);
   if (sizeof(T) == 2 && n >= (int64_t)1 << 24)
-    return launch_quantize4_units<T, 2, false>(x, packed, absmax, n, blocksize, table, stream);
-  return launch_quantize4_units<T, 1, false>(x, packed, absmax, n, blocksize, table, stream);
+    return launch_quantize4_units<T, 2, 0>(x, packed, absmax, n, blocksize, table, stream);
+  return launch_quantize4_units<T, 1, 0>(x, packed, absmax, n, blocksize, table, stream);
 }
 
 }  // namespace

@@ -98,3 +98,22 @@ def test_quantize_4bit_units(hq, oracle, n, blocksize, dtype, table):
     wp, wa = oracle.quantize_4bit(x, blocksize, table)
     assert np.array_equal(absmax.cpu().numpy(), wa)
     assert np.array_equal(packed.cpu().numpy(), wp)
+
+
+@pytest.mark.parametrize("table", [0, 1])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("blocksize", [1024, 2048, 4096])
+def test_blocks_shared_by_waves(hq, oracle, blocksize, dtype, table):
+    """Blocks that the waves of a workgroup share: the largest magnitude in every wave's part in turn, a block of zeros,
+    NaN and infinite elements, and lengths that end in any part of the last block."""
+    import torch
+    rng = np.random.default_rng(blocksize + table)
+    x = rng.standard_normal(17 * blocksize).astype(dtype)
+    for b in range(8):  # one peak per eighth of a block
+        x[b * blocksize + (2 * b + 1) * blocksize // 16] = 9.0 + b
+    x[8 * blocksize:9 * blocksize] = 0
+    x[10 * blocksize + 3], x[11 * blocksize - 1] = np.nan, np.inf
+    for n in (17 * blocksize, 16 * blocksize + 1, 12 * blocksize + blocksize // 4 + 5, 9 * blocksize + blocksize // 2, blocksize - 8):
+        got, amax = hq.quantize_4bit(torch.from_numpy(x[:n]).cuda(), blocksize, table)
+        want, wmax = oracle.quantize_4bit(x[:n], blocksize, table)
+        assert np.array_equal(got.cpu().numpy(), want) and np.array_equal(amax.cpu().numpy(), wmax), n
