@@ -63,13 +63,13 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(HQ_ARGS24) {
   for (int i = 0; i < 4; ++i) a.cb_sizes[i] = r;
   a.scales = r; a.y = r;
   const int lane = threadIdx.x & 63;
-  // Workgroups b, b + 8, b + 16, ... run on the same XCD; inside every 64 of them the row blocks are dealt
-  // out so that the eight workgroups whose results share a 128-byte line of y are on one XCD (its L2 then
-  // writes the line back whole instead of eight XCDs writing 16 bytes of it each).
-  const int b = blockIdx.x;
+  // An XCD takes consecutive row blocks: it gathers from one or two of the code books instead of all (each has 1 MB, its L2 4), and the
+  // workgroups whose results share a 128-byte line of y are on one XCD, whose L2 writes the line back whole.  (Dealt out in runs of
+  // eight instead, three code books: 1119 x 2496 6.9 / 5.85 us, 864 x 7360 8.4 / 7.7, 1311 x 9536 11.9 / 10.8, 7513 x 4160 20.4 / 19.9;
+  // one: 778 x 4160 5.5 / 5.3, 4096 x 4096 no difference.)
   constexpr int kPerBlock = SPLIT ? ROWS : 4 * ROWS;
-  const int blocks = (a.M + kPerBlock - 1) / kPerBlock;  // (as the host: gridDim is a load of its own, ahead of every address)
-  const int blk = b < (blocks & ~63) ? ((b & ~63) | ((b & 7) << 3) | ((b >> 3) & 7)) : b;
+  // (the number of workgroups as the host has it: gridDim is a load of its own, ahead of every address, 0.5 us a call)
+  const int blk = hq_column_tile(blockIdx.x, (a.M + kPerBlock - 1) / kPerBlock, true);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int row0 = (SPLIT ? blk : blk * 4 + wv) * ROWS;
   const int chunk0 = SPLIT ? wv * 64 : 0, step = SPLIT ? 256 : 64;  // units: this wave's first chunk, and to its next

@@ -195,7 +195,7 @@ __device__ __forceinline__ float hq_sum_partials(const float* p, size_t stride, 
 // Packed rows that start at any multiple of four or one column (N not a multiple of 32 words): the 128-byte lines at the edges of
 // a column tile belong to its neighbour too.
 __device__ __forceinline__ bool hq_tiles_share_lines(const void* w, int N) { return ((N & 31) | ((int)(uintptr_t)w & 127)) != 0; }
-// Column tile of workgroup x of a row of ntiles workgroups.  Workgroup x runs on XCD x mod 8, so tile x would have its neighbours
+// Column tile (or block of rows) of workgroup x of a row of ntiles workgroups.  Workgroup x runs on XCD x mod 8, so tile x would have its neighbours
 // on two other XCDs, and both would fetch the lines between them from memory.  Where there are such lines an XCD takes consecutive
 // tiles and finds them in its L2; where there are none the plain order stays, which spreads an XCD's reads over more of the memory.
 // (ntiles from the arguments, not from gridDim: that is a load of its own ahead of every address, 0.3 us.)
