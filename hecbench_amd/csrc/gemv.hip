@@ -316,7 +316,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
   }
   __syncthreads();
   if (threadIdx.x < R && row0 + (int)threadIdx.x < a.rows) {
-    const int waves = (units + 63) >> 6;  // as the host (blockDim is a load of its own, here at the exposed end)
+    const int waves = blockDim.x >> 6;  // preloaded behind the plain arguments
     float s = 0.f, vs = 0.f;
     for (int k = 0; k < waves; ++k) {
       s += part[k][threadIdx.x];

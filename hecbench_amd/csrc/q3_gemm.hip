@@ -75,9 +75,10 @@ __device__ __forceinline__ float prep_wave(float v) {
 // with K.  The kernels keep the negated pairs in accumulators of their own (odd waves, odd parts of K) and subtract those at
 // the end, so that the cuts of the two halves cancel.  Error of the result against 64 bits (2-norm): 300 rows, K=4096, N=4100
 // 9.1e-6 -> 1.8e-6; 128 rows, K=8192, N=2048 1.28e-5 -> 1.8e-6; 295 rows, K=1376, N=11252 5.5e-6 -> 1.8e-6; same time.
-__device__ __forceinline__ void q3_gemm_prep_body(const _Float16* __restrict__ A, _Float16* __restrict__ Ap,
-                                                  float* __restrict__ rowsum, float* __restrict__ rowinv, int M, int K, int Mpad,
-                                                  int Gpad, unsigned* __restrict__ counters, int ncounters) {
+__global__ __launch_bounds__(256) void q3_gemm_prep(const _Float16* __restrict__ A, _Float16* __restrict__ Ap,
+                                                   float* __restrict__ rowsum, float* __restrict__ rowinv,
+                                                   int M, int K, int Mpad, int Gpad, unsigned* __restrict__ counters,
+                                                   int ncounters) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int G = K >> 5;
   // Eight consecutive rows share the 128-byte lines of Ap; workgroups b, b + 8, b + 16, ... run on the same
@@ -149,16 +150,6 @@ __device__ __forceinline__ void q3_gemm_prep_body(const _Float16* __restrict__ A
   }
   for (int i = m * 256 + (int)threadIdx.x; i < ncounters; i += Mpad * 256) counters[i] = 0u;
 }
-__global__ __launch_bounds__(256) void q3_gemm_prep(HQ_ARGS16) {
-  HqReader r(HQ_PASS16);
-  const _Float16* const A = r;
-  _Float16* const Ap = r;
-  float *const rowsum = r, *const rowinv = r;
-  const int M = r, K = r, Mpad = r, Gpad = r;
-  unsigned* const counters = r;
-  const int ncounters = r;
-  q3_gemm_prep_body(A, Ap, rowsum, rowinv, M, K, Mpad, Gpad, counters, ncounters);
-}
 
 // Sixteen two-field registers of one column's k-group (see q3_recipe.h).
 __device__ __forceinline__ void unpack16(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t (&a)[16]) {
@@ -197,12 +188,15 @@ struct GemmArgs {
 // depth itself, 2 to 5 steps, changes little: what a workgroup moves through its CU's L1 - all of the
 // re-ordered activations, 1 MB, next to 0.4 MB of weights - bounds the loop, not the latency.)
 template <int MB>  // 32-row blocks of activations
-__global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(HQ_ARGS28) {
-  // the first 14 dwords of the arguments arrive preloaded in scalar registers
-  HqReader r(HQ_PASS28);
+__global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_, const u4v* Ap_, int M_, int K_, int N_,
+                                                             int Gpad_, int nsplit_, int spp_, unsigned flags_,
+                                                             const float* scales_, const float* zeros_,
+                                                             const float* rowsum_, const float* rowinv_, float* out_,
+                                                             float* partial_, unsigned* counters_) {
+  // leading scalars, not the struct: the first 14 dwords of the arguments arrive preloaded in scalar registers
   GemmArgs a;
-  a.w = r; a.Ap = r; a.M = r; a.K = r; a.N = r; a.Gpad = r; a.nsplit = r; a.spp = r; a.scales = r; a.zeros = r; a.rowsum = r;
-  a.rowinv = r; a.out = r; a.partial = r; a.counters = r; a.flags = r;
+  a.w = w_; a.Ap = Ap_; a.rowsum = rowsum_; a.rowinv = rowinv_; a.scales = scales_; a.zeros = zeros_; a.out = out_;
+  a.partial = partial_; a.counters = counters_; a.M = M_; a.K = K_; a.N = N_; a.Gpad = Gpad_; a.nsplit = nsplit_; a.spp = spp_; a.flags = flags_;
   constexpr int Mpad = 32 * MB;
   extern __shared__ u4v lds[];  // used by the final reduction only
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -409,8 +403,10 @@ int launch_gemm(const GemmArgs& a, hipStream_t stream) {
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (attr != hipSuccess) return (int)attr;
   const int ntiles = (a.N + kTileN - 1) / kTileN;
-  const int rc = hq_launch(q3_gemm_kernel<MB>, dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K, a.N,
-                           a.Gpad, a.nsplit, a.spp, a.scales, a.zeros, a.rowsum, a.rowinv, a.out, a.partial, a.counters, a.flags);
+  hipLaunchKernelGGL((q3_gemm_kernel<MB>), dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K,
+                     a.N, a.Gpad, a.nsplit, a.spp, a.flags, a.scales, a.zeros, a.rowsum, a.rowinv, a.out, a.partial,
+                     a.counters);
+  int rc = hq_launch_status();
   if (rc != HQ_OK || a.nsplit == 1 || a.counters) return rc;
   hipLaunchKernelGGL(q3_gemm_reduce, dim3(ntiles, (a.M + 7) / 8 < 8 ? (a.M + 7) / 8 : 8), dim3(256), 0, stream, a, 32 * MB);
   return hq_launch_status();
@@ -449,8 +445,9 @@ GemmPlan gemm_plan(int cus, int K, int N) {
 
 int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad,
                            unsigned* counters, size_t ncounters, hipStream_t stream) {
-  return hq_launch(q3_gemm_prep, dim3((Mpad + 63) / 64 * 64), dim3(256), 0, stream, A, Ap, rowsum, rowinv, M, K, Mpad, Gpad, counters,
-                   (int)ncounters);
+  hipLaunchKernelGGL(q3_gemm_prep, dim3((Mpad + 63) / 64 * 64), dim3(256), 0, stream, reinterpret_cast<const _Float16*>(A),
+                     reinterpret_cast<_Float16*>(Ap), rowsum, rowinv, M, K, Mpad, Gpad, counters, (int)ncounters);
+  return hq_launch_status();
 }
 
 namespace {
