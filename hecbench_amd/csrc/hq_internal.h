@@ -93,8 +93,9 @@ static inline int hq_launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t 
   return e == hipSuccess ? HQ_OK : (int)e;
 }
 template <typename T> struct HqSame { typedef T type; };  // keeps the arguments out of the deduction
-// A kernel that takes its arguments as they are: a structure, which it loads for itself, or pointers whose __restrict__ the
-// generated code turns to account (the 8-bit quantiser of 10^7 floats 10.9 us, 11.7 with packed arguments).
+// A kernel that takes its arguments as they are: a structure, which it loads for itself; pointers whose __restrict__ the generated
+// code turns to account (the 8-bit quantiser of 10^7 floats 10.9 us, 11.7 with packed arguments); or a kernel whose instructions
+// the compiler orders better so (the dense column kernel, the 64-row product) and whose calls wait for the device anyway.
 template <typename... P>
 static inline int hq_launch_as_is(void (*kernel)(P...), dim3 grid, dim3 block, size_t smem, hipStream_t stream, typename HqSame<P>::type... args) {
   void* params[] = {const_cast<void*>(static_cast<const void*>(&args))...};
@@ -194,7 +195,7 @@ __device__ __forceinline__ float hq_sum_partials(const float* p, size_t stride, 
 
 // Packed rows that start at any multiple of four or one column (N not a multiple of 32 words): the 128-byte lines at the edges of
 // a column tile belong to its neighbour too.
-__device__ __forceinline__ bool hq_tiles_share_lines(const void* w, int N) { return ((N & 31) | ((int)(uintptr_t)w & 127)) != 0; }
+__host__ __device__ __forceinline__ bool hq_tiles_share_lines(const void* w, int N) { return ((N & 31) | ((int)(uintptr_t)w & 127)) != 0; }
 // Column tile (or block of rows) of workgroup x of a row of ntiles workgroups.  Workgroup x runs on XCD x mod 8, so tile x would have its neighbours
 // on two other XCDs, and both would fetch the lines between them from memory.  Where there are such lines an XCD takes consecutive
 // tiles and finds them in its L2; where there are none the plain order stays, which spreads an XCD's reads over more of the memory.

@@ -15,8 +15,9 @@
 //     its own operands through a ring of its own in LDS without ever meeting the others before the end (with operands shared
 //     between waves and a barrier per step 13.4 instead of 10.3 us at 341 rows, K=4416, N=644);
 //   - the rows' sums for the zero term come out of the operand registers (v_dot2_f32_f16).
-// Measured, before -> now: 70 x 4096 x 4096 17 -> 9 us; 341 x 4416 x 644 21.6 -> 10.4; 39 x 4160 x 3176 16.6 -> 9.5; 128 x 4096 x
-// 4096 17.8 -> 9.4; 64 x 4096 x 11008 18.5 -> 12.3; 210 x 6976 x 4592 28 -> 19; 23 x 1952 x 12980 11.7 -> 7.4.
+// Measured, before -> now: 70 x 4096 x 4096 17.6 -> 8.7 us; 341 x 4416 x 644 21.6 -> 10.4; 39 x 4160 x 3176 16.6 -> 9.0; 128 x 4096 x
+// 4096 18.0 -> 9.3; 64 x 4096 x 11008 18.4 -> 12.0; 210 x 6976 x 4592 28.7 -> 20.2; 23 x 1952 x 12980 12.6 -> 6.9; 0.3 of each of these
+// by arguments that arrive in registers instead of a structure that is loaded first.
 // Codes that are normal numbers also lose less in the matrix instruction, which aligns the products of a sum by their
 // exponents: error against 64 bits 2e-7 of the result (2-norm) instead of 1.8e-6.
 #include <type_traits>
@@ -373,7 +374,8 @@ struct DirectPlan {
   size_t partial_floats, counters;
 };
 
-// The workgroups and what they cost, fitted to 5700 timings of 520 problems on MI355X (spread about the fit: 7 %): a workgroup
+// The workgroups and what they cost, fitted to 5700 timings of 520 problems on MI355X (spread about the fit: 7 %; the bases 0.25 lower since the arguments come
+// in registers): a workgroup
 // takes base_us and step_us for every step of 64 ks elements; workgroups that share a compute unit take their steps one after
 // the other (their operands come through one queue), beyond per_cu of them in rounds; dividing a tile's K among c workgroups costs
 // share_us + c * per_share_us.  Eight waves per workgroup where every compute unit has but one, four otherwise; 128 columns load

@@ -187,7 +187,9 @@ struct GemmArgs {
 // (Two waves per SIMD with one step in flight measured 38.4 us at M=64, K=8192, N=28672 against 36.2; the
 // depth itself, 2 to 5 steps, changes little: what a workgroup moves through its CU's L1 - all of the
 // re-ordered activations, 1 MB, next to 0.4 MB of weights - bounds the loop, not the latency.)
-template <int MB>  // 32-row blocks of activations
+// MB: 32-row blocks of activations.  SHARED: column tiles share 128-byte lines (hq_column_tile; a kernel of its own, so that nothing
+// stands in front of the other's first loads).
+template <int MB, bool SHARED>
 __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_, const u4v* Ap_, int M_, int K_, int N_,
                                                              int Gpad_, int nsplit_, int spp_, unsigned flags_,
                                                              const float* scales_, const float* zeros_,
@@ -206,7 +208,7 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
   // Gpad is a multiple of 32 k-groups) and the last of the tile to arrive, or q3_gemm_reduce, adds them up
   const int t_begin = blockIdx.y * a.spp;
   const int nsteps = min(a.spp, a.Gpad / kStepGroups - t_begin);
-  const int tile = hq_column_tile(blockIdx.x, (a.N + kTileN - 1) / kTileN, hq_tiles_share_lines(a.w, a.N));
+  const int tile = SHARED ? hq_column_tile(blockIdx.x, (a.N + kTileN - 1) / kTileN, true) : (int)blockIdx.x;
   const int col0 = tile * kTileN;
   const int col = min(col0 + 4 * nl, a.N - 4);
   const size_t row_stride = (size_t)a.N;
@@ -396,17 +398,21 @@ __global__ __launch_bounds__(256) void q3_gemm_reduce(GemmArgs a, int Mpad) {
   }
 }
 
-template <int MB>
-int launch_gemm(const GemmArgs& a, hipStream_t stream) {
+template <int MB, bool SHARED>
+int launch_gemm_t(const GemmArgs& a, int ntiles, hipStream_t stream) {
   const size_t smem = (size_t)kWaves * 32 * kTileN * 4;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_gemm_kernel<MB>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_gemm_kernel<MB, SHARED>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (attr != hipSuccess) return (int)attr;
-  const int ntiles = (a.N + kTileN - 1) / kTileN;
-  hipLaunchKernelGGL((q3_gemm_kernel<MB>), dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K,
+  hipLaunchKernelGGL((q3_gemm_kernel<MB, SHARED>), dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K,
                      a.N, a.Gpad, a.nsplit, a.spp, a.flags, a.scales, a.zeros, a.rowsum, a.rowinv, a.out, a.partial,
                      a.counters);
-  int rc = hq_launch_status();
+  return hq_launch_status();
+}
+template <int MB>
+int launch_gemm(const GemmArgs& a, hipStream_t stream) {
+  const int ntiles = (a.N + kTileN - 1) / kTileN;
+  const int rc = hq_tiles_share_lines(a.w, a.N) ? launch_gemm_t<MB, true>(a, ntiles, stream) : launch_gemm_t<MB, false>(a, ntiles, stream);
   if (rc != HQ_OK || a.nsplit == 1 || a.counters) return rc;
   hipLaunchKernelGGL(q3_gemm_reduce, dim3(ntiles, (a.M + 7) / 8 < 8 ? (a.M + 7) / 8 : 8), dim3(256), 0, stream, a, 32 * MB);
   return hq_launch_status();
