@@ -155,13 +155,19 @@ void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);
 int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
 float hq_q3_tiles_us(int cus, int K, int N, int M);  // estimate of a call, pre-pass included
-// The same product in one launch (small and medium problems): estimate of a call, a test's override, scratch, launch.  Always able
-// to do without scratch.
-float hq_q3_direct_us(int cus, int K, int N, int M);
-bool hq_q3_direct_forced();
-void hq_q3_direct_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
-int hq_q3_direct_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
-                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
+// The same product in one launch (small and medium problems), always able to do without scratch.  Making the plan tries up to 32
+// forms and shares (0.25 us), so whoever chooses this kernel makes it once, after everything that can be decided without it, and
+// hands it to the launch.
+struct HqQ3DirectPlan {
+  int kind, tm, tn, ks, nmt, ntiles, T, nshare, L;
+  float us;  // estimate of a call
+  size_t partial_floats, counters;
+};
+bool hq_q3_direct_can(int K, int N);  // whether the kernel can take the matrix at all
+bool hq_q3_direct_forced();           // a test's override
+HqQ3DirectPlan hq_q3_direct_plan(int cus, int K, int N, int M, bool undivided);
+int hq_q3_direct_launch(HqQ3DirectPlan plan, int cus, const void* x, const int32_t* qweight, const float* scales, const float* zeros,
+                        float* y, int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
 // Resolves the current device's copy of the fixed scratch array (once per device).
 int hq_noalloc_setup(void);
 

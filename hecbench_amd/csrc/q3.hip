@@ -580,8 +580,9 @@ int q3_block_row_blocks(int cus, int K, int N, int batch_M, int nsplit, int rpw)
 // 8.3 (16 rows, K=5120, N=3068); 2.5: 9.9 / 6.8 (12 rows, K=1696, N=13684); 3.7: 14.6 / 8.9 (45 rows, K=3648, N=5028).  Up to eight rows of
 // a large matrix are as fast either way (7e7 weights and more: 14.3 / 14.4, 19.2 / 19.6, 25.2 / 25.0) and stay where they were.
 bool q3_block_yields(int cus, int K, int N, int batch_M) {
+  if (!hq_q3_direct_can(K, N)) return false;
   if (hq_q3_direct_forced()) return true;
-  if (batch_M <= 4 || hq_tune(HQ_TUNE_Q3_ROW_BLOCKS, -1) >= 0 || hq_q3_direct_us(cus, K, N, batch_M) > 1e29f) return false;
+  if (batch_M <= 4 || hq_tune(HQ_TUNE_Q3_ROW_BLOCKS, -1) >= 0) return false;
   int nsplit, rpw;
   q3_block_split(cus, K, N, batch_M, &nsplit, &rpw);
   if (batch_M <= 8 && (int64_t)K * N >= 70000000) return false;
@@ -770,10 +771,9 @@ int hq_q3_workspace_need_impl(int cus, int K, int N, int batch_M, size_t* floats
     *floats = b.split.floats;
     *counters = b.split.nsplit > 1 ? (size_t)b.split.ntiles : 0;
     if (q3_block_yields(cus, K, N, batch_M)) {
-      size_t f, c;
-      hq_q3_direct_need(cus, K, N, batch_M, &f, &c);
-      if (f > *floats) *floats = f;
-      if (c > *counters) *counters = c;
+      const HqQ3DirectPlan d = hq_q3_direct_plan(cus, K, N, batch_M, false);
+      if (d.partial_floats > *floats) *floats = d.partial_floats;
+      if (d.counters > *counters) *counters = d.counters;
     }
     return HQ_OK;
   }
@@ -827,7 +827,8 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
       const Q3BlockPlan b = q3_block_shape(dev->cus, K, N, batch_M, lim);
       if (b.split.nsplit != b.nsplit) return HQ_ERR_BAD_SHAPE;
       if (!b.split.too_large && q3_block_yields(dev->cus, K, N, batch_M))
-        return hq_q3_direct_launch(x, qweight, scales, zeros, y, K, N, batch_M, flags, stream, fixed);
+        return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, batch_M, false), dev->cus, x, qweight, scales, zeros, y, K, N,
+                                   batch_M, flags, stream, fixed);
       rc = q3_split_acquire(b.split, fixed, stream, &sp);
       if (rc != HQ_OK) return rc;
       return hq_q3_block_launch(x, qweight, scales, zeros, y, K, N, batch_M, b.nsplit, b.rpw, b.mblocks, sp.partial,

@@ -368,11 +368,6 @@ __global__ __launch_bounds__(256) void clear_counters(unsigned* p, int n) {
 }
 
 // Host arithmetic of a launch (the launch, the choice between the kernels and the size query share it).
-struct DirectPlan {
-  int kind, tm, tn, ks, nmt, ntiles, T, nshare, L;
-  float us;
-  size_t partial_floats, counters;
-};
 
 // The workgroups and what they cost, fitted to 5700 timings of 520 problems on MI355X (spread about the fit: 7 %; the bases 0.25 lower since the arguments come
 // in registers): a workgroup
@@ -388,9 +383,9 @@ constexpr DirectKind kKinds[4] = {{32, 64, 4, 3, 3.58f, 0.385f, 1.36f, 0.17f}, {
                                   {32, 128, 4, 2, 3.81f, 0.574f, 1.2f, 0.35f}, {32, 128, 8, 1, 4.65f, 0.904f, 1.9f, 0.15f}};
 constexpr int kMaxShares = 8;
 
-DirectPlan direct_plan_of(int cus, int K, int N, int M, int kind, int nshare) {
+HqQ3DirectPlan direct_plan_of(int cus, int K, int N, int M, int kind, int nshare) {
   const DirectKind& kd = kKinds[kind];
-  DirectPlan p;
+  HqQ3DirectPlan p;
   p.kind = kind;
   p.tm = kd.tm; p.tn = kd.tn; p.ks = kd.ks;
   p.nmt = (M + p.tm - 1) / p.tm;
@@ -407,23 +402,6 @@ DirectPlan direct_plan_of(int cus, int K, int N, int M, int kind, int nshare) {
   return p;
 }
 
-DirectPlan direct_plan(int cus, int K, int N, int M, bool undivided) {
-  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: 3 + kind + 10 * shares
-  if (force >= 0 && force % 10 >= 3 && force % 10 < 7)
-    return direct_plan_of(cus, K, N, M, force % 10 - 3, undivided || force < 10 ? 1 : force / 10);
-  DirectPlan best = direct_plan_of(cus, K, N, M, 0, 1);
-  for (int kind = 0; kind < 4; ++kind)
-    for (int c = 1; c <= (undivided ? 1 : kMaxShares); ++c) {
-      const DirectPlan p = direct_plan_of(cus, K, N, M, kind, c);
-      if (p.nshare != c) continue;
-      const int64_t wgs = (int64_t)p.ntiles * c;
-      if (c > 1 && wgs > 2 * cus) break;                       // bounds the workspace: 2 * cus * 32 * 128 floats
-      if (kKinds[kind].per_cu == 1 && wgs > cus) continue;
-      if (p.us < best.us) best = p;
-    }
-  return best;
-}
-
 template <int CB, int KS>
 int launch(const DirectArgs& a, hipStream_t stream) {
   using S = Form<CB, KS>;
@@ -436,31 +414,37 @@ int launch(const DirectArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Estimate of one call (us), and whether the kernel can take it at all: offsets inside a step are 32-bit.
-float hq_q3_direct_us(int cus, int K, int N, int M) {
-  return K > (1 << 24) || N > (1 << 22) ? 1e30f : direct_plan(cus, K, N, M, false).us;
-}
+bool hq_q3_direct_can(int K, int N) { return K <= (1 << 24) && N <= (1 << 22); }  // offsets inside a step are 32-bit
 bool hq_q3_direct_forced() {
-  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);
+  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: 3 + kind + 10 * shares
   return force >= 0 && force % 10 >= 3 && force % 10 < 7;
 }
 
-void hq_q3_direct_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
-  const DirectPlan p = direct_plan(cus, K, N, M, false);
-  *floats = p.partial_floats;
-  *counters = p.counters;
+HqQ3DirectPlan hq_q3_direct_plan(int cus, int K, int N, int M, bool undivided) {
+  if (hq_q3_direct_forced()) {
+    const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);
+    return direct_plan_of(cus, K, N, M, force % 10 - 3, undivided || force < 10 ? 1 : force / 10);
+  }
+  HqQ3DirectPlan best = direct_plan_of(cus, K, N, M, 0, 1);
+  for (int kind = 0; kind < 4; ++kind)
+    for (int c = 1; c <= (undivided ? 1 : kMaxShares); ++c) {
+      const HqQ3DirectPlan p = direct_plan_of(cus, K, N, M, kind, c);
+      if (p.nshare != c) continue;
+      const int64_t wgs = (int64_t)p.ntiles * c;
+      if (c > 1 && wgs > 2 * cus) break;                       // bounds the workspace: 2 * cus * 32 * 128 floats
+      if (kKinds[kind].per_cu == 1 && wgs > cus) continue;
+      if (p.us < best.us) best = p;
+    }
+  return best;
 }
 
-int hq_q3_direct_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
-                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
-  const HqDevice* dev = nullptr;
-  int rc = hq_current_device(&dev);
-  if (rc != HQ_OK) return rc;
-  DirectPlan p = direct_plan(dev->cus, K, N, M, false);
+int hq_q3_direct_launch(HqQ3DirectPlan p, int cus, const void* x, const int32_t* qweight, const float* scales, const float* zeros,
+                        float* y, int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
   // without room for the shares' sums no tile is divided
   if (p.nshare > 1 && (fixed ? p.partial_floats > fixed->tiles_floats || p.counters > fixed->ncounters
                              : hq_workspace_out_of_reach(stream, p.partial_floats, p.counters)))
-    p = direct_plan(dev->cus, K, N, M, true);
+    p = hq_q3_direct_plan(cus, K, N, M, true);
+  int rc = HQ_OK;
   DirectArgs a;
   a.partial = nullptr; a.counters = nullptr;
   if (p.nshare > 1 && fixed) {

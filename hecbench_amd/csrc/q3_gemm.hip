@@ -462,13 +462,14 @@ namespace {
 // rows, K=4896, N=21956 25.5 -> 30.0); beyond, by the two estimates (over 270 timed problems of 97 and more rows the choice
 // costs 0.3 % on average against the better of the two, 15 % at most).  65 to 96 rows that the tiles do not serve were two passes of
 // the 64-row kernel: 78 rows, K=6880, N=584 19.5 -> 8.6.
-bool direct_serves(int cus, int K, int N, int M) {
-  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);
-  if (hq_q3_direct_forced()) return true;
-  const float us = hq_q3_direct_us(cus, K, N, M);
-  if (force >= 0 || us > 1e29f) return false;
-  if (M <= 64) return M <= 32 || (int64_t)K * N < 90000000;
-  return !hq_q3_tiles_serve(cus, K, N, M) || us < hq_q3_tiles_us(cus, K, N, M);
+// The plan is made only where it is looked at: by the estimates, or by the launch of a batch that the kernel serves.
+bool direct_serves(int cus, int K, int N, int M, HqQ3DirectPlan* plan) {
+  if (!hq_q3_direct_can(K, N)) return false;
+  const bool forced = hq_q3_direct_forced();
+  if (!forced && hq_tune(HQ_TUNE_Q3_TILES, -1) >= 0) return false;
+  if (!forced && M > 32 && M <= 64 && (int64_t)K * N >= 90000000) return false;
+  *plan = hq_q3_direct_plan(cus, K, N, M, false);
+  return forced || M <= 64 || !hq_q3_tiles_serve(cus, K, N, M) || plan->us < hq_q3_tiles_us(cus, K, N, M);
 }
 }  // namespace
 
@@ -481,11 +482,10 @@ int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counte
     *floats = p.ap_halves / 2 + 128 + p.partial_floats;
     *counters = p.counters;
   }
-  if (direct_serves(cus, K, N, M)) {
-    size_t f, c;
-    hq_q3_direct_need(cus, K, N, M, &f, &c);
-    if (f > *floats) *floats = f;
-    if (c > *counters) *counters = c;
+  HqQ3DirectPlan d;
+  if (direct_serves(cus, K, N, M, &d)) {
+    if (d.partial_floats > *floats) *floats = d.partial_floats;
+    if (d.counters > *counters) *counters = d.counters;
   }
   return HQ_OK;
 }
@@ -497,8 +497,9 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   const HqDevice* dev = nullptr;
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
-  if (direct_serves(dev->cus, K, N, M) && !(fixed && K > kFixedMaxK))  // (which is refused below)
-    return hq_q3_direct_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
+  HqQ3DirectPlan direct;
+  if (!(fixed && K > kFixedMaxK) && direct_serves(dev->cus, K, N, M, &direct))  // (a longer K is refused below)
+    return hq_q3_direct_launch(direct, dev->cus, x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   bool tiles = hq_q3_tiles_serve(dev->cus, K, N, M);
   if (tiles) {
     // 64 rows at a time need less: under capture without room for all rows' activations, and where the fixed array cannot hold
@@ -510,8 +511,9 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   if (tiles) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   const GemmPlan plan = gemm_plan(dev->cus, K, N);
   if (!fixed && hq_workspace_out_of_reach(stream, plan.ap_halves / 2 + 128 + plan.partial_floats, plan.counters) &&
-      hq_q3_direct_us(dev->cus, K, N, M) < 1e29f)  // under capture without room for these activations: none are needed there
-    return hq_q3_direct_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
+      hq_q3_direct_can(K, N))  // under capture without room for these activations: none are needed there
+    return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, M, false), dev->cus, x, qweight, scales, zeros, y, K, N, M, flags,
+                               stream, fixed);
   const int Gpad = plan.Gpad, nsplit = plan.nsplit, spp = plan.spp;
   const size_t ap_halves = plan.ap_halves, partial_floats = plan.partial_floats;
   _Float16* Ap;
