@@ -168,6 +168,10 @@ bool hq_q3_direct_forced();           // a test's override
 HqQ3DirectPlan hq_q3_direct_plan(int cus, int K, int N, int M, bool undivided);
 int hq_q3_direct_launch(HqQ3DirectPlan plan, int cus, const void* x, const int32_t* qweight, const float* scales, const float* zeros,
                         float* y, int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
+// The kernel of a batch where scratch is no question (so that a test can say what it runs).
+enum HqQ3Kernel { HQ_Q3_KERNEL_BLOCK, HQ_Q3_KERNEL_DIRECT, HQ_Q3_KERNEL_ROWS64, HQ_Q3_KERNEL_TILES };
+int hq_q3_batch_kernel(int cus, int K, int N, int M);
+int hq_q3_gemm_kernel_of(int cus, int K, int N, int M);  // of those that hq_q3_gemm_launch chooses from
 // Resolves the current device's copy of the fixed scratch array (once per device).
 int hq_noalloc_setup(void);
 

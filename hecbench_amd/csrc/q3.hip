@@ -754,6 +754,11 @@ extern "C" int hq_q3_matvec_plan(int K, int N, int batch_M) {
   return rc != HQ_OK ? rc : q3_plan(dev->cus, K, N, batch_M);
 }
 
+int hq_q3_batch_kernel(int cus, int K, int N, int M) {
+  if (q3_plan(cus, K, N, M) != HQ_Q3_PLAN_BLOCK) return hq_q3_gemm_kernel_of(cus, K, N, M);
+  return q3_block_yields(cus, K, N, M) ? HQ_Q3_KERNEL_DIRECT : HQ_Q3_KERNEL_BLOCK;
+}
+
 // Workspace one hq_q3_matvec call takes from its stream on a device of `cus` compute units: the same plan
 // functions as the launch (host arithmetic only, no device is touched).
 int hq_q3_workspace_need_impl(int cus, int K, int N, int batch_M, size_t* floats, size_t* counters) {

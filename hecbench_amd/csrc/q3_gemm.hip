@@ -466,12 +466,18 @@ namespace {
 bool direct_serves(int cus, int K, int N, int M, HqQ3DirectPlan* plan) {
   if (!hq_q3_direct_can(K, N)) return false;
   const bool forced = hq_q3_direct_forced();
-  if (!forced && hq_tune(HQ_TUNE_Q3_TILES, -1) >= 0) return false;
+  if (!forced && hq_tune(HQ_TUNE_Q3_TILES, -1) >= 0) return false;  // tests: the other kernels
   if (!forced && M > 32 && M <= 64 && (int64_t)K * N >= 90000000) return false;
   *plan = hq_q3_direct_plan(cus, K, N, M, false);
   return forced || M <= 64 || !hq_q3_tiles_serve(cus, K, N, M) || plan->us < hq_q3_tiles_us(cus, K, N, M);
 }
 }  // namespace
+
+int hq_q3_gemm_kernel_of(int cus, int K, int N, int M) {
+  HqQ3DirectPlan d;
+  if (direct_serves(cus, K, N, M, &d)) return HQ_Q3_KERNEL_DIRECT;
+  return hq_q3_tiles_serve(cus, K, N, M) ? HQ_Q3_KERNEL_TILES : HQ_Q3_KERNEL_ROWS64;
+}
 
 // What the kernel of the plan takes, or the one that stands in for it where that is more.
 int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {

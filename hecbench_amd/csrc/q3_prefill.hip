@@ -396,8 +396,8 @@ bool few_rows(int cus, int K, int N, int M) {
 
 TilePlan tile_plan(int cus, int K, int N, int M) {
   if (few_rows(cus, K, N, M)) return tile_plan_of(cus, K, N, M, kKinds[2], 0);
-  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: kind + 10 * shares
-  if (force >= 0) return tile_plan_of(cus, K, N, M, kKinds[force % 10 % 3], force / 10);
+  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: kind + 10 * shares (3 to 6 the one-launch kernel's, 9 none in particular)
+  if (force >= 0 && force % 10 < 3) return tile_plan_of(cus, K, N, M, kKinds[force % 10], force / 10);
   TilePlan best = tile_plan_of(cus, K, N, M, kKinds[0], 0);
   for (int i = 1; i < 3; ++i) {
     const TilePlan p = tile_plan_of(cus, K, N, M, kKinds[i], 0);

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from tests import oracle_api as oa
+from tests.q3_kernel import kernel_of
 from tests.tol import FLOOR_F16, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -84,6 +85,7 @@ def test_default_plans(hq, oracle, M, K, N):
     import torch
     from hecbench_amd import _lib
     lib = _lib.load()
+    assert kernel_of(M, K, N) == "direct"
     codes, scales, zeros, A = oa.make_q3_problem(M + K, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
     a, w, s, z = _t(A), _t(mat), _t(scales), _t(zeros)
@@ -103,11 +105,17 @@ def test_default_plans(hq, oracle, M, K, N):
     assert torch.equal(got[1, True], got[0, True] + 3.0)
 
 
-def test_capture_without_any_workspace(hq, oracle):
+@pytest.mark.parametrize("stands_in", [False, True])
+def test_capture_without_any_workspace(hq, oracle, tunable, stands_in):
     """Under capture nothing can be allocated: on a stream that has no workspace the call divides no tile, and replays give the
-    eager result's values to the last bits but the order of the sums."""
+    eager result's values to the last bits but the order of the sums.  The same for a batch of the 64-row kernel, whose re-ordered
+    activations have no place there."""
     import torch
     M, K, N = 39, 4160, 1176
+    if stands_in:
+        tunable("HQ_Q3_SMALL_BATCH", 0)
+        tunable("HQ_Q3_TILES", 9)
+    assert kernel_of(M, K, N) == ("rows64" if stands_in else "direct")
     codes, scales, zeros, A = oa.make_q3_problem(11, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
     a, w, s, z = _t(A), _t(mat), _t(scales), _t(zeros)

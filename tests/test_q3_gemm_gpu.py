@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from tests import oracle_api as oa
+from tests.q3_kernel import kernel_of
 from tests.tol import FLOOR_F16, TOL_F16_ACC, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -12,13 +13,17 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(autouse=True)
 def _the_gemm_kernel_only(tunable):
-    """Small launches of up to 64 rows would take the matvec's four-rows-per-workgroup kernel by default
-    (tests/test_q3_small_batch_gpu.py covers that): this file is about the MFMA GEMM, so every batch takes it."""
+    """Most problems of these sizes would take the matvec's four-rows-per-workgroup kernel (tests/test_q3_small_batch_gpu.py
+    covers that) or the one-launch kernel (tests/test_q3_direct_gpu.py): this file is about the MFMA GEMM behind a pre-pass, so
+    every batch takes it, up to 64 rows on the 64-row kernel, more on the tiles (or 64 at a time)."""
     tunable("HQ_Q3_SMALL_BATCH", 0)
+    tunable("HQ_Q3_TILES", 9)
 
 
 def _run(hq, A, mat, scales, zeros):
     import torch
+    M, K, N = len(A), A.shape[1], mat.shape[1]
+    assert kernel_of(M, K, N) in (("rows64",) if M <= 64 else ("rows64", "tiles")), (M, K, N)
     dev = torch.device("cuda:0")
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
     y = hq.q3_gemm(t(A), t(mat), t(scales), t(zeros))
@@ -64,6 +69,7 @@ def test_split_sums_by_the_last_workgroup(hq, oracle, M, K, N):
     mat = oracle.q3_pack(codes)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
     args = t(A), t(mat), t(scales), t(zeros)
+    assert kernel_of(M, K, N) == "rows64"
     y = hq.q3_gemm(*args)
     for _ in range(3):
         assert torch.equal(y, hq.q3_gemm(*args))
@@ -119,6 +125,27 @@ def test_dynamic_range(hq, oracle, scale_exp):
     for m in (0, 5, 7):
         yv = hq.q3_matvec(t(A[m]), t(mat), t(scales), t(zeros)).cpu().numpy()
         assert rel_err(y[m], yv) <= 5e-3, (scale_exp, m)
+
+
+@pytest.mark.parametrize("M,K,N", [(40, 16384, 8192), (48, 24576, 4096)])
+def test_divided_by_default(hq, oracle, tunable, M, K, N):
+    """Without any knob: 33 to 64 rows of 9e7 weights and more whose column tiles leave compute units idle; four shares of K
+    summed by the last workgroup, eight by the kernel behind."""
+    import torch
+    from hecbench_amd import _lib
+    for knob in (b"HQ_Q3_SMALL_BATCH", b"HQ_Q3_TILES"):
+        assert _lib.load().hq_set_tunable(knob, 0, 1) == 0
+    assert kernel_of(M, K, N) == "rows64"
+    g = torch.Generator(device="cuda:0").manual_seed(K)
+    mat = torch.randint(-2 ** 31, 2 ** 31, (3 * K // 32, N), dtype=torch.int32, device="cuda:0", generator=g)
+    scales = torch.rand(N, device="cuda:0", generator=g).mul_(0.01).add_(0.002)
+    A = torch.empty((M, K), dtype=torch.float16, device="cuda:0").normal_(generator=g)
+    y = hq.q3_gemm(A, mat, scales, scales * 3)
+    assert torch.equal(y, hq.q3_gemm(A, mat, scales, scales * 3))
+    cols = np.unique(np.concatenate([np.arange(0, 68), np.arange(N // 2, N // 2 + 8), np.arange(N - 68, N)]))
+    sc = scales.cpu().numpy()[cols]
+    exact = oracle.q3_gemm(A.cpu().numpy(), np.ascontiguousarray(mat.cpu().numpy()[:, cols]), sc, (scales * 3).cpu().numpy()[cols], mode=0)
+    assert rel_err(y.cpu().numpy()[:, cols], exact, FLOOR_F16) <= 1e-4
 
 
 def test_config4_sampled_columns(hq, oracle):

@@ -15,7 +15,8 @@ MATVEC = {"default": {}, "unsplit": {"HQ_Q3_KSPLIT": 1}, "tiles32": {"HQ_Q3_TILE
           "steps2": {"HQ_Q3_STEPS": 2}}
 LONG_K = {"default": {}, "unsplit": {"HQ_Q3_KSPLIT": 1}, "three_ranges": {"HQ_Q3_KSPLIT": 3}}
 BATCH = {"default": {}, "gemm": {"HQ_Q3_SMALL_BATCH": 0}, "passes": {"HQ_Q3_ROW_BLOCKS": 0},
-         "row_blocks": {"HQ_Q3_ROW_BLOCKS": 1}}
+         "row_blocks": {"HQ_Q3_ROW_BLOCKS": 1}, "pre_pass": {"HQ_Q3_SMALL_BATCH": 0, "HQ_Q3_TILES": 9},
+         "one_launch": {"HQ_Q3_TILES": 5}, "one_launch_halves": {"HQ_Q3_TILES": 25}}
 CASES = [
     (4096, 11008, 1, MATVEC),
     (4096, 11008, 4, BATCH),

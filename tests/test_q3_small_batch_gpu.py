@@ -1,13 +1,14 @@
-"""Batches 2 ... 16 of the GPTQ 3-bit product (hq_q3_matvec with batch_M > 1): batches 2 ... 8 (up to 12 on
-small launches) run on the matvec's matrix-core kernel with every activation as four small fp8 terms under
-one scale per 32 activations (four rows side by side in the operand per pass over the weights, K split across
-workgroups as for batch 1), all others on the batched GEMM.  Every batch size is checked against the CPU oracle through the C ABI,
-and the kernel that ran is asserted through hq_q3_matvec_plan.  The reference has no batched kernel:
+"""Small batches of the GPTQ 3-bit product (hq_q3_matvec with batch_M > 1): batches 2 ... 4, and up to 64 rows while every
+workgroup has a compute unit of its own, run on the matvec's matrix-core kernel with every activation as four small fp8 terms under
+one scale per 32 activations (four rows side by side in the operand per pass over the weights or workgroup, K split across
+workgroups as for batch 1), all others on the batched GEMM's kernels.  Every batch size is checked against the CPU oracle through
+the C ABI, and the kernel that ran is asserted through hq_q3_matvec_plan or the library's own choice.  The reference has no batched kernel:
 the oracle is the matvec formula applied row by row (parity unpinned by the reference)."""
 import numpy as np
 import pytest
 
 from tests import oracle_api as oa
+from tests.q3_kernel import kernel_of
 from tests.tol import FLOOR_F16, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -49,8 +50,9 @@ _EVERY_BATCH = [(M, K, N) for (K, N) in [(512, 16388), (4128, 8192), (1024, 132)
 def test_every_batch_vs_oracle(hq, oracle, M, K, N):
     codes, scales, zeros, A = oa.make_q3_problem(1000 + 16 * M + (K % 7), K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
-    # more than four rows: row blocks of four where that makes at most four workgroups per compute unit (the
-    # wide shape: up to three blocks of its 257 tiles), up to 64 rows
+    # more than four rows: row blocks of four, up to 64 rows, where every workgroup has a compute unit of its own (the narrow
+    # shape); the wide shape's 257 tiles go to the one-launch kernel, which has no plan number of its own
+    assert kernel_of(M, K, N) == ("block" if M <= 4 or (N < 1000 and M <= 64) else "direct")
     want_plan = PLAN_BLOCK if M <= (12 if N > 1000 else 64) else PLAN_GEMM
     assert _plan(K, N, M) == want_plan
     y = _run(hq, A, mat, scales, zeros)
@@ -217,12 +219,18 @@ def test_batch2_split_k_accumulates_and_strict_fences(hq, oracle, tunable):
 
 @pytest.mark.parametrize("M,K,N", [(M, K, N) for (K, N) in [(1024, 196), (4128, 8192)] for M in (2, 3, 4, 5, 8, 11)])
 def test_small_batches_on_the_gemm(hq, oracle, tunable, M, K, N):
-    """HQ_Q3_SMALL_BATCH=0 keeps the digit kernels out: the GEMM serves the small batches as well."""
+    """HQ_Q3_SMALL_BATCH=0 keeps the digit kernels out: the GEMM's kernels serve the small batches as well, in one launch and,
+    that kernel kept out too, behind a pre-pass."""
     tunable("HQ_Q3_SMALL_BATCH", 0)
     assert _plan(K, N, M) == PLAN_GEMM
     codes, scales, zeros, A = oa.make_q3_problem(1300 + M, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
-    _check(_run(hq, A, mat, scales, zeros), oracle.q3_gemm(A, mat, scales, zeros, mode=0))
+    exact = oracle.q3_gemm(A, mat, scales, zeros, mode=0)
+    assert kernel_of(M, K, N) == "direct"
+    _check(_run(hq, A, mat, scales, zeros), exact)
+    tunable("HQ_Q3_TILES", 9)
+    assert kernel_of(M, K, N) == "rows64"
+    _check(_run(hq, A, mat, scales, zeros), exact)
 
 
 # one and two passes of four rows, full and partly filled; K of one round, a K the rounds do not divide
@@ -234,11 +242,14 @@ _BLOCK_CASES = [(M, K, N) for (K, N) in [(4128, 1028), (160, 16388)] for M in (3
 
 
 @pytest.mark.parametrize("M,K,N", _BLOCK_CASES)
-def test_block_kernel_vs_oracle(hq, oracle, M, K, N):
+def test_block_kernel_vs_oracle(hq, oracle, tunable, M, K, N):
     """Four rows per pass, four fp8 terms per activation: against the oracle at the batch-1 kernel's bound
     (N(0,1) activations enter exactly) and, row by row, the batch-1 matvec; a second call gives the same bits
     (partial sums and counters are left ready)."""
     assert _plan(K, N, M) == PLAN_BLOCK
+    if kernel_of(M, K, N) != "block":
+        tunable("HQ_Q3_ROW_BLOCKS", 0)  # passes in one workgroup, in place of the one-launch kernel
+    assert kernel_of(M, K, N) == "block"
     codes, scales, zeros, A = oa.make_q3_problem(1500 + 16 * M + K % 11, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
     y = _run(hq, A, mat, scales, zeros)
@@ -250,6 +261,23 @@ def test_block_kernel_vs_oracle(hq, oracle, M, K, N):
     for m in (0, M - 1):
         yv = hq.q3_matvec(_t(A[m]), dm, ds, dz).cpu().numpy()
         assert rel_err(y[m], yv) <= 1e-3
+
+
+@pytest.mark.parametrize("M,K,N", [(6, 4096, 17092), (8, 4096, 17092), (7, 8256, 8500), (5, 36864, 2052), (12, 36864, 516)])
+def test_batches_that_stay_with_the_block_kernel(hq, oracle, M, K, N):
+    """Five and more rows with more workgroups than compute units go to the one-launch kernel, up to eight rows of 7e7 weights and
+    more do not: two passes of one workgroup (six rows), row blocks (seven and eight); and more than eight rounds of K: two and
+    three passes."""
+    import torch
+    assert kernel_of(M, K, N) == "block"
+    g = torch.Generator(device="cuda:0").manual_seed(K)
+    mat = torch.randint(-2 ** 31, 2 ** 31, (3 * K // 32, N), dtype=torch.int32, device="cuda:0", generator=g)
+    scales = torch.rand(N, device="cuda:0", generator=g).mul_(0.01).add_(0.002)
+    A = torch.empty((M, K), dtype=torch.float16, device="cuda:0").normal_(generator=g)
+    y = hq.q3_gemm(A, mat, scales, scales * 3).cpu().numpy()
+    cols = np.unique(np.concatenate([np.arange(0, 68), np.arange(N // 2, N // 2 + 8), np.arange(N - 68, N)]))
+    _check(y[:, cols], oracle.q3_gemm(A.cpu().numpy(), np.ascontiguousarray(mat.cpu().numpy()[:, cols]), scales.cpu().numpy()[cols],
+                                      (scales * 3).cpu().numpy()[cols], mode=0))
 
 
 @pytest.mark.parametrize("M,K,N", [(5, 4128, 1028), (8, 512, 4100), (11, 4128, 1028), (12, 160, 16388), (13, 1024, 132),

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from tests import oracle_api as oa
+from tests.q3_kernel import kernel_of
 from tests.tol import FLOOR_F16, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -56,6 +57,8 @@ def test_outlier_at_any_code(hq, oracle, tunable, M, K, N, k, pos, amp):
     the sum so far below the 24th bit of that: 17 cuts of at most 2^(10 - pos) * 2^-24 of the outlier's power of two, times the
     column's scale (seen: a quarter of that).  The rest of the row: 1e-5 of its RMS."""
     tunable("HQ_Q3_SMALL_BATCH", 0)
+    tunable("HQ_Q3_TILES", 9)
+    assert kernel_of(M, K, N) == ("rows64" if M <= 64 else "tiles")
     codes, scales, zeros, A = oa.make_q3_problem(M + K + N, K, N, x_dtype=np.float16, batch=M)
     A[9, K // 64 * 32 + k] = np.float16(amp)
     mat = oracle.q3_pack(codes)
@@ -65,11 +68,17 @@ def test_outlier_at_any_code(hq, oracle, tunable, M, K, N, k, pos, amp):
     assert np.all(np.abs(y - exact) <= 17 * cut * scales + 1e-5 * np.sqrt(np.mean(exact ** 2)))
 
 
-@pytest.mark.parametrize("M,K,N", [(100, 4096, 4096), (700, 512, 3000), (1030, 16416, 8), (70, 256, 8200)])
-def test_default_plans(hq, oracle, M, K, N):
-    """The library's own choice: few tiles, several full rounds with a rest, several passes over the rows, 65 ... 96 rows of a
-    wide matrix.  Rows of one magnitude: the RMS of the whole result is the measure, as in the 64-row kernel's tests (a few
-    columns of one row are no sample of it)."""
+@pytest.mark.parametrize("M,K,N,default", [(100, 4096, 4096, 0), (700, 512, 3000, 0), (1030, 16416, 8, 0), (70, 256, 8200, 0),
+                                           (100, 6112, 17848, 1), (1100, 5376, 4468, 1), (72, 576, 49700, 1), (1100, 16384, 4100, 1),
+                                           (163, 8416, 10948, 1)])
+def test_default_plans(hq, oracle, tunable, M, K, N, default):
+    """The library's own choice of the tiles' plan: few tiles, several full rounds with a rest, several passes over the rows,
+    65 ... 96 rows of a wide matrix; problems that the tiles serve by default, and smaller ones that are the one-launch kernel's.
+    Rows of one magnitude: the RMS of the whole result is the measure, as in the 64-row kernel's tests (a few columns of one row
+    are no sample of it)."""
+    if not default:
+        tunable("HQ_Q3_TILES", 9)
+    assert kernel_of(M, K, N) == "tiles"
     codes, scales, zeros, A = oa.make_q3_problem(M + K, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
     y = hq.q3_gemm(_t(A), _t(mat), _t(scales), _t(zeros)).cpu().numpy()
@@ -77,11 +86,13 @@ def test_default_plans(hq, oracle, M, K, N):
     _check(y[:, cols], oracle.q3_gemm(A, np.ascontiguousarray(mat[:, cols]), scales[cols], zeros[cols], mode=0), rows=False)
 
 
-def test_accumulate_and_the_call_that_allocates_nothing(hq, oracle):
+def test_accumulate_and_the_call_that_allocates_nothing(hq, oracle, tunable):
     import torch
     from hecbench_amd import _lib
     lib = _lib.load()
     M, K, N = 200, 1024, 516
+    tunable("HQ_Q3_TILES", 9)
+    assert kernel_of(M, K, N) == "tiles"
     codes, scales, zeros, A = oa.make_q3_problem(3, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
     exact = oracle.q3_gemm(A, mat, scales, zeros, mode=0)
@@ -94,9 +105,11 @@ def test_accumulate_and_the_call_that_allocates_nothing(hq, oracle):
         _check(y.cpu().numpy() - 3.0, exact)
 
 
-def test_capture_with_the_workspace_of_a_smaller_call(hq, oracle):
+def test_capture_with_the_workspace_of_a_smaller_call(hq, oracle, tunable):
     """Under capture nothing can be allocated: where the stream's workspace holds what 64 rows need and not what all do, the
-    call goes 64 rows at a time."""
+    call goes 64 rows at a time, and gives the bits of such calls."""
+    tunable("HQ_Q3_TILES", 9)  # the workspace of the 64-row kernel, which this matrix is too small to take by itself
+    tunable("HQ_Q3_SMALL_BATCH", 0)
     import torch
     M, K, N = 1000, 4096, 16512
     codes, scales, zeros, A = oa.make_q3_problem(11, K, N, x_dtype=np.float16, batch=M)
@@ -107,6 +120,8 @@ def test_capture_with_the_workspace_of_a_smaller_call(hq, oracle):
     torch.cuda.synchronize()
     with torch.cuda.stream(stream):
         hq.q3_gemm(a[:32].contiguous(), w, s, z)
+        first, last = hq.q3_gemm(a[:64].contiguous(), w, s, z), hq.q3_gemm(a[960:].contiguous(), w, s, z)
+    assert kernel_of(64, K, N) == "rows64" and kernel_of(M, K, N) == "tiles"
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g, stream=stream):
@@ -118,3 +133,4 @@ def test_capture_with_the_workspace_of_a_smaller_call(hq, oracle):
         g.replay()
         torch.cuda.synchronize()
         _check(out.cpu().numpy()[:, cols], exact, rows=False)
+        assert torch.equal(out[:64], first) and torch.equal(out[960:], last)

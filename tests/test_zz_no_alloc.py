@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from tests import oracle_api as oa
+from tests.q3_kernel import kernel_of
 from tests.tol import rel_err
 
 pytestmark = pytest.mark.gpu
@@ -35,7 +36,15 @@ def _call(fn, p, batch):
     return y.cpu().numpy()
 
 
-def test_noalloc_matches_workspace_path(hq, oracle):
+@pytest.fixture(params=["default", "pre-pass"])
+def pre_pass(request, tunable):
+    """Once as the library chooses, and once with the kernels behind a pre-pass in place of the one-launch kernel."""
+    if request.param == "pre-pass":
+        tunable("HQ_Q3_TILES", 9)
+    return request.param == "pre-pass"
+
+
+def test_noalloc_matches_workspace_path(hq, oracle, pre_pass):
     from hecbench_amd import _lib
     lib = _lib.load()
     # 32 and 8 column tiles: far fewer than half the compute units, so both calls split K across
@@ -44,7 +53,7 @@ def test_noalloc_matches_workspace_path(hq, oracle):
     small = _problem(oracle, 302, 2048, 512, 66)
     for p in (big, small):                      # two calls in a row, the second with a smaller input
         # the matvec (narrow tiles), the small-batch kernel with one workgroup per tile and with two, three and
-        # ten row blocks, the GEMM (64 rows and the rest)
+        # ten row blocks, the one-launch kernel, the GEMM (64 rows and the rest)
         for batch in (1, 2, 6, 11, 40, p["M"]):
             want = _call(lib.hq_q3_matvec, p, batch)
             got = _call(lib.hq_q3_matvec_noalloc, p, batch)
@@ -61,9 +70,9 @@ def test_noalloc_matches_workspace_path(hq, oracle):
 
 @pytest.mark.parametrize("K,N,M", [(4096, 11008, 65), (8192, 4096, 72), (1024, 2048, 97), (4096, 4096, 128), (8192, 28672, 200),
                                    (16384, 6148, 300), (512, 260, 9000), (2080, 1028, 1100), (4160, 28672, 1030)])
-def test_many_rows_give_the_bits_of_the_workspace_path(hq, oracle, K, N, M):
+def test_many_rows_give_the_bits_of_the_workspace_path(hq, oracle, pre_pass, K, N, M):
     """Batches that hq_q3_matvec takes in tiles (and one that it takes 64 rows at a time): whole rounds, divided rests, several
-    passes over the rows, the longest K."""
+    passes over the rows, the longest K; the smaller of them on the one-launch kernel by default."""
     import torch
     from hecbench_amd import _lib
     lib = _lib.load()
@@ -85,13 +94,17 @@ class _Scratch(ctypes.Structure):  # HqQ3Scratch of csrc/hq_internal.h
                 ("sums_floats", ctypes.c_size_t), ("tiles", ctypes.c_void_p), ("tiles_floats", ctypes.c_size_t)]
 
 
-@pytest.mark.parametrize("K,N,M", [(4096, 516, 40), (8192, 516, 20), (8192, 2048, 64), (4096, 4096, 70), (8192, 512, 66)])
-def test_batched_call_after_one_that_was_cut_short(hq, oracle, K, N, M):
+@pytest.mark.parametrize("K,N,M", [(4096, 516, 40), (8192, 516, 20), (8192, 2048, 64), (4096, 4096, 70), (8192, 512, 66),
+                                   (4096, 1028, 130)])
+def test_batched_call_after_one_that_was_cut_short(hq, oracle, tunable, pre_pass, K, N, M):
     """A call that does not finish leaves its arrival counters part of the way up.  The next call must not count on from
-    there: the library's own launch function with a scratch of the test's, counters as such a call leaves them; 64-row kernel
-    (K split, sums by the last workgroup and, eight splits of 64 rows, by the second kernel) and tiles."""
+    there: the library's own launch function with a scratch of the test's, counters as such a call leaves them; one-launch kernel,
+    64-row kernel (K split, sums by the last workgroup and, eight splits of 64 rows, by the second kernel) and tiles."""
     import torch
     from hecbench_amd import _lib
+    if pre_pass:
+        tunable("HQ_Q3_SMALL_BATCH", 0)
+        assert kernel_of(M, K, N) == ("rows64" if M <= 64 else "tiles")
     launch = getattr(_lib.load(), "_Z17hq_q3_gemm_launchPKvPKiPKfS4_PfiiijP12ihipStream_tPK11HqQ3Scratch")
     p = _problem(oracle, 303, K, N, M)
     dev = "cuda:0"
