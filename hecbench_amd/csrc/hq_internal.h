@@ -149,7 +149,7 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
 // 1 / row scale; the product's arrival counters cleared), and the tiled kernels for many rows.
 int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad,
                            unsigned* counters, size_t ncounters, hipStream_t stream);
-bool hq_q3_tiles_serve(int cus, int K, int N, int M);
+bool hq_q3_tiles_serve(int N, int M);
 int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
 void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);
 int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,

@@ -460,8 +460,8 @@ namespace {
 // Which batches take the one-launch kernel (q3_direct.hip).  Up to 32 rows every one; up to 64, which are two of its row tiles, as
 // long as reading the weights twice costs less than the pre-pass (9e7 weights: 63 rows, K=5984, N=13008 23.1 -> 19.8 us, but 57
 // rows, K=4896, N=21956 25.5 -> 30.0); beyond, by the two estimates (over 270 timed problems of 97 and more rows the choice
-// costs 0.3 % on average against the better of the two, 15 % at most).  65 to 96 rows that the tiles do not serve were two passes of
-// the 64-row kernel: 78 rows, K=6880, N=584 19.5 -> 8.6.
+// costs 0.3 % on average against the better of the two, 15 % at most).  65 to 96 rows of a narrow matrix (N <= 4096) always, where
+// the 64-row kernel reads the weights twice: 78 rows, K=6880, N=584 19.5 -> 8.6.
 // The plan is made only where it is looked at: by the estimates, or by the launch of a batch that the kernel serves.
 bool direct_serves(int cus, int K, int N, int M, HqQ3DirectPlan* plan) {
   if (!hq_q3_direct_can(K, N)) return false;
@@ -469,19 +469,19 @@ bool direct_serves(int cus, int K, int N, int M, HqQ3DirectPlan* plan) {
   if (!forced && hq_tune(HQ_TUNE_Q3_TILES, -1) >= 0) return false;  // tests: the other kernels
   if (!forced && M > 32 && M <= 64 && (int64_t)K * N >= 90000000) return false;
   *plan = hq_q3_direct_plan(cus, K, N, M, false);
-  return forced || M <= 64 || !hq_q3_tiles_serve(cus, K, N, M) || plan->us < hq_q3_tiles_us(cus, K, N, M);
+  return forced || M <= 64 || !hq_q3_tiles_serve(N, M) || plan->us < hq_q3_tiles_us(cus, K, N, M);
 }
 }  // namespace
 
 int hq_q3_gemm_kernel_of(int cus, int K, int N, int M) {
   HqQ3DirectPlan d;
   if (direct_serves(cus, K, N, M, &d)) return HQ_Q3_KERNEL_DIRECT;
-  return hq_q3_tiles_serve(cus, K, N, M) ? HQ_Q3_KERNEL_TILES : HQ_Q3_KERNEL_ROWS64;
+  return hq_q3_tiles_serve(N, M) ? HQ_Q3_KERNEL_TILES : HQ_Q3_KERNEL_ROWS64;
 }
 
 // What the kernel of the plan takes, or the one that stands in for it where that is more.
 int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
-  if (hq_q3_tiles_serve(cus, K, N, M)) {
+  if (hq_q3_tiles_serve(N, M)) {
     hq_q3_tiles_need(cus, K, N, M, floats, counters);
   } else {
     const GemmPlan p = gemm_plan(cus, K, N);
@@ -506,7 +506,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   HqQ3DirectPlan direct;
   if (!(fixed && K > kFixedMaxK) && direct_serves(dev->cus, K, N, M, &direct))  // (a longer K is refused below)
     return hq_q3_direct_launch(direct, dev->cus, x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
-  bool tiles = hq_q3_tiles_serve(dev->cus, K, N, M);
+  bool tiles = hq_q3_tiles_serve(N, M);
   if (tiles) {
     // 64 rows at a time need less: under capture without room for all rows' activations, and where the fixed array cannot hold
     // the tiles' plan (a device of more compute units than it was sized for; K beyond its limit, which is refused below)

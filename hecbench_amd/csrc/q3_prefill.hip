@@ -386,16 +386,7 @@ TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int wa
   return p;
 }
 
-// 65 to 96 rows of a narrow matrix of less than 2^25 weights are served here as well, with the smallest tile.  The 64-row kernel
-// reads the weights twice and launches six times: 70 rows, K=4096, N=4096 27.2 -> 17.6 us; 90 rows, K=512, N=2048 18.4 -> 10.5; 66
-// rows, K=8192, N=512 26.0 -> 20.3.  The line at 2^25 weights and K=8192 is where the workspace of such a call was once agreed on
-// and not where the times cross: beyond it as much would be gained (96 rows, K=8192, N=4096 33.1 -> 22.5).
-bool few_rows(int cus, int K, int N, int M) {
-  return M > 64 && M <= 96 && N <= 4096 && K <= 8192 && (int64_t)K * N < (1 << 25) && cus <= 256;
-}
-
 TilePlan tile_plan(int cus, int K, int N, int M) {
-  if (few_rows(cus, K, N, M)) return tile_plan_of(cus, K, N, M, kKinds[2], 0);
   const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: kind + 10 * shares (3 to 6 the one-launch kernel's, 9 none in particular)
   if (force >= 0 && force % 10 < 3) return tile_plan_of(cus, K, N, M, kKinds[force % 10], force / 10);
   TilePlan best = tile_plan_of(cus, K, N, M, kKinds[0], 0);
@@ -425,10 +416,9 @@ int launch_tiles(const TileArgs& a, int nwg, hipStream_t stream) {
 }  // namespace
 
 // Batches the tiled kernels serve.  Up to 64 rows go through the 64-row kernel of q3_gemm.hip (64 rows, K=8192, N=28672: 36.8 us
-// there, 40.2 here; 32 rows 26.5 and 35.4; 58 rows, K=6464, N=13924 28.7 and 25.9).
-bool hq_q3_tiles_serve(int cus, int K, int N, int M) {
-  return few_rows(cus, K, N, M) || M > 96 || (M > 64 && N > 4096);
-}
+// there, 40.2 here; 32 rows 26.5 and 35.4; 58 rows, K=6464, N=13924 28.7 and 25.9), 65 to 96 rows of a narrow matrix through the
+// one-launch kernel of q3_direct.hip (70 rows, K=4096, N=4096 8.7 us there, 17.6 here).
+bool hq_q3_tiles_serve(int N, int M) { return M > 96 || (M > 64 && N > 4096); }
 
 // What such a call takes (us): the tiles as planned, and the pre-pass in front of them (3.2 us, more for a long K and for its bytes).
 float hq_q3_tiles_us(int cus, int K, int N, int M) {

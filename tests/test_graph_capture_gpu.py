@@ -33,7 +33,7 @@ def test_replays_match_eager(hq, oracle, pre_pass):
     codes, scales, zeros, x = oa.make_q3_problem(901, K, N)
     mat = oracle.q3_pack(codes)
     Kg, Ng, M = 1024, 516, 72               # batched GEMM (more than 64 rows): one launch, or pre-pass and main kernel that meet in the workspace
-    assert kernel_of(M, Kg, Ng) == ("tiles" if pre_pass else "direct")
+    assert kernel_of(M, Kg, Ng) == ("rows64" if pre_pass else "direct")
     codes_g, scales_g, zeros_g, A = oa.make_q3_problem(902, Kg, Ng, x_dtype=np.float16, batch=M)
     mat_g = oracle.q3_pack(codes_g)
     dx, dm, ds, dz = _t(x), _t(mat), _t(scales), _t(zeros)

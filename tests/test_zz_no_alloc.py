@@ -104,7 +104,7 @@ def test_batched_call_after_one_that_was_cut_short(hq, oracle, tunable, pre_pass
     from hecbench_amd import _lib
     if pre_pass:
         tunable("HQ_Q3_SMALL_BATCH", 0)
-        assert kernel_of(M, K, N) == ("rows64" if M <= 64 else "tiles")
+        assert kernel_of(M, K, N) == ("tiles" if M > 96 else "rows64")
     launch = getattr(_lib.load(), "_Z17hq_q3_gemm_launchPKvPKiPKfS4_PfiiijP12ihipStream_tPK11HqQ3Scratch")
     p = _problem(oracle, 303, K, N, M)
     dev = "cuda:0"
