@@ -41,6 +41,7 @@ constexpr int kDeep = 3;        // steps of operands in flight ahead of the one 
 constexpr int kBufs = kDeep + 1;
 constexpr int kChunk = kStepGroups * kBufs;  // the pre-pass pads K to a multiple of this many k-groups
 constexpr int kTileN = 128;     // output columns per workgroup
+constexpr int kRowBlocks = 2, kRows = 32 * kRowBlocks;  // activation rows of a pass over the weights
 constexpr int kMaxSplitGroups = 256;  // workgroups of a K-split launch (tiles times splits)
 constexpr int kFixedMaxK = 16384;     // longest K of a batched call in the fixed scratch
 
@@ -187,9 +188,9 @@ struct GemmArgs {
 // (Two waves per SIMD with one step in flight measured 38.4 us at M=64, K=8192, N=28672 against 36.2; the
 // depth itself, 2 to 5 steps, changes little: what a workgroup moves through its CU's L1 - all of the
 // re-ordered activations, 1 MB, next to 0.4 MB of weights - bounds the loop, not the latency.)
-// MB: 32-row blocks of activations.  SHARED: column tiles share 128-byte lines (hq_column_tile; a kernel of its own, so that nothing
-// stands in front of the other's first loads).
-template <int MB, bool SHARED>
+// SHARED: column tiles share 128-byte lines (hq_column_tile; a kernel of its own, so that nothing stands in front of the other's
+// first loads).
+template <bool SHARED>
 __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_, const u4v* Ap_, int M_, int K_, int N_,
                                                              int Gpad_, int nsplit_, int spp_, unsigned flags_,
                                                              const float* scales_, const float* zeros_,
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
   GemmArgs a;
   a.w = w_; a.Ap = Ap_; a.rowsum = rowsum_; a.rowinv = rowinv_; a.scales = scales_; a.zeros = zeros_; a.out = out_;
   a.partial = partial_; a.counters = counters_; a.M = M_; a.K = K_; a.N = N_; a.Gpad = Gpad_; a.nsplit = nsplit_; a.spp = spp_; a.flags = flags_;
-  constexpr int Mpad = 32 * MB;
+  constexpr int MB = kRowBlocks, Mpad = kRows;
   extern __shared__ u4v lds[];  // used by the final reduction only
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int nl = lane & 31, kb = lane >> 5;
@@ -367,7 +368,8 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
 
 // K split: sums the workgroups' raw sums of a tile in split order and applies scale, zero and the row's power
 // of two.  A thread owns four adjacent columns of one row.
-__global__ __launch_bounds__(256) void q3_gemm_reduce(GemmArgs a, int Mpad) {
+__global__ __launch_bounds__(256) void q3_gemm_reduce(GemmArgs a) {
+  constexpr int Mpad = kRows;
   const int tile = blockIdx.x;
   const int nl = threadIdx.x & 31;
   const int n_out = tile * kTileN + 4 * nl;
@@ -398,23 +400,22 @@ __global__ __launch_bounds__(256) void q3_gemm_reduce(GemmArgs a, int Mpad) {
   }
 }
 
-template <int MB, bool SHARED>
+template <bool SHARED>
 int launch_gemm_t(const GemmArgs& a, int ntiles, hipStream_t stream) {
   const size_t smem = (size_t)kWaves * 32 * kTileN * 4;
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_gemm_kernel<MB, SHARED>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&q3_gemm_kernel<SHARED>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (attr != hipSuccess) return (int)attr;
-  hipLaunchKernelGGL((q3_gemm_kernel<MB, SHARED>), dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K,
+  hipLaunchKernelGGL(q3_gemm_kernel<SHARED>, dim3(ntiles, a.nsplit), dim3(kWaves * 64), smem, stream, a.w, a.Ap, a.M, a.K,
                      a.N, a.Gpad, a.nsplit, a.spp, a.flags, a.scales, a.zeros, a.rowsum, a.rowinv, a.out, a.partial,
                      a.counters);
   return hq_launch_status();
 }
-template <int MB>
 int launch_gemm(const GemmArgs& a, hipStream_t stream) {
   const int ntiles = (a.N + kTileN - 1) / kTileN;
-  const int rc = hq_tiles_share_lines(a.w, a.N) ? launch_gemm_t<MB, true>(a, ntiles, stream) : launch_gemm_t<MB, false>(a, ntiles, stream);
+  const int rc = hq_tiles_share_lines(a.w, a.N) ? launch_gemm_t<true>(a, ntiles, stream) : launch_gemm_t<false>(a, ntiles, stream);
   if (rc != HQ_OK || a.nsplit == 1 || a.counters) return rc;
-  hipLaunchKernelGGL(q3_gemm_reduce, dim3(ntiles, (a.M + 7) / 8 < 8 ? (a.M + 7) / 8 : 8), dim3(256), 0, stream, a, 32 * MB);
+  hipLaunchKernelGGL(q3_gemm_reduce, dim3(ntiles, (a.M + 7) / 8 < 8 ? (a.M + 7) / 8 : 8), dim3(256), 0, stream, a);
   return hq_launch_status();
 }
 
@@ -434,7 +435,7 @@ GemmPlan gemm_plan(int cus, int K, int N) {
   GemmPlan p;
   const int G = K / 32;
   p.Gpad = (G + kChunk - 1) / kChunk * kChunk;
-  p.ap_halves = (size_t)p.Gpad * 4 * 64 * 8;
+  p.ap_halves = (size_t)p.Gpad * 4 * kRows * 8;
   const int ntiles = (N + kTileN - 1) / kTileN;
   const int nsteps = p.Gpad / kStepGroups;
   p.nsplit = (cus < kMaxSplitGroups ? cus : kMaxSplitGroups) / ntiles;
@@ -443,7 +444,7 @@ GemmPlan gemm_plan(int cus, int K, int N) {
   p.spp = (nsteps + p.nsplit - 1) / p.nsplit;
   p.spp = (p.spp + kBufs - 1) / kBufs * kBufs;
   p.nsplit = (nsteps + p.spp - 1) / p.spp;
-  p.partial_floats = p.nsplit > 1 ? (size_t)ntiles * p.nsplit * 64 * kTileN : 0;
+  p.partial_floats = p.nsplit > 1 ? (size_t)ntiles * p.nsplit * kRows * kTileN : 0;
   p.counters = p.nsplit > 1 ? (size_t)ntiles : 1;
   return p;
 }
@@ -485,7 +486,7 @@ int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counte
     hq_q3_tiles_need(cus, K, N, M, floats, counters);
   } else {
     const GemmPlan p = gemm_plan(cus, K, N);
-    *floats = p.ap_halves / 2 + 128 + p.partial_floats;
+    *floats = p.ap_halves / 2 + 2 * kRows + p.partial_floats;
     *counters = p.counters;
   }
   HqQ3DirectPlan d;
@@ -516,7 +517,7 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   }
   if (tiles) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   const GemmPlan plan = gemm_plan(dev->cus, K, N);
-  if (!fixed && hq_workspace_out_of_reach(stream, plan.ap_halves / 2 + 128 + plan.partial_floats, plan.counters) &&
+  if (!fixed && hq_workspace_out_of_reach(stream, plan.ap_halves / 2 + 2 * kRows + plan.partial_floats, plan.counters) &&
       hq_q3_direct_can(K, N))  // under capture without room for these activations: none are needed there
     return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, M, false), dev->cus, x, qweight, scales, zeros, y, K, N, M, flags,
                                stream, fixed);
@@ -529,26 +530,24 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
     if (ap_halves / 2 > fixed->partial_floats || partial_floats > fixed->sums_floats || plan.counters > fixed->ncounters) return HQ_ERR_TOO_LARGE;
     Ap = reinterpret_cast<_Float16*>(fixed->partial);
     rowsum = fixed->rows;
-    rowinv = fixed->rows + 64;
+    rowinv = fixed->rows + kRows;
     partial = fixed->sums;
     counters = fixed->counters;
   } else {
     HqWorkspace ws;
-    rc = hq_get_workspace(stream, ap_halves / 2 + 128 + partial_floats, plan.counters, &ws);
+    rc = hq_get_workspace(stream, ap_halves / 2 + 2 * kRows + partial_floats, plan.counters, &ws);
     if (rc != HQ_OK) return rc;
     Ap = reinterpret_cast<_Float16*>(ws.partial);
     rowsum = ws.partial + ap_halves / 2;
-    rowinv = rowsum + 64;
-    partial = rowsum + 128;
+    rowinv = rowsum + kRows;
+    partial = rowsum + 2 * kRows;
     counters = ws.counters;
   }
   // up to 64 rows per pass over the weights
-  for (int m0 = 0; m0 < M; m0 += 64) {
-    const int Mb = M - m0 < 64 ? M - m0 : 64;
-    const int MB = Mb > 32 ? 2 : 1;
-    const int Mpad = 32 * MB;
+  for (int m0 = 0; m0 < M; m0 += kRows) {
+    const int Mb = M - m0 < kRows ? M - m0 : kRows;
     const _Float16* A = reinterpret_cast<const _Float16*>(x) + (size_t)m0 * K;
-    rc = hq_q3_gemm_prep_launch(A, Ap, rowsum, rowinv, Mb, K, Mpad, Gpad, counters, nsplit > 1 ? plan.counters : 0, stream);
+    rc = hq_q3_gemm_prep_launch(A, Ap, rowsum, rowinv, Mb, K, kRows, Gpad, counters, nsplit > 1 ? plan.counters : 0, stream);
     if (rc != HQ_OK) return rc;
     GemmArgs a;
     a.w = reinterpret_cast<const uint32_t*>(qweight);
@@ -559,8 +558,8 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
     a.zeros = zeros;
     a.out = y + (size_t)m0 * N;
     a.M = Mb; a.K = K; a.N = N; a.Gpad = Gpad; a.flags = flags;
-    a.partial = partial; a.counters = MB == 2 && nsplit > 4 ? nullptr : counters; a.nsplit = nsplit; a.spp = spp;
-    rc = MB == 2 ? launch_gemm<2>(a, stream) : launch_gemm<1>(a, stream);
+    a.partial = partial; a.counters = nsplit > 4 ? nullptr : counters; a.nsplit = nsplit; a.spp = spp;
+    rc = launch_gemm(a, stream);
     if (rc != HQ_OK) return rc;
   }
   return HQ_OK;
