@@ -55,14 +55,14 @@ struct Form {
   static constexpr int kWLoads = (kWBytes + 1023) / 1024;  // and packed rows, the last load by half of the lanes if CB is 2
   static constexpr int kLoads = kALoads + kWLoads, kStageBytes = kABytes + kWBytes;
   static constexpr int kUnits = 4 * CB;                    // groups of eight rows, every CB-th column
-  static constexpr int kMeetUnits = kUnits * KS > 128 ? 128 / KS : kUnits;  // of which so many meet at a time,
-  static constexpr int kRounds = kUnits / kMeetUnits, kFinal = kMeetUnits / KS;  // and a wave finishes some of them
-  static constexpr int kWaveBytes = 2 * kStageBytes, kRing = KS * kWaveBytes, kMeet = KS * kMeetUnits * 1024;
+  static constexpr int kFinal = kUnits / KS;               // of which a wave finishes so many
+  static constexpr int kWaveBytes = 2 * kStageBytes, kRing = KS * kWaveBytes, kMeet = KS * kUnits * 1024;
   static constexpr int kBulk = kRing > kMeet ? kRing : kMeet;
   static constexpr int kSums = 2 * KS * kTileM;            // floats: parts of the row sums
   static constexpr int kSmem = kBulk + (kSums + kTileM) * 4 + 16;
   static_assert(KS % 2 == 0, "odd parts of K enter negated");
   static_assert(CB == 2 || CB == 4, "a lane's columns are one LDS read");
+  static_assert(kUnits % KS == 0, "every wave finishes as many units");
   static_assert(kSmem <= 160 * 1024, "LDS");
 };
 
@@ -261,48 +261,45 @@ __global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
 
   // ---- the parts of K meet: wave p finishes units p * kFinal and up (no load is in flight into LDS any more: the last steps
   // waited for theirs) ----
-  constexpr int F = S::kFinal, R = S::kRounds;
+  constexpr int F = S::kFinal;
   constexpr int V = F < CB ? F : CB;  // adjacent columns of a wave's units
   typedef float fv_t __attribute__((ext_vector_type(V)));
   float* const sums = reinterpret_cast<float*>(lds + S::kBulk);  // [2 KS][kTileM], then the rows' sums
   float* const total = sums + S::kSums;
   f4v* const meet = reinterpret_cast<f4v*>(lds) + lane;
-  auto first_row = [&](int r, int i) { return (r * S::kMeetUnits + kp * F + i) / CB * 8 + 4 * kb; };  // of unit i of round r
+  auto first_row = [&](int i) { return (kp * F + i) / CB * 8 + 4 * kb; };  // of this wave's unit i
   const int first_col = ct * S::kTileN + CB * nl + kp * F % CB;
-  f4v fin[R][F];
+  f4v fin[F];
   sums[(2 * kp + kb) * S::kTileM + nl] = rs;
+  __syncthreads();  // every wave is done with its stages
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    __syncthreads();  // every wave is done with its stages, and with the round before
+  for (int u = 0; u < S::kUnits; ++u) {
+    f4v x;
 #pragma unroll
-    for (int v = 0; v < S::kMeetUnits; ++v) {
-      const int u = r * S::kMeetUnits + v;
-      f4v x;
+    for (int e = 0; e < 4; ++e) x[e] = acc[u % CB][4 * (u / CB) + e];
+    meet[(u * KS + kp) * 64] = x;
+  }
+  if (tid < S::kTileM) {  // (the sums' parts were written ahead of the barrier)
+    float t = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) x[e] = acc[u % CB][4 * (u / CB) + e];
-      meet[(v * KS + kp) * 64] = x;
+    for (int i = 0; i < 2 * KS; ++i) t += sums[i * S::kTileM + tid];
+    total[tid] = t;
+  }
+  asm volatile("" ::"s"(a.flags));  // the last arguments are here with the others, not behind the first LDS reads' wait
+  __syncthreads();
+  const int nc = min(first_col, a.N - V);
+  const fv_t sc = *reinterpret_cast<const fv_t*>(a.scales + nc), zr = *reinterpret_cast<const fv_t*>(a.zeros + nc);
+#pragma unroll
+  for (int i = 0; i < F; ++i) {
+    f4v x = meet[((kp * F + i) * KS) * 64];
+#pragma unroll
+    for (int p = 1; p < KS; ++p) {
+      const f4v other = meet[((kp * F + i) * KS + p) * 64];
+      x = p & 1 ? x - other : x + other;  // odd parts are the negated ones
     }
-    if (r == 0 && tid < S::kTileM) {  // (the sums' parts were written ahead of the barrier)
-      float t = 0.f;
+    const f4v t = *reinterpret_cast<const f4v*>(total + first_row(i));
 #pragma unroll
-      for (int i = 0; i < 2 * KS; ++i) t += sums[i * S::kTileM + tid];
-      total[tid] = t;
-    }
-    __syncthreads();
-    const int nc = min(first_col, a.N - V);
-    const fv_t sc = *reinterpret_cast<const fv_t*>(a.scales + nc), zr = *reinterpret_cast<const fv_t*>(a.zeros + nc);
-#pragma unroll
-    for (int i = 0; i < F; ++i) {
-      f4v x = meet[((kp * F + i) * KS) * 64];
-#pragma unroll
-      for (int p = 1; p < KS; ++p) {
-        const f4v other = meet[((kp * F + i) * KS + p) * 64];
-        x = p & 1 ? x - other : x + other;  // odd parts are the negated ones
-      }
-      const f4v t = *reinterpret_cast<const f4v*>(total + first_row(r, i));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) fin[r][i][e] = sc[i % V] * (x[e] * 8.f) - zr[i % V] * t[e];  // codes enter as eighths
-    }
+    for (int e = 0; e < 4; ++e) fin[i][e] = sc[i % V] * (x[e] * 8.f) - zr[i % V] * t[e];  // codes enter as eighths
   }
 
   if (a.nshare > 1) {
@@ -313,7 +310,7 @@ __global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
     };
     f4v* dst = slot_of_share(share);
 #pragma unroll
-    for (int i = 0; i < R * F; ++i) hq_store_share(dst + i * S::kThreads, fin[i / F][i % F]);
+    for (int i = 0; i < F; ++i) hq_store_share(dst + i * S::kThreads, fin[i]);
     unsigned* last = reinterpret_cast<unsigned*>(total + S::kTileM);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -325,41 +322,38 @@ __global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
     }
     __syncthreads();
     if (!*last) return;
-    constexpr int kAtOnce = R * F >= 16 ? 1 : (F >= 8 ? 2 : (F >= 4 ? 4 : 8));
+    constexpr int kAtOnce = F >= 4 ? 4 : 8;
     for (int c0 = 0; c0 < a.nshare; c0 += kAtOnce) {
-      f4v x[kAtOnce * R * F];
+      f4v x[kAtOnce * F];
 #pragma unroll
       for (int k = 0; k < kAtOnce; ++k)
 #pragma unroll
-        for (int i = 0; i < R * F; ++i)
-          x[k * R * F + i] = hq_load_share(slot_of_share(min(c0 + k, a.nshare - 1)) + i * S::kThreads);
+        for (int i = 0; i < F; ++i)
+          x[k * F + i] = hq_load_share(slot_of_share(min(c0 + k, a.nshare - 1)) + i * S::kThreads);
       hq_wait_shares(x);
 #pragma unroll
       for (int k = 0; k < kAtOnce; ++k)
         if (c0 + k < a.nshare) {
 #pragma unroll
-          for (int i = 0; i < R * F; ++i)
-            fin[i / F][i % F] = c0 + k == 0 ? x[k * R * F + i] : fin[i / F][i % F] + x[k * R * F + i];
+          for (int i = 0; i < F; ++i) fin[i] = c0 + k == 0 ? x[k * F + i] : fin[i] + x[k * F + i];
         }
     }
   }
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+  for (int i = 0; i < F; i += V) {
+    const int m0 = mt * S::kTileM + first_row(i), n = first_col;
 #pragma unroll
-    for (int i = 0; i < F; i += V) {
-      const int m0 = mt * S::kTileM + first_row(r, i), n = first_col;
+    for (int e = 0; e < 4; ++e) {
+      if (m0 + e < a.M && n < a.N) {
+        fv_t* p = reinterpret_cast<fv_t*>(a.out + (size_t)(m0 + e) * a.N + n);
+        fv_t o;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (m0 + e < a.M && n < a.N) {
-          fv_t* p = reinterpret_cast<fv_t*>(a.out + (size_t)(m0 + e) * a.N + n);
-          fv_t o;
-#pragma unroll
-          for (int c = 0; c < V; ++c) o[c] = fin[r][i + c][e];
-          if (a.flags & HQ_FLAG_ACCUMULATE) o += *p;
-          __builtin_nontemporal_store(o, p);
-        }
+        for (int c = 0; c < V; ++c) o[c] = fin[i + c][e];
+        if (a.flags & HQ_FLAG_ACCUMULATE) o += *p;
+        __builtin_nontemporal_store(o, p);
       }
     }
+  }
 }
 
 __global__ __launch_bounds__(256) void clear_counters(unsigned* p, int n) {
