@@ -54,23 +54,6 @@ __device__ __forceinline__ float dot8(u4v e, u4v xv, float acc) {
 constexpr int kMaxLdsK = 24576;  // 48 KB
 __host__ __device__ constexpr int aqlm_x_stride(int units) { return (units + 7) / 8 * 8 + 1; }
 
-// Sum over the wave without LDS traffic: four DPP butterfly steps inside each 16-lane row, the four row results as scalars (as a
-// butterfly of shuffles 0.2 us more, exposed at every wave's end: 1311 x 9536 three code books 10.75 / 10.45 us, 4096 x 4096 11.2 / 11.05).
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lane_f(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  v += dpp_f<0x140>(v);  // row_mirror
-  return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
-}
-
 template <int ROWS, bool XLDS, bool SPLIT>
 __global__ __launch_bounds__(256) void aqlm_matvec_kernel(HQ_ARGS24) {
   // the first 14 dwords of the arguments arrive preloaded in scalar registers: all but scales and y
@@ -146,7 +129,7 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(HQ_ARGS24) {
   __shared__ float part[4][ROWS];
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
-    float v = wave_sum(acc[r]);
+    float v = hq_wave_sum(acc[r]);
     if (SPLIT) {
       if (lane == 0) part[wv][r] = v;
     } else if (lane == 0 && row0 + r < a.M) {

@@ -27,21 +27,6 @@ typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ h2v as_h2(uint32_t v) { return __builtin_bit_cast(h2v, v); }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lane_f(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp_f<0x141>(v);  // row_half_mirror
-  v += dpp_f<0x140>(v);  // row_mirror
-  return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
-}
-
 enum { kF16 = 0, kI8 = 1, kI4 = 2 };
 
 struct GemvArgs {
@@ -146,7 +131,7 @@ __device__ __forceinline__ void gemv_finish(const GemvArgs& a, int row0, const f
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    float s = wave_sum(MODE == kI4 ? fmaf(acc16[r], 0.0625f, acc[r]) : acc[r]);
+    float s = hq_wave_sum(MODE == kI4 ? fmaf(acc16[r], 0.0625f, acc[r]) : acc[r]);
     if (MODE == kI8) s = a.scale * (s - a.zp * vs);
     if (MODE == kI4) s = a.scale * (s * 16777216.f - a.zp * vs);  // codes were fp16 subnormals code * 2^-24
     if (lane == 0 && row0 + r < a.rows) a.res[row0 + r] = (_Float16)s;
@@ -183,7 +168,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(HQ_ARGS12) {
     gemv_step<MODE, R, true>(m, v, acc, acc16, vsum);
   }
 
-  gemv_finish<MODE, R>(a, row0, acc, acc16, MODE == kF16 ? 0.f : wave_sum(vsum));
+  gemv_finish<MODE, R>(a, row0, acc, acc16, MODE == kF16 ? 0.f : hq_wave_sum(vsum));
 }
 
 // Rows cut across the waves of a workgroup.  On this part a stream moves fastest when every wave issues a
@@ -228,11 +213,11 @@ __global__ __launch_bounds__(SPLIT * 64) void gemv_split_kernel(HQ_ARGS12) {
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const float s = wave_sum(MODE == kI4 ? fmaf(acc16[r], 0.0625f, acc[r]) : acc[r]);
+    const float s = hq_wave_sum(MODE == kI4 ? fmaf(acc16[r], 0.0625f, acc[r]) : acc[r]);
     if (lane == 0) part[wv][r] = s;
   }
   if (MODE != kF16) {
-    const float vs = wave_sum(vsum);
+    const float vs = hq_wave_sum(vsum);
     if (lane == 0) part[wv][R] = vs;
   }
   __syncthreads();
@@ -265,12 +250,8 @@ template <int R>
 __device__ __forceinline__ void row_sums(const float (&s)[R], float (&w)[R / 4]) {
 #pragma unroll
   for (int i = 0; i < R / 4; ++i) {
-    float v = swap_add_16(swap_add_32(s[i], s[i + R / 2]), swap_add_32(s[i + R / 4], s[i + R / 2 + R / 4]));
-    v += dpp_f<0xB1>(v);
-    v += dpp_f<0x4E>(v);
-    v += dpp_f<0x141>(v);
-    v += dpp_f<0x140>(v);
-    w[i] = v;
+    const float v = swap_add_16(swap_add_32(s[i], s[i + R / 2]), swap_add_32(s[i + R / 4], s[i + R / 2 + R / 4]));
+    w[i] = hq_row(v, HqAdd());
   }
 }
 
@@ -311,7 +292,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
   for (int i = 0; i < R / 4; ++i)
     if ((lane & 15) == i) part[wv][i + R / 4 * (lane >> 4)] = w[i];
   if (MODE != kF16) {
-    const float vs = wave_sum(vsum);
+    const float vs = hq_wave_sum(vsum);
     if (lane == 0) part[wv][R] = vs;
   }
   __syncthreads();
@@ -394,7 +375,7 @@ __global__ __launch_bounds__(1024) void gemv_lds_kernel(HQ_ARGS12) {
       if (first) gemv_step<MODE, R, true>(cur, v, acc, acc16, vsum);
       else gemv_step<MODE, R, false>(cur, v, acc, acc16, vsum);
     }
-    if (first && MODE != kF16) vs = wave_sum(vsum);
+    if (first && MODE != kF16) vs = hq_wave_sum(vsum);
     first = false;
     gemv_finish<MODE, R>(a, grp * R, acc, acc16, vs);
   }

@@ -184,6 +184,45 @@ enum HqTunable {
 };
 int hq_tune(HqTunable id, int dflt);
 
+// ---- the lanes of a wave together ----------------------------------------------------------------------------------------
+// On the data path's own lane exchanges (DPP) inside each row of 16 lanes, then the four rows' results as scalars: no LDS.  As a
+// butterfly of shuffles, which go through the LDS crossbar, 0.2 us more where it is exposed (the AQLM matvec's waves end with one:
+// 1311 x 9536, three code books, 10.75 / 10.45 us; the batched product's pre-pass has two: 32 x 4096 x 11008 13.55 / 13.3).
+template <int CTRL>
+__device__ __forceinline__ float hq_dpp(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float hq_lane(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
+template <typename OP>
+__device__ __forceinline__ float hq_quad(float v, OP op) {
+  v = op(v, hq_dpp<0xB1>(v));     // quad_perm [1,0,3,2]
+  return op(v, hq_dpp<0x4E>(v));  // quad_perm [2,3,0,1]
+}
+template <typename OP>
+__device__ __forceinline__ float hq_row(float v, OP op) {
+  v = hq_quad(v, op);
+  v = op(v, hq_dpp<0x141>(v));     // row_half_mirror
+  return op(v, hq_dpp<0x140>(v));  // row_mirror
+}
+template <typename OP>
+__device__ __forceinline__ float hq_wave(float v, OP op) {
+  v = hq_row(v, op);
+  return op(op(hq_lane(v, 0), hq_lane(v, 16)), op(hq_lane(v, 32), hq_lane(v, 48)));
+}
+struct HqAdd {
+  __device__ __forceinline__ float operator()(float x, float y) const { return x + y; }
+};
+struct HqMax {
+  __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); }
+};
+struct HqMin {
+  __device__ __forceinline__ float operator()(float x, float y) const { return fminf(x, y); }
+};
+__device__ __forceinline__ float hq_wave_sum(float v) { return hq_wave(v, HqAdd()); }
+__device__ __forceinline__ float hq_wave_max(float v) { return hq_wave(v, HqMax()); }
+
 // Sum of the nsplit partial sums p[s * stride] of a K split, added in split order (the result does not depend
 // on which workgroup arrived last).  The loads are device-scope atomic loads, which bypass the non-coherent
 // cache levels; eight of them are in flight at a time - one after the other each costs a trip to memory, and

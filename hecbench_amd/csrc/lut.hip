@@ -209,33 +209,6 @@ __device__ __forceinline__ v8i unpack_bits_fp4(uint32_t w) {
   return a;
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lane_f(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-// Maximum over 16 lanes (four DPP butterfly steps), and over all 64: then the row results.
-__device__ __forceinline__ float row_max(float v) {
-  v = fmaxf(v, dpp_f<0xB1>(v));   // quad_perm [1,0,3,2]
-  v = fmaxf(v, dpp_f<0x4E>(v));   // quad_perm [2,3,0,1]
-  v = fmaxf(v, dpp_f<0x141>(v));  // row_half_mirror
-  return fmaxf(v, dpp_f<0x140>(v));  // row_mirror
-}
-__device__ __forceinline__ float wave_max(float v) {
-  v = row_max(v);
-  return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_f<0xB1>(v);
-  v += dpp_f<0x4E>(v);
-  v += dpp_f<0x141>(v);
-  v += dpp_f<0x140>(v);
-  return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
-}
-
 // 128-bit loads for rows that start at any element (N not a multiple of 8 or 4): the types carry
 // the element's own alignment, the hardware reads unaligned global addresses.
 typedef uint32_t u4v_any __attribute__((ext_vector_type(4), aligned(4)));
@@ -459,7 +432,7 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(HQ_ARGS24) {
       }
     }
     // GROUPED: a quad's scale is its own (its sixteen lanes are one DPP row), otherwise the round's
-    const float xmax = GROUPED ? row_max(amax) : wave_max(amax);
+    const float xmax = GROUPED ? hq_row(amax, HqMax()) : hq_wave_max(amax);
     // 2^E * max|x| lies in [2^14, 2^15): u = rint(|x| * 2^E) <= 2^15 stays inside 16 bits
     int E = 14 - ((int)((__float_as_uint(xmax) >> 23) & 255u) - 127);
     E = xmax > 0.f ? max(-120, min(120, E)) : 0;
@@ -530,7 +503,7 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(HQ_ARGS24) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) run[q] = fmaf((float)r.cf[t][COEFS - 1][q], xh, run[q]);
         }
-        const float descale = lane_f(descale_lane, 16 * t);
+        const float descale = hq_lane(descale_lane, 16 * t);
 #pragma unroll
         for (int q = 0; q < 4; ++q) { tot[q] = fmaf(run[q], descale, tot[q]); run[q] = 0.f; }
         continue;
@@ -579,7 +552,7 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(HQ_ARGS24) {
   }
   // ---- combine lane quarters (planes, bias) and waves --------------------------------------------------
   {
-    const float wp = wave_sum(poison);
+    const float wp = hq_wave_sum(poison);
     if (lane == 0) poison_w[wv] = wp;
   }
   *reinterpret_cast<f4*>(red + (wv * 4 + kb) * 64 + 4 * c) = f4{tot[0], tot[1], tot[2], tot[3]};

@@ -126,17 +126,12 @@ __global__ __launch_bounds__(256) void quantize4_kernel(const T* __restrict__ x,
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_max(float v) {
-  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true)));
-}
-
 // Maximum over groups of `lanes` (1, 2, 4, ... 64; wave-uniform) adjacent lanes; every lane of a group gets it.
 __device__ __forceinline__ float group_max(float v, int lanes) {
-  if (lanes >= 2) v = dpp_max<0xB1>(v);    // quad_perm [1,0,3,2]
-  if (lanes >= 4) v = dpp_max<0x4E>(v);    // quad_perm [2,3,0,1]
-  if (lanes >= 8) v = dpp_max<0x141>(v);   // row_half_mirror
-  if (lanes >= 16) v = dpp_max<0x140>(v);  // row_mirror
+  if (lanes >= 2) v = fmaxf(v, hq_dpp<0xB1>(v));    // quad_perm [1,0,3,2]
+  if (lanes >= 4) v = fmaxf(v, hq_dpp<0x4E>(v));    // quad_perm [2,3,0,1]
+  if (lanes >= 8) v = fmaxf(v, hq_dpp<0x141>(v));   // row_half_mirror
+  if (lanes >= 16) v = fmaxf(v, hq_dpp<0x140>(v));  // row_mirror
   if (lanes >= 32) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));

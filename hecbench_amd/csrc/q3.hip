@@ -58,30 +58,6 @@ struct Q3Args {
 
 __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
-// Cross-lane reductions without LDS traffic: four DPP butterfly steps inside each
-// 16-lane row, then the four row results are read into scalars.
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float lane_f(float v, int l) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, dpp_f<0xB1>(v));   // quad_perm [1,0,3,2]
-  v = fmaxf(v, dpp_f<0x4E>(v));   // quad_perm [2,3,0,1]
-  v = fmaxf(v, dpp_f<0x141>(v));  // row_half_mirror
-  v = fmaxf(v, dpp_f<0x140>(v));  // row_mirror
-  return fmaxf(fmaxf(lane_f(v, 0), lane_f(v, 16)), fmaxf(lane_f(v, 32), lane_f(v, 48)));
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_f<0xB1>(v);
-  v += dpp_f<0x4E>(v);
-  v += dpp_f<0x141>(v);
-  v += dpp_f<0x140>(v);
-  return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
-}
-
 // Bits of word `word` of the 96-bit string that belong to the low three bits of a 6-bit field.
 constexpr uint32_t low3_mask(int word) {
   uint32_t m = 0;
@@ -91,7 +67,7 @@ constexpr uint32_t low3_mask(int word) {
 }
 
 // Row-wise broadcast of lane 8 of each 16-lane row (DPP row_newbcast:8).
-__device__ __forceinline__ float row_bcast8(float v) { return dpp_f<0x158>(v); }
+__device__ __forceinline__ float row_bcast8(float v) { return hq_dpp<0x158>(v); }
 
 // 4x4 byte transpose: in[j] holds four digits of value j, out[i] digit i of the four values.
 __device__ __forceinline__ void transpose4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t (&o)[4]) {
@@ -282,8 +258,8 @@ __global__ __launch_bounds__(WAVES * 64) void q3_matvec_kernel(HQ_ARGS24) {
         asum += xr[p][j];
       }
     }
-    const float xmax = wave_max(amax);
-    asum_total += wave_sum(asum);
+    const float xmax = hq_wave_max(amax);
+    asum_total += hq_wave_sum(asum);
     // 2^E * max|x| lies in [2^29, 2^30): v = rint(x * 2^E) + 0x88888888 never wraps, and its
     // nibbles n_d satisfy v = sum_d 16^d (n_d - 8).
     int E = 29 - ((int)((__float_as_uint(xmax) >> 23) & 255u) - 127);

@@ -58,19 +58,6 @@ struct BlockArgs {
   int prow;            // rows of partial sums a (virtual) column tile has per split
 };
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-__device__ __forceinline__ float quad_max(float v) {
-  v = fmaxf(v, dpp_f<0xB1>(v));  // quad_perm [1,0,3,2]
-  return fmaxf(v, dpp_f<0x4E>(v));  // quad_perm [2,3,0,1]
-}
-__device__ __forceinline__ float quad_sum(float v) {
-  v += dpp_f<0xB1>(v);
-  return v + dpp_f<0x4E>(v);
-}
-
 constexpr uint32_t low3_mask(int word) {
   uint32_t m = 0;
   for (int b = 0; b < 32; ++b)
@@ -209,7 +196,7 @@ __device__ __forceinline__ void q3_block_body(const BlockArgs& a, const int tile
 #pragma unroll
       for (int i = 0; i < 4; ++i) mx = __builtin_elementwise_max(mx, __builtin_elementwise_abs(pr[i]));
       const float amax = fmaxf((float)mx[0], (float)mx[1]);
-      const float gmax = quad_max(amax);  // the k-group's largest magnitude (its four lanes)
+      const float gmax = hq_quad(amax, HqMax());  // the k-group's largest magnitude (its four lanes)
       // 2^E * max|x| lies in [2^-3, 2^-2): 64 ... 127 subnormal steps of the fp8 format.  fp16 magnitudes: E in -18 ... 21.
       int E = -3 - ((int)((__float_as_uint(gmax) >> 23) & 255u) - 127);
       E = gmax > 0.f ? max(-18, min(21, E)) : 0;
@@ -284,12 +271,13 @@ __device__ __forceinline__ void q3_block_body(const BlockArgs& a, const int tile
     // sum of its four columns (four neighbouring lanes).  Lane c keeps the sums of i = c & 3.
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const float v0 = quad_sum(acc[q][0]), v1 = quad_sum(acc[q][1]), v2 = quad_sum(acc[q][2]), v3 = quad_sum(acc[q][3]);
+      const float v0 = hq_quad(acc[q][0], HqAdd()), v1 = hq_quad(acc[q][1], HqAdd());
+      const float v2 = hq_quad(acc[q][2], HqAdd()), v3 = hq_quad(acc[q][3], HqAdd());
       float v = (c & 2) ? ((c & 1) ? v3 : v2) : ((c & 1) ? v1 : v0);
       asm volatile("" : "+v"(v));  // selected here, not where it is stored (four candidates alive until then)
       keep[p][q] += v;
     }
-    rowsum[p] += quad_sum(colsum[0]);  // every result row holds the column sums
+    rowsum[p] += hq_quad(colsum[0], HqAdd());  // every result row holds the column sums
   };
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) {

@@ -22,7 +22,6 @@
 // no LDS traffic and no barrier in the loop.  The four waves' accumulators are
 // summed through LDS at the end and scale/zero are applied once per output.
 #include <mutex>
-#include <type_traits>
 
 #include "hq_internal.h"
 #include "q3_recipe.h"
@@ -44,23 +43,6 @@ constexpr int kTileN = 128;     // output columns per workgroup
 constexpr int kRowBlocks = 2, kRows = 32 * kRowBlocks;  // activation rows of a pass over the weights
 constexpr int kMaxSplitGroups = 256;  // workgroups of a K-split launch (tiles times splits)
 constexpr int kFixedMaxK = 16384;     // longest K of a batched call in the fixed scratch
-
-
-// Sum or maximum over the 64 lanes on the data path's own lane exchanges (two times six rounds of shuffles through the LDS
-// crossbar took 0.2 us longer: 32 rows, K=4096, N=11008 13.55 -> 13.3 us per call).
-template <bool MAX>
-__device__ __forceinline__ float prep_wave(float v) {
-  auto pick = [](float x, float y) { return MAX ? fmaxf(x, y) : x + y; };
-  auto dpp = [](float x, auto ctrl) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true));
-  };
-  auto at = [](float x, int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l)); };
-  v = pick(v, dpp(v, std::integral_constant<int, 0xB1>()));   // quad_perm [1,0,3,2]
-  v = pick(v, dpp(v, std::integral_constant<int, 0x4E>()));   // quad_perm [2,3,0,1]
-  v = pick(v, dpp(v, std::integral_constant<int, 0x141>()));  // row_half_mirror
-  v = pick(v, dpp(v, std::integral_constant<int, 0x140>()));  // row_mirror
-  return pick(pick(at(v, 0), at(v, 16)), pick(at(v, 32), at(v, 48)));
-}
 
 // ---- pre-pass: activations -> operand-slot order, scaled by P[m] * 2^-pos; row sums ------------
 // Ap[((g*4 + j)*Mpad + m)*8 + e] = A[m][32g + k] * P[m] * 2^-pos(k) with slot(k) = 8j + e; rows >= M and
@@ -115,8 +97,8 @@ __global__ __launch_bounds__(256) void q3_gemm_prep(const _Float16* __restrict__
       }
     }
   }
-  sum = prep_wave<false>(sum);
-  amax = prep_wave<true>(amax);
+  sum = hq_wave_sum(sum);
+  amax = hq_wave_max(amax);
   if (lane == 0) { s_sum[wv] = sum; s_max[wv] = amax; }
   __syncthreads();
   amax = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
