@@ -77,6 +77,10 @@ int hq_init(void);
  * re-ordered rows and the shares of divided tiles among them - on 256 compute units 8 MiB for max_K = 512, 16 MiB for
  * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152.  A stream that only ever sees smaller calls takes less without a
  * reservation: a workspace grows with the calls (hq_q3_workspace_need; batch 1 at most a few MiB, up to 64 rows 16 MiB).
+ * A captured call keeps the workspace of the stream it was captured on, whatever stream its graph is replayed on: replays must not
+ * overlap with each other or with calls on that stream where both use it.  Calls that overlap in one workspace give wrong results,
+ * and they may leave its arrival counters, which the kernels expect at zero and return to zero, at other values; hq_shutdown()
+ * and calls (and captures) anew start from fresh ones.
  * No counterpart in the reference. */
 int hq_reserve_workspace(void* stream, int max_K, int max_N);
 
@@ -145,22 +149,25 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  * (src/quant3MatMul-hip/kernels.h:171-217) — pass HQ_FLAG_ACCUMULATE for their
  * "mul +=" behaviour.  batch_M > 1 requires HQ_DTYPE_F16 and has no counterpart in
  * the reference; which kernel serves it (hq_q3_matvec_plan tells):
- *   - the matvec's kernel, four rows side by side: batches 2 ... 4 (at 0.1 ... 0.6 us more than
- *     batch 1); batches up to 64 as row blocks of four, one workgroup per column tile, 4096
- *     elements of K and row block, where that makes at most four workgroups per compute unit
- *     (5 and 6 rows: at most one) and K <= 32768; otherwise 5 ... 8 rows as two passes of one
- *     workgroup unless N / 128 is at least 7/8 of the compute units or K is longer than that;
- *     every activation enters with an error of at most 2^-19 of the largest magnitude
- *     among its 32 neighbours (exactly, if within 2^8 of it);
- *   - everything else: the MFMA GEMM path.  Up to 64 rows go in one pass over the weights; more than 96 rows, and 65 to 96
- *     rows where N > 4096 or where K <= 8192 and K * N < 2^25, in tiles of 64 or 128 rows, up to thousands of rows per pass;
- *     the remaining 65 to 96 rows in two passes of up to 64.  Under stream capture, where the stream's workspace is too small
- *     for the tiles' scratch and cannot grow, the call still succeeds with the workspace of a call of 64 rows: it goes 64 rows at a
- *     time, with results equal to rounding (not bit for bit) and slower, 1.3 to 5 times at hundreds of rows;
- *     hq_reserve_workspace keeps calls off that path.  Every activation row is pre-scaled by a
- *     power of two, so accuracy does not depend on the magnitude of the activations:
- *     entries within 2^21 of their row's largest magnitude enter the matrix cores
- *     exactly, smaller ones lose low bits (those 2^32 below it vanish).
+ *   - the matvec's kernel, four rows side by side: batches 2 ... 4 (at 0.1 ... 0.6 us more than batch 1); up to 64 rows as row
+ *     blocks of four, one workgroup per column tile, 4096 elements of K and row block, while every workgroup has a compute unit of
+ *     its own (beyond K = 32768: 5 ... 12 rows as two or three passes of one workgroup, by the same count); and 5 ... 8 rows of
+ *     7e7 weights and more as row blocks or two passes, unless N / 128 is at least 7/8 of the compute units.  Every activation
+ *     enters with an error of at most 2^-19 of the largest magnitude among its 32 neighbours (exactly, if within 2^8 of it);
+ *   - the matrix cores in one launch: all other batches of up to 32 rows, 33 to 64 rows of less than 9e7 weights, 65 to 96 rows
+ *     where N <= 4096, and more rows as long as the estimated time is below the tiles' (hundreds of rows of small matrices).  A
+ *     tile's K may be divided among up to eight workgroups.  Activations enter as they are;
+ *   - 33 to 64 rows of 9e7 weights and more: the matrix cores behind a pre-pass that re-orders the activations;
+ *   - the rest: tiles of 64 or 128 rows behind such a pre-pass, up to thousands of rows per pass over the weights.
+ * The pre-pass scales every activation row by a power of two, so accuracy does not depend on the magnitude of the activations:
+ * entries within 2^21 of their row's largest magnitude enter the matrix cores exactly, smaller ones lose low bits (those 2^32 below
+ * it vanish).
+ * Under stream capture, where a stream's workspace cannot grow, a call that finds too little room for its plan succeeds on another
+ * one: one launch with K undivided where a tile's K would have been divided or a pre-pass would have no place for its result, and,
+ * in place of the tiles, 64 rows at a time where there is the workspace of a call of 64 rows.  The results equal those of the
+ * eager call to rounding, not bit for bit, and the call is slower (64 rows at a time 1.3 to 5 times at hundreds of rows).
+ * hq_reserve_workspace keeps calls off these ways; batch 1 and the matvec's kernel have none and fail where K is divided and there is
+ * no room.
  */
 int hq_q3_matvec(const void* x, int x_dtype, const int32_t* qweight, const float* scales,
                  const float* zeros, float* y, int K, int N, int batch_M, unsigned flags,
@@ -179,8 +186,8 @@ int hq_q3_matvec_plan(int K, int N, int batch_M);
 /*
  * hq_q3_matvec for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): same arguments, same kernels and bit-identical results, but the
- * scratch the kernels need (split-K partial sums and arrival counters of batches 1 and 2, the batched
- * path's re-ordered activations, row sums, row scales and K-split sums) is a fixed 68 MiB + 128 KiB array in device
+ * scratch the kernels need (partial sums and arrival counters of a divided K, the batched
+ * path's re-ordered activations, row sums and row scales) is a fixed 68 MiB + 128 KiB array in device
  * memory that each GPU holds from library load to process end, instead of the stream's workspace (the runtime clears it
  * when it loads the library onto a GPU: about 25 ms of the first hq_init).
  * The call runs no hipMalloc, hipFree or allocating library routine.  Limits: a batch that the MFMA
