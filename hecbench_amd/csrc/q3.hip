@@ -553,16 +553,22 @@ int q3_block_row_blocks(int cus, int K, int N, int batch_M, int nsplit, int rpw)
 // Small launches of more than four rows: row blocks while every workgroup has a compute unit of its own (then 5 to 7 us, ahead of
 // anything else by a quarter), beyond that the one-launch matrix-core kernel of q3_direct.hip.  Workgroups per compute unit that
 // row blocks would need, and both (us): 0.86: 5.3 / 7.3 (26 rows, K=2528, N=1960); 1.04: 6.9 / 6.7 (11 rows, K=1824, N=5640); 1.5: 9.6 /
-// 8.3 (16 rows, K=5120, N=3068); 2.5: 9.9 / 6.8 (12 rows, K=1696, N=13684); 3.7: 14.6 / 8.9 (45 rows, K=3648, N=5028).  Up to eight rows of
-// a large matrix are as fast either way (7e7 weights and more: 14.3 / 14.4, 19.2 / 19.6, 25.2 / 25.0) and stay where they were.
+// 8.3 (16 rows, K=5120, N=3068); 2.5: 9.9 / 6.8 (12 rows, K=1696, N=13684); 3.7: 14.6 / 8.9 (45 rows, K=3648, N=5028).
+// Five to eight rows stay, as passes of one workgroup (five and six) or row blocks, where four rows would have a compute unit for
+// every workgroup and the matrix is large: the one-launch kernel's time grows with it, theirs hardly does (us, theirs / one launch:
+// 5 rows, K=4096, N=11008 7.5 / 8.7, K=8192, N=8192 9.9 / 11.5, K=2816, N=12736 6.85 / 7.5, K=5184, N=5008 8.8 / 8.9, K=4480, N=4516 8.9 / 8.4; 6
+// rows 4096 x 11008 8.0 / 8.7, 6048 x 6824 9.65 / 9.8, 2272 x 15704 7.4 / 7.2, 5440 x 5372 9.4 / 8.8; 8 rows 8192 x 8192 10.5 / 11.5, 7680 x
+// 6328 10.1 / 11.6, 4096 x 11008 8.55 / 8.7, 6048 x 6824 9.7 / 9.8, 8608 x 4376 10.2 / 9.6).  So do up to eight rows of 7e7 weights and
+// more (8 rows, K=4096, N=22016 11.7 / 12.3, K=28672, N=8192 26.8 / 28.0, but K=8192, N=9000 13.2 / 12.6).
 bool q3_block_yields(int cus, int K, int N, int batch_M) {
   if (!hq_q3_direct_can(K, N)) return false;
   if (hq_q3_direct_forced()) return true;
   if (batch_M <= 4 || hq_tune(HQ_TUNE_Q3_ROW_BLOCKS, -1) >= 0) return false;
   int nsplit, rpw;
   q3_block_split(cus, K, N, batch_M, &nsplit, &rpw);
-  if (batch_M <= 8 && (int64_t)K * N >= 70000000) return false;
-  return (int64_t)((N + 63) / 64) * nsplit * ((batch_M + 3) / 4) > cus;
+  const int64_t groups = (int64_t)((N + 63) / 64) * nsplit, weights = (int64_t)K * N;
+  if (batch_M <= 8 && (weights >= 70000000 || (groups <= cus && weights >= (batch_M <= 6 ? 35000000 : 40000000)))) return false;
+  return groups * ((batch_M + 3) / 4) > cus;
 }
 
 int q3_plan(int cus, int K, int N, int batch_M) {

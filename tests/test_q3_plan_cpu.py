@@ -27,3 +27,14 @@ def test_a_batch_that_keeps_its_row_blocks_makes_no_other_plan(K, N, M):
     long again as all else (0.33 us with the call through ctypes, four rows, which no other kernel competes for; 0.61 with it)."""
     lib = _lib.load()
     assert _us(lib, K, N, M) <= 1.4 * _us(lib, K, N, 4)
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(5, 4096, 11008, "block"), (6, 4096, 11008, "block"), (5, 8192, 8192, "block"),
+                                          (6, 11008, 4096, "block"), (8, 8192, 8192, "block"), (7, 7680, 6328, "block"),
+                                          (5, 5184, 5008, "direct"), (6, 5440, 5372, "direct"), (8, 8608, 4376, "direct"),
+                                          (9, 4096, 11008, "direct"), (5, 4224, 14336, "direct")])
+def test_five_to_eight_rows_of_a_large_matrix_stay_with_the_block_kernel(M, K, N, kernel):
+    """On 256 compute units: its passes and row blocks take 2 to 17 % less than the one-launch kernel while four rows would have a
+    compute unit for every workgroup (not the last: 448 of them) and the matrix has 3.5e7 weights and more (seven and eight rows: 4e7)."""
+    choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
+    assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel

@@ -20,7 +20,9 @@ BATCH = {"default": {}, "gemm": {"HQ_Q3_SMALL_BATCH": 0}, "passes": {"HQ_Q3_ROW_
 CASES = [
     (4096, 11008, 1, MATVEC),
     (4096, 11008, 4, BATCH),
+    (4096, 11008, 5, BATCH),
     (4096, 11008, 8, BATCH),
+    (8192, 8192, 8, BATCH),
     (4096, 11008, 16, BATCH),
     (4096, 4096, 1, MATVEC),
     (4096, 4096, 12, BATCH),
