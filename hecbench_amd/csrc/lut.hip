@@ -662,8 +662,9 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
     // 34 quads, 12.2 / 13.1): every round is a workgroup of its own, which has half the registers, so that two share
     // a compute unit and the work is even whatever the tiles (us, walked / apart: 10880 x 17510 three planes 29.0 / 22.8; 14208 x 16512
     // 28.5 / 21.5; 8448 x 7943 two planes 9.3 / 7.9; 10624 x 25368 group 64 37.8 / 33.2; not 4864 x 26591 one plane, 416 tiles, 7.6 / 9.2;
-    // not 4224 x 12997, 204 tiles, 8.7 / 9.8), with three or more planes in small groups one quad per wave (6656 x 18823 group 32 30.9,
-    // 25.0, fine 22.3; 13568 x 4444 group 64 14.3, 13.5, 12.1).
+    // not 4224 x 12997, 204 tiles, 8.7 / 9.8), with three or more planes in small groups one quad per wave (three planes, walked / apart /
+    // fine: 6656 x 18823 group 32 30.9 / 25.0 / 22.3 in the plain order of tiles, apart 20.8 and fine 18.1 in hq_column_tile's; 13568 x
+    // 4444 group 64 14.3 / 13.5 / 12.1, and 12.3, 11.1).
     const int waves_of_tiles = (ntiles + cus - 1) / cus;
     const bool full_end = 2 * nquads >= (2 * rounds - 1) * 8 * QUADS;
     apart = !fine && rpw > 1 &&

@@ -306,11 +306,11 @@ int launch_quantize4_units(const T* x, uint8_t* packed, float* absmax, int64_t n
 
 // Units per lane.  Blocks up to 512 elements: one, as the wave launcher is the better load scheduler (2^23 fp16 elements
 // 5.2 / 5.5 / 6.5 us with 1 / 2 / 4; fp32 4096 x 11008 33.9 / 36.2 / 37.9), except for large fp16 inputs, where a
-// workgroup's table and barrier weigh more (4096 x 11008: 20.2 / 18.9 / 19.6).  Longer blocks keep to one (fp32) or two (fp16) units
-// and are shared by the waves of a workgroup, which exchange their maxima at the barrier that the cells need anyway (us with one
-// wave per block, of 2, 4, 8 units a lane / this: blocksize 4096 of 5521 fp16 elements 5.4 / 2.9, 1 M 4.9 / 3.0, 8.4 M 6.9 / 5.7, 45 M
-// 22.5 / 20.3, fp32 38.6 / 35.2; 2048 of 45 M fp16 21.9 / 20.35, fp32 37.4 / 33.4; 1024 fp32 35.2 / 33.7.  One unit of fp16: 2048 22.4,
-// 1024 22.3 instead of 20.3).
+// workgroup's table and barrier weigh more (4096 x 11008: 20.2 / 18.9 / 19.6).  Longer blocks keep to one (fp32) or two (fp16, and
+// fp32 blocks of 4096, which have no more than four waves) units and are shared by the waves of a workgroup, which exchange their
+// maxima at the barrier that the cells need anyway (us with one wave per block, of 2, 4, 8 units a lane / this: blocksize 4096 of
+// 5521 fp16 elements 5.4 / 2.9, 1 M 4.9 / 3.0, 8.4 M 6.9 / 5.7, 45 M 22.5 / 20.3, fp32 38.6 / 35.2; 2048 of 45 M fp16 21.9 / 20.35,
+// fp32 37.4 / 33.4; 1024 fp32 35.2 / 33.7.  One unit of fp16: 2048 22.4, 1024 22.3 instead of 20.3).
 template <typename T>
 int quantize4_units(const T* x, uint8_t* packed, float* absmax, int64_t n, int blocksize, int table, hipStream_t stream) {
   constexpr bool kHalf = sizeof(T) == 2;

@@ -505,7 +505,7 @@ namespace {
 // applied to every caller so that both entry points run the same kernel on the same shape.
 constexpr size_t kBlockPartialRows = 8192;
 
-// How the kernel for 2 ... 8 rows cuts K: up to eight rounds of 4096 elements, one workgroup per round (as the
+// How the block kernel cuts K: up to eight rounds of 4096 elements, one workgroup per round (as the
 // batch-1 kernel); beyond that as many workgroups per column tile as give every compute unit two, each taking
 // several rounds one after the other.
 void q3_block_split(int cus, int K, int N, int batch_M, int* nsplit, int* rpw) {
@@ -530,13 +530,13 @@ constexpr int kRowBlockBatchMax = 64;  // rows a batch may have as row blocks of
 // one workgroup; 0: the four-rows-per-pass kernel does not take this batch at all.
 int q3_block_row_blocks(int cus, int K, int N, int batch_M, int nsplit, int rpw) {
   (void)K;
-  // Measured (us per call, passes in one workgroup or the GEMM -> row blocks): with a CU for every workgroup,
-  // K=4096, N=4096: 5 rows 7.2 -> 5.2, 8 rows 8.4 -> 5.3, 12 rows 11.7 -> 5.3, 16 rows 12.7 -> 5.6; with up to
-  // four workgroups per CU, K=4096, N=4096, 32 rows 12.8 -> 8.4; K=4096, N=11008: 8 rows 9.0 -> 8.5, 12 rows
-  // 12.3 -> 11.0, 16 rows 14.3 -> 11.4; K=11008, N=4096: 12 rows 15.0 -> 12.8, 16 rows 17.6 -> 13.0; K=4096,
-  // N=22016: 7 rows 14.4 -> 11.9, 8 rows 15.2 -> 11.7; K=8192, N=8192: 16 rows 16.5 -> 16.2.  Five and six
-  // rows in more workgroups than CUs do not gain (K=4096, N=11008, 5 rows: 7.8 -> 8.4): the second block's one
-  // or two rows cost a whole workgroup where a second pass costs two rows of staging.
+  // Measured (us per call, passes in one workgroup -> row blocks): with a CU for every workgroup, K=4096, N=4096: 5
+  // rows 6.9 -> 5.2, 8 rows 8.2 -> 5.3, 12 rows 11.5 -> 5.3; with up to four workgroups per CU, K=4096, N=11008: 8 rows
+  // 8.8 -> 8.5, 12 rows 12.1 -> 11.05; K=11008, N=4096: 12 rows 14.2 -> 12.4; K=4096, N=22016: 7 rows 14.4 -> 11.7, 8 rows
+  // 15.1 -> 11.7.  Five and six rows in more workgroups than CUs do not gain (K=4096, N=11008, 5 rows: 7.5 -> 8.4): the
+  // second block's one or two rows cost a whole workgroup where a second pass costs two rows of staging.  Most batches
+  // with more workgroups than CUs then go to the one-launch kernel all the same (q3_block_yields: 12 rows 8.65, 16 rows 8.75
+  // at K=4096, N=11008).
   const int mode = hq_tune(HQ_TUNE_Q3_ROW_BLOCKS, -1);  // 0: never, 1: wherever possible (tests)
   if (batch_M <= 4) return 1;
   const int mb = (batch_M + 3) / 4;
@@ -580,17 +580,16 @@ int q3_plan(int cus, int K, int N, int batch_M) {
   const int mb = q3_block_row_blocks(cus, K, N, batch_M, nsplit, rpw);
   if (mb > 1) return HQ_Q3_PLAN_BLOCK;
   if (mb == 0) return HQ_Q3_PLAN_GEMM;
-  // 2 ... 8 rows in one workgroup per tile and K range.  Five to eight rows take
-  // two passes per workgroup, which beats the GEMM (7.8-12.4 us against 13-19 us at 4096 x 4096 ... 14336 x
-  // 4096, 20.7-24.9 against 24.7 at K=8192, N=22016, 26.5-31.9 against 31.6 at K=28672, N=8192) except where
-  // the GEMM's 128-column tiles fill the device without a K split (K=8192, N=28672: 27.8-31.1 against 25.3 us).
+  // 2 ... 8 rows in one workgroup per tile and K range, five to eight rows as two passes, except where 128-column tiles fill
+  // the device without a K split (K=8192, N=28672, 8 rows: 27.8-31.1 us, the 64-row kernel 25.3, the one-launch kernel, which
+  // takes those batches, 22); which of them leave this kernel for the one-launch kernel is q3_block_yields' matter.
   const size_t groups = (size_t)((N + 63) / 64) * nsplit;
   const size_t tiles128 = (size_t)(N + 127) / 128;
   if (batch_M <= 8 && (nsplit == 1 || groups * batch_M <= kBlockPartialRows) &&
       (batch_M <= 4 || (rpw == 1 && 8 * tiles128 < 7 * (size_t)cus)))
     return HQ_Q3_PLAN_BLOCK;
-  // 9 ... 12 rows, three passes: where the launch has at most one workgroup per compute unit (it is a matter
-  // of latency there, and the GEMM needs three launches)
+  // 9 ... 12 rows, three passes: where the launch has at most one workgroup per compute unit.  Up to K=32768 such a batch goes on as
+  // row blocks or to the one-launch kernel; three passes are what is left of it beyond.
   if (batch_M <= 12 && rpw == 1 && groups <= (size_t)cus) return HQ_Q3_PLAN_BLOCK;
   return HQ_Q3_PLAN_GEMM;
 }

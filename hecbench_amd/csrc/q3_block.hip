@@ -24,14 +24,14 @@
 // the matrix core does not add products that far apart exactly, 5e-5 of the output RMS was lost.)
 // Five to eight rows take two passes over the weights held in registers: terms of four rows staged in LDS,
 // sixteen MFMAs per wave, the pass's sums folded into four registers, next four rows; nine to twelve rows
-// take three passes where the launch is small (see q3_block_kernel_many below).
+// of a K beyond 32768 take three passes where the launch is small (see q3_block_kernel_many below).
 // Everything else follows q3.hip: a workgroup owns a 64-column tile and one round of K (8 waves x 4 steps x
 // 4 k-groups = 4096 elements), a wave's 16-lane quarter streams one k-group per step as three 128-bit loads,
 // every wave stages its own operand behind a wave-local fence, the waves meet once at the end, and K beyond
 // one round is split across workgroups whose partial sums the last one to arrive adds up in split order.
 // The weights are read once for all rows at nine VALU instructions per 32 weights and pass, in one launch,
-// where the batched GEMM (q3_gemm.hip) needs a pre-pass, twenty per 32 weights, and a third launch when it
-// splits K.  No counterpart in the reference (its kernels are batch 1: src/quant3MatMul-hip/kernels.h:12-217).
+// where the 64-row kernel (q3_gemm.hip) needs a pre-pass and twenty per 32 weights, and the one-launch kernel
+// (q3_direct.hip) takes its time for 32 rows whatever their number.  No counterpart in the reference (its kernels are batch 1: src/quant3MatMul-hip/kernels.h:12-217).
 #include "hq_internal.h"
 
 namespace {

@@ -5,7 +5,9 @@
 //
 // The reference benchmark has only the batch-1 matvec
 // (src/quant3MatMul-hip/kernels.h in the HeCBench tree); this is the same
-// arithmetic applied to up to 64 activation rows per pass on the matrix cores.
+// arithmetic applied to up to 64 activation rows per pass on the matrix cores.  It serves 33 to 64 rows of 9e7 weights and more, and
+// stands in where a captured call finds room for 64 rows' activations only; fewer rows and smaller matrices go through
+// q3_direct.hip, more rows through q3_prefill.hip, whose pre-pass is the one here.
 //
 // As in the matvec, the packed codes are never converted: an AND turns a 32-bit
 // window of the packed string into two subnormal-fp16 MFMA operands
@@ -312,8 +314,8 @@ __global__ __launch_bounds__(kWaves * 64) void q3_gemm_kernel(const uint32_t* w_
   if (a.nsplit == 1 || !a.counters) return;
   // Every wave waits for the acknowledgement of its write-through stores, the workgroup counts itself at the memory side,
   // and the last of the tile adds the raw sums in split order, four splits' loads in flight.  (As a kernel of its own this took
-  // 3.4 to 5.1 us and a launch: 23 rows, K=1952, N=12980 13.7 -> 11.7 us, 64 rows, K=4096, N=11008 19.9 -> 18.5; with eight splits of 64
-  // rows, 256 KB for one workgroup, the kernel of its own stays ahead, 24.4 against 25.4 at K=16384, N=4096.)
+  // 3.4 to 5.1 us and a launch: 64 rows, K=4096, N=11008, which the one-launch kernel has taken over since, 19.9 -> 18.5 us; with eight
+  // splits of 64 rows, 256 KB for one workgroup, the kernel of its own stays ahead, 24.4 against 25.4 at K=16384, N=4096.)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // also: nobody reads the waves' sums in LDS any more
   unsigned* flag = reinterpret_cast<unsigned*>(lds);

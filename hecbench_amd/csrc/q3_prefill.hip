@@ -17,7 +17,7 @@
 //     matrix instructions, and unpacking fills the slots between those.
 //   - Tiles that do not fill a round of the compute units are divided along K (tile_plan).
 // K=8192, N=28672, 1021 rows: 574 -> 363-390 us (1.22-1.32 PFLOP/s; the library's fp16 product of 8192^3 runs at 1.2 here);
-// 512 rows, K=4096, N=11008: 153 -> 52-57; 463 rows, K=5408, N=660: 118 -> 24; 128 rows, K=8192, N=28672: 75 -> 58.
+// 512 rows, K=4096, N=11008: 153 -> 52-57; 128 rows, K=8192, N=28672: 75 -> 58.
 #include <type_traits>
 
 #include "hq_internal.h"
@@ -341,9 +341,9 @@ struct TilePlan {
 // The three tiles and what they cost, measured on MI355X (us): a step (64 * ks elements of K; between a launch of few
 // workgroups and a full device, whose clock the power limit lowers), and dividing a tile's K into c shares.  A tile costs
 // 3 us beside its steps (first loads from HBM, the parts of K meeting, results).  The large tile multiplies most per
-// load and unpacked weight: K=8192, N=28672, 1021 rows 363-379 us against 406 and 510 with the smaller ones; 512 rows, K=4096,
-// N=11008 52 / 59 / 64.  Small problems want more workgroups: 128 rows, K=8192, N=28672 64 / 58 / 73; 463 rows, K=5408, N=660
-// 39 / 27 / 24; 100 rows, K=1024, N=2048 21.6 / 14.6 / 12.1.
+// load and unpacked weight: K=8192, N=28672, 1021 rows 367 us against 397 and 520 with the smaller ones; 512 rows, K=4096,
+// N=11008 52 / 58 / 68.  Smaller problems want more workgroups: 128 rows, K=8192, N=28672 61 / 57 / 78; 98 rows, K=4512, N=8712
+// 33 / 24 / 27; 397 rows, K=2720, N=9220 41 / 40 / 37.  (The smallest are the one-launch kernel's: q3_direct.hip.)
 struct TileKind {
   int tm, tn, ks;
   float step_us, share_us, per_share_us;
