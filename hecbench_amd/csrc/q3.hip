@@ -812,7 +812,12 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
     if (q3_plan(dev->cus, K, N, batch_M) == HQ_Q3_PLAN_BLOCK) {
       const Q3BlockPlan b = q3_block_shape(dev->cus, K, N, batch_M, lim);
       if (b.split.nsplit != b.nsplit) return HQ_ERR_BAD_SHAPE;
-      if (!b.split.too_large && q3_block_yields(dev->cus, K, N, batch_M))
+      // (under capture without room for the sums of a divided K: the one-launch kernel can do without)
+      const auto no_room = [&] {
+        return !fixed && b.split.nsplit > 1 && hq_q3_direct_can(K, N) &&
+               hq_workspace_out_of_reach(stream, b.split.floats, (size_t)b.split.ntiles);
+      };
+      if (!b.split.too_large && (q3_block_yields(dev->cus, K, N, batch_M) || no_room()))
         return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, batch_M, false), dev->cus, x, qweight, scales, zeros, y, K, N,
                                    batch_M, flags, stream, fixed);
       rc = q3_split_acquire(b.split, fixed, stream, &sp);

@@ -152,8 +152,9 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  *   - the matvec's kernel, four rows side by side: batches 2 ... 4 (at 0.1 ... 0.6 us more than batch 1); up to 64 rows as row
  *     blocks of four, one workgroup per column tile, 4096 elements of K and row block, while every workgroup has a compute unit of
  *     its own (beyond K = 32768: 5 ... 12 rows as two or three passes of one workgroup, by the same count); and 5 ... 8 rows of
- *     7e7 weights and more as row blocks or two passes, unless N / 128 is at least 7/8 of the compute units.  Every activation
- *     enters with an error of at most 2^-19 of the largest magnitude among its 32 neighbours (exactly, if within 2^8 of it);
+ *     large matrices (3.5e7 weights, 7 and 8 rows 4e7, while four rows would have a compute unit for every workgroup; 7e7 at any
+ *     size) as two passes or row blocks, unless N / 128 is at least 7/8 of the compute units.  Every activation enters with an
+ *     error of at most 2^-19 of the largest magnitude among its 32 neighbours (exactly, if within 2^8 of it);
  *   - the matrix cores in one launch: all other batches of up to 32 rows, 33 to 64 rows of less than 9e7 weights, 65 to 96 rows
  *     where N <= 4096, and more rows as long as the estimated time is below the tiles' (hundreds of rows of small matrices).  A
  *     tile's K may be divided among up to eight workgroups.  Activations enter as they are;
@@ -163,11 +164,10 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  * entries within 2^21 of their row's largest magnitude enter the matrix cores exactly, smaller ones lose low bits (those 2^32 below
  * it vanish).
  * Under stream capture, where a stream's workspace cannot grow, a call that finds too little room for its plan succeeds on another
- * one: one launch with K undivided where a tile's K would have been divided or a pre-pass would have no place for its result, and,
- * in place of the tiles, 64 rows at a time where there is the workspace of a call of 64 rows.  The results equal those of the
- * eager call to rounding, not bit for bit, and the call is slower (64 rows at a time 1.3 to 5 times at hundreds of rows).
- * hq_reserve_workspace keeps calls off these ways; batch 1 and the matvec's kernel have none and fail where K is divided and there is
- * no room.
+ * one: the matrix cores in one launch with K undivided where K would have been divided or a pre-pass would have no place for its
+ * result, and, in place of the tiles, 64 rows at a time where there is the workspace of a call of 64 rows.  The results equal
+ * those of the eager call to rounding, not bit for bit, and the call is slower (64 rows at a time 1.3 to 5 times at hundreds of
+ * rows).  hq_reserve_workspace keeps calls off these ways; batch 1 has none and fails where K is divided and there is no room.
  */
 int hq_q3_matvec(const void* x, int x_dtype, const int32_t* qweight, const float* scales,
                  const float* zeros, float* y, int K, int N, int batch_M, unsigned flags,

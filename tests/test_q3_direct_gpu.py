@@ -105,17 +105,17 @@ def test_default_plans(hq, oracle, M, K, N):
     assert torch.equal(got[1, True], got[0, True] + 3.0)
 
 
-@pytest.mark.parametrize("stands_in", [False, True])
-def test_capture_without_any_workspace(hq, oracle, tunable, stands_in):
+@pytest.mark.parametrize("M,K,N,kernel", [(39, 4160, 1176, "direct"), (39, 4160, 1176, "rows64"), (6, 11008, 4096, "block"),
+                                          (8, 8192, 8192, "block")])
+def test_capture_without_any_workspace(hq, oracle, tunable, M, K, N, kernel):
     """Under capture nothing can be allocated: on a stream that has no workspace the call divides no tile, and replays give the
     eager result's values to the last bits but the order of the sums.  The same for a batch of the 64-row kernel, whose re-ordered
-    activations have no place there."""
+    activations have no place there, and for the block kernel where it would divide K."""
     import torch
-    M, K, N = 39, 4160, 1176
-    if stands_in:
+    if kernel == "rows64":
         tunable("HQ_Q3_SMALL_BATCH", 0)
         tunable("HQ_Q3_TILES", 9)
-    assert kernel_of(M, K, N) == ("rows64" if stands_in else "direct")
+    assert kernel_of(M, K, N) == kernel
     codes, scales, zeros, A = oa.make_q3_problem(11, K, N, x_dtype=np.float16, batch=M)
     mat = oracle.q3_pack(codes)
     a, w, s, z = _t(A), _t(mat), _t(scales), _t(zeros)
