@@ -136,8 +136,8 @@ bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t ne
   return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
 }
 
-// Upper bound of what any hq_q3_matvec call with K <= max_K, N <= max_N (any batch) and any hq_lut_gemv call
-// of those sizes takes from its stream's workspace on a device of `cus` compute units, with the default launch
+// Upper bound of what any hq_q3_matvec call with K <= max_K, N <= max_N (any batch) and any hq_lut_gemv or hq_aqlm_matvec
+// call of those sizes (rows as columns) takes from its stream's workspace on a device of `cus` compute units, with the default launch
 // policy.  Host arithmetic only.  (tests/test_workspace_cpu.py checks it against the per-call need over a
 // sweep of shapes.)
 static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t* counters) {
@@ -161,6 +161,8 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   // batches 2 ... 64 on the matvec-like kernel: one partial row per tile, range of K and activation row, at most
   // 8192 of them whatever the shape
   if ((size_t)8192 * 64 > split_floats) split_floats = (size_t)8192 * 64;
+  // the AQLM kernel in slices: eight sums a row, rows padded to whole groups (an eighth of the compute units)
+  if ((size_t)8 * (max_N + cus / 8) > split_floats) split_floats = (size_t)8 * (max_N + cus / 8);
   *floats = gemm_floats > split_floats ? gemm_floats : split_floats;
   // many rows: the tiled kernels
   size_t tile_floats = 0, tile_counters = 0;
@@ -169,6 +171,7 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   // arrival counters: one per column tile, narrow tiles four per 64 columns, row blocks sixteen per tile
   *counters = tiles > 1 ? tiles * 16 : 16;
   if (tile_counters > *counters) *counters = tile_counters;
+  if ((size_t)cus / 8 > *counters) *counters = cus / 8;  // and one per group of rows of the AQLM kernel
 }
 
 extern "C" int hq_reserve_need(int compute_units, int max_K, int max_N, int64_t* floats, int64_t* counters) {

@@ -237,7 +237,9 @@ int hq_lut_gemv_plan(const uint32_t* bW, const void* alpha_fp16, const void* q_b
  * with m < codebook_a_sizes[j] (4 where there is none).  scales_fp16 may be NULL (the reference kernel
  * applies no scale).  K % 64 == 0 (as in the reference).  fp32 accumulation, one rounding.  Replaces
  * code1x16_matvec, src/quantAQLM-hip/main.cu:103-139 (without its internal
- * synchronisation, timing and printing).
+ * synchronisation, timing and printing).  Calls of several million codes leave partial sums in the stream's workspace (eight
+ * floats a row; hq_reserve_workspace with max_N >= M makes room); under stream capture, or where there is no room and none can be
+ * had, they run on the kernel that needs none.
  */
 int hq_aqlm_matvec(const int16_t* codes, const void* codebooks_fp16, const void* scales_fp16,
                    const void* x_fp16, void* y_fp16, int M, int K,

@@ -50,6 +50,72 @@ def test_default_rules(hq, oracle, M, K):
     assert rel_err(y, ref64, FLOOR_F16) <= 2e-3
 
 
+@pytest.mark.parametrize("sub", [0, 1, 2])
+@pytest.mark.parametrize("M,K,ncb", [(1, 64, 1), (31, 1024, 1), (33, 1088, 3), (2049, 2112, 1), (2100, 4096, 3), (8193, 1600, 1), (70, 15872, 3)])
+def test_code_book_in_slices(hq, oracle, tunable, M, K, ncb, sub):
+    """Groups of rows without rows, of one and of several trips, the last with waves that have none; rows of one run of lanes and of
+    several, the last cut; the longest K; groups with rows of several code books, one of them empty."""
+    codes, cb, scales, x = oa.make_aqlm_problem(M + 3 * K, M, K, ncb=ncb)
+    sizes = (M, 0, 0, 0) if ncb == 1 else (M // 3, M // 3, M // 2, M)
+    if ncb == 3:
+        cb = np.concatenate([cb, cb[:1] * np.float16(2)])
+    tunable("HQ_AQLM_ROWS", 20 + sub)
+    y = _run(hq, codes, cb, scales, x, sizes)
+    _, ref64 = oracle.aqlm_matvec(codes, cb, scales, x, sizes, 65536, mode=0)
+    assert rel_err(y, ref64, FLOOR_F16) <= 2e-3
+    assert np.array_equal(y.view(np.uint16), _run(hq, codes, cb, scales, x, sizes).view(np.uint16))
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_slices_and_numbers_that_are_none(hq, tunable, bad):
+    """An infinity or NaN among the activations, or in a code book, reaches the outputs that it reaches without slices, as it does there."""
+    M, K = 300, 640
+    codes, cb, scales, x = oa.make_aqlm_problem(77, M, K)
+    for in_x in (True, False):
+        xs, cbs = x.copy(), cb.copy()
+        if in_x:
+            xs[K // 2] = bad
+            cbs[0, codes[5, K // 16].astype(np.uint16), (K // 2) % 8] = 0  # times zero: NaN there
+        else:
+            cbs[0, codes[7, 3].astype(np.uint16), 2] = bad
+            xs[8 * np.arange(K // 8)[codes[9] == codes[7, 3]] + 2] = 0
+        got = []
+        for knob in (1, 21):
+            tunable("HQ_AQLM_ROWS", knob)
+            got.append(_run(hq, codes, cbs, scales, xs, (M, 0, 0, 0)).astype(np.float64))
+        fin = np.isfinite(got[0])
+        assert not fin.all() and np.array_equal(got[0][~fin], got[1][~fin], equal_nan=True)
+        assert not fin.any() or rel_err(got[1][fin], got[0][fin], FLOOR_F16) <= 2e-3
+
+
+def test_default_takes_slices_but_not_under_capture(hq, tunable):
+    import torch
+    M, K = 8192, 4096
+    codes, cb, scales, x = oa.make_aqlm_problem(8, M, K)
+    t = [torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0") for a in (codes, x, cb, scales)]
+    call = lambda: hq.code1x16_matvec(t[0], t[1], t[2], (M, 0, 0, 0), 65536, scales=t[3])
+    y = call()
+    want = {}
+    for knob in (2, 22):
+        tunable("HQ_AQLM_ROWS", knob)
+        want[knob] = call()
+    assert torch.equal(y, call())           # as forced: in slices
+    assert not torch.equal(want[2], want[22])  # (sums in another order round differently somewhere among 8192)
+    from hecbench_amd import _lib
+    _lib.load().hq_set_tunable(b"HQ_AQLM_ROWS", 0, 1)
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            out = call()
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_err(out.cpu().numpy(), y.cpu().numpy().astype(np.float64), FLOOR_F16) <= 2e-3
+        assert torch.equal(call(), y)
+
+
 def test_three_codebooks_and_no_scale(hq, oracle):
     """Reference default geometry: 3 code books of 4096 rows each, no scale."""
     M, K = 12288, 1024
