@@ -17,6 +17,8 @@ std::map<int, HqDevice> g_devices;
 constexpr int kListedDevices = 64;
 std::atomic<const HqDevice*> g_known[kListedDevices];  // entries of g_devices that are gfx950 parts
 std::map<std::pair<int, hipStream_t>, HqWorkspace> g_workspaces;
+std::map<std::pair<int, hipStream_t>, std::pair<unsigned long long*, size_t>> g_slots;  // of hq_exchange_slots, and how many
+constexpr size_t kMostSlots = (size_t)4 << 20;  // 32 MB
 std::vector<std::pair<int, void*>> g_retired;  // outgrown buffers, freed by hq_shutdown()
 }  // namespace
 
@@ -124,6 +126,31 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
   return HQ_OK;
 }
 
+unsigned long long* hq_exchange_slots(hipStream_t stream, size_t n) {
+  int dev = 0;
+  if (n > kMostSlots || hipGetDevice(&dev) != hipSuccess) return nullptr;
+  std::lock_guard<std::mutex> lk(g_mu);
+  auto& s = g_slots[std::make_pair(dev, stream)];
+  if (s.second >= n) return s.first;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
+  size_t room = s.second ? s.second * 2 : (size_t)1 << 17;
+  while (room < n) room *= 2;
+  unsigned long long* p = nullptr;
+  if (hipMalloc((void**)&p, room * sizeof(*p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (hipMemsetAsync(p, 0, room * sizeof(*p), stream) != hipSuccess) {  // in front of every call that can use them
+    (void)hipGetLastError();
+    g_retired.push_back(std::make_pair(dev, (void*)p));
+    return nullptr;
+  }
+  if (s.first) g_retired.push_back(std::make_pair(dev, (void*)s.first));
+  s = std::make_pair(p, room);
+  return p;
+}
+
 bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
@@ -191,6 +218,11 @@ extern "C" int hq_reserve_workspace(void* stream, int max_K, int max_N) {
   if (rc != HQ_OK) return rc;
   size_t floats = 0, counters = 0;
   reserve_bound(d->cus, max_K, max_N, &floats, &counters);
+  // and the slots in which the shares of K meet: a column's, per tile, row and share but one (at most 8192 rows of partial sums for
+  // batches, two workgroups per compute unit where tiles are narrow).  Calls go on without where there are none.
+  const size_t tiles = ((size_t)max_N + 63) / 64;
+  const size_t rows = tiles * (kHqMeetMost - 1) > 8192 ? tiles * (kHqMeetMost - 1) : 8192;
+  (void)hq_exchange_slots((hipStream_t)stream, (rows > 2 * (size_t)d->cus ? rows : 2 * (size_t)d->cus) * 64);
   HqWorkspace ws;
   return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, true);
 }
@@ -212,6 +244,8 @@ extern "C" int hq_shutdown(void) {
     release(kv.first.first, kv.second.partial);
     release(kv.first.first, kv.second.counters);
   }
+  for (auto& kv : g_slots) release(kv.first.first, kv.second.first);
+  g_slots.clear();
   for (auto& r : g_retired) release(r.first, r.second);
   g_workspaces.clear();
   g_retired.clear();

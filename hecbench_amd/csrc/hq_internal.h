@@ -114,6 +114,10 @@ struct HqDevice {
 // Device facts for the current device (cached per ordinal).  Returns an hq code.
 int hq_current_device(const HqDevice** out);
 
+// The sums of a divided K that meet by exchange (hq_meet): `n` slots, zero between calls, of (current device, stream).  Null where
+// there are not as many and none can be had (under capture): the shares then meet through a workspace and a counter.
+unsigned long long* hq_exchange_slots(hipStream_t stream, size_t n);
+
 struct HqWorkspace {
   float* partial;      // split-K partial sums
   unsigned* counters;  // arrival counters, zero between calls (self-resetting)
@@ -223,12 +227,21 @@ struct HqMin {
 __device__ __forceinline__ float hq_wave_sum(float v) { return hq_wave(v, HqAdd()); }
 __device__ __forceinline__ float hq_wave_max(float v) { return hq_wave(v, HqMax()); }
 
-// Sum of the nsplit partial sums p[s * stride] of a K split, added in split order (the result does not depend
-// on which workgroup arrived last).  The loads are device-scope atomic loads, which bypass the non-coherent
+// Sum of the nsplit partial sums p[s * stride] of a K split, added in split order, up to eight in hq_meet's tree (the result does
+// not depend on which workgroup arrived last, nor on which way the sums met).  The loads are device-scope atomic loads, which bypass the non-coherent
 // cache levels; eight of them are in flight at a time - one after the other each costs a trip to memory, and
 // the last workgroup of a tile is the last thing a kernel does.
 __device__ __forceinline__ float hq_sum_partials(const float* p, size_t stride, int nsplit) {
   float sum = 0.f;
+  if (nsplit <= 8) {  // in the tree of hq_meet
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      v[j] = __hip_atomic_load(p + (size_t)min(j, nsplit - 1) * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int j = 2; j < 8; ++j) v[j] = j < nsplit ? v[j] : 0.f;
+    return 0.f + (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
+  }
   for (int s0 = 0; s0 < nsplit; s0 += 8) {
     float v[8];
 #pragma unroll
@@ -241,6 +254,30 @@ __device__ __forceinline__ float hq_sum_partials(const float* p, size_t stride, 
   }
   return sum;
 }
+
+// A few shares of K meet without a count: two and two in a slot of their column, {1, a sum} in one 64-bit exchange at the memory
+// side.  Whoever finds the slot empty is done; whoever finds the other's sum goes on with both, to the next pair, and the one that
+// goes through all holds the total.  Where the shares arrive together that is one trip to memory for two of them and two for four,
+// in place of three (the partial sums' acknowledgement, the count, and the sums back).  Nobody waits for anybody, and the sums are
+// added in the same tree whoever comes first: (0 + 1) + (2 + 3).  A slot is empty again when its second visitor has gone.
+// slots: this column's, `stride` apart, nsplit - 1 of them.  True in the lanes that hold the total.
+__device__ __forceinline__ bool hq_meet(unsigned long long* slots, size_t stride, int share, int nsplit, float& v) {
+  for (int n = nsplit, first = 0; n > 1; first += n >> 1, n = (n + 1) >> 1, share >>= 1) {
+    if ((share ^ 1) >= n) continue;  // the last of an odd number goes on by itself
+    unsigned long long* slot = slots + (size_t)(first + (share >> 1)) * stride;
+    const unsigned long long other =
+        __hip_atomic_exchange(slot, 1ull << 32 | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!(other >> 32)) return false;
+    v += __uint_as_float((uint32_t)other);
+    __hip_atomic_store(slot, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  return true;
+}
+// Up to eight shares, three trips at most.  3-bit matvec, count / exchange, us: two shares 8192 x 640 5.1 / 4.2, 8192 x 28672 18.1 / 17.2;
+// three 11008 x 4096 6.45 / 6.2; five 20480 x 4096 9.55 / 8.85; eight 32768 x 2048 7.7 / 7.4; ten 39136 x 364 7.0 / 7.3 (four trips: not
+// taken).  Four rows, two shares, 4224 x 2200 6.9 / 6.05.  LUT-GEMM: two shares 8192 x 8192 8.15 / 7.35, three 11008 x 4096 7.8 / 7.1,
+// six 6016 x 2265 (two planes) 5.8 / 5.0, eight 7552 x 2166 (groups of 64) 6.9 / 6.2.
+constexpr int kHqMeetMost = 8;
 
 // Packed rows that start at any multiple of four or one column (N not a multiple of 32 words): the 128-byte lines at the edges of
 // a column tile belong to its neighbour too.

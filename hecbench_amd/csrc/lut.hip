@@ -567,11 +567,15 @@ __global__ __launch_bounds__(WAVES * 64) void bcq_planes_kernel(HQ_ARGS24) {
       v += poison_w[w];
     }
     // operand units 2^-10, and the sums hold half of sum s*x
-    if (a.nsplit == 1) a.y[n] = (_Float16)(v * 2048.f);
-    else __hip_atomic_store(&a.partial[((size_t)tile * a.nsplit + blockIdx.y) * 64 + tid], v, __ATOMIC_RELAXED,
+    if (a.nsplit == 1) {
+      a.y[n] = (_Float16)(v * 2048.f);
+    } else if (!a.counters) {  // a few shares: partial holds exchange slots
+      if (hq_meet(reinterpret_cast<unsigned long long*>(a.partial) + (size_t)tile * (a.nsplit - 1) * 64 + tid, 64, blockIdx.y, a.nsplit, v))
+        a.y[n] = (_Float16)(v * 2048.f);
+    } else __hip_atomic_store(&a.partial[((size_t)tile * a.nsplit + blockIdx.y) * 64 + tid], v, __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (a.nsplit > 1) {
+  if (a.nsplit > 1 && a.counters) {
     // Arrival counting as in the table kernel above and in q3.hip: write-through partial sums, every wave waits
     // for their acknowledgement, a barrier, one device-scope fetch-add per workgroup, and the last workgroup
     // to arrive adds the partial sums in split order with loads that bypass the non-coherent cache levels.
@@ -611,7 +615,12 @@ int launch_bcq_planes(LutArgs a, bool ragged, int nsplit, hipStream_t stream) {
   a.kslice = rpw * WAVES * QUADS * 128;
   a.nsplit = nsplit;
   a.strict = hq_tune(HQ_TUNE_SPLITK_FENCES, 0);
-  if (nsplit > 1) {
+  unsigned long long* slots = nullptr;
+  if (nsplit > 1 && nsplit <= kHqMeetMost && !a.strict) slots = hq_exchange_slots(stream, (size_t)ntiles * (nsplit - 1) * 64);
+  if (slots) {
+    a.partial = reinterpret_cast<float*>(slots);
+    a.counters = nullptr;
+  } else if (nsplit > 1) {
     HqWorkspace ws;
     const int rc = hq_get_workspace(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles, &ws);
     if (rc != HQ_OK) return rc;

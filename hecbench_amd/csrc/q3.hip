@@ -28,8 +28,8 @@
 // stages its own activation digits in LDS without a workgroup barrier, and meets
 // the other waves only in the final reduction.  When one workgroup covers all of
 // K no cross-workgroup reduction is needed; otherwise (split-K) the partial sums
-// go to a workspace and the last workgroup to arrive at a tile adds them in a
-// fixed order, so results do not depend on arrival order.
+// meet by exchange (up to eight shares), or go to a workspace and the last workgroup to arrive
+// at a tile adds them; in a fixed order, so results do not depend on arrival order.
 #include "hq_internal.h"
 #include "q3_recipe.h"
 
@@ -400,6 +400,9 @@ __global__ __launch_bounds__(WAVES * 64) void q3_matvec_kernel(HQ_ARGS24) {
       // Write-through store: the result is on its way to memory at once instead of waiting in this
       // XCD's L2 for the write-back at the end of the kernel (the last store of a kernel is exposed).
       __hip_atomic_store(&a.y[n], y_old + val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (!a.counters) {  // a few shares: partial holds exchange slots
+      if (hq_meet(reinterpret_cast<unsigned long long*>(a.partial) + (size_t)tile * (a.nsplit - 1) * 64 + tid, 64, split, a.nsplit, val))
+        __hip_atomic_store(&a.y[n], ((a.flags & HQ_FLAG_ACCUMULATE) ? a.y[n] : 0.f) + val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
       // Device-coherent (write-through) store: visible to the other XCDs' workgroups
       // without flushing or invalidating this XCD's L2.
@@ -407,7 +410,7 @@ __global__ __launch_bounds__(WAVES * 64) void q3_matvec_kernel(HQ_ARGS24) {
                          __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  if (a.nsplit > 1) {
+  if (a.nsplit > 1 && a.counters) {
     // Arrival counting.  Default protocol, relaxed device-scope atomics only:
     //  (1) the partial sums above are device-scope atomic stores, i.e. write-through stores that are
     //      acknowledged only once they are visible to every XCD;
@@ -658,6 +661,13 @@ int q3_split_acquire(const Q3SplitPlan& p, const HqQ3Scratch* fixed, hipStream_t
     out->partial = fixed->partial;
     out->counters = fixed->counters;
     return HQ_OK;
+  }
+  if (p.nsplit <= kHqMeetMost && !hq_tune(HQ_TUNE_SPLITK_FENCES, 0)) {
+    // (floats: a row of 64 per tile, share and row of results)
+    if (unsigned long long* slots = hq_exchange_slots(stream, p.floats / p.nsplit * (p.nsplit - 1))) {
+      out->partial = reinterpret_cast<float*>(slots);
+      return HQ_OK;
+    }
   }
   HqWorkspace ws;
   const int rc = hq_get_workspace(stream, p.floats, (size_t)p.ntiles, &ws);

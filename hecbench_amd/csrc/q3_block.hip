@@ -28,7 +28,7 @@
 // Everything else follows q3.hip: a workgroup owns a 64-column tile and one round of K (8 waves x 4 steps x
 // 4 k-groups = 4096 elements), a wave's 16-lane quarter streams one k-group per step as three 128-bit loads,
 // every wave stages its own operand behind a wave-local fence, the waves meet once at the end, and K beyond
-// one round is split across workgroups whose partial sums the last one to arrive adds up in split order.
+// one round is split across workgroups whose partial sums meet as in q3.hip.
 // The weights are read once for all rows at nine VALU instructions per 32 weights and pass, in one launch,
 // where the 64-row kernel (q3_gemm.hip) needs a pre-pass and twenty per 32 weights, and the one-launch kernel
 // (q3_direct.hip) takes its time for 32 rows whatever their number.  No counterpart in the reference (its kernels are batch 1: src/quant3MatMul-hip/kernels.h:12-217).
@@ -318,13 +318,18 @@ __device__ __forceinline__ void q3_block_body(const BlockArgs& a, const int tile
         float* yp = &a.y[(size_t)m * a.N + ncol];
         const float y_old = (a.flags & HQ_FLAG_ACCUMULATE) ? *yp : 0.f;
         __hip_atomic_store(yp, y_old + val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      } else if (!a.counters) {  // a few shares: partial holds exchange slots (hq_meet)
+        float* yp = &a.y[(size_t)m * a.N + ncol];
+        if (hq_meet(reinterpret_cast<unsigned long long*>(a.partial) + ((size_t)vtile * (a.nsplit - 1) * a.prow + m) * 64 + col,
+                    (size_t)a.prow * 64, split, a.nsplit, val))
+          __hip_atomic_store(yp, ((a.flags & HQ_FLAG_ACCUMULATE) ? *yp : 0.f) + val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       } else {
         __hip_atomic_store(&a.partial[(((size_t)vtile * a.nsplit + split) * a.prow + m) * 64 + col], val, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   }
-  if (a.nsplit > 1) {
+  if (a.nsplit > 1 && a.counters) {
     // Arrival counting as in q3.hip: write-through partial sums, every wave waits for their acknowledgement,
     // a barrier, one device-scope fetch-add per workgroup, and the last workgroup to arrive adds the partial
     // sums in split order with loads that bypass the non-coherent cache levels.

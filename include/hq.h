@@ -18,7 +18,7 @@
  *   - a NaN or an infinity among the activations makes the affected outputs non-finite (the
  *     fixed-point matrix-core paths give NaN where the reference arithmetic would give +-Inf);
  *   - the library keeps one workspace per (device, stream) pair (split-K
- *     partial sums, arrival counters, re-ordered GEMM activations), allocated by
+ *     partial sums, arrival counters, exchange slots, re-ordered GEMM activations), allocated by
  *     hq_init() / hq_reserve_workspace() or by the first call that needs more than
  *     is there (that call then runs hipMalloc, which fails under stream capture:
  *     reserve first).  A workspace grows geometrically (a reservation to what it names), lives until hq_shutdown()
@@ -75,11 +75,12 @@ int hq_init(void);
  * batched GEMMs up to max_K input features, so that later calls on that stream never allocate
  * (needed before stream capture).  It allocates what hq_reserve_need tells: room for batches of any size, thousands of
  * re-ordered rows and the shares of divided tiles among them - on 256 compute units 8 MiB for max_K = 512, 16 MiB for
- * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152.  A stream that only ever sees smaller calls takes less without a
+ * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152 - and 4 MiB and more (3.5 KiB per 64 columns) in which the sums of a K
+ * divided among a few workgroups meet.  A stream that only ever sees smaller calls takes less without a
  * reservation: a workspace grows with the calls (hq_q3_workspace_need; batch 1 at most a few MiB, up to 64 rows 16 MiB).
  * A captured call keeps the workspace of the stream it was captured on, whatever stream its graph is replayed on: replays must not
  * overlap with each other or with calls on that stream where both use it.  Calls that overlap in one workspace give wrong results,
- * and they may leave its arrival counters, which the kernels expect at zero and return to zero, at other values; hq_shutdown()
+ * and they may leave its arrival counters and slots, which the kernels expect at zero and return to zero, at other values; hq_shutdown()
  * and calls (and captures) anew start from fresh ones.
  * No counterpart in the reference. */
 int hq_reserve_workspace(void* stream, int max_K, int max_N);
