@@ -644,13 +644,22 @@ int launch_bcq_planes(LutArgs a, bool ragged, int nsplit, hipStream_t stream) {
 
 // Split of K over workgroups.  Ordinary: rounds of QUADS quads (128 elements of K) per wave, and as many workgroups as there
 // are compute units to take them (K=11008, N=4096, three planes: 64 tiles x 3 rounds).  Fine: one quad per wave, one round per
-// workgroup, all rounds side by side.  From measurements of both over thirty shapes (MI355X): a quad takes a wave 0.11 us per
-// plane (0.23 with groups of 64 or 32), the exchange of a split 1.4 us and 0.16 more for every part.  Fine splits are taken
-// where they save more than they cost and all workgroups are on the device at once, two per compute unit (us, ordinary / fine:
-// 4224 x 5562 four planes 9.1 / 7.9; 4352 x 622 two planes 5.9 / 4.9; 7552 x 2166 group 64 8.5 / 7.3; 1024 x 1024 group 32 5.8 /
-// 4.6; not 11008 x 4096 7.9 / 8.7, 13184 x 1025 7.2 / 7.7, 4096 x 4096 5.7 / 6.1), and where several rounds of few more tiles than
-// compute units would leave most of those idle behind the first tile (2432 x 20485 four planes group 32 18.7 / 13.7; 5120 x 20480
-// 14.2 / 13.0; not 4096 x 28672 four planes 15.6 / 16.6).
+// workgroup, all rounds side by side.  Groups of 128 and more, from 180 drawn problems timed both ways (MI355X; the choice costs 0.6 %
+// on average against the better one, 10 % at most): a quad takes a wave 0.11 us per plane, the exchange of a split 0.3 us and 0.1 more
+// for every part, workgroups beyond one per compute unit 0.9, and more than eight parts, which meet through a count, 1.0.  Fine
+// splits are taken where they save more than they cost and all workgroups are on the device at once, two per compute unit (us,
+// ordinary / fine: 3072 x 1776 three planes 5.35 / 4.45; 3968 x 1911 5.3 / 4.6; 4352 x 622 two planes 5.9 / 4.9; not 3200 x 6705
+// 5.5 / 6.0, 13184 x 1025 7.2 / 7.7), and where several rounds of few more tiles than compute units would leave most of those idle
+// behind the first tile (5120 x 20480 14.2 / 13.0; not 4096 x 28672 four planes 15.6 / 16.6).
+// Groups of 64 and 32 take twice the arithmetic, and an even share of it counts more: both ways are estimated (grouped_us; 140
+// problems, spread 5 and 8 %, the choice costs 1.3 % on average): 2432 x 25507 four planes 17.6 / 12.3; 4736 x 23517 two planes 17.2 /
+// 13.1; 5760 x 9363 four planes 16.2 / 12.2; 7552 x 10028 18.2 / 14.1; not 8448 x 7872 three planes 10.25 / 11.7, 15872 x 22799 40.7 / 42.4.
+// quads: a wave's in a row, in the average over the compute units where they are even.
+inline float grouped_us(bool fine, float quads, int NB, float stream_us, int parts) {
+  if (!fine) return 3.1f + 0.276f * quads * NB + 0.54f * stream_us + (parts > 1 ? 0.72f : 0.f);
+  const int trips = parts > 8 ? 0 : (parts > 4 ? 3 : (parts > 2 ? 2 : (parts > 1 ? 1 : 0)));
+  return 2.9f + 0.2f * quads * NB + 0.68f * stream_us + 0.56f * trips + (parts > 8 ? 2.7f : 0.f);
+}
 template <int NB, bool GROUPED>
 int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t stream) {
   constexpr int QUADS = NB <= 3 ? 4 : (NB <= 6 ? 2 : 1);  // bounded by the register budget
@@ -662,8 +671,9 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
   const int rpw = (rounds + nsplit - 1) / nsplit;
   bool fine = false, apart = false;
   if (QUADS > 1) {
-    const float saves = (GROUPED ? 0.23f : 0.11f) * NB * (rpw * QUADS - 1);
-    const float costs = parts == 1 ? 0.f : (nsplit == 1 ? 1.4f : 0.f) + 0.16f * (parts - nsplit);
+    const float saves = 0.11f * NB * (rpw * QUADS - 1);
+    const float costs = parts == 1 ? 0.f : (nsplit == 1 ? 0.3f : 0.f) + 0.1f * (parts - nsplit) +
+                                               (ntiles * (int64_t)parts > cus ? 0.9f : 0.f) + (parts > 8 ? 1.f : 0.f);
     fine = (int64_t)ntiles * parts <= 2 * cus && saves > costs;
     if (ntiles > cus && ntiles * 8 <= cus * 11 && rpw > 1 && parts <= 5) fine = true;
     // Several rounds per workgroup, and the exchange paid for anyway (nsplit > 1) or a last wave of tiles that would leave more
@@ -671,14 +681,23 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
     // 34 quads, 12.2 / 13.1): every round is a workgroup of its own, which has half the registers, so that two share
     // a compute unit and the work is even whatever the tiles (us, walked / apart: 10880 x 17510 three planes 29.0 / 22.8; 14208 x 16512
     // 28.5 / 21.5; 8448 x 7943 two planes 9.3 / 7.9; 10624 x 25368 group 64 37.8 / 33.2; not 4864 x 26591 one plane, 416 tiles, 7.6 / 9.2;
-    // not 4224 x 12997, 204 tiles, 8.7 / 9.8), with three or more planes in small groups one quad per wave (three planes, walked / apart /
-    // fine: 6656 x 18823 group 32 30.9 / 25.0 / 22.3 in the plain order of tiles, apart 20.8 and fine 18.1 in hq_column_tile's; 13568 x
-    // 4444 group 64 14.3 / 13.5 / 12.1, and 12.3, 11.1).
+    // not 4224 x 12997, 204 tiles, 8.7 / 9.8).
     const int waves_of_tiles = (ntiles + cus - 1) / cus;
     const bool full_end = 2 * nquads >= (2 * rounds - 1) * 8 * QUADS;
-    apart = !fine && rpw > 1 &&
+    apart = (GROUPED || !fine) && rpw > 1 &&
             (nsplit > 1 || (ntiles > cus && (int64_t)ntiles * 32 <= (int64_t)waves_of_tiles * cus * (full_end ? 25 : 20)));
-    fine = fine || (apart && GROUPED && NB >= 3);
+    if (GROUPED) {
+      const float planes = (float)a.K * (float)a.N * NB / 8.f;
+      const float stream_us = planes * (1.f + 16.f / a.G * (1.f + 1.f / NB)) / 6e6f;
+      const float even = (float)ntiles / cus;
+      const int quads1 = (nquads + 7) / 8;  // of a wave, in one round of all
+      float ordinary;
+      if (apart) ordinary = (even * rounds > 1.f ? even * rounds : 1.f) * (QUADS < nquads / 8.f ? QUADS : nquads / 8.f);
+      else if (rounds > 1) ordinary = (float)((ntiles * nsplit + cus - 1) / cus) * rpw * QUADS;
+      else ordinary = (float)waves_of_tiles * (QUADS < quads1 ? QUADS : quads1);
+      fine = grouped_us(true, even * parts > 1.f ? even * parts : 1.f, NB, stream_us, parts) <
+             grouped_us(false, ordinary, NB, stream_us, apart ? rounds : nsplit);
+    }
     fine = hq_tune(HQ_TUNE_LUT_FINE, fine) != 0;
   }
   if (fine) nsplit = parts;

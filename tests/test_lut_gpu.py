@@ -63,6 +63,17 @@ def test_k_split_of_the_plane_kernel(hq, oracle, tunable, K, N, nb):
     assert np.array_equal(y, _run(hq, bW, alpha, qbias, x, 128))
 
 
+@pytest.mark.parametrize("K,N,nb,group", [(1792, 5350, 4, 32), (2432, 6500, 3, 64), (1408, 19519, 3, 32), (3072, 1777, 3, 128), (9216, 700, 2, 64),
+                                          (1152, 130, 6, 32)])
+def test_split_by_estimate(hq, oracle, K, N, nb, group):
+    """The library's own choice where a quad per wave has become the faster one, on one and on several workgroups per compute unit,
+    and in more parts than meet by exchange."""
+    bW, alpha, qbias, x = oa.make_lut_problem(K + 3 * N + nb, K, N, nb, group, False)
+    y = _run(hq, bW, alpha, qbias, x, group)
+    assert rel_err(y, oracle.lut_gemv_f64(bW, alpha, qbias, x, group), FLOOR_F16) <= 2e-3
+    assert np.array_equal(y, _run(hq, bW, alpha, qbias, x, group))
+
+
 @pytest.mark.parametrize("split", [1, 2])
 @pytest.mark.parametrize("K,N,nb,group", [(128, 64, 1, 32), (1024, 100, 3, 64), (1152, 130, 3, 32), (2304, 200, 4, 64),
                                           (3200, 64, 6, 32), (4224, 321, 2, 128), (8192, 65, 5, 64), (1280, 192, 8, 64)])
