@@ -5,8 +5,8 @@
 //
 // The reference benchmark has only the batch-1 matvec
 // (src/quant3MatMul-hip/kernels.h in the HeCBench tree); this is the same
-// arithmetic applied to up to 64 activation rows per pass on the matrix cores.  It serves 33 to 64 rows of 9e7 weights and more, and
-// stands in where a captured call finds room for 64 rows' activations only; fewer rows and smaller matrices go through
+// arithmetic applied to up to 64 activation rows per pass on the matrix cores.  It serves 33 to 64 rows of 9e7 weights and more that
+// leave it column tiles for half the compute units or have a K of 16384, and stands in where a captured call finds room for 64 rows' activations only; fewer rows and smaller matrices go through
 // q3_direct.hip, more rows through q3_prefill.hip, whose pre-pass is the one here.
 //
 // As in the matvec, the packed codes are never converted: an AND turns a 32-bit
@@ -444,7 +444,11 @@ int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv
 namespace {
 // Which batches take the one-launch kernel (q3_direct.hip).  Up to 32 rows every one; up to 64, which are two of its row tiles, as
 // long as reading the weights twice costs less than the pre-pass (9e7 weights: 63 rows, K=5984, N=13008 23.1 -> 19.8 us, but 57
-// rows, K=4896, N=21956 25.5 -> 30.0); beyond, by the two estimates (over 270 timed problems of 97 and more rows the choice
+// rows, K=4896, N=21956 25.5 -> 30.0), and, where the 64-row kernel has too few column tiles and cuts K, than its shares as well
+// (64 rows, K=6016, N=16380 23.4 -> 19.9; 37, K=12032, N=8176 24.8 -> 21.9; 58, K=13824, N=11568 36.1 -> 34.3; 45, K=12864, N=8612 30.3 ->
+// 26.2).  A K of 16384 and more stays with that kernel: 2.5e8 weights and more are as fast there (64 rows, K=32768, N=8192 45.7 / 46.4,
+// K=49152, N=12288 94.7 / 106; 40, K=16384, N=8192 28.4 / 28.0), few columns are not (48, K=24576, N=4096 28.8 / 24.7).  Beyond 64 rows by the
+// two estimates (over 270 timed problems of 97 and more rows the choice
 // costs 0.3 % on average against the better of the two, 15 % at most).  65 to 96 rows of a narrow matrix (N <= 4096) always, where
 // the 64-row kernel reads the weights twice: 78 rows, K=6880, N=584 19.5 -> 8.6.
 // The plan is made only where it is looked at: by the estimates, or by the launch of a batch that the kernel serves.
@@ -452,7 +456,8 @@ bool direct_serves(int cus, int K, int N, int M, HqQ3DirectPlan* plan) {
   if (!hq_q3_direct_can(K, N)) return false;
   const bool forced = hq_q3_direct_forced();
   if (!forced && hq_tune(HQ_TUNE_Q3_TILES, -1) >= 0) return false;  // tests: the other kernels
-  if (!forced && M > 32 && M <= 64 && (int64_t)K * N >= 90000000) return false;
+  const bool cut = 2 * ((N + kTileN - 1) / kTileN) <= cus && K < 16384;  // the 64-row kernel would cut K
+  if (!forced && M > 32 && M <= 64 && (int64_t)K * N >= (cut ? 250000000 : 90000000)) return false;
   *plan = hq_q3_direct_plan(cus, K, N, M, false);
   return forced || M <= 64 || !hq_q3_tiles_serve(N, M) || plan->us < hq_q3_tiles_us(cus, K, N, M);
 }

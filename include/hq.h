@@ -156,10 +156,10 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  *     large matrices (3.5e7 weights, 7 and 8 rows 4e7, while four rows would have a compute unit for every workgroup; 7e7 at any
  *     size) as two passes or row blocks, unless N / 128 is at least 7/8 of the compute units.  Every activation enters with an
  *     error of at most 2^-19 of the largest magnitude among its 32 neighbours (exactly, if within 2^8 of it);
- *   - the matrix cores in one launch: all other batches of up to 32 rows, 33 to 64 rows of less than 9e7 weights, 65 to 96 rows
- *     where N <= 4096, and more rows as long as the estimated time is below the tiles' (hundreds of rows of small matrices).  A
- *     tile's K may be divided among up to eight workgroups.  Activations enter as they are;
- *   - 33 to 64 rows of 9e7 weights and more: the matrix cores behind a pre-pass that re-orders the activations;
+ *   - the matrix cores in one launch: all other batches of up to 32 rows, 33 to 64 rows of less than 9e7 weights (2.5e8, if K <
+ *     16384 and 128-column tiles are too few for half the compute units), 65 to 96 rows where N <= 4096, and more rows as long as
+ *     the estimated time is below the tiles' (hundreds of rows of small matrices).  A tile's K may be divided among up to eight workgroups.  Activations enter as they are;
+ *   - 33 to 64 rows of larger matrices: the matrix cores behind a pre-pass that re-orders the activations;
  *   - the rest: tiles of 64 or 128 rows behind such a pre-pass, up to thousands of rows per pass over the weights.
  * The pre-pass scales every activation row by a power of two, so accuracy does not depend on the magnitude of the activations:
  * entries within 2^21 of their row's largest magnitude enter the matrix cores exactly, smaller ones lose low bits (those 2^32 below

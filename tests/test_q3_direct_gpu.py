@@ -105,6 +105,11 @@ def test_default_plans(hq, oracle, M, K, N):
     assert torch.equal(got[1, True], got[0, True] + 3.0)
 
 
+@pytest.mark.parametrize("M,K,N", [(33, 11008, 8192), (64, 6016, 16380), (64, 16352, 5632)])
+def test_default_plans_where_the_other_kernel_would_cut_k(hq, oracle, M, K, N):
+    test_default_plans(hq, oracle, M, K, N)
+
+
 @pytest.mark.parametrize("M,K,N,kernel", [(39, 4160, 1176, "direct"), (39, 4160, 1176, "rows64"), (6, 11008, 4096, "block"),
                                           (8, 8192, 8192, "block")])
 def test_capture_without_any_workspace(hq, oracle, tunable, M, K, N, kernel):
