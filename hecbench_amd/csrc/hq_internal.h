@@ -154,7 +154,8 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
 int hq_q3_gemm_prep_launch(const void* A, void* Ap, float* rowsum, float* rowinv, int M, int K, int Mpad, int Gpad,
                            unsigned* counters, size_t ncounters, hipStream_t stream);
 bool hq_q3_tiles_serve(int N, int M);
-int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters);
+// (cut_off: and the columns that the tiles leave to the one-launch kernel, which does without where there is no room)
+int hq_q3_tiles_need(int cus, int K, int N, int M, bool cut_off, size_t* floats, size_t* counters);
 void hq_q3_tiles_bound(int cus, int max_K, size_t* floats, size_t* counters);
 int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scales, const float* zeros, float* y, int K, int N,
                        int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
@@ -170,8 +171,9 @@ struct HqQ3DirectPlan {
 bool hq_q3_direct_can(int K, int N);  // whether the kernel can take the matrix at all
 bool hq_q3_direct_forced();           // a test's override
 HqQ3DirectPlan hq_q3_direct_plan(int cus, int K, int N, int M, bool undivided);
+// Columns col0 (a multiple of 256) to N; the plan is one of N - col0 columns.
 int hq_q3_direct_launch(HqQ3DirectPlan plan, int cus, const void* x, const int32_t* qweight, const float* scales, const float* zeros,
-                        float* y, int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
+                        float* y, int K, int N, int M, int col0, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed);
 // The kernel of a batch where scratch is no question (so that a test can say what it runs).
 enum HqQ3Kernel { HQ_Q3_KERNEL_BLOCK, HQ_Q3_KERNEL_DIRECT, HQ_Q3_KERNEL_ROWS64, HQ_Q3_KERNEL_TILES };
 int hq_q3_batch_kernel(int cus, int K, int N, int M);

@@ -829,7 +829,7 @@ int hq_q3_matvec_impl(const void* x, int x_dtype, const int32_t* qweight, const 
       };
       if (!b.split.too_large && (q3_block_yields(dev->cus, K, N, batch_M) || no_room()))
         return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, batch_M, false), dev->cus, x, qweight, scales, zeros, y, K, N,
-                                   batch_M, flags, stream, fixed);
+                                   batch_M, 0, flags, stream, fixed);
       rc = q3_split_acquire(b.split, fixed, stream, &sp);
       if (rc != HQ_OK) return rc;
       return hq_q3_block_launch(x, qweight, scales, zeros, y, K, N, batch_M, b.nsplit, b.rpw, b.mblocks, sp.partial,

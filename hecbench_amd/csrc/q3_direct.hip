@@ -75,6 +75,7 @@ struct DirectArgs {
   float* partial;      // [tile][nshare][kTileM * kTileN]
   unsigned* counters;  // [tile], zero between calls
   int M, N, K, nmt, T, nshare, L, nwg;  // row tiles; steps of K, shares of L steps each; workgroups
+  int ct0;             // column tiles in front of the first
   unsigned flags;
 };
 
@@ -83,8 +84,8 @@ __global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
   // the first 14 dwords of the arguments (all that the loads need) arrive preloaded in scalar registers
   HqReader r(HQ_PASS24);
   DirectArgs a;
-  a.w = r; a.x = r; a.M = r; a.N = r; a.K = r; a.nmt = r; a.T = r; a.nshare = r; a.L = r; a.nwg = r; a.scales = r; a.zeros = r;
-  a.out = r; a.partial = r; a.counters = r; a.flags = r;
+  a.w = r; a.x = r; a.M = r; a.N = r; a.K = r; a.nmt = r; a.T = r; a.nshare = r; a.L = r; a.nwg = r; a.ct0 = r; a.flags = r; a.scales = r; a.zeros = r;
+  a.out = r; a.partial = r; a.counters = r;
   using S = Form<CB, KS>;
   typedef uint32_t wv_t __attribute__((ext_vector_type(CB)));
   extern __shared__ unsigned char lds[];
@@ -97,7 +98,8 @@ __global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
   const int xcd = blockIdx.x & 7;
   const int v = xcd * (a.nwg >> 3) + min(xcd, a.nwg & 7) + (int)(blockIdx.x >> 3);
   const int tile = v / a.nshare, share = v - tile * a.nshare;
-  const int ct = __builtin_amdgcn_readfirstlane(tile / a.nmt), mt = __builtin_amdgcn_readfirstlane(tile - ct * a.nmt);
+  const int ct_here = __builtin_amdgcn_readfirstlane(tile / a.nmt), mt = __builtin_amdgcn_readfirstlane(tile - ct_here * a.nmt);
+  const int ct = a.ct0 + ct_here;
   const int t0 = share * a.L, len = min(a.L, a.T - t0);
 
   // ---- loader ----
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(64 * KS, 2) void q3_direct_kernel(HQ_ARGS24) {
     for (int i = 0; i < 2 * KS; ++i) t += sums[i * S::kTileM + tid];
     total[tid] = t;
   }
-  asm volatile("" ::"s"(a.flags));  // the last arguments are here with the others, not behind the first LDS reads' wait
+  asm volatile("" ::"s"(a.counters));  // the last arguments are here with the others, not behind the first LDS reads' wait
   __syncthreads();
   const int nc = min(first_col, a.N - V);
   const fv_t sc = *reinterpret_cast<const fv_t*>(a.scales + nc), zr = *reinterpret_cast<const fv_t*>(a.zeros + nc);
@@ -403,7 +405,7 @@ int launch(const DirectArgs& a, hipStream_t stream) {
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, S::kSmem);
   if (attr != hipSuccess) return (int)attr;
   return hq_launch(q3_direct_kernel<CB, KS>, dim3(a.nwg), dim3(S::kThreads), S::kSmem, stream, a.w, a.x, a.M, a.N, a.K, a.nmt, a.T,
-                   a.nshare, a.L, a.nwg, a.scales, a.zeros, a.out, a.partial, a.counters, a.flags);
+                   a.nshare, a.L, a.nwg, a.ct0, a.flags, a.scales, a.zeros, a.out, a.partial, a.counters);
 }
 
 }  // namespace
@@ -433,11 +435,11 @@ HqQ3DirectPlan hq_q3_direct_plan(int cus, int K, int N, int M, bool undivided) {
 }
 
 int hq_q3_direct_launch(HqQ3DirectPlan p, int cus, const void* x, const int32_t* qweight, const float* scales, const float* zeros,
-                        float* y, int K, int N, int M, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
+                        float* y, int K, int N, int M, int col0, unsigned flags, hipStream_t stream, const HqQ3Scratch* fixed) {
   // without room for the shares' sums no tile is divided
   if (p.nshare > 1 && (fixed ? p.partial_floats > fixed->tiles_floats || p.counters > fixed->ncounters
                              : hq_workspace_out_of_reach(stream, p.partial_floats, p.counters)))
-    p = hq_q3_direct_plan(cus, K, N, M, true);
+    p = hq_q3_direct_plan(cus, K, N - col0, M, true);
   int rc = HQ_OK;
   DirectArgs a;
   a.partial = nullptr; a.counters = nullptr;
@@ -459,6 +461,7 @@ int hq_q3_direct_launch(HqQ3DirectPlan p, int cus, const void* x, const int32_t*
   a.x = reinterpret_cast<const _Float16*>(x);
   a.scales = scales; a.zeros = zeros; a.out = y;
   a.M = M; a.N = N; a.K = K; a.nmt = p.nmt; a.T = p.T; a.nshare = p.nshare; a.L = p.L; a.nwg = p.ntiles * p.nshare;
+  a.ct0 = col0 / p.tn;
   a.flags = flags;
   switch (p.kind) {
     case 0: return launch<2, 4>(a, stream);

@@ -472,7 +472,7 @@ int hq_q3_gemm_kernel_of(int cus, int K, int N, int M) {
 // What the kernel of the plan takes, or the one that stands in for it where that is more.
 int hq_q3_gemm_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
   if (hq_q3_tiles_serve(N, M)) {
-    hq_q3_tiles_need(cus, K, N, M, floats, counters);
+    hq_q3_tiles_need(cus, K, N, M, true, floats, counters);
   } else {
     const GemmPlan p = gemm_plan(cus, K, N);
     *floats = p.ap_halves / 2 + 2 * kRows + p.partial_floats;
@@ -495,21 +495,21 @@ int hq_q3_gemm_launch(const void* x, const int32_t* qweight, const float* scales
   if (rc != HQ_OK) return rc;
   HqQ3DirectPlan direct;
   if (!(fixed && K > kFixedMaxK) && direct_serves(dev->cus, K, N, M, &direct))  // (a longer K is refused below)
-    return hq_q3_direct_launch(direct, dev->cus, x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
+    return hq_q3_direct_launch(direct, dev->cus, x, qweight, scales, zeros, y, K, N, M, 0, flags, stream, fixed);
   bool tiles = hq_q3_tiles_serve(N, M);
   if (tiles) {
     // 64 rows at a time need less: under capture without room for all rows' activations, and where the fixed array cannot hold
     // the tiles' plan (a device of more compute units than it was sized for; K beyond its limit, which is refused below)
     size_t floats, counters;
-    hq_q3_tiles_need(dev->cus, K, N, M, &floats, &counters);
+    hq_q3_tiles_need(dev->cus, K, N, M, false, &floats, &counters);
     tiles = fixed ? K <= kFixedMaxK && floats <= fixed->tiles_floats : !hq_workspace_out_of_reach(stream, floats, counters);
   }
   if (tiles) return hq_q3_tiles_launch(x, qweight, scales, zeros, y, K, N, M, flags, stream, fixed);
   const GemmPlan plan = gemm_plan(dev->cus, K, N);
   if (!fixed && hq_workspace_out_of_reach(stream, plan.ap_halves / 2 + 2 * kRows + plan.partial_floats, plan.counters) &&
       hq_q3_direct_can(K, N))  // under capture without room for these activations: none are needed there
-    return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, M, false), dev->cus, x, qweight, scales, zeros, y, K, N, M, flags,
-                               stream, fixed);
+    return hq_q3_direct_launch(hq_q3_direct_plan(dev->cus, K, N, M, false), dev->cus, x, qweight, scales, zeros, y, K, N, M, 0,
+                               flags, stream, fixed);
   const int Gpad = plan.Gpad, nsplit = plan.nsplit, spp = plan.spp;
   const size_t ap_halves = plan.ap_halves, partial_floats = plan.partial_floats;
   _Float16* Ap;

@@ -15,7 +15,8 @@
 //     a barrier comes once per 128 or 256 elements.
 //   - Operand reads run one to three quarters of a step ahead, the LDS loads of a stage go out one by one between the
 //     matrix instructions, and unpacking fills the slots between those.
-//   - Tiles that do not fill a round of the compute units are divided along K (tile_plan).
+//   - Tiles that do not fill a round of the compute units are divided along K (tile_plan), or, where they are few, left to the
+//     one-launch kernel (cut_plan).
 // K=8192, N=28672, 1021 rows: 574 -> 363-390 us (1.22-1.32 PFLOP/s; the library's fp16 product of 8192^3 runs at 1.2 here);
 // 512 rows, K=4096, N=11008: 153 -> 52-57; 128 rows, K=8192, N=28672: 75 -> 58.
 #include <type_traits>
@@ -334,6 +335,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 // Host arithmetic of a launch (the launch, the workspace reservation and the size query share it).
 struct TilePlan {
   int tm, tn, ks, nmt, T, nwg, rounds, rest, nshare, L, Mpad;
+  int cut;  // columns from here on go through the one-launch kernel; N: none
+  HqQ3DirectPlan direct;
   float us;
   size_t ap_floats, row_floats, partial_floats, counters;
 };
@@ -360,6 +363,7 @@ float tile_us(const TileKind& kind, int T, int c) {
 TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int want_shares) {
   TilePlan p;
   const int G = K / 32;
+  p.cut = N;
   p.tm = kind.tm; p.tn = kind.tn; p.ks = kind.ks;
   p.T = (G + 2 * p.ks - 1) / (2 * p.ks);
   p.nmt = (M + p.tm - 1) / p.tm;
@@ -386,12 +390,32 @@ TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int wa
   return p;
 }
 
+// The same with the column tiles beyond the last full round left to the one-launch kernel, in a launch of its own behind this one,
+// where that is less by the two estimates; otherwise the plan as it is.  Dividing a few tiles along K costs most of a round whatever
+// their number (shares of 128 x 256 sums go out to memory and come back): 1024 rows, K=2048, 33 column tiles of 256, the 33rd
+// divided 59.3 us, as 32 x 64 tiles of the one-launch kernel 44.7.  1271 rows, K=2048, N=26476 (four rounds and 16 tiles) 159 -> 147;
+// 1902, K=1056, N=13184 89 -> 77.6; 1580, K=1504, N=25548 162 -> 150; 290, K=6272, N=14240 64.3 -> 58.4; 1595, K=1600, N=21980 (94
+// tiles) 148 -> 144.  From two fifths of a round on nothing is gained (1975, K=1632, N=10760, 176 tiles: 92.0 / 99.4), and with the
+// smallest tile never.
+TilePlan cut_plan(int cus, int K, int N, int M, const TileKind& kind, const TilePlan& whole, bool forced) {
+  const int cols = whole.rounds * whole.nwg / whole.nmt;
+  if (!forced && (5 * whole.rest > 2 * whole.nwg || kind.ks != 2)) return whole;
+  if (whole.rounds < 1 || cols < 1 || cols * kind.tn >= N || !hq_q3_direct_can(K, N)) return whole;
+  TilePlan p = tile_plan_of(cus, K, cols * kind.tn, M, kind, 0);
+  p.direct = hq_q3_direct_plan(cus, K, N - p.cut, M, false);
+  p.us += p.direct.us;
+  return forced || p.us < whole.us ? p : whole;
+}
+
 TilePlan tile_plan(int cus, int K, int N, int M) {
-  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: kind + 10 * shares (3 to 6 the one-launch kernel's, 9 none in particular)
+  const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: kind + 10 * shares (3 to 6 the one-launch kernel's, 9 none in particular; 100 + kind: cut)
+  if (force >= 100 && force < 103) return cut_plan(cus, K, N, M, kKinds[force - 100], tile_plan_of(cus, K, N, M, kKinds[force - 100], 0), true);
   if (force >= 0 && force % 10 < 3) return tile_plan_of(cus, K, N, M, kKinds[force % 10], force / 10);
   TilePlan best = tile_plan_of(cus, K, N, M, kKinds[0], 0);
+  best = cut_plan(cus, K, N, M, kKinds[0], best, false);
   for (int i = 1; i < 3; ++i) {
-    const TilePlan p = tile_plan_of(cus, K, N, M, kKinds[i], 0);
+    TilePlan p = tile_plan_of(cus, K, N, M, kKinds[i], 0);
+    p = cut_plan(cus, K, N, M, kKinds[i], p, false);
     if (p.us < best.us) best = p;
   }
   return best;
@@ -425,14 +449,18 @@ float hq_q3_tiles_us(int cus, int K, int N, int M) {
   return tile_plan(cus, K, N, M).us + 3.2f + 0.0002f * K + (float)M * (float)K * (4.f / 4.5e6f);
 }
 
-int hq_q3_tiles_need(int cus, int K, int N, int M, size_t* floats, size_t* counters) {
+int hq_q3_tiles_need(int cus, int K, int N, int M, bool cut_off, size_t* floats, size_t* counters) {
   *floats = *counters = 0;
   const int rows = rows_per_pass(K, M);
   for (int m0 = M > rows ? (M - 1) / rows * rows - rows : 0; m0 < M; m0 += rows) {  // the full pass and the last one
     const TilePlan p = tile_plan(cus, K, N, M - m0 < rows ? M - m0 : rows);
-    const size_t f = p.ap_floats + p.row_floats + p.partial_floats;
+    size_t f = p.ap_floats + p.row_floats + p.partial_floats, c = p.counters;
+    if (cut_off && p.cut < N) {  // one after the other in the same place
+      if (p.direct.partial_floats > f) f = p.direct.partial_floats;
+      if (p.direct.counters > c) c = p.direct.counters;
+    }
     if (f > *floats) *floats = f;
-    if (p.counters > *counters) *counters = p.counters;
+    if (c > *counters) *counters = c;
   }
   return HQ_OK;
 }
@@ -464,7 +492,7 @@ int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scale
   int rc = hq_current_device(&dev);
   if (rc != HQ_OK) return rc;
   size_t floats, ncounters;
-  hq_q3_tiles_need(dev->cus, K, N, M, &floats, &ncounters);
+  hq_q3_tiles_need(dev->cus, K, N, M, false, &floats, &ncounters);
   float* ap;
   unsigned* counters;
   if (fixed) {
@@ -496,6 +524,9 @@ int hq_q3_tiles_launch(const void* x, const int32_t* qweight, const float* scale
     a.nshare = p.nshare; a.L = p.L; a.flags = flags;
     rc = p.tm == 128 ? launch_tiles<4, 2>(a, p.nwg, stream)
                      : (p.tn == 256 ? launch_tiles<2, 2>(a, p.nwg, stream) : launch_tiles<2, 4>(a, p.nwg, stream));
+    if (rc == HQ_OK && p.cut < N)
+      rc = hq_q3_direct_launch(p.direct, dev->cus, reinterpret_cast<const _Float16*>(x) + (size_t)m0 * K, qweight, scales, zeros,
+                               y + (size_t)m0 * N, K, N, Mb, p.cut, flags, stream, fixed);
     if (rc != HQ_OK) return rc;
   }
   return HQ_OK;

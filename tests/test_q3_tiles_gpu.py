@@ -48,6 +48,30 @@ def test_kinds_and_shares(hq, oracle, tunable, kind, shares, M, K, N):
     _check(y.cpu().numpy(), exact)
 
 
+@pytest.mark.parametrize("M,K,N,kind", [(1024, 96, 8196, 0), (1000, 1376, 8452, 0), (97, 416, 66052, 0), (1090, 288, 7684, 0), (512, 1056, 8452, 1),
+                                        (300, 2080, 13316, 1)])
+def test_columns_beyond_the_last_round(hq, oracle, tunable, M, K, N, kind):
+    """Columns cut off for the one-launch kernel: four columns, a tile of 256 and four, 516 behind whole rounds that row tiles do
+    not divide, and on top of what is in the output.  Bounds of the tiles."""
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    codes, scales, zeros, A = oa.make_q3_problem(M + K + N, K, N, x_dtype=np.float16, batch=M)
+    mat = oracle.q3_pack(codes)
+    a, w, s, z = _t(A), _t(mat), _t(scales), _t(zeros)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    tunable("HQ_Q3_TILES", 100 + kind)
+    y = hq.q3_gemm(a, w, s, z)
+    for fn in (lib.hq_q3_matvec, lib.hq_q3_matvec_noalloc):
+        on_top = torch.full((M, N), 3.0, device="cuda:0")
+        assert fn(a.data_ptr(), 1, w.data_ptr(), s.data_ptr(), z.data_ptr(), on_top.data_ptr(), K, N, M, 1, stream) == 0
+        assert torch.allclose(on_top - 3.0, y, rtol=0, atol=2.0 ** -22 * float(y.abs().max() + 3))  # one rounding of the sum and one back
+    row_tiles = -(-M // (128 >> kind))
+    cut = 256 // row_tiles * 256 if N // 256 * row_tiles < 512 else 512 // row_tiles * 256
+    cols = np.r_[0:40, cut - 40:min(cut + 40, N), N - 4:N]
+    _check(y[:, cols].cpu().numpy(), oracle.q3_gemm(A, np.ascontiguousarray(mat[:, cols]), scales[cols], zeros[cols], mode=0), rows=False)
+
+
 @pytest.mark.parametrize("M,K,N", [(40, 2080, 516), (64, 8192, 132), (129, 2080, 260), (300, 1024, 1028)])
 @pytest.mark.parametrize("k,pos", [(0, 0), (19, 0), (29, 0), (14, 1), (3, 5)])
 @pytest.mark.parametrize("amp", [64.0, 4096.0, -60000.0])
