@@ -38,3 +38,15 @@ def test_five_to_eight_rows_of_a_large_matrix_stay_with_the_block_kernel(M, K, N
     compute unit for every workgroup (not the last: 448 of them) and the matrix has 3.5e7 weights and more (seven and eight rows: 4e7)."""
     choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
     assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(8, 4160, 19972, "direct"), (7, 4960, 24904, "direct"), (5, 5120, 13824, "direct"),
+                                          (6, 15936, 12176, "block"), (8, 15936, 12176, "direct"), (6, 10976, 12176, "direct"),
+                                          (5, 12128, 17920, "direct"), (5, 12128, 16384, "block"), (6, 15936, 10176, "direct"),
+                                          (8, 4096, 19648, "block"), (8, 4096, 19652, "direct"), (7, 8256, 8500, "block"),
+                                          (7, 8704, 8500, "direct"), (8, 16416, 9000, "block")])
+def test_five_to_eight_rows_in_more_workgroups_than_compute_units(M, K, N, kernel):
+    """7e7 weights and more, on either side of each line: up to a fifth more workgroups than compute units (307 of 64 columns; a last
+    range of K that is nearly empty counts for nothing), five and six rows of K >= 11000 in evenly filled rounds, K beyond 16384."""
+    choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
+    assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel
