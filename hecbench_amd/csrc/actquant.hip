@@ -17,7 +17,7 @@
 // The division by a scale shared by many elements: fp32 elements are multiplied by its reciprocal wherever that provably
 // rounds to the same integer (the product is further from a tie than its error bound, or saturates either way), the other
 // lanes divide; 16-bit elements, among which ties are common, get the rounded quotient in three operations (fast8).
-// 4096 x 5137, us, before -> now: bf16 static 14.7 -> 11.6, with zero point 15.7 -> 11.7, dynamic with zero point 17.5 -> 14.4;
+// 4096 x 5137, us, before -> now: bf16 static 14.7 -> 11.6, with zero point 15.7 -> 11.7, dynamic with zero point 17.5 -> 13.5;
 // fp16 12.4 -> 11.8, 13.0 -> 12.0, 15.9 -> 14.0.
 #include "hq_internal.h"
 
@@ -143,6 +143,48 @@ struct UnitScan<_Float16, AZP> {
   __device__ __forceinline__ void fold(float& mx, float& mn) {
     mx = fmaxf(mx, fmaxf((float)hi.x, (float)hi.y));
     if (AZP) mn = fminf(mn, fminf((float)lo.x, (float)lo.y));
+  }
+};
+
+// Running maximum and minimum of bf16 units as packed integers, a unit of eight in twelve instructions (as converted floats in 16; without
+// a zero point eight, 12): a float is a sign and a magnitude, so the largest number, where one is positive, is the largest signed
+// integer (the maximum begins above zero), and the smallest the largest unsigned one, or, where none is negative, the smallest.  What is
+// not in the row counts as zeros, or as ones for that smallest.  A wave with a NaN scans again as floats, which drop it; that the others
+// have none spares the second pass its test.
+// With zero point, us, floats -> bits: 4096 x 5137 14.2 -> 13.6, 2000 x 1399 5.61 -> 5.29, 8192 x 401 8.30 -> 7.87, 1452 x 14519 14.6 ->
+// 13.65, without 6001 x 1003 6.61 -> 6.26.  Rows of whole 512 elements up to 4096 do not gain (4096 x 4096 10.5 -> 10.6, 6000 x 2048
+// 10.2 -> 10.2, but 4096 x 8192 18.7 -> 18.1) and are scanned as floats, as is fp16, whose packed maximum is as short.
+typedef short s2v __attribute__((ext_vector_type(2)));
+typedef unsigned short us2v __attribute__((ext_vector_type(2)));
+template <bool AZP>
+struct BitScan {
+  static constexpr uint32_t kInf = 0x7f80u;
+  s2v hi = {0, 0};
+  us2v most = {0, 0}, least = {0xffff, 0xffff};  // most, without a zero point: of the magnitudes
+  // The bits of word i that belong to the row: elements [lo, end) of the unit.
+  static __device__ __forceinline__ uint32_t inside(int i, int lo, int end) {
+    return (lo <= 2 * i && end > 2 * i ? 0xffffu : 0u) | (lo <= 2 * i + 1 && end > 2 * i + 1 ? 0xffff0000u : 0u);
+  }
+  template <bool CUT>  // the row's first or last unit
+  __device__ __forceinline__ void add(const Raw<bf16_t>& r, int lo, int end) {
+#pragma unroll
+    for (int i = 0; i < kVec / 2; ++i) {
+      const uint32_t in = CUT ? inside(i, lo, end) : 0xffffffffu;
+      const uint32_t x = r.w[0][i] & (AZP ? in : in & 0x7fff7fffu);
+      if (AZP) {
+        hi = __builtin_elementwise_max(hi, __builtin_bit_cast(s2v, x));
+        least = __builtin_elementwise_min(least, __builtin_bit_cast(us2v, x | ~in));
+      }
+      most = __builtin_elementwise_max(most, __builtin_bit_cast(us2v, x));
+    }
+  }
+  // The lane's maximum and minimum; whether the wave has a NaN.
+  __device__ __forceinline__ bool fold(float& mx, float& mn) {
+    const uint32_t h = (uint32_t)max((int)hi.x, (int)hi.y), m = max((uint32_t)most.x, (uint32_t)most.y);
+    const uint32_t l = m >= 0x8000u ? m : min((uint32_t)least.x, (uint32_t)least.y);
+    mx = fmaxf(mx, __uint_as_float((AZP ? h : m) << 16));
+    if (AZP && l != 0xffffu) mn = fminf(mn, __uint_as_float(l << 16));  // (all ones: no element at all)
+    return __builtin_amdgcn_ballot_w64(h > kInf || m > ((AZP ? 0x8000u : 0u) | kInf)) != 0;
   }
 };
 
@@ -305,8 +347,8 @@ __device__ __forceinline__ void residues(const Raw<_Float16>& r, const float (&q
   }
 }
 
-// The eight results of a unit, as low bytes; false if a quotient is a NaN (a NaN element, or an overflow on the way).
-template <FastMode MODE, typename T>
+// The eight results of a unit, as low bytes; CHECKED: false if a quotient is a NaN (a NaN element, or an overflow on the way).
+template <bool CHECKED, FastMode MODE, typename T>
 __device__ __forceinline__ bool fast8(const Raw<T>& raw, const FastRow<MODE>& row, int (&q)[kVec]) {
   float t[kVec];
   bool ordered = true;
@@ -319,7 +361,7 @@ __device__ __forceinline__ bool fast8(const Raw<T>& raw, const FastRow<MODE>& ro
 #pragma clang fp contract(off)
       t[i] = fmaf(rest[i], row.m, q0[i]) + kMagic;
       if (MODE == kQuotientAzp) t[i] = t[i] + row.azp;
-      any = __builtin_elementwise_maximum(any, t[i]);  // a NaN stays
+      if (CHECKED) any = __builtin_elementwise_maximum(any, t[i]);  // a NaN stays
     }
     ordered = any == any;
 #pragma unroll
@@ -363,7 +405,7 @@ __device__ __forceinline__ void static_quant_body(const T* __restrict__ in, int8
     for (int k = 0; k < kStaticUnroll; ++k) {
       const int64_t u = u0 + k * stride;
       int q[kVec];
-      if (!(sizeof(T) == 2 && row.usable && !__builtin_amdgcn_ballot_w64(!fast8(raw[k], row, q))))
+      if (!(sizeof(T) == 2 && row.usable && !__builtin_amdgcn_ballot_w64(!fast8<true>(raw[k], row, q))))
         quantise8<AZP>(raw[k], d, azp, q);
       if (u < units) store_unit<true>(out, u, q, 0, (int)min((int64_t)kVec, total - u * kVec), aligned);
     }
@@ -405,11 +447,12 @@ __device__ __forceinline__ void row_max_min(float& a, float& b, float* lds) {
 // needed twice the registers for half the waves per CU and measured 18.8 us where this takes 14.0, 4096
 // rows of 5137 fp16: the hardware overlaps one row's stores with another's loads by itself when enough
 // workgroups fit a CU.)
-// WHOLE: both pointers are aligned and the tensor is a whole number of units, so every unit is loaded whole; TAIL: aligned,
+// WHOLE: both pointers are aligned and the tensor is a whole number of units, so every unit is loaded whole; EVEN: so is every row, of up
+// to 4096 elements (bf16 only, see BitScan); TAIL: aligned,
 // but the tensor's last unit is cut (it alone, in the last row, is loaded element by element); ANY: other pointers.  (With
 // ANY in the place of TAIL 1452 rows of 14519 bf16 took 35.6 us.)
 // 64 registers for the 16-bit types, i.e. eight waves per SIMD, where nothing spills for it (one more register cost bf16 rows of 16384 22.3 -> 26.2 us).
-enum RowMode { WHOLE, TAIL, ANY };
+enum RowMode { WHOLE, EVEN, TAIL, ANY };
 constexpr int row_threads(int lanes) { return lanes < 256 ? 256 : lanes; }
 
 template <typename T, bool AZP, int LANES, int KEEP, RowMode MODE>
@@ -437,7 +480,7 @@ __device__ __forceinline__ void dynamic_quant_body(const T* __restrict__ in, int
   // the last unit of the row that lies in the tensor whole (the tensor has one)
   const int last = MODE == TAIL ? (int)(min(ubase + end, total / kVec) - ubase) - 1 : end - 1;
   auto fetch = [&](int j) {
-    return MODE == WHOLE || (MODE == TAIL && j <= last) ? load_unit(row_in, j) : load_unit_tail(in, ubase + j, total);
+    return MODE == WHOLE || MODE == EVEN || (MODE == TAIL && j <= last) ? load_unit(row_in, j) : load_unit_tail(in, ubase + j, total);
   };
 
   Raw<T> keep[KEEP];
@@ -459,30 +502,65 @@ __device__ __forceinline__ void dynamic_quant_body(const T* __restrict__ in, int
   // (reference.h:71-72); the symmetric variant starts its absmax at 0 (reference.h:43)
   float mx = AZP ? 1.17549435e-38f : 0.f;
   float mn = 3.40282347e+38f;
-  UnitScan<T, AZP> whole;
-  auto scan = [&](const Raw<T>& raw, int j) {
+  auto part = [&](int j, int& lo, int& hi) {  // elements of unit j that belong to the row
     const int rel = (j - first) * kVec - head;  // row position of the unit's element 0
-    const int lo = max(-rel, 0), hi = min(hidden - rel, kVec);
-    if (lo == 0 && hi == kVec) {  // all but the row's first and last unit
-      whole.add(raw, mx, mn);
-    } else {
-      float v[kVec];
-      unpack(raw, v);
+    lo = max(-rel, 0);
+    hi = min(hidden - rel, kVec);
+  };
+  auto scan_kept = [&](auto&& scan) {
 #pragma unroll
-      for (int i = 0; i < kVec; ++i)
-        if (i >= lo && i < hi) {
-          if (AZP) { mx = fmaxf(mx, v[i]); mn = fminf(mn, v[i]); }
-          else mx = fmaxf(mx, fabsf(v[i]));
-        }
+    for (int k = 0; k < KEEP; ++k) {
+      const int j = lane + k * LANES;
+      if (j >= first && j < end) scan(keep[k], j);
     }
   };
+  auto scan_rest = [&](auto&& scan) {
+    for (int j = lane + KEEP * LANES; j < end; j += LANES) scan(fetch(j), j);
+  };
+  auto scan_floats = [&](const Raw<T>& raw, int j) {
+    int lo, hi;
+    part(j, lo, hi);
+    float v[kVec];
+    unpack(raw, v);
 #pragma unroll
-  for (int k = 0; k < KEEP; ++k) {
-    const int j = lane + k * LANES;
-    if (j >= first && j < end) scan(keep[k], j);
+    for (int i = 0; i < kVec; ++i)
+      if (i >= lo && i < hi) {
+        if (AZP) { mx = fmaxf(mx, v[i]); mn = fminf(mn, v[i]); }
+        else mx = fmaxf(mx, fabsf(v[i]));
+      }
+  };
+  constexpr bool by_bits = __is_same(T, bf16_t) && MODE != EVEN;
+  bool nan = false;  // by_bits: among the elements of the wave
+  if constexpr (by_bits) {
+    const float mx0 = mx, mn0 = mn;
+    BitScan<AZP> bits;
+    auto add = [&](const Raw<T>& raw, int j) {
+      int lo, hi;
+      part(j, lo, hi);
+      if (lo == 0 && hi == kVec) bits.template add<false>(raw, 0, kVec);  // all but the row's first and last unit
+      else bits.template add<true>(raw, lo, hi);
+    };
+    scan_kept(add);
+    scan_rest(add);
+    nan = bits.fold(mx, mn);
+    if (nan) {
+      mx = mx0;
+      mn = mn0;
+      scan_kept(scan_floats);
+      scan_rest(scan_floats);
+    }
+  } else {
+    UnitScan<T, AZP> whole;
+    auto scan = [&](const Raw<T>& raw, int j) {
+      int lo, hi;
+      part(j, lo, hi);
+      if (lo == 0 && hi == kVec) whole.add(raw, mx, mn);  // all but the row's first and last unit
+      else scan_floats(raw, j);
+    };
+    scan_kept(scan);
+    scan_rest(scan);
+    whole.fold(mx, mn);
   }
-  for (int j = lane + KEEP * LANES; j < end; j += LANES) scan(fetch(j), j);
-  whole.fold(mx, mn);
   row_max_min<LANES>(mx, mn, lds);
 
   float scale_val, mul = 0.f;
@@ -504,7 +582,15 @@ __device__ __forceinline__ void dynamic_quant_body(const T* __restrict__ in, int
     int q[kVec];
     forget(raw);
     bool done = false;
-    if (sizeof(T) == 2 && row.usable) done = !__builtin_amdgcn_ballot_w64(!fast8(raw, row, q));
+    if constexpr (by_bits) {
+      // no NaN among the wave's elements, and none on the way: the largest magnitude is ordinary and a quotient within 2^20
+      if (row.usable && !(AZP && nan)) {
+        fast8<false>(raw, row, q);
+        done = true;
+      }
+    } else if (sizeof(T) == 2 && row.usable) {
+      done = !__builtin_amdgcn_ballot_w64(!fast8<true>(raw, row, q));
+    }
     if (done) {
     } else if (AZP) {
       quantise8<true>(raw, d, azp_val, q);
@@ -525,7 +611,7 @@ __device__ __forceinline__ void dynamic_quant_body(const T* __restrict__ in, int
   for (int j = lane + KEEP * LANES; j < end; j += LANES) emit(fetch(j), j);
 }
 template <typename T, bool AZP, int LANES, int KEEP, RowMode MODE>
-__global__ __launch_bounds__(row_threads(LANES)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && LANES >= 256 ? (MODE == WHOLE || !AZP ? 8 : 7) : 1)))
+__global__ __launch_bounds__(row_threads(LANES)) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && LANES >= 256 ? (MODE == WHOLE || MODE == EVEN || !AZP ? 8 : 7) : 1)))
 void dynamic_quant_kernel(HQ_ARGS12) {
   HqReader r(HQ_PASS12);
   const T* const in = r;
@@ -599,6 +685,9 @@ int launch_dynamic_azp(const T* in, int8_t* out, float* scales, int32_t* azps, i
     return launch_dynamic_mode<T, AZP, ANY>(in, out, scales, azps, tokens, hidden, dev, stream);
   if (total % kVec)
     return launch_dynamic_mode<T, AZP, TAIL>(in, out, scales, azps, tokens, hidden, dev, stream);
+  if constexpr (__is_same(T, bf16_t)) {
+    if (hidden % (64 * kVec) == 0 && hidden <= 4096) return launch_dynamic_mode<T, AZP, EVEN>(in, out, scales, azps, tokens, hidden, dev, stream);
+  }
   return launch_dynamic_mode<T, AZP, WHOLE>(in, out, scales, azps, tokens, hidden, dev, stream);
 }
 

@@ -281,3 +281,42 @@ def test_quotients_of_16_bit_rows(hq, oracle, dtype):
         want, ws, wz = oracle.int8_quant_dynamic(x, with_azp)
         assert np.array_equal(gs.cpu().numpy(), ws) and np.array_equal(got.cpu().numpy(), want)
         assert not with_azp or np.array_equal(gz.cpu().numpy(), wz)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hidden", [1, 7, 8, 9, 515, 1541, 2055, 5137, 13001, 41999])
+def test_scan_of_16_bit_rows_by_their_bits(hq, oracle, dtype, hidden):
+    """Rows of one sign, with either zero, with a NaN of either sign and with their extremes at the row's ends, next to rows of the
+    other kind (whose elements share their first and last units): scales, zero points and results are the oracle's."""
+    import torch
+    rng = np.random.default_rng(hidden)
+    n = rng.standard_normal((12, hidden)).astype(np.float32)
+    n[0] = np.abs(n[0]) + 1
+    n[1] = -np.abs(n[1]) - 1
+    n[2] = np.maximum(n[2], 0)
+    n[3] = np.minimum(n[3], -0.0)
+    n[4] = np.abs(n[4]) + 1
+    n[4, hidden // 2] = -0.0
+    n[5, 0], n[5, -1] = 50, -60
+    n[6] = np.abs(n[6]) * 1e-6 + 1e-7  # fp16: subnormal
+    n[7] = np.abs(n[7]) + 2
+    n[7, -1] = 1.5
+    n[9] = -np.abs(n[9]) - 3
+    nan = {8: [0], 9: [hidden // 3], 10: [hidden - 1], 11: [0, hidden - 1]} if hidden > 2 else {}
+    x = torch.from_numpy(n).to({"f16": torch.float16, "bf16": torch.bfloat16}[dtype])
+    keep = np.ones(n.shape, bool)
+    for row, at in nan.items():
+        for i, sign in zip(at, (0, -0x8000) if row != 10 else (-0x8000,)):
+            x.view(torch.int16)[row, i] = sign + 0x7fc1
+            keep[row, i] = False
+    x = x if dtype == "bf16" else x.numpy()
+    for with_azp in (False, True):
+        got, gs, gz = hq.dynamic_scaled_int8_quant(_dev(x), with_azp)
+        want, ws, wz = oracle.int8_quant_dynamic(x, with_azp)
+        ok = np.ones(len(n), bool)
+        if with_azp:  # a row of one value has a scale of zero: the quotients are no numbers
+            ok = ws != 0
+            assert np.array_equal(gz.cpu().numpy()[ok], wz[ok])
+        assert np.array_equal(gs.cpu().numpy(), ws)
+        both = keep & ok[:, None]
+        assert np.array_equal(got.cpu().numpy()[both], want[both]), with_azp
