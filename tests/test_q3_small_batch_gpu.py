@@ -266,8 +266,8 @@ def test_block_kernel_vs_oracle(hq, oracle, tunable, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(6, 4096, 17092), (8, 4096, 17092), (7, 8256, 8500), (5, 36864, 2052), (12, 36864, 516),
                                    (5, 4096, 11008), (8, 8192, 8192)])
 def test_batches_that_stay_with_the_block_kernel(hq, oracle, M, K, N):
-    """Five and more rows with more workgroups than compute units go to the one-launch kernel, up to eight rows of 7e7 weights and
-    more (and of less while four rows have a compute unit for every workgroup) do not: two passes of one workgroup (six rows), row blocks (seven and eight); and more than eight rounds of K: two and
+    """Five and more rows with more workgroups than compute units go to the one-launch kernel, up to eight rows of large
+    matrices while four rows have a compute unit for every workgroup, or nearly so, do not: two passes of one workgroup (six rows), row blocks (seven and eight); and more than eight rounds of K: two and
     three passes."""
     import torch
     assert kernel_of(M, K, N) == "block"
