@@ -702,7 +702,12 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
   }
   if (fine) nsplit = parts;
   else if (apart) nsplit = rounds;
-  if (nsplit > 1 && hq_workspace_out_of_reach(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles)) nsplit = 1;
+  if (nsplit > 1 && hq_workspace_out_of_reach(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles)) {
+    // A workgroup walks all of K, in rounds of as many quads as there are registers for (one quad a round / this, under capture, us: 8192 x
+    // 128 group 64 15.1 / 11.3, 4096 x 4096 7.3 / 5.5, 4224 x 5562 four planes 8.9 / 7.8, 3072 x 1776 6.0 / 5.4; 2432 x 25507 group 32 15.1 / 16.2).
+    nsplit = 1;
+    fine = false;
+  }
   return fine ? launch_bcq_planes<NB, 1, GROUPED>(a, ragged, nsplit, stream)
               : launch_bcq_planes<NB, QUADS, GROUPED>(a, ragged, nsplit, stream);
 }
