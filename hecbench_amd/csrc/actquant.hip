@@ -153,7 +153,9 @@ struct UnitScan<_Float16, AZP> {
 // have none spares the second pass its test.
 // With zero point, us, floats -> bits: 4096 x 5137 14.2 -> 13.6, 2000 x 1399 5.61 -> 5.29, 8192 x 401 8.30 -> 7.87, 1452 x 14519 14.6 ->
 // 13.65, without 6001 x 1003 6.61 -> 6.26.  Rows of whole 512 elements up to 4096 do not gain (4096 x 4096 10.5 -> 10.6, 6000 x 2048
-// 10.2 -> 10.2, but 4096 x 8192 18.7 -> 18.1) and are scanned as floats, as is fp16, whose packed maximum is as short.
+// 10.2 -> 10.2, but 4096 x 8192 18.7 -> 18.1), nor those that divide 512, whose lanes have one unit each (8000 x 128 4.47 -> 4.59, 20000 x
+// 32 8.10 -> 8.28), nor, without a zero point, those of whole units (1992 x 168 2.78 -> 2.83, 4000 x 264 3.61 -> 3.66): these are scanned
+// as floats, as is fp16, whose packed maximum is as short.
 typedef short s2v __attribute__((ext_vector_type(2)));
 typedef unsigned short us2v __attribute__((ext_vector_type(2)));
 template <bool AZP>
@@ -448,7 +450,7 @@ __device__ __forceinline__ void row_max_min(float& a, float& b, float* lds) {
 // rows of 5137 fp16: the hardware overlaps one row's stores with another's loads by itself when enough
 // workgroups fit a CU.)
 // WHOLE: both pointers are aligned and the tensor is a whole number of units, so every unit is loaded whole; EVEN: so is every row, of up
-// to 4096 elements (bf16 only, see BitScan); TAIL: aligned,
+// to 4096 elements, as far as floats scan it as fast (bf16 only, see BitScan); TAIL: aligned,
 // but the tensor's last unit is cut (it alone, in the last row, is loaded element by element); ANY: other pointers.  (With
 // ANY in the place of TAIL 1452 rows of 14519 bf16 took 35.6 us.)
 // 64 registers for the 16-bit types, i.e. eight waves per SIMD, where nothing spills for it (one more register cost bf16 rows of 16384 22.3 -> 26.2 us).
@@ -686,7 +688,10 @@ int launch_dynamic_azp(const T* in, int8_t* out, float* scales, int32_t* azps, i
   if (total % kVec)
     return launch_dynamic_mode<T, AZP, TAIL>(in, out, scales, azps, tokens, hidden, dev, stream);
   if constexpr (__is_same(T, bf16_t)) {
-    if (hidden % (64 * kVec) == 0 && hidden <= 4096) return launch_dynamic_mode<T, AZP, EVEN>(in, out, scales, azps, tokens, hidden, dev, stream);
+    // with a zero point only rows that begin and end with blocks of 64 units, or never cross one
+    const bool even = !AZP || hidden % (64 * kVec) == 0 || (64 * kVec) % hidden == 0;
+    if (hidden % kVec == 0 && even && hidden <= 4096)
+      return launch_dynamic_mode<T, AZP, EVEN>(in, out, scales, azps, tokens, hidden, dev, stream);
   }
   return launch_dynamic_mode<T, AZP, WHOLE>(in, out, scales, azps, tokens, hidden, dev, stream);
 }

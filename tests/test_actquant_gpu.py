@@ -284,7 +284,7 @@ def test_quotients_of_16_bit_rows(hq, oracle, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
-@pytest.mark.parametrize("hidden", [1, 7, 8, 9, 515, 1541, 2055, 5137, 13001, 41999])
+@pytest.mark.parametrize("hidden", [1, 7, 8, 9, 64, 168, 256, 515, 1541, 2055, 4096, 4104, 5137, 13001, 41999])
 def test_scan_of_16_bit_rows_by_their_bits(hq, oracle, dtype, hidden):
     """Rows of one sign, with either zero, with a NaN of either sign and with their extremes at the row's ends, next to rows of the
     other kind (whose elements share their first and last units): scales, zero points and results are the oracle's."""
