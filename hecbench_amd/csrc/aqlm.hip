@@ -195,6 +195,7 @@ __global__ __launch_bounds__(kSlicedThreads) void aqlm_sliced_kernel(HQ_ARGS28) 
   const int per_xcd = (groups + 7) >> 3, group = (int)(blockIdx.x & 7) * per_xcd + place / kSlices;
   if (group >= groups) return;
   const int g0 = (int)((int64_t)a.M * group / groups), g1 = (int)((int64_t)a.M * (group + 1) / groups);
+  if (g0 == g1) return;  // fewer rows than groups: none here, and no row whose codes could be read ahead of the first trip
   const int group_rows = (a.M + groups - 1) / groups;
   float* const mine = partial + (size_t)(group * kSlices + slice) * group_rows;
 
