@@ -94,6 +94,19 @@ int hq_current_device(const HqDevice** out) {
   return HQ_OK;
 }
 
+namespace {
+// Device memory that is zero when this returns: nothing of it is left to a stream, so a graph that was captured on one stream and is
+// replayed on another finds it zero whatever its own stream has still to do.
+hipError_t alloc_zeroed(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) return e;
+  e = hipMemset(*p, 0, bytes);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  if (e != hipSuccess) (void)hipFree(*p);
+  return e;
+}
+}  // namespace
+
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
                      HqWorkspace* out, bool reserve) {
   int dev = 0;
@@ -116,8 +129,7 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
     size_t n = ws.ncounters ? ws.ncounters * 2 : (size_t)1 << 14;
     while (n < need_counters) n *= 2;
     unsigned* c = nullptr;
-    HQ_HIP_TRY(hipMalloc((void**)&c, n * sizeof(unsigned)));
-    HQ_HIP_TRY(hipMemset(c, 0, n * sizeof(unsigned)));
+    HQ_HIP_TRY(alloc_zeroed((void**)&c, n * sizeof(unsigned)));
     if (ws.counters) g_retired.push_back(std::make_pair(dev, (void*)ws.counters));
     ws.counters = c;
     ws.ncounters = n;
@@ -137,13 +149,8 @@ unsigned long long* hq_exchange_slots(hipStream_t stream, size_t n) {
   size_t room = s.second ? s.second * 2 : (size_t)1 << 17;
   while (room < n) room *= 2;
   unsigned long long* p = nullptr;
-  if (hipMalloc((void**)&p, room * sizeof(*p)) != hipSuccess) {
+  if (alloc_zeroed((void**)&p, room * sizeof(*p)) != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
-  }
-  if (hipMemsetAsync(p, 0, room * sizeof(*p), stream) != hipSuccess) {  // in front of every call that can use them
-    (void)hipGetLastError();
-    g_retired.push_back(std::make_pair(dev, (void*)p));
     return nullptr;
   }
   if (s.first) g_retired.push_back(std::make_pair(dev, (void*)s.first));

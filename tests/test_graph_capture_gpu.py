@@ -129,3 +129,51 @@ def test_capture_after_reserve_only(hq, pre_pass):
         torch.cuda.synchronize()
         for (M, *_), o, w in zip(probs, outs, want):
             assert torch.equal(o, w), (rep, M, tuple(o.shape))
+
+
+def _q3(M, K, N, g):
+    import torch
+    mat = torch.randint(-2 ** 31, 2 ** 31 - 1, (3 * K // 32, N), dtype=torch.int32, device="cuda:0", generator=g)
+    s = torch.empty(N, device="cuda:0").uniform_(0.005, 0.02, generator=g)
+    x = torch.randn(M, K, device="cuda:0", generator=g).half()
+    return (x[0].contiguous() if M == 1 else x), mat, s, 4 * s
+
+
+def test_replay_ahead_of_the_capture_stream(hq):
+    """A reservation on a stream that is busy, a capture there, replays on another stream while it is still busy: the slots and
+    counters are ready when the reservation returns."""
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    torch.cuda.synchronize()
+    assert lib.hq_shutdown() == 0  # torch hands streams out again: none has a workspace from here on
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(3)
+    K, N = 8192, 8256
+    x, mat, s, z = _q3(1, K, N, g)
+    want = hq.q3_matvec(x, mat, s, z)
+    out = torch.zeros_like(want)
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    big = torch.zeros(8192, 8192, dtype=torch.float16, device="cuda:0")
+    sink = torch.mm(big, big)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(busy):
+        for _ in range(300):  # of half a millisecond and more
+            torch.mm(big, big, out=sink)
+    assert lib.hq_reserve_workspace(ctypes.c_void_p(busy.cuda_stream), K, N) == 0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(busy):
+        graph.capture_begin()
+        hq.q3_matvec(x, mat, s, z, out=out)
+        graph.capture_end()
+    with torch.cuda.stream(other):
+        for rep in range(4):
+            out.fill_(float(rep))
+            graph.replay()
+            other.synchronize()
+            assert torch.equal(out, want), rep
+    assert not busy.query()
+    torch.cuda.synchronize()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
