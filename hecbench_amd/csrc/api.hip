@@ -17,7 +17,9 @@ std::map<int, HqDevice> g_devices;
 constexpr int kListedDevices = 64;
 std::atomic<const HqDevice*> g_known[kListedDevices];  // entries of g_devices that are gfx950 parts
 std::map<std::pair<int, hipStream_t>, HqWorkspace> g_workspaces;
-std::map<std::pair<int, hipStream_t>, std::pair<unsigned long long*, size_t>> g_slots;  // of hq_exchange_slots, and how many
+// Counters that a workspace begins with.  With exchange slots for every batch (8192 rows of partial sums) and up to 75,000 columns they
+// grow no later than the partial sums: an allocation is an error while any other stream is being captured.
+constexpr size_t kLeastCounters = (size_t)1 << 20;
 constexpr size_t kMostSlots = (size_t)4 << 20;  // 32 MB
 std::vector<std::pair<int, void*>> g_retired;  // outgrown buffers, freed by hq_shutdown()
 }  // namespace
@@ -107,8 +109,8 @@ hipError_t alloc_zeroed(void** p, size_t bytes) {
 }
 }  // namespace
 
-int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
-                     HqWorkspace* out, bool reserve) {
+int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters, HqWorkspace* out, size_t want_slots,
+                     bool reserve) {
   int dev = 0;
   HQ_HIP_TRY(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_mu);
@@ -125,37 +127,42 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
     ws.partial = p;
     ws.partial_floats = n;
   }
-  if (ws.ncounters < need_counters) {
-    size_t n = ws.ncounters ? ws.ncounters * 2 : (size_t)1 << 14;
-    while (n < need_counters) n *= 2;
+  size_t want = want_slots <= kMostSlots && 2 * want_slots > need_counters ? 2 * want_slots : need_counters;
+  if (want > need_counters && ws.ncounters < want) {  // slots can be done without: none of them while capturing
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      want = need_counters;
+    }
+  }
+  if (ws.ncounters < want) {
+    size_t n = ws.ncounters ? ws.ncounters * 2 : kLeastCounters;
+    while (n < want) n *= 2;
+    if (reserve) n = want > (size_t)1 << 14 ? want : (size_t)1 << 14;
     unsigned* c = nullptr;
-    HQ_HIP_TRY(alloc_zeroed((void**)&c, n * sizeof(unsigned)));
-    if (ws.counters) g_retired.push_back(std::make_pair(dev, (void*)ws.counters));
-    ws.counters = c;
-    ws.ncounters = n;
+    const hipError_t e = alloc_zeroed((void**)&c, n * sizeof(unsigned));
+    if (e == hipSuccess) {
+      if (ws.counters) g_retired.push_back(std::make_pair(dev, (void*)ws.counters));
+      ws.counters = c;
+      ws.ncounters = n;
+    } else {
+      (void)hipGetLastError();
+      if (ws.ncounters < need_counters) return (int)e;
+    }
   }
   *out = ws;
   return HQ_OK;
 }
 
-unsigned long long* hq_exchange_slots(hipStream_t stream, size_t n) {
-  int dev = 0;
-  if (n > kMostSlots || hipGetDevice(&dev) != hipSuccess) return nullptr;
-  std::lock_guard<std::mutex> lk(g_mu);
-  auto& s = g_slots[std::make_pair(dev, stream)];
-  if (s.second >= n) return s.first;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return nullptr;
-  size_t room = s.second ? s.second * 2 : (size_t)1 << 17;
-  while (room < n) room *= 2;
-  unsigned long long* p = nullptr;
-  if (alloc_zeroed((void**)&p, room * sizeof(*p)) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  if (s.first) g_retired.push_back(std::make_pair(dev, (void*)s.first));
-  s = std::make_pair(p, room);
-  return p;
+int hq_get_split(hipStream_t stream, size_t floats, size_t counters, int nsplit, float** partial, unsigned** arrivals) {
+  const size_t slots = hq_tune(HQ_TUNE_SPLITK_FENCES, 0) ? 0 : hq_split_slots(floats, nsplit);
+  HqWorkspace ws;
+  const int rc = hq_get_workspace(stream, floats, counters, &ws, slots);
+  if (rc != HQ_OK) return rc;
+  const bool meet = slots > 0 && ws.ncounters >= 2 * slots;
+  *partial = meet ? reinterpret_cast<float*>(ws.counters) : ws.partial;
+  *arrivals = meet ? nullptr : ws.counters;
+  return HQ_OK;
 }
 
 bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters) {
@@ -229,9 +236,9 @@ extern "C" int hq_reserve_workspace(void* stream, int max_K, int max_N) {
   // batches, two workgroups per compute unit where tiles are narrow).  Calls go on without where there are none.
   const size_t tiles = ((size_t)max_N + 63) / 64;
   const size_t rows = tiles * (kHqMeetMost - 1) > 8192 ? tiles * (kHqMeetMost - 1) : 8192;
-  (void)hq_exchange_slots((hipStream_t)stream, (rows > 2 * (size_t)d->cus ? rows : 2 * (size_t)d->cus) * 64);
+  const size_t slots = (rows > 2 * (size_t)d->cus ? rows : 2 * (size_t)d->cus) * 64;
   HqWorkspace ws;
-  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, true);
+  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, slots, true);
 }
 
 extern "C" int hq_shutdown(void) {
@@ -251,8 +258,6 @@ extern "C" int hq_shutdown(void) {
     release(kv.first.first, kv.second.partial);
     release(kv.first.first, kv.second.counters);
   }
-  for (auto& kv : g_slots) release(kv.first.first, kv.second.first);
-  g_slots.clear();
   for (auto& r : g_retired) release(r.first, r.second);
   g_workspaces.clear();
   g_retired.clear();

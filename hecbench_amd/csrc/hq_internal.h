@@ -114,24 +114,25 @@ struct HqDevice {
 // Device facts for the current device (cached per ordinal).  Returns an hq code.
 int hq_current_device(const HqDevice** out);
 
-// The sums of a divided K that meet by exchange (hq_meet): `n` slots, zero between calls, of (current device, stream).  Null where
-// there are not as many and none can be had (under capture): the shares then meet through a workspace and a counter.
-unsigned long long* hq_exchange_slots(hipStream_t stream, size_t n);
-
 struct HqWorkspace {
   float* partial;      // split-K partial sums
-  unsigned* counters;  // arrival counters, zero between calls (self-resetting)
+  unsigned* counters;  // zero between calls: arrival counters (self-resetting), or exchange slots of two each (hq_meet)
   size_t partial_floats;
   size_t ncounters;
 };
 
-// Workspace of (current device, stream) holding at least the requested sizes.
+// Workspace of (current device, stream) holding at least the requested sizes, and counters for want_slots slots unless the stream is
+// being captured or they cannot be had.
 // Allocated on first use, grown geometrically on demand (reserve: to no more than the request), freed by hq_shutdown().
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
-                     HqWorkspace* out, bool reserve = false);
+                     HqWorkspace* out, size_t want_slots = 0, bool reserve = false);
 // Whether that would allocate while the stream is being captured, where an allocation is an error: a plan that can do
 // without a workspace then does.
 bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters);
+// Where the `nsplit` shares of a divided K meet, `floats` partial sums in all: in exchange slots (*arrivals null, *partial the slots,
+// up to kHqMeetMost shares and no formal fences), or through partial sums and arrival counters.  The workspace has room for those
+// either way, so a captured call finds what an eager one has left behind, and gives the same bits on both ways.
+int hq_get_split(hipStream_t stream, size_t floats, size_t counters, int nsplit, float** partial, unsigned** arrivals);
 
 // Caller-provided scratch of the GPTQ 3-bit paths (the entry point that allocates nothing passes its
 // fixed device array here; a null pointer means "use the stream's workspace").
@@ -280,6 +281,7 @@ __device__ __forceinline__ bool hq_meet(unsigned long long* slots, size_t stride
 // taken).  Four rows, two shares, 4224 x 2200 6.9 / 6.05.  LUT-GEMM: two shares 8192 x 8192 8.15 / 7.35, three 11008 x 4096 7.8 / 7.1,
 // six 6016 x 2265 (two planes) 5.8 / 5.0, eight 7552 x 2166 (groups of 64) 6.9 / 6.2.
 constexpr int kHqMeetMost = 8;
+inline size_t hq_split_slots(size_t floats, int nsplit) { return nsplit > 1 && nsplit <= kHqMeetMost ? floats / nsplit * (nsplit - 1) : 0; }
 
 // Packed rows that start at any multiple of four or one column (N not a multiple of 32 words): the 128-byte lines at the edges of
 // a column tile belong to its neighbour too.

@@ -615,17 +615,9 @@ int launch_bcq_planes(LutArgs a, bool ragged, int nsplit, hipStream_t stream) {
   a.kslice = rpw * WAVES * QUADS * 128;
   a.nsplit = nsplit;
   a.strict = hq_tune(HQ_TUNE_SPLITK_FENCES, 0);
-  unsigned long long* slots = nullptr;
-  if (nsplit > 1 && nsplit <= kHqMeetMost && !a.strict) slots = hq_exchange_slots(stream, (size_t)ntiles * (nsplit - 1) * 64);
-  if (slots) {
-    a.partial = reinterpret_cast<float*>(slots);
-    a.counters = nullptr;
-  } else if (nsplit > 1) {
-    HqWorkspace ws;
-    const int rc = hq_get_workspace(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles, &ws);
+  if (nsplit > 1) {
+    const int rc = hq_get_split(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles, nsplit, &a.partial, &a.counters);
     if (rc != HQ_OK) return rc;
-    a.partial = ws.partial;
-    a.counters = ws.counters;
   }
   const dim3 grid(ntiles, nsplit), block(WAVES * 64);
   const size_t smem = (size_t)WAVES * QUADS * kDigQuad + (size_t)WAVES * 4 * 64 * 4 + (size_t)WAVES * 4 + 16;

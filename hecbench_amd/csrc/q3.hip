@@ -674,19 +674,7 @@ int q3_split_acquire(const Q3SplitPlan& p, const HqQ3Scratch* fixed, hipStream_t
     out->counters = fixed->counters;
     return HQ_OK;
   }
-  if (p.nsplit <= kHqMeetMost && !hq_tune(HQ_TUNE_SPLITK_FENCES, 0)) {
-    // (floats: a row of 64 per tile, share and row of results)
-    if (unsigned long long* slots = hq_exchange_slots(stream, p.floats / p.nsplit * (p.nsplit - 1))) {
-      out->partial = reinterpret_cast<float*>(slots);
-      return HQ_OK;
-    }
-  }
-  HqWorkspace ws;
-  const int rc = hq_get_workspace(stream, p.floats, (size_t)p.ntiles, &ws);
-  if (rc != HQ_OK) return rc;
-  out->partial = ws.partial;
-  out->counters = ws.counters;
-  return HQ_OK;
+  return hq_get_split(stream, p.floats, (size_t)p.ntiles, p.nsplit, &out->partial, &out->counters);
 }
 
 // Launch shape of the batch-1 kernel (pure arithmetic).

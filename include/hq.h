@@ -77,7 +77,7 @@ int hq_init(void);
  * re-ordered rows and the shares of divided tiles among them - on 256 compute units 8 MiB for max_K = 512, 16 MiB for
  * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152 - and 4 MiB and more (3.5 KiB per 64 columns) in which the sums of a K
  * divided among a few workgroups meet.  A stream that only ever sees smaller calls takes less without a
- * reservation: a workspace grows with the calls (hq_q3_workspace_need; batch 1 at most a few MiB, up to 64 rows 16 MiB).
+ * reservation: a workspace grows with the calls (hq_q3_workspace_need; 8 MiB to begin with, nearly always enough for batch 1; up to 64 rows 20 MiB).
  * A captured call keeps the workspace of the stream it was captured on, whatever stream its graph is replayed on: replays must not
  * overlap with each other or with calls on that stream where both use it.  Calls that overlap in one workspace give wrong results,
  * and they may leave its arrival counters and slots, which the kernels expect at zero and return to zero, at other values; hq_shutdown()

@@ -177,3 +177,51 @@ def test_replay_ahead_of_the_capture_stream(hq):
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+def _lut(K, N, nb, group, g):
+    import torch
+    bW = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 32, nb, N), dtype=torch.int32, device="cuda:0", generator=g)
+    alpha = torch.rand(K // group, nb, N, device="cuda:0", generator=g).mul_(0.02).half()
+    return torch.randn(K, device="cuda:0", generator=g).half(), bW, alpha, None, group
+
+
+@pytest.mark.parametrize("first,op,shape", [
+    (None, "lut", (8192, 8192, 3, 128)), (None, "lut", (2432, 25507, 4, 32)), (None, "lut", (13184, 256, 2, 64)),
+    (None, "q3", (4, 8192, 8256)), (None, "q3", (7, 8192, 640)), (None, "q3", (1, 8192, 28672)),
+    ((1, 8192, 640), "q3", (1, 39136, 364)),      # ten shares, which meet through a count, after a call of two
+    ((1, 8192, 640), "q3", (1, 28672, 28672)),    # more shares than the first call of the stream had
+    ((4, 8192, 640), "lut", (8192, 8192, 3, 128))])
+def test_capture_after_an_eager_call(hq, first, op, shape):
+    """No reservation: what a stream's eager calls have allocated serves the same call under capture, and any other that takes no
+    more than the least a workspace holds.  The same kernel on the same shares of K: the eager call's bits."""
+    import torch
+    from hecbench_amd import _lib
+    torch.cuda.synchronize()
+    assert _lib.load().hq_shutdown() == 0  # torch hands streams out again: none has a workspace from here on
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(sum(shape))
+    data = _lut(*shape, g) if op == "lut" else _q3(*shape, g)
+    call = lambda d=data: (hq.lut_matmul if op == "lut" else hq.q3_matvec if d[0].dim() == 1 else hq.q3_gemm)(*d)
+    if first is None:
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            want = call()
+    else:
+        want = call()
+        stream = torch.cuda.Stream()
+        d = _q3(*first, g)
+        with torch.cuda.stream(stream):
+            stream.wait_stream(torch.cuda.default_stream())
+            (hq.q3_matvec if first[0] == 1 else hq.q3_gemm)(*d)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = call()
+    for rep in range(3):
+        out.fill_(float(rep))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), rep
+        assert torch.equal(call(), want)
