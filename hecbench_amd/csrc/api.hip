@@ -1,4 +1,5 @@
 // Library-wide state of libhq: device facts, per-stream workspaces, error text.
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <cstdio>
@@ -20,7 +21,6 @@ std::map<std::pair<int, hipStream_t>, HqWorkspace> g_workspaces;
 // Counters that a workspace begins with.  With exchange slots for every batch (8192 rows of partial sums) and up to 75,000 columns they
 // grow no later than the partial sums: an allocation is an error while any other stream is being captured.
 constexpr size_t kLeastCounters = (size_t)1 << 20;
-constexpr size_t kMostSlots = (size_t)4 << 20;  // 32 MB
 std::vector<std::pair<int, void*>> g_retired;  // outgrown buffers, freed by hq_shutdown()
 }  // namespace
 
@@ -127,7 +127,7 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
     ws.partial = p;
     ws.partial_floats = n;
   }
-  size_t want = want_slots <= kMostSlots && 2 * want_slots > need_counters ? 2 * want_slots : need_counters;
+  size_t want = std::max(need_counters, 2 * want_slots);
   if (want > need_counters && ws.ncounters < want) {  // slots can be done without: none of them while capturing
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
@@ -212,6 +212,14 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   // arrival counters: one per column tile, narrow tiles four per 64 columns, row blocks sixteen per tile
   *counters = tiles > 1 ? tiles * 16 : 16;
   if (tile_counters > *counters) *counters = tile_counters;
+  // and the slots in which up to eight shares of K meet, two counters each: a row of 64 per column tile and share but one, of 1024
+  // elements of K at least (the LUT kernels; narrow tiles of the matvec stay within the compute units) or of 4096 and for every
+  // row of a batch, where partial sums take 8192 rows at most
+  auto shares = [&](size_t k) { return std::min<size_t>(((size_t)max_K + k - 1) / k, kHqMeetMost); };
+  size_t slots = 0;
+  if (max_K > 1024) slots = tiles * (shares(1024) - 1) * 64;
+  if (max_K > 4096) slots = std::max({slots, (size_t)cus * 64, std::min<size_t>(tiles * (shares(4096) - 1) * 64, 8192) * 64});
+  *counters = std::max(*counters, 2 * std::min(slots, kHqMostSlots));
   if ((size_t)cus / 8 > *counters) *counters = cus / 8;  // and one per group of rows of the AQLM kernel
 }
 
@@ -232,13 +240,8 @@ extern "C" int hq_reserve_workspace(void* stream, int max_K, int max_N) {
   if (rc != HQ_OK) return rc;
   size_t floats = 0, counters = 0;
   reserve_bound(d->cus, max_K, max_N, &floats, &counters);
-  // and the slots in which the shares of K meet: a column's, per tile, row and share but one (at most 8192 rows of partial sums for
-  // batches, two workgroups per compute unit where tiles are narrow).  Calls go on without where there are none.
-  const size_t tiles = ((size_t)max_N + 63) / 64;
-  const size_t rows = tiles * (kHqMeetMost - 1) > 8192 ? tiles * (kHqMeetMost - 1) : 8192;
-  const size_t slots = (rows > 2 * (size_t)d->cus ? rows : 2 * (size_t)d->cus) * 64;
   HqWorkspace ws;
-  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, slots, true);
+  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, 0, true);
 }
 
 extern "C" int hq_shutdown(void) {

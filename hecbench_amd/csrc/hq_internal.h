@@ -281,7 +281,12 @@ __device__ __forceinline__ bool hq_meet(unsigned long long* slots, size_t stride
 // taken).  Four rows, two shares, 4224 x 2200 6.9 / 6.05.  LUT-GEMM: two shares 8192 x 8192 8.15 / 7.35, three 11008 x 4096 7.8 / 7.1,
 // six 6016 x 2265 (two planes) 5.8 / 5.0, eight 7552 x 2166 (groups of 64) 6.9 / 6.2.
 constexpr int kHqMeetMost = 8;
-inline size_t hq_split_slots(size_t floats, int nsplit) { return nsplit > 1 && nsplit <= kHqMeetMost ? floats / nsplit * (nsplit - 1) : 0; }
+constexpr size_t kHqMostSlots = (size_t)4 << 20;  // 32 MB
+// The slots of `floats` partial sums in nsplit shares; 0: they do not meet by exchange.
+inline size_t hq_split_slots(size_t floats, int nsplit) {
+  const size_t n = nsplit > 1 && nsplit <= kHqMeetMost ? floats / nsplit * (nsplit - 1) : 0;
+  return n <= kHqMostSlots ? n : 0;
+}
 
 // Packed rows that start at any multiple of four or one column (N not a multiple of 32 words): the 128-byte lines at the edges of
 // a column tile belong to its neighbour too.

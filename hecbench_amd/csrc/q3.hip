@@ -30,6 +30,8 @@
 // K no cross-workgroup reduction is needed; otherwise (split-K) the partial sums
 // meet by exchange (up to eight shares), or go to a workspace and the last workgroup to arrive
 // at a tile adds them; in a fixed order, so results do not depend on arrival order.
+#include <algorithm>
+
 #include "hq_internal.h"
 #include "q3_recipe.h"
 
@@ -756,16 +758,18 @@ int hq_q3_workspace_need_impl(int cus, int K, int N, int batch_M, size_t* floats
   if (K <= 0 || N <= 0 || batch_M <= 0 || (K & 31) || (N & 3) || cus <= 0) return HQ_ERR_BAD_SHAPE;
   *floats = 0;
   *counters = 0;
+  // (as hq_get_split takes them: a few shares meet in slots of two counters)
+  auto counters_of = [](const Q3SplitPlan& p) { return std::max(p.nsplit > 1 ? (size_t)p.ntiles : 0, 2 * hq_split_slots(p.floats, p.nsplit)); };
   if (batch_M == 1) {
     const Q3MatvecPlan m = q3_matvec_shape(cus, K, N, nullptr);
     *floats = m.split.floats;
-    *counters = m.split.nsplit > 1 ? (size_t)m.split.ntiles : 0;
+    *counters = counters_of(m.split);
     return HQ_OK;
   }
   if (q3_plan(cus, K, N, batch_M) == HQ_Q3_PLAN_BLOCK) {
     const Q3BlockPlan b = q3_block_shape(cus, K, N, batch_M, nullptr);
     *floats = b.split.floats;
-    *counters = b.split.nsplit > 1 ? (size_t)b.split.ntiles : 0;
+    *counters = counters_of(b.split);
     if (q3_block_yields(cus, K, N, batch_M)) {
       const HqQ3DirectPlan d = hq_q3_direct_plan(cus, K, N, batch_M, false);
       if (d.partial_floats > *floats) *floats = d.partial_floats;

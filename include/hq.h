@@ -75,8 +75,8 @@ int hq_init(void);
  * batched GEMMs up to max_K input features, so that later calls on that stream never allocate
  * (needed before stream capture).  It allocates what hq_reserve_need tells: room for batches of any size, thousands of
  * re-ordered rows and the shares of divided tiles among them - on 256 compute units 8 MiB for max_K = 512, 16 MiB for
- * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152 - and 4 MiB and more (3.5 KiB per 64 columns) in which the sums of a K
- * divided among a few workgroups meet.  A stream that only ever sees smaller calls takes less without a
+ * 1024, 64 to 68 MiB from 2048 to 16384, 128 MiB for 49152, and up to 4 MiB (beyond 75,000 columns 3.5 KiB per 64) of counters.
+ * A stream that only ever sees smaller calls takes less without a
  * reservation: a workspace grows with the calls (hq_q3_workspace_need; 8 MiB to begin with, nearly always enough for batch 1; up to 64 rows 20 MiB).
  * A captured call keeps the workspace of the stream it was captured on, whatever stream its graph is replayed on: replays must not
  * overlap with each other or with calls on that stream where both use it.  Calls that overlap in one workspace give wrong results,
@@ -86,9 +86,10 @@ int hq_init(void);
 int hq_reserve_workspace(void* stream, int max_K, int max_N);
 
 /* Host-only size queries behind hq_reserve_workspace (plain arithmetic: no device is touched, so they also
- * answer for a device that is not present).  hq_q3_workspace_need: floats and arrival counters one
- * hq_q3_matvec(K, N, batch_M) call takes from its stream's workspace on a device of compute_units compute
- * units, computed by the very plan functions of the launch.  hq_reserve_need: what
+ * answer for a device that is not present).  hq_q3_workspace_need: floats and counters (32-bit words that are zero between
+ * calls: arrival counters, or exchange slots of two words each) that one hq_q3_matvec(K, N, batch_M) call makes sure of in its
+ * stream's workspace on a device of compute_units compute units, computed by the very plan functions of the launch (slots up to
+ * 32 MiB, and not under capture: a call goes on without).  hq_reserve_need: what
  * hq_reserve_workspace(stream, max_K, max_N) makes sure of - at least the need of every call with K <= max_K
  * and N <= max_N, whatever the batch.  Counterpart of the compute-unit query that sizes the launch in
  * src/quantAQLM-hip/main.cu:108-121. */

@@ -58,3 +58,31 @@ def test_a_reservation_allocates_what_it_names(hq):
         assert lib.hq_reserve_workspace(ctypes.c_void_p(stream.cuda_stream), K, N) == 0
         taken = free - torch.cuda.mem_get_info()[0]
         assert taken <= f.value * 4 + c.value * 4 + (6 << 20), (K, N, taken, f.value * 4)
+
+
+def test_a_reservation_is_enough_for_the_lut_kernels(hq):
+    """Whatever the split of K and the meeting of its shares: no call of those sizes allocates."""
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    torch.cuda.synchronize()
+    assert lib.hq_shutdown() == 0
+    stream = torch.cuda.Stream()
+    maxK, maxN = 8192, 9000
+    buf = torch.zeros(maxK * maxN // 8 * 4, dtype=torch.uint8, device="cuda:0")
+    alpha = torch.zeros(maxK // 32 * 4 * maxN, dtype=torch.float16, device="cuda:0")
+    x, y = torch.zeros(maxK, device="cuda:0").half(), torch.zeros(maxN, device="cuda:0").half()
+    vp = lambda t: ctypes.c_void_p(t.data_ptr())
+    call = lambda K, N, nb, G, s: lib.hq_lut_gemv(vp(buf), vp(alpha), None, vp(x), vp(y), K, N, nb, G, ctypes.c_void_p(s))
+    shapes = [(K, N, nb, G) for K in (1152, 2304, 4224, 8192) for N in (64, 700, 2166, 4096, 9000) for nb, G in ((1, 128), (3, 128), (2, 64), (4, 32))]
+    for s in shapes:
+        assert call(*s, 0) == 0  # (code objects, and the default stream's workspace)
+    with torch.cuda.stream(stream):
+        y.zero_()  # (the stream's own queue)
+    torch.cuda.synchronize()
+    assert lib.hq_reserve_workspace(ctypes.c_void_p(stream.cuda_stream), maxK, maxN) == 0
+    free = torch.cuda.mem_get_info()[0]
+    for s in shapes:
+        assert call(*s, stream.cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 4 << 20  # (to grow is to take 8 MiB)
