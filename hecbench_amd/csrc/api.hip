@@ -18,6 +18,7 @@ std::map<int, HqDevice> g_devices;
 constexpr int kListedDevices = 64;
 std::atomic<const HqDevice*> g_known[kListedDevices];  // entries of g_devices that are gfx950 parts
 std::map<std::pair<int, hipStream_t>, HqWorkspace> g_workspaces;
+std::map<std::pair<int, hipStream_t>, HqWorkspace> g_eager;  // of hq_get_eager_workspace
 // Counters that a workspace begins with.  With exchange slots for every batch (8192 rows of partial sums) and up to 75,000 columns they
 // grow no later than the partial sums: an allocation is an error while any other stream is being captured.
 constexpr size_t kLeastCounters = (size_t)1 << 20;
@@ -154,6 +155,31 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
   return HQ_OK;
 }
 
+int hq_get_eager_workspace(hipStream_t stream, size_t need_floats, size_t need_counters, HqWorkspace* out, bool reserve) {
+  int dev = 0;
+  HQ_HIP_TRY(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(g_mu);
+  HqWorkspace& ws = g_eager[std::make_pair(dev, stream)];
+  if (ws.partial_floats < need_floats || ws.ncounters < need_counters) {
+    size_t n = ws.partial_floats ? ws.partial_floats * 2 : (size_t)1 << 18;
+    while (n < need_floats) n *= 2;
+    if (reserve) n = std::max(need_floats, ws.partial_floats);
+    const size_t c = std::max(need_counters, ws.ncounters);
+    // one buffer, the counters in front; cleared in front of every call that can use them.
+    unsigned* p = nullptr;
+    hipError_t e = hipMalloc((void**)&p, (c + n) * sizeof(unsigned));
+    if (e == hipSuccess && (e = hipMemsetAsync(p, 0, c * sizeof(unsigned), stream)) != hipSuccess) (void)hipFree(p);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return (int)e;
+    }
+    if (ws.counters) g_retired.push_back(std::make_pair(dev, (void*)ws.counters));
+    ws = HqWorkspace{reinterpret_cast<float*>(p + c), p, n, c};
+  }
+  *out = ws;
+  return HQ_OK;
+}
+
 int hq_get_split(hipStream_t stream, size_t floats, size_t counters, int nsplit, float** partial, unsigned** arrivals) {
   const size_t slots = hq_tune(HQ_TUNE_SPLITK_FENCES, 0) ? 0 : hq_split_slots(floats, nsplit);
   HqWorkspace ws;
@@ -177,8 +203,8 @@ bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t ne
   return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
 }
 
-// Upper bound of what any hq_q3_matvec call with K <= max_K, N <= max_N (any batch) and any hq_lut_gemv or hq_aqlm_matvec
-// call of those sizes (rows as columns) takes from its stream's workspace on a device of `cus` compute units, with the default launch
+// Upper bound of what any hq_q3_matvec call with K <= max_K, N <= max_N (any batch) and any hq_lut_gemv call
+// of those sizes takes from its stream's workspace on a device of `cus` compute units, with the default launch
 // policy.  Host arithmetic only.  (tests/test_workspace_cpu.py checks it against the per-call need over a
 // sweep of shapes.)
 static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t* counters) {
@@ -202,8 +228,6 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   // batches 2 ... 64 on the matvec-like kernel: one partial row per tile, range of K and activation row, at most
   // 8192 of them whatever the shape
   if ((size_t)8192 * 64 > split_floats) split_floats = (size_t)8192 * 64;
-  // the AQLM kernel in slices: eight sums a row, rows padded to whole groups (an eighth of the compute units)
-  if ((size_t)8 * (max_N + cus / 8) > split_floats) split_floats = (size_t)8 * (max_N + cus / 8);
   *floats = gemm_floats > split_floats ? gemm_floats : split_floats;
   // many rows: the tiled kernels
   size_t tile_floats = 0, tile_counters = 0;
@@ -220,7 +244,12 @@ static void reserve_bound(int cus, int max_K, int max_N, size_t* floats, size_t*
   if (max_K > 1024) slots = tiles * (shares(1024) - 1) * 64;
   if (max_K > 4096) slots = std::max({slots, (size_t)cus * 64, std::min<size_t>(tiles * (shares(4096) - 1) * 64, 8192) * 64});
   *counters = std::max(*counters, 2 * std::min(slots, kHqMostSlots));
-  if ((size_t)cus / 8 > *counters) *counters = cus / 8;  // and one per group of rows of the AQLM kernel
+}
+// The same of an eager hq_aqlm_matvec call of max_N rows, from memory of its own: eight sums a row, rows padded to whole groups (an
+// eighth of the compute units), a counter for each group.
+static void reserve_bound_eager(int cus, int max_N, size_t* floats, size_t* counters) {
+  *counters = (size_t)cus / 8;
+  *floats = 8 * (std::min<size_t>(max_N, 1 << 20) + *counters);
 }
 
 extern "C" int hq_reserve_need(int compute_units, int max_K, int max_N, int64_t* floats, int64_t* counters) {
@@ -228,8 +257,10 @@ extern "C" int hq_reserve_need(int compute_units, int max_K, int max_N, int64_t*
   if (max_K < 0 || max_N < 0 || compute_units <= 0) return HQ_ERR_BAD_SHAPE;
   size_t f = 0, c = 0;
   reserve_bound(compute_units, max_K, max_N, &f, &c);
-  *floats = (int64_t)f;
-  *counters = (int64_t)c;
+  size_t ef = 0, ec = 0;
+  reserve_bound_eager(compute_units, max_N, &ef, &ec);
+  *floats = (int64_t)(f + ef);
+  *counters = (int64_t)(c + ec);
   return HQ_OK;
 }
 
@@ -241,7 +272,10 @@ extern "C" int hq_reserve_workspace(void* stream, int max_K, int max_N) {
   size_t floats = 0, counters = 0;
   reserve_bound(d->cus, max_K, max_N, &floats, &counters);
   HqWorkspace ws;
-  return hq_get_workspace((hipStream_t)stream, floats, counters, &ws, 0, true);
+  rc = hq_get_workspace((hipStream_t)stream, floats, counters, &ws, 0, true);
+  if (rc != HQ_OK) return rc;
+  reserve_bound_eager(d->cus, max_N, &floats, &counters);
+  return hq_get_eager_workspace((hipStream_t)stream, floats, counters, &ws, true);
 }
 
 extern "C" int hq_shutdown(void) {
@@ -261,8 +295,10 @@ extern "C" int hq_shutdown(void) {
     release(kv.first.first, kv.second.partial);
     release(kv.first.first, kv.second.counters);
   }
+  for (auto& kv : g_eager) release(kv.first.first, kv.second.counters);
   for (auto& r : g_retired) release(r.first, r.second);
   g_workspaces.clear();
+  g_eager.clear();
   g_retired.clear();
   (void)hipSetDevice(cur);
   return rc;

@@ -402,15 +402,16 @@ extern "C" int hq_aqlm_matvec(const int16_t* codes, const void* codebooks, const
   a.codes = (const u4v*)codes; a.codebooks = (const u4v*)codebooks; a.scales = (const _Float16*)scales;
   a.x = (const u4v*)x; a.y = (_Float16*)y; a.M = M; a.K = K; a.cb_stride = cb_stride_int4;
   for (int j = 0; j < 4; ++j) a.cb_sizes[j] = cb_a_sizes[j];
-  // Many codes: in slices.  That kernel takes memory of the stream's workspace, so a captured call, whose graph may be replayed beside
-  // anything, and a call that finds none stay with the other one.
+  // Many codes: in slices.  That kernel takes memory of its stream.  A captured call, whose graph may be replayed beside calls on that
+  // stream and beside other graphs captured there (nobody had to order calls of this operator), and one that finds no memory stay with the other one.
+  // Nor does one on the per-thread stream take it: one handle for as many streams as there are threads.
   const SlicedPlan sliced = sliced_plan(dev, M, K, cb_a_sizes[0] < M);
-  if (sliced.groups > 0) {
+  if (sliced.groups > 0 && stream != hipStreamPerThread) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     HqWorkspace ws;
     const size_t group_rows = (M + sliced.groups - 1) / sliced.groups;
     if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
-        hq_get_workspace(stream, (size_t)sliced.groups * kSlices * group_rows, sliced.groups, &ws) == HQ_OK) {
+        hq_get_eager_workspace(stream, (size_t)sliced.groups * kSlices * group_rows, sliced.groups, &ws) == HQ_OK) {
       static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&aqlm_sliced_kernel),
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kSlicedMaxLds);
       if (attr != hipSuccess) return (int)attr;

@@ -126,6 +126,9 @@ struct HqWorkspace {
 // Allocated on first use, grown geometrically on demand (reserve: to no more than the request), freed by hq_shutdown().
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters,
                      HqWorkspace* out, size_t want_slots = 0, bool reserve = false);
+// A second one of the stream, for kernels that do without under capture: no graph uses it, so its calls are ordered with everything
+// that does, whatever is replayed elsewhere.
+int hq_get_eager_workspace(hipStream_t stream, size_t need_floats, size_t need_counters, HqWorkspace* out, bool reserve = false);
 // Whether that would allocate while the stream is being captured, where an allocation is an error: a plan that can do
 // without a workspace then does.
 bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters);

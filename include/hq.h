@@ -90,7 +90,7 @@ int hq_reserve_workspace(void* stream, int max_K, int max_N);
  * calls: arrival counters, or exchange slots of two words each) that one hq_q3_matvec(K, N, batch_M) call makes sure of in its
  * stream's workspace on a device of compute_units compute units, computed by the very plan functions of the launch (slots up to
  * 32 MiB, and not under capture: a call goes on without).  hq_reserve_need: what
- * hq_reserve_workspace(stream, max_K, max_N) makes sure of - at least the need of every call with K <= max_K
+ * hq_reserve_workspace(stream, max_K, max_N) makes sure of (hq_aqlm_matvec's part, 32 bytes a row, included) - at least the need of every call with K <= max_K
  * and N <= max_N, whatever the batch.  Counterpart of the compute-unit query that sizes the launch in
  * src/quantAQLM-hip/main.cu:108-121. */
 int hq_q3_workspace_need(int compute_units, int K, int N, int batch_M, int64_t* floats, int64_t* counters);
@@ -240,9 +240,10 @@ int hq_lut_gemv_plan(const uint32_t* bW, const void* alpha_fp16, const void* q_b
  * with m < codebook_a_sizes[j] (4 where there is none).  scales_fp16 may be NULL (the reference kernel
  * applies no scale).  K % 64 == 0 (as in the reference).  fp32 accumulation, one rounding.  Replaces
  * code1x16_matvec, src/quantAQLM-hip/main.cu:103-139 (without its internal
- * synchronisation, timing and printing).  Calls of several million codes leave partial sums in the stream's workspace (eight
- * floats a row; hq_reserve_workspace with max_N >= M makes room); under stream capture, or where there is no room and none can be
- * had, they run on the kernel that needs none.
+ * synchronisation, timing and printing).  Calls of several million codes leave partial sums in memory of their stream that no
+ * other operator and no graph uses (eight floats a row; hq_reserve_workspace with max_N >= M makes room); under stream capture, or
+ * where there is no room and none can be had, they run on the kernel that needs none, whose sums are added in another order: captured
+ * and eager results are equal to rounding.
  */
 int hq_aqlm_matvec(const int16_t* codes, const void* codebooks_fp16, const void* scales_fp16,
                    const void* x_fp16, void* y_fp16, int M, int K,

@@ -116,6 +116,62 @@ def test_default_takes_slices_but_not_under_capture(hq, tunable):
         assert torch.equal(call(), y)
 
 
+def _many_codes(seed, M=8192, K=4096):
+    import torch
+    codes, cb, scales, x = oa.make_aqlm_problem(seed, M, K)
+    t = [torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0") for a in (codes, cb, scales, x)]
+    y = torch.zeros(M, dtype=torch.float16, device="cuda:0")
+    sizes = (ctypes.c_int * 4)(M, M, M, M)
+    vp = lambda a: ctypes.c_void_p(a.data_ptr())
+
+    def call(stream):
+        from hecbench_amd import _lib
+        assert _lib.load().hq_aqlm_matvec(vp(t[0]), vp(t[1]), vp(t[2]), vp(t[3]), vp(y), M, K, sizes, 65536, ctypes.c_void_p(stream)) == 0
+        return y
+    return call
+
+
+def test_slices_beside_replays_of_the_same_stream(hq, tunable):
+    """A graph with a divided K captured on a stream, replayed on another one beside eager calls in slices on the first: neither
+    touches what the other leaves in memory.  The same with calls of this operator in the graph."""
+    import torch
+    torch.cuda.synchronize()
+    call = _many_codes(12)
+    K, N = 8192, 28672
+    mat = torch.randint(-2 ** 31, 2 ** 31 - 1, (3 * K // 32, N), dtype=torch.int32, device="cuda:0")
+    s = torch.full((N,), 0.01, device="cuda:0")
+    x = torch.randn(K, device="cuda:0")
+    captured, other = torch.cuda.Stream(), torch.cuda.Stream()
+    want_q3 = hq.q3_matvec(x, mat, s, 4 * s)
+    with torch.cuda.stream(captured):
+        captured.wait_stream(torch.cuda.default_stream())
+        hq.q3_matvec(x, mat, s, 4 * s)
+        y = call(captured.cuda_stream)
+    torch.cuda.synchronize()
+    want, outs = y.clone(), [torch.zeros_like(want_q3) for _ in range(8)]
+    beside = _many_codes(13)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        for o in outs:
+            hq.q3_matvec(x, mat, s, 4 * s, out=o)
+            y_beside = beside(captured.cuda_stream)
+    with torch.cuda.stream(other):
+        graph.replay()
+    torch.cuda.synchronize()
+    want_beside = y_beside.clone()
+    assert not torch.equal(want, want_beside)
+    for rep in range(30):
+        with torch.cuda.stream(other):
+            graph.replay()
+        got = []
+        with torch.cuda.stream(captured):
+            for _ in range(8):
+                got.append(call(captured.cuda_stream).clone())
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want_q3) for o in outs) and torch.equal(y_beside, want_beside), rep
+        assert all(torch.equal(g, want) for g in got), rep
+
+
 def test_three_codebooks_and_no_scale(hq, oracle):
     """Reference default geometry: 3 code books of 4096 rows each, no scale."""
     M, K = 12288, 1024
