@@ -98,16 +98,40 @@ int hq_current_device(const HqDevice** out) {
 }
 
 namespace {
-// Device memory that is zero when this returns: nothing of it is left to a stream, so a graph that was captured on one stream and is
-// replayed on another finds it zero whatever its own stream has still to do.
-hipError_t alloc_zeroed(void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
+// Device memory that is zero when this returns: nothing of it is left to a caller's stream, so a graph that was captured on one stream and
+// is replayed on another finds it zero whatever its own stream has still to do.  Cleared on a stream of the library's own: the
+// default stream may not be touched while another is being captured.
+std::map<int, hipStream_t> g_fill;  // per device
+hipError_t alloc_zeroed(int dev, void** p, size_t bytes) {
+  hipStream_t& fill = g_fill[dev];
+  hipError_t e = fill ? hipSuccess : hipStreamCreateWithFlags(&fill, hipStreamNonBlocking);
+  if (e != hipSuccess) {
+    fill = nullptr;
+    return e;
+  }
+  e = hipMalloc(p, bytes);
   if (e != hipSuccess) return e;
-  e = hipMemset(*p, 0, bytes);
-  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+  e = hipMemsetAsync(*p, 0, bytes, fill);
+  if (e == hipSuccess) e = hipStreamSynchronize(fill);
   if (e != hipSuccess) (void)hipFree(*p);
   return e;
 }
+// Around the allocations of a call on a stream that is not being captured: they do not make a capture invalid that another stream is
+// in the middle of.  (On a stream that is, an allocation stays the error that it is.)
+struct BesideCaptures {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool exchanged = false;
+  explicit BesideCaptures(hipStream_t stream) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone)
+      exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    else
+      (void)hipGetLastError();
+  }
+  ~BesideCaptures() {
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
 }  // namespace
 
 int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counters, HqWorkspace* out, size_t want_slots,
@@ -122,6 +146,7 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
     while (n < need_floats) n *= 2;
     if (reserve) n = need_floats;
     float* p = nullptr;
+    const BesideCaptures beside(stream);
     HQ_HIP_TRY(hipMalloc((void**)&p, n * sizeof(float)));
     // kernels in flight may still read the previous buffer: it is kept until hq_shutdown()
     if (ws.partial) g_retired.push_back(std::make_pair(dev, (void*)ws.partial));
@@ -141,7 +166,8 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
     while (n < want) n *= 2;
     if (reserve) n = want > (size_t)1 << 14 ? want : (size_t)1 << 14;
     unsigned* c = nullptr;
-    const hipError_t e = alloc_zeroed((void**)&c, n * sizeof(unsigned));
+    const BesideCaptures beside(stream);
+    const hipError_t e = alloc_zeroed(dev, (void**)&c, n * sizeof(unsigned));
     if (e == hipSuccess) {
       if (ws.counters) g_retired.push_back(std::make_pair(dev, (void*)ws.counters));
       ws.counters = c;
@@ -167,6 +193,7 @@ int hq_get_eager_workspace(hipStream_t stream, size_t need_floats, size_t need_c
     const size_t c = std::max(need_counters, ws.ncounters);
     // one buffer, the counters in front; cleared in front of every call that can use them.
     unsigned* p = nullptr;
+    const BesideCaptures beside(stream);
     hipError_t e = hipMalloc((void**)&p, (c + n) * sizeof(unsigned));
     if (e == hipSuccess && (e = hipMemsetAsync(p, 0, c * sizeof(unsigned), stream)) != hipSuccess) (void)hipFree(p);
     if (e != hipSuccess) {
@@ -295,6 +322,12 @@ extern "C" int hq_shutdown(void) {
     release(kv.first.first, kv.second.partial);
     release(kv.first.first, kv.second.counters);
   }
+  for (auto& kv : g_fill) {
+    hipError_t e = kv.second ? hipSetDevice(kv.first) : hipSuccess;
+    if (e == hipSuccess && kv.second) e = hipStreamDestroy(kv.second);
+    if (e != hipSuccess && rc == HQ_OK) rc = (int)e;
+  }
+  g_fill.clear();
   for (auto& kv : g_eager) release(kv.first.first, kv.second.counters);
   for (auto& r : g_retired) release(r.first, r.second);
   g_workspaces.clear();

@@ -172,6 +172,30 @@ def test_slices_beside_replays_of_the_same_stream(hq, tunable):
         assert all(torch.equal(g, want) for g in got), rep
 
 
+def test_the_first_call_in_slices_beside_a_capture(hq):
+    """A stream's first call of millions of codes, while another stream is being captured: it runs, and the capture is whole."""
+    import torch
+    from hecbench_amd import _lib
+    call, inside = _many_codes(14), _many_codes(15)
+    call(0), inside(0)
+    torch.cuda.synchronize()
+    assert _lib.load().hq_shutdown() == 0
+    want, want_inside = call(0).clone(), inside(0).clone()
+    captured, eager = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        y = inside(captured.cuda_stream)
+        got = call(eager.cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_err(y.cpu().numpy(), want_inside.cpu().numpy().astype(np.float64), FLOOR_F16) <= 2e-3
+
+
 def test_three_codebooks_and_no_scale(hq, oracle):
     """Reference default geometry: 3 code books of 4096 rows each, no scale."""
     M, K = 12288, 1024
