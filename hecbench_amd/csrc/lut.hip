@@ -695,10 +695,13 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
   if (fine) nsplit = parts;
   else if (apart) nsplit = rounds;
   if (nsplit > 1 && hq_workspace_out_of_reach(stream, (size_t)ntiles * nsplit * 64, (size_t)ntiles)) {
-    // A workgroup walks all of K, in rounds of as many quads as there are registers for (one quad a round / this, under capture, us: 8192 x
-    // 128 group 64 15.1 / 11.3, 4096 x 4096 7.3 / 5.5, 4224 x 5562 four planes 8.9 / 7.8, 3072 x 1776 6.0 / 5.4; 2432 x 25507 group 32 15.1 / 16.2).
+    // A workgroup walks all of K.  Under capture, us, one quad a round / as many as there are registers for: 8192 x 128 group 64 15.2 /
+    // 11.3, 4096 x 4096 8.2 / 6.1, 4224 x 5562 four planes 10.1 / 8.8, 8704 x 24420 two planes group 32 23.2 / 19.0.  In small groups,
+    // one where it was chosen and more would leave half of a round's registers empty (1280 x 10413 5.1 / 5.9), and, with three planes or
+    // more, where more than one tile per compute unit is walked in few rounds (2432 x 25507 four planes 15.6 / 17.2, 2432 x 20485 15.1 /
+    // 16.6; not 4736 x 24052 two planes 14.1 / 12.4) or in a few more that are even (6656 x 18823 22.5 / 23.9; not 12800 x 17707 38.0 / 37.2).
     nsplit = 1;
-    fine = false;
+    fine = fine && GROUPED && (2 * parts <= QUADS || (NB >= 3 && ntiles > cus && rpw > 1 && (parts <= 5 || (apart && parts <= 8))));
   }
   return fine ? launch_bcq_planes<NB, 1, GROUPED>(a, ragged, nsplit, stream)
               : launch_bcq_planes<NB, QUADS, GROUPED>(a, ragged, nsplit, stream);

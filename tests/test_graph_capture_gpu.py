@@ -252,3 +252,26 @@ def test_the_first_divided_call_beside_a_capture(hq, shape):
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(scaled, want * 2)
+
+
+@pytest.mark.parametrize("shape", [(1280, 700, 3, 64), (2048, 100, 2, 32), (2432, 20485, 4, 32), (4736, 17000, 3, 64), (6656, 16500, 3, 32), (8192, 128, 3, 64)])
+def test_lut_under_capture_without_any_workspace(hq, shape):
+    """All of K in one workgroup, in rounds of one quad (the first five) or of several: equal to the eager call but for the order of the sum."""
+    import torch
+    from hecbench_amd import _lib
+    from tests.tol import FLOOR_F16, rel_err
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(shape[1])
+    data = _lut(*shape, g)
+    want = hq.lut_matmul(*data).cpu().numpy().astype(np.float64)
+    torch.cuda.synchronize()
+    assert _lib.load().hq_shutdown() == 0  # torch hands streams out again: none has a workspace from here on
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        out = hq.lut_matmul(*data)
+    for rep in range(3):
+        out.fill_(float(rep))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_err(out.cpu().numpy(), want, FLOOR_F16) <= 2e-3, rep
