@@ -98,11 +98,11 @@ int hq_current_device(const HqDevice** out) {
 }
 
 namespace {
-// Device memory that is zero when this returns: nothing of it is left to a caller's stream, so a graph that was captured on one stream and
+// Device memory whose first `zero` bytes are zero when this returns: nothing of it is left to a caller's stream, so a graph that was captured on one stream and
 // is replayed on another finds it zero whatever its own stream has still to do.  Cleared on a stream of the library's own: the
 // default stream may not be touched while another is being captured.
 std::map<int, hipStream_t> g_fill;  // per device
-hipError_t alloc_zeroed(int dev, void** p, size_t bytes) {
+hipError_t alloc_zeroed(int dev, void** p, size_t bytes, size_t zero) {
   hipStream_t& fill = g_fill[dev];
   hipError_t e = fill ? hipSuccess : hipStreamCreateWithFlags(&fill, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -111,7 +111,7 @@ hipError_t alloc_zeroed(int dev, void** p, size_t bytes) {
   }
   e = hipMalloc(p, bytes);
   if (e != hipSuccess) return e;
-  e = hipMemsetAsync(*p, 0, bytes, fill);
+  e = hipMemsetAsync(*p, 0, zero, fill);
   if (e == hipSuccess) e = hipStreamSynchronize(fill);
   if (e != hipSuccess) (void)hipFree(*p);
   return e;
@@ -167,7 +167,7 @@ int hq_get_workspace(hipStream_t stream, size_t need_floats, size_t need_counter
     if (reserve) n = want > (size_t)1 << 14 ? want : (size_t)1 << 14;
     unsigned* c = nullptr;
     const BesideCaptures beside(stream);
-    const hipError_t e = alloc_zeroed(dev, (void**)&c, n * sizeof(unsigned));
+    const hipError_t e = alloc_zeroed(dev, (void**)&c, n * sizeof(unsigned), n * sizeof(unsigned));
     if (e == hipSuccess) {
       if (ws.counters) g_retired.push_back(std::make_pair(dev, (void*)ws.counters));
       ws.counters = c;
@@ -191,11 +191,11 @@ int hq_get_eager_workspace(hipStream_t stream, size_t need_floats, size_t need_c
     while (n < need_floats) n *= 2;
     if (reserve) n = std::max(need_floats, ws.partial_floats);
     const size_t c = std::max(need_counters, ws.ncounters);
-    // one buffer, the counters in front; cleared in front of every call that can use them.
+    // one buffer, the counters in front; not cleared on the stream, which may be in the middle of a capture where one allows
+    // allocations: a reservation's memset would wait for a replay
     unsigned* p = nullptr;
     const BesideCaptures beside(stream);
-    hipError_t e = hipMalloc((void**)&p, (c + n) * sizeof(unsigned));
-    if (e == hipSuccess && (e = hipMemsetAsync(p, 0, c * sizeof(unsigned), stream)) != hipSuccess) (void)hipFree(p);
+    const hipError_t e = alloc_zeroed(dev, (void**)&p, (c + n) * sizeof(unsigned), c * sizeof(unsigned));
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return (int)e;

@@ -196,6 +196,39 @@ def test_the_first_call_in_slices_beside_a_capture(hq):
         assert rel_err(y.cpu().numpy(), want_inside.cpu().numpy().astype(np.float64), FLOOR_F16) <= 2e-3
 
 
+def test_a_reservation_inside_a_relaxed_capture(hq):
+    """Where a capture allows allocations, a reservation of the captured stream is no part of the graph: the stream's eager calls
+    find their counters at zero although nothing is ever replayed."""
+    import torch
+    from hecbench_amd import _lib
+    lib = _lib.load()
+    call = _many_codes(16)
+    call(0)
+    torch.cuda.synchronize()
+    assert lib.hq_shutdown() == 0  # torch hands streams out again: none has a workspace from here on
+    want = call(0).clone()
+    torch.cuda.synchronize()
+    used = []
+    for n in (1 << 16, 1 << 18, 1 << 20, 1 << 21) * 8:  # what the reservation is likely to be given: not zero
+        p = ctypes.c_void_p()
+        assert lib.hipMalloc(ctypes.byref(p), ctypes.c_size_t(n)) == 0 and lib.hipMemset(p, 0xff, ctypes.c_size_t(n)) == 0
+        used.append(p)
+    torch.cuda.synchronize()
+    for p in used:
+        assert lib.hipFree(p) == 0
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+        want + 1
+        assert lib.hq_reserve_workspace(ctypes.c_void_p(stream.cuda_stream), 4096, 8192) == 0
+    torch.cuda.synchronize()
+    for _ in range(3):
+        got = call(0).zero_()
+        torch.cuda.synchronize()
+        call(stream.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
 def test_three_codebooks_and_no_scale(hq, oracle):
     """Reference default geometry: 3 code books of 4096 rows each, no scale."""
     M, K = 12288, 1024
