@@ -636,21 +636,25 @@ int launch_bcq_planes(LutArgs a, bool ragged, int nsplit, hipStream_t stream) {
 
 // Split of K over workgroups.  Ordinary: rounds of QUADS quads (128 elements of K) per wave, and as many workgroups as there
 // are compute units to take them (K=11008, N=4096, three planes: 64 tiles x 3 rounds).  Fine: one quad per wave, one round per
-// workgroup, all rounds side by side.  Groups of 128 and more, from 180 drawn problems timed both ways (MI355X; the choice costs 0.6 %
-// on average against the better one, 10 % at most): a quad takes a wave 0.11 us per plane, the exchange of a split 0.3 us and 0.1 more
-// for every part, workgroups beyond one per compute unit 0.9, and more than eight parts, which meet through a count, 1.0.  Fine
-// splits are taken where they save more than they cost and all workgroups are on the device at once, two per compute unit (us,
+// workgroup, all rounds side by side.  Groups of 128 and more, from problems drawn and timed both ways (MI355X; over 1239 of them the
+// choice costs 0.6 % on average against the better one): a quad takes a wave 0.11 us per plane, the exchange of a split 0.3 us and 0.1
+// more for every part, workgroups beyond one per compute unit 0.9, and more than eight parts, which meet through a count, 2.0 where they
+// fill the compute units and ever less where they are few, down to a gain of 1.0 (8320 x 384 three planes 6.4 / 5.4, 8704 x 256 six
+// planes 7.0 / 5.8; not 11392 x 1778 two planes 5.6 / 7.1).  Fine splits are taken where they save more than they cost and all
+// workgroups are on the device at once, two per compute unit (us,
 // ordinary / fine: 3072 x 1776 three planes 5.35 / 4.45; 3968 x 1911 5.3 / 4.6; 4352 x 622 two planes 5.9 / 4.9; not 3200 x 6705
 // 5.5 / 6.0, 13184 x 1025 7.2 / 7.7), and where several rounds of few more tiles than compute units would leave most of those idle
 // behind the first tile (5120 x 20480 14.2 / 13.0; not 4096 x 28672 four planes 15.6 / 16.6).
-// Groups of 64 and 32 take twice the arithmetic, and an even share of it counts more: both ways are estimated (grouped_us; 140
-// problems, spread 5 and 8 %, the choice costs 1.3 % on average): 2432 x 25507 four planes 17.6 / 12.3; 4736 x 23517 two planes 17.2 /
-// 13.1; 5760 x 9363 four planes 16.2 / 12.2; 7552 x 10028 18.2 / 14.1; not 8448 x 7872 three planes 10.25 / 11.7, 15872 x 22799 40.7 / 42.4.
-// quads: a wave's in a row, in the average over the compute units where they are even.
-inline float grouped_us(bool fine, float quads, int NB, float stream_us, int parts) {
-  if (!fine) return 3.1f + 0.276f * quads * NB + 0.54f * stream_us + (parts > 1 ? 0.72f : 0.f);
-  const int trips = parts > 8 ? 0 : (parts > 4 ? 3 : (parts > 2 ? 2 : (parts > 1 ? 1 : 0)));
-  return 2.9f + 0.2f * quads * NB + 0.68f * stream_us + 0.56f * trips + (parts > 8 ? 2.7f : 0.f);
+// Groups of 64 and 32 take twice the arithmetic, and an even share of it counts more: both ways are estimated (grouped_us), fitted to 1466
+// drawn problems of up to six planes timed both ways; over 1763 others the choice costs 0.5 % on average against the better one (2432 x
+// 25507 four planes 17.4 / 12.7; 13312 x 192 five planes 7.85 / 6.35; 5888 x 5562 four planes 10.4 / 9.1; 17664 x 1814 six planes 15.3 / 12.3;
+// not 4480 x 26432 group 64 two planes 9.8 / 12.0, 14208 x 10688 two planes 14.4 / 15.9).
+// quads: a wave's in a row, in the average over the compute units where they are even; busy: compute units with work, of one.
+inline float grouped_us(bool fine, float quads, int NB, float stream_us, int parts, bool apart, float busy) {
+  const float trips = parts > 4 ? 3.f : (parts > 2 ? 2.f : (parts > 1 ? 1.f : 0.f));
+  const float meet = parts > 8 ? 1.8f + busy : 0.41f * trips;
+  if (!fine) return 3.2f + quads * (0.28f * NB - 0.15f) + 0.5f * stream_us + (apart ? 1.f : 0.f) + meet;
+  return 2.55f + quads * (0.29f * NB + 0.24f) + 0.25f * stream_us + 0.5f * busy + meet;
 }
 template <int NB, bool GROUPED>
 int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t stream) {
@@ -663,9 +667,11 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
   const int rpw = (rounds + nsplit - 1) / nsplit;
   bool fine = false, apart = false;
   if (QUADS > 1) {
+    auto busy = [&](int shares) { return (int64_t)ntiles * shares < cus ? (float)(ntiles * shares) / cus : 1.f; };
     const float saves = 0.11f * NB * (rpw * QUADS - 1);
     const float costs = parts == 1 ? 0.f : (nsplit == 1 ? 0.3f : 0.f) + 0.1f * (parts - nsplit) +
-                                               (ntiles * (int64_t)parts > cus ? 0.9f : 0.f) + (parts > 8 ? 1.f : 0.f);
+                                               (ntiles * (int64_t)parts > cus ? 0.9f : 0.f) +
+                                               (parts > 8 ? 3.f * busy(parts) - 1.f : 0.f);
     fine = (int64_t)ntiles * parts <= 2 * cus && saves > costs;
     if (ntiles > cus && ntiles * 8 <= cus * 11 && rpw > 1 && parts <= 5) fine = true;
     // Several rounds per workgroup, and the exchange paid for anyway (nsplit > 1) or a last wave of tiles that would leave more
@@ -682,13 +688,12 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
       const float planes = (float)a.K * (float)a.N * NB / 8.f;
       const float stream_us = planes * (1.f + 16.f / a.G * (1.f + 1.f / NB)) / 6e6f;
       const float even = (float)ntiles / cus;
-      const int quads1 = (nquads + 7) / 8;  // of a wave, in one round of all
-      float ordinary;
+      const int shares = apart ? rounds : (rounds + rpw - 1) / rpw;
+      float ordinary;  // (a wave has no more quads in a row than K holds: a last round may be nearly empty)
       if (apart) ordinary = (even * rounds > 1.f ? even * rounds : 1.f) * (QUADS < nquads / 8.f ? QUADS : nquads / 8.f);
-      else if (rounds > 1) ordinary = (float)((ntiles * nsplit + cus - 1) / cus) * rpw * QUADS;
-      else ordinary = (float)waves_of_tiles * (QUADS < quads1 ? QUADS : quads1);
-      fine = grouped_us(true, even * parts > 1.f ? even * parts : 1.f, NB, stream_us, parts) <
-             grouped_us(false, ordinary, NB, stream_us, apart ? rounds : nsplit);
+      else ordinary = (float)((ntiles * shares + cus - 1) / cus) * (rpw * QUADS < parts ? rpw * QUADS : parts);
+      fine = grouped_us(true, even * parts > 1.f ? even * parts : 1.f, NB, stream_us, parts, false, busy(parts)) <
+             grouped_us(false, ordinary, NB, stream_us, shares, apart, busy(shares));
     }
     fine = hq_tune(HQ_TUNE_LUT_FINE, fine) != 0;
   }
