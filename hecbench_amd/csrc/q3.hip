@@ -564,12 +564,16 @@ int q3_block_row_blocks(int cus, int K, int N, int batch_M, int nsplit, int rpw)
 // 5 rows, K=4096, N=11008 7.5 / 8.7, K=8192, N=8192 9.9 / 11.5, K=2816, N=12736 6.85 / 7.5, K=5184, N=5008 8.8 / 8.9, K=4480, N=4516 8.9 / 8.4; 6
 // rows 4096 x 11008 8.0 / 8.7, 6048 x 6824 9.65 / 9.8, 2272 x 15704 7.4 / 7.2, 5440 x 5372 9.4 / 8.8; 8 rows 8192 x 8192 10.5 / 11.5, 7680 x
 // 6328 10.1 / 11.6, 4096 x 11008 8.55 / 8.7, 6048 x 6824 9.7 / 9.8, 8608 x 4376 10.2 / 9.6).  Of 7e7
-// weights and more, which are more workgroups than compute units, K up to 16384 yields too (133 drawn problems, theirs / one launch:
-// 7 rows 4960 x 24904 22.0 / 14.1, 8 rows 4160 x 19972 19.5 / 12.7, 7136 x 11060 14.8 / 12.0, 13728 x 10872 21.0 / 16.4, 6 rows 4160 x
-// 26824 20.9 / 13.1, 5 rows 5120 x 13824 12.1 / 9.6) but for up to a fifth more workgroups than compute units (8 rows 3808 x 18680 11.8 /
-// 12.5, 7520 x 9588 12.5 / 12.9) and five and six rows of a K of 11000 and more in up to three rounds of workgroups, the last at least half
-// full (5 rows 12128 x 15584 18.0 / 21.2, 6 rows 15936 x 12176 20.4 / 22.2): 1.10 in the geometric mean, the choice
-// costs 0.4 % on average against the better way.  A longer K stays (8 rows 28672 x 8192 26.8 / 28.0).
+// weights and more, which are more workgroups than compute units, K up to 16384 yields too (1113 drawn problems, weights from memory,
+// theirs / one launch: 7 rows 4960 x 24904 21.6 / 15.9, 8 rows 4160 x 19972 19.1 / 14.0, 7136 x 11060 15.2 / 12.8, 13728 x 10872 21.3 /
+// 20.2, 6 rows 4160 x 26824 21.2 / 14.6, 5 rows 5120 x 13824 11.8 / 10.5) but for
+//  - up to a fifth more workgroups than compute units, half as many again where K is less than a round (8 rows 3808 x 18680 11.8 / 12.5, 7520 x
+//    9588 12.5 / 12.9; 3680 x 19904 11.4 / 13.8, 3264 x 24080 11.5 / 12.3),
+//  - five rows of K from 7000 on in rounds of workgroups of which the last is three fifths full, or in up to three rounds with a last range of
+//    K that is nearly whole (10368 x 10116 14.6 / 17.2, 15872 x 15488 24.6 / 27.6, 7968 x 21376 19.3 / 22.0), and
+//  - five and six rows of a K of 11000 and more in up to three rounds of workgroups, the last at least half full (5 rows 12128 x 15584 18.0 /
+//    21.2, 6 rows 15936 x 12176 20.8 / 24.3).
+// 1.063 in the geometric mean; the choice costs 0.4 % on average against the better way.  A longer K stays (8 rows 28672 x 8192 26.8 / 28.0).
 bool q3_block_yields(int cus, int K, int N, int batch_M) {
   if (!hq_q3_direct_can(K, N)) return false;
   if (hq_q3_direct_forced()) return true;
@@ -580,10 +584,11 @@ bool q3_block_yields(int cus, int K, int N, int batch_M) {
   if (batch_M <= 8 && groups <= cus && weights >= (batch_M <= 6 ? 35000000 : 40000000)) return false;
   if (batch_M <= 8 && weights >= 70000000) {
     const int64_t rounds = (groups + cus - 1) / cus;
-    const int tail = K % 4096;  // a last range of K that is nearly empty costs nothing
-    const int64_t busy = groups - (nsplit > 1 && tail > 0 && tail < 512 ? (N + 63) / 64 : 0);
-    if (K > 16384 || 5 * busy <= 6 * cus || (batch_M <= 6 && K >= 11000 && rounds <= 3 && 2 * groups >= (2 * rounds - 1) * cus))
-      return false;
+    const int last = (K - 1) % 4096 + 1;  // a last range of K that is nearly empty costs nothing
+    const int64_t busy = groups - (nsplit > 1 && last < 512 ? (N + 63) / 64 : 0);
+    if (K > 16384 || 5 * busy <= 6 * cus || (K < 4096 && 2 * groups <= 3 * cus)) return false;
+    if (batch_M == 5 && K >= 7000 && (5 * groups >= (5 * rounds - 2) * cus || (last >= 3072 && rounds <= 3))) return false;
+    if (batch_M <= 6 && K >= 11000 && rounds <= 3 && 2 * groups >= (2 * rounds - 1) * cus) return false;
   }
   return groups * ((batch_M + 3) / 4) > cus;
 }

@@ -155,7 +155,8 @@ int hq_quantize_dynamic8(const float* code, const float* A, uint8_t* out, int64_
  *     blocks of four, one workgroup per column tile, 4096 elements of K and row block, while every workgroup has a compute unit of
  *     its own (beyond K = 32768: 5 ... 12 rows as two or three passes of one workgroup, by the same count); and 5 ... 8 rows of
  *     large matrices (3.5e7 weights, 7 and 8 rows 4e7) as two passes or row blocks, while four rows would have a compute unit for every
- *     workgroup, or nearly so, or K is beyond 16384 (five and six rows: beyond 11000, where that fills the compute units evenly),
+ *     workgroup, or nearly so, or K is beyond 16384 (five and six rows: beyond 11000, five rows from 7000 on, where that fills the compute units
+ *     evenly),
  *     unless N / 128 is at least 7/8 of the compute units.  Every activation enters with an
  *     error of at most 2^-19 of the largest magnitude among its 32 neighbours (exactly, if within 2^8 of it);
  *   - the matrix cores in one launch: all other batches of up to 32 rows, 33 to 64 rows of less than 9e7 weights (2.5e8, if K <

@@ -50,3 +50,13 @@ def test_five_to_eight_rows_in_more_workgroups_than_compute_units(M, K, N, kerne
     range of K that is nearly empty counts for nothing), five and six rows of K >= 11000 in evenly filled rounds, K beyond 16384."""
     choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
     assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(8, 3680, 19904, "block"), (8, 4064, 24576, "block"), (8, 4064, 24580, "direct"), (5, 10368, 10116, "block"),
+                                          (5, 15872, 15488, "block"), (5, 7968, 21376, "block"), (5, 6976, 21376, "direct"),
+                                          (5, 7968, 25000, "direct"), (6, 7968, 21376, "direct")])
+def test_more_workgroups_than_compute_units_that_stay(M, K, N, kernel):
+    """On either side of each line: a K of less than a round in up to half as many workgroups again; five rows of K >= 7000 in evenly
+    filled rounds, or in up to three with a last range of K that is nearly whole."""
+    choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
+    assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel
