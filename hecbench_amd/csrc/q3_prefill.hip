@@ -390,33 +390,41 @@ TilePlan tile_plan_of(int cus, int K, int N, int M, const TileKind& kind, int wa
   return p;
 }
 
-// The same with the column tiles beyond the last full round left to the one-launch kernel, in a launch of its own behind this one,
-// where that is less by the two estimates; otherwise the plan as it is.  Dividing a few tiles along K costs most of a round whatever
-// their number (shares of 128 x 256 sums go out to memory and come back): 1024 rows, K=2048, 33 column tiles of 256, the 33rd
-// divided 59.3 us, as 32 x 64 tiles of the one-launch kernel 44.7.  1271 rows, K=2048, N=26476 (four rounds and 16 tiles) 159 -> 147;
-// 1902, K=1056, N=13184 89 -> 77.6; 1580, K=1504, N=25548 162 -> 150; 290, K=6272, N=14240 64.3 -> 58.4; 1595, K=1600, N=21980 (94
-// tiles) 148 -> 144.  From two fifths of a round on nothing is gained (1975, K=1632, N=10760, 176 tiles: 92.0 / 99.4), and with the
-// smallest tile never.
-TilePlan cut_plan(int cus, int K, int N, int M, const TileKind& kind, const TilePlan& whole, bool forced) {
+// The same with the column tiles beyond the last full round left to the one-launch kernel, in a launch of its own behind this one.
+// Dividing a few tiles along K costs most of a round whatever their number (shares of 128 x 256 sums go out to memory and come back):
+// 1024 rows, K=2048, 33 column tiles of 256, the 33rd divided 50.7 us, as 32 x 64 tiles of the one-launch kernel 44.2.  1271 rows, K=2048,
+// N=26476 (four rounds and 16 tiles) 155 -> 143; 1902, K=1056, N=13184 85 -> 74; 1580, K=1504, N=25548 156 -> 146; 290, K=6272, N=14240 66 ->
+// 60.6.  From two fifths of a round on nothing is gained (1975, K=1632, N=10760, 176 tiles: 92.0 / 99.4), and with the smallest tile never.
+// Without such columns the plan as it is.
+TilePlan cut_plan(int cus, int K, int N, int M, const TileKind& kind, bool forced) {
+  const TilePlan whole = tile_plan_of(cus, K, N, M, kind, 0);
   const int cols = whole.rounds * whole.nwg / whole.nmt;
-  if (!forced && (5 * whole.rest > 2 * whole.nwg || kind.ks != 2)) return whole;
-  if (whole.rounds < 1 || cols < 1 || cols * kind.tn >= N || !hq_q3_direct_can(K, N)) return whole;
+  if ((!forced && (5 * whole.rest > 2 * whole.nwg || kind.ks != 2)) || whole.rounds < 1 || cols < 1 || cols * kind.tn >= N ||
+      !hq_q3_direct_can(K, N))
+    return whole;
   TilePlan p = tile_plan_of(cus, K, cols * kind.tn, M, kind, 0);
   p.direct = hq_q3_direct_plan(cus, K, N - p.cut, M, false);
   p.us += p.direct.us;
-  return forced || p.us < whole.us ? p : whole;
+  return p;
 }
 
+// The least of the estimates; columns are cut off where that is less by 7 us, which the second launch takes beside its own estimate (it
+// begins when the last tile has gone out), or by 1 where the call is longer than 36 us and the tile the large one, whose rounds then take
+// more than theirs.  452 drawn problems for which the estimates alone are for the cut: 1.037 times as fast in the geometric mean as without any
+// (all of them cut 1.032), 14 more than 3 % slower than without (76; 263 rows, 2240 x 13548 27.1 / 33.2, 1848 rows, 288 x 9420 40.6 / 49.5).
 TilePlan tile_plan(int cus, int K, int N, int M) {
   const int force = hq_tune(HQ_TUNE_Q3_TILES, -1);  // tests: kind + 10 * shares (3 to 6 the one-launch kernel's, 9 none in particular; 100 + kind: cut)
-  if (force >= 100 && force < 103) return cut_plan(cus, K, N, M, kKinds[force - 100], tile_plan_of(cus, K, N, M, kKinds[force - 100], 0), true);
+  if (force >= 100 && force < 103) return cut_plan(cus, K, N, M, kKinds[force - 100], true);
   if (force >= 0 && force % 10 < 3) return tile_plan_of(cus, K, N, M, kKinds[force % 10], force / 10);
-  TilePlan best = tile_plan_of(cus, K, N, M, kKinds[0], 0);
-  best = cut_plan(cus, K, N, M, kKinds[0], best, false);
+  TilePlan whole = tile_plan_of(cus, K, N, M, kKinds[0], 0);
   for (int i = 1; i < 3; ++i) {
-    TilePlan p = tile_plan_of(cus, K, N, M, kKinds[i], 0);
-    p = cut_plan(cus, K, N, M, kKinds[i], p, false);
-    if (p.us < best.us) best = p;
+    const TilePlan p = tile_plan_of(cus, K, N, M, kKinds[i], 0);
+    if (p.us < whole.us) whole = p;
+  }
+  TilePlan best = whole;
+  for (int i = 0; i < 3; ++i) {
+    const TilePlan p = cut_plan(cus, K, N, M, kKinds[i], false);
+    if (p.cut < N && p.us < best.us && p.us < whole.us - (i == 0 && whole.us > 36.f ? 1.f : 7.f)) best = p;
   }
   return best;
 }

@@ -60,3 +60,14 @@ def test_more_workgroups_than_compute_units_that_stay(M, K, N, kernel):
     filled rounds, or in up to three with a last range of K that is nearly whole."""
     choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
     assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel
+
+
+@pytest.mark.parametrize("M,K,N,tiles_us,cut", [(263, 2240, 13548, 28.2, False), (1848, 288, 9420, 21.6, False), (135, 3584, 25704, 42.1, False),
+                                                (1024, 2048, 8448, 45.9, True), (1902, 1056, 13184, 62.4, True), (129, 2304, 23920, 28.2, False)])
+def test_columns_are_cut_off_where_that_gains_more_than_a_launch(M, K, N, tiles_us, cut):
+    """The estimate of a call beside that of whole tiles (tiles_us, and the pre-pass): less by a microsecond and more, or the same."""
+    import ctypes
+    us = getattr(_lib.load(), "_Z14hq_q3_tiles_usiiii")
+    us.restype = ctypes.c_float
+    whole = tiles_us + 3.2 + 0.0002 * K + M * K * 4 / 4.5e6
+    assert (us(256, K, N, M) < whole - 1) if cut else abs(us(256, K, N, M) - whole) < 0.1
