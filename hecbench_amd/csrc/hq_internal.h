@@ -133,7 +133,7 @@ int hq_get_eager_workspace(hipStream_t stream, size_t need_floats, size_t need_c
 // without a workspace then does.
 bool hq_workspace_out_of_reach(hipStream_t stream, size_t need_floats, size_t need_counters);
 // Where the `nsplit` shares of a divided K meet, `floats` partial sums in all: in exchange slots (*arrivals null, *partial the slots,
-// up to kHqMeetMost shares and no formal fences), or through partial sums and arrival counters.  The workspace has room for those
+// up to kHqMeetMost shares and no formal fences), or (nsplit 0: in any case) through partial sums and arrival counters.  The workspace has room for those
 // either way, so a captured call finds what an eager one has left behind, and gives the same bits on both ways.
 int hq_get_split(hipStream_t stream, size_t floats, size_t counters, int nsplit, float** partial, unsigned** arrivals);
 
@@ -280,7 +280,7 @@ __device__ __forceinline__ bool hq_meet(unsigned long long* slots, size_t stride
   return true;
 }
 // Up to eight shares, three trips at most.  3-bit matvec, count / exchange, us: two shares 8192 x 640 5.1 / 4.2, 8192 x 28672 18.1 / 17.2;
-// three 11008 x 4096 6.45 / 6.2; five 20480 x 4096 9.55 / 8.85; eight 32768 x 2048 7.7 / 7.4; ten 39136 x 364 7.0 / 7.3 (four trips: not
+// three 11008 x 4096 6.45 / 6.2; five 20480 x 4096 9.4 / 9.1; eight 32768 x 2048 7.9 / 7.5; ten 39136 x 364 7.0 / 7.3 (four trips: not
 // taken).  Four rows, two shares, 4224 x 2200 6.9 / 6.05.  LUT-GEMM: two shares 8192 x 8192 8.15 / 7.35, three 11008 x 4096 7.8 / 7.1,
 // six 6016 x 2265 (two planes) 5.8 / 5.0, eight 7552 x 2166 (groups of 64) 6.9 / 6.2.
 constexpr int kHqMeetMost = 8;

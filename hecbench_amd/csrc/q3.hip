@@ -626,6 +626,7 @@ struct Q3SplitPlan {
   int nsplit;       // workgroups per column tile
   int ntiles;       // column tiles (times row blocks) = arrival counters
   size_t floats;    // partial sums: 0 without a split
+  int meet;         // shares that meet by exchange: all of them or 0
   bool too_large;   // the fixed scratch cannot hold this plan
 };
 struct Q3Limits {  // what a fixed scratch holds; null pointer = the stream's workspace (grows on demand)
@@ -658,6 +659,11 @@ Q3SplitPlan q3_split_plan(int cus, int G, int gpr, int ntiles, int rows_out, boo
   p.nsplit = (G + p.gpw - 1) / p.gpw;
   p.ntiles = ntiles;
   p.floats = p.nsplit > 1 ? tile_floats * p.nsplit : 0;
+  // Six to eight shares in more than three workgroups per compute unit come one after the other, and the third trip is nothing beside that:
+  // they count (us, exchange / count: eight shares 30432 x 8964 22.2 / 21.0, 32160 x 14336 32.1 / 30.8, three rows 25.5 / 24.5; seven 28064 x
+  // 8964 20.4 / 19.6; six 23968 x 14336 25.0 / 24.6; not eight 32160 x 5632 14.5 / 14.45, six 23968 x 5632 12.3 / 12.8, five 19872 x 14336 20.55 /
+  // 21.05).
+  p.meet = p.nsplit <= 5 || (int64_t)ntiles * p.nsplit <= 3 * cus ? p.nsplit : 0;
   p.too_large = p.nsplit > 1 && fixed && (p.floats > fixed->partial_floats || (size_t)ntiles > fixed->ncounters);
   return p;
 }
@@ -681,7 +687,7 @@ int q3_split_acquire(const Q3SplitPlan& p, const HqQ3Scratch* fixed, hipStream_t
     out->counters = fixed->counters;
     return HQ_OK;
   }
-  return hq_get_split(stream, p.floats, (size_t)p.ntiles, p.nsplit, &out->partial, &out->counters);
+  return hq_get_split(stream, p.floats, (size_t)p.ntiles, p.meet, &out->partial, &out->counters);
 }
 
 // Launch shape of the batch-1 kernel (pure arithmetic).
@@ -764,7 +770,7 @@ int hq_q3_workspace_need_impl(int cus, int K, int N, int batch_M, size_t* floats
   *floats = 0;
   *counters = 0;
   // (as hq_get_split takes them: a few shares meet in slots of two counters)
-  auto counters_of = [](const Q3SplitPlan& p) { return std::max(p.nsplit > 1 ? (size_t)p.ntiles : 0, 2 * hq_split_slots(p.floats, p.nsplit)); };
+  auto counters_of = [](const Q3SplitPlan& p) { return std::max(p.nsplit > 1 ? (size_t)p.ntiles : 0, 2 * hq_split_slots(p.floats, p.meet)); };
   if (batch_M == 1) {
     const Q3MatvecPlan m = q3_matvec_shape(cus, K, N, nullptr);
     *floats = m.split.floats;

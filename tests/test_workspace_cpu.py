@@ -90,7 +90,7 @@ def test_the_case_that_used_to_fall_short():
     assert _bound(lib, 256, 16384, 65536)[0] >= f2
 
 
-@pytest.mark.parametrize("M,K,N,shares,rows", [(1, 8192, 640, 2, 40), (1, 8192, 28672, 2, 448), (1, 28672, 8192, 7, 128), (4, 8192, 8256, 2, 129 * 4),
+@pytest.mark.parametrize("M,K,N,shares,rows", [(1, 8192, 640, 2, 40), (1, 8192, 28672, 2, 448), (1, 28672, 4096, 7, 64), (4, 8192, 8256, 2, 129 * 4),
                                                (7, 8192, 640, 2, 10 * 8)])
 def test_the_slots_of_a_few_shares_are_told(M, K, N, shares, rows):
     """A few shares of K meet in slots, of two counters each: a row of 64 per column tile (16 columns, where they are few), share but
@@ -100,12 +100,18 @@ def test_the_slots_of_a_few_shares_are_told(M, K, N, shares, rows):
     assert f == rows * shares * 64 and c == 2 * rows * (shares - 1) * 64
 
 
+@pytest.mark.parametrize("M,K,N,counters", [(1, 28672, 8192, 128), (3, 32768, 8192, 128), (1, 32768, 6144, 2 * 96 * 7 * 64)])
+def test_many_workgroups_of_many_shares_count(M, K, N, counters):
+    """Six to eight shares in more than three workgroups per compute unit (the last: just not): arrival counters, and no slots."""
+    assert _need(_lib.load(), 256, K, N, M)[1] == counters
+
+
 def test_a_reservation_for_very_many_columns_has_slots_for_fewer():
     """Beyond 32 MiB of slots a call does without; a reservation that would take more holds those 32 MiB."""
     lib = _lib.load()
     assert _bound(lib, 256, 65536, 2000000)[1] == 2 * (4 << 20) + 256 // 8  # (and the arrival counters of AQLM calls in slices)
-    assert _need(lib, 256, 28672, 65536, 1)[1] == 2 * 1024 * 6 * 64
-    assert _need(lib, 256, 28672, 1000000, 1)[1] == 15625  # arrival counters
+    assert _need(lib, 256, 20480, 65536, 1)[1] == 2 * 1024 * 4 * 64
+    assert _need(lib, 256, 20480, 1200000, 1)[1] == 18750  # arrival counters
 
 
 def test_bad_arguments():
