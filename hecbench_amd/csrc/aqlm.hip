@@ -156,11 +156,12 @@ __global__ __launch_bounds__(256) void aqlm_matvec_kernel(HQ_ARGS24) {
 // eighth of the code book fits a compute unit's LDS, so here the workgroups of eight compute units, each with its eighth, go over
 // the same rows: every code is read by all eight (a cached 2 bytes instead of a request of 16) and answered by the one that holds its
 // entry; for the others it points at an entry of zeros.  Their sums meet through memory.  What bounds it now are the vector
-// instructions, six for a code in each of the eight, and the LDS reads under them.
+// instructions, 6.5 for a code in the loop and 7.7 in all, in each of the eight, and the LDS reads under them.
 // The eight of a group of rows run on one XCD, whose L2 reads the group's codes from memory once.
-// Gathers from L2 -> in slices: 8192 x 4096 19.6 -> 15.5 us, 18359 x 3840 37.1 -> 25.4, 28672 x 4096 with three code books 59.5 -> 36.6,
-// 16234 x 10496 88.9 -> 48.6, 28672 x 15872 228 -> 106 (580 G codes/s without the 8 us in front and behind; the vector units 0.8 busy, an
-// LDS read 4.7 cycles of which 0.7 are conflicts).
+// Gathers from L2 -> in slices, weights from memory: 8192 x 4096 19.8 -> 16.1 us, 18359 x 3840 37.7 -> 25.7, 28672 x 4096 with three code
+// books 60.3 -> 36.5, 16234 x 10496 89.2 -> 48.5, 28672 x 15872 228 -> 111 (550 G codes/s without the 8 us in front and behind; the vector
+// units 0.8 busy, an LDS read 4.7 cycles of which 0.7 are conflicts).  That is after a quarter of a second of such calls: the first sixty
+// after idle take 125 to 148, at the clock that the power management begins with; the gathers, bound by the L2, 228 to 240 throughout.
 constexpr int kSlices = 8, kEntries = 65536 / kSlices;
 constexpr int kSlicedThreads = 1024, kSlicedWaves = kSlicedThreads / 64, kSlicedRows = 4;
 constexpr size_t kSlicedBytes = (size_t)(kEntries + 1) * 16;  // a slice and the entry of zeros; behind it the activations
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(kSlicedThreads) void aqlm_sliced_kernel(HQ_ARGS28) 
 // against the better of the two): the gathers' 2.4 us and 242 G codes/s; in slices 8.1 us for the first data, the slice's way into LDS and
 // the meeting of the eight, 1.86 us for a trip of the sixteen waves over one run of lanes and 0.5 beside for its sums, the last
 // trip for its share of waves and a fifth more, 0.6 where there are several code books.  The line lies at 3 to 4.5 M codes: 2001 x 10240
-// and 4096 x 4096 stay (10.3 us against 11.7), 8192 x 4096 19.6 -> 15.5, 28672 x 1024 18.3 -> 15.5.
+// and 4096 x 4096 stay (10.3 us against 11.7), 8192 x 4096 19.8 -> 16.1, 28672 x 1024 18.6 -> 16.6.
 struct SlicedPlan {
   int groups, sub_bits;  // groups 0: not in slices
 };
