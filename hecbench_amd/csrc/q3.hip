@@ -659,11 +659,13 @@ Q3SplitPlan q3_split_plan(int cus, int G, int gpr, int ntiles, int rows_out, boo
   p.nsplit = (G + p.gpw - 1) / p.gpw;
   p.ntiles = ntiles;
   p.floats = p.nsplit > 1 ? tile_floats * p.nsplit : 0;
-  // Six to eight shares in more than three workgroups per compute unit come one after the other, and the third trip is nothing beside that:
-  // they count (us, exchange / count: eight shares 30432 x 8964 22.2 / 21.0, 32160 x 14336 32.1 / 30.8, three rows 25.5 / 24.5; seven 28064 x
-  // 8964 20.4 / 19.6; six 23968 x 14336 25.0 / 24.6; not eight 32160 x 5632 14.5 / 14.45, six 23968 x 5632 12.3 / 12.8, five 19872 x 14336 20.55 /
-  // 21.05).
-  p.meet = p.nsplit <= 5 || (int64_t)ntiles * p.nsplit <= 3 * cus ? p.nsplit : 0;
+  // Six to eight shares in more than two and three quarters workgroups per compute unit come one after the other, and the third trip is
+  // nothing beside that: they count (us, exchange / count: eight shares 30432 x 8964 22.2 / 21.0, 32160 x 14336 32.1 / 30.8, 32768 x 6144 15.2 /
+  // 15.0, two rows 17.1 / 16.2; seven 28064 x 8964 20.4 / 19.6, two rows 28672 x 6976 16.7 / 15.7; six 23968 x 14336 25.0 / 24.6, 24576 x
+  // 8192 15.6 / 15.1, two rows 17.5 / 16.4, four 16.6 / 16.5; not six 24576 x 5632 12.3 / 12.85, two rows 7168 columns 14.9 / 15.15, four
+  // 15.4 / 15.6, seven 28672 x 5632 13.45 / 13.7, two rows 14.25 / 14.7, eight 32768 x 5632 14.3 / 14.2, two rows 15.4 / 15.4, five 19872 x
+  // 14336 20.55 / 21.05).
+  p.meet = p.nsplit <= 5 || (int64_t)ntiles * p.nsplit * 4 <= 11 * cus ? p.nsplit : 0;
   p.too_large = p.nsplit > 1 && fixed && (p.floats > fixed->partial_floats || (size_t)ntiles > fixed->ncounters);
   return p;
 }

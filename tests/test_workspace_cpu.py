@@ -100,9 +100,11 @@ def test_the_slots_of_a_few_shares_are_told(M, K, N, shares, rows):
     assert f == rows * shares * 64 and c == 2 * rows * (shares - 1) * 64
 
 
-@pytest.mark.parametrize("M,K,N,counters", [(1, 28672, 8192, 128), (3, 32768, 8192, 128), (1, 32768, 6144, 2 * 96 * 7 * 64)])
+@pytest.mark.parametrize("M,K,N,counters", [(1, 28672, 8192, 128), (3, 32768, 8192, 128), (2, 24576, 8192, 128), (1, 32768, 5696, 89),
+                                            (1, 32768, 5632, 2 * 88 * 7 * 64)])
 def test_many_workgroups_of_many_shares_count(M, K, N, counters):
-    """Six to eight shares in more than three workgroups per compute unit (the last: just not): arrival counters, and no slots."""
+    """Six to eight shares in more than two and three quarters workgroups per compute unit (the last: just not): arrival counters,
+    and no slots."""
     assert _need(_lib.load(), 256, K, N, M)[1] == counters
 
 
