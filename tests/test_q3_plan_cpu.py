@@ -71,3 +71,11 @@ def test_columns_are_cut_off_where_that_gains_more_than_a_launch(M, K, N, tiles_
     us.restype = ctypes.c_float
     whole = tiles_us + 3.2 + 0.0002 * K + M * K * 4 / 4.5e6
     assert (us(256, K, N, M) < whole - 1) if cut else abs(us(256, K, N, M) - whole) < 0.1
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(576, 1280, 14524, "direct"), (1999, 960, 4492, "direct"), (1179, 1216, 7208, "direct"),
+                                          (1654, 2144, 5056, "tiles"), (324, 2432, 23040, "tiles"), (1992, 768, 16592, "tiles")])
+def test_cut_tiles_beside_the_one_launch_kernel(M, K, N, kernel):
+    """The estimate of tiles with their last columns cut off stands against that of the one-launch kernel for all columns."""
+    choose = getattr(_lib.load(), "_Z18hq_q3_batch_kerneliiii")
+    assert ("block", "direct", "rows64", "tiles")[choose(256, K, N, M)] == kernel
