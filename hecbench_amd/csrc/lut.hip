@@ -692,8 +692,9 @@ int launch_bcq_planes_of(const LutArgs& a, bool ragged, int cus, hipStream_t str
       float ordinary;  // (a wave has no more quads in a row than K holds: a last round may be nearly empty)
       if (apart) ordinary = (even * rounds > 1.f ? even * rounds : 1.f) * (QUADS < nquads / 8.f ? QUADS : nquads / 8.f);
       else ordinary = (float)((ntiles * shares + cus - 1) / cus) * (rpw * QUADS < parts ? rpw * QUADS : parts);
-      fine = grouped_us(true, even * parts > 1.f ? even * parts : 1.f, NB, stream_us, parts, false, busy(parts)) <
-             grouped_us(false, ordinary, NB, stream_us, shares, apart, busy(shares));
+      // (up to K = 1024 no wave has a second quad, and the registers for several cost occupancy: 512 x 11964 three planes 5.4 / 3.3)
+      fine = parts == 1 || grouped_us(true, even * parts > 1.f ? even * parts : 1.f, NB, stream_us, parts, false, busy(parts)) <
+                               grouped_us(false, ordinary, NB, stream_us, shares, apart, busy(shares));
     }
     fine = hq_tune(HQ_TUNE_LUT_FINE, fine) != 0;
   }

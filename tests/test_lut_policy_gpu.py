@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("K,N,nb,group", [(13312, 192, 5, 32), (5888, 5562, 4, 32), (17664, 1814, 6, 32), (4480, 26432, 2, 64),
-                                          (14208, 10688, 2, 32), (8320, 384, 3, 128), (8704, 256, 6, 128), (11392, 1778, 2, 128)])
+                                          (14208, 10688, 2, 32), (8320, 384, 3, 128), (8704, 256, 6, 128), (11392, 1778, 2, 128),
+                                          (512, 11964, 3, 64), (512, 23848, 2, 32), (256, 10475, 4, 64), (512, 40000, 3, 32)])
 def test_own_choice_is_the_faster_walk(hq, tunable, K, N, nb, group):
     import torch
     from hecbench_amd import _lib
