@@ -79,7 +79,8 @@ int hq_init(void);
  * A stream that only ever sees smaller calls takes less without a
  * reservation: a workspace grows with the calls (hq_q3_workspace_need; 8 MiB to begin with, nearly always enough for batch 1; up to 64 rows 20 MiB).
  * A captured call keeps the workspace of the stream it was captured on, whatever stream its graph is replayed on: replays must not
- * overlap with each other or with calls on that stream where both use it.  Calls that overlap in one workspace give wrong results,
+ * overlap with each other or with calls on that stream where both use it.  hipStreamPerThread is one handle and so one
+ * workspace: calls of several threads on it must not overlap either (hq_aqlm_matvec leaves nothing there).  Calls that overlap in one workspace give wrong results,
  * and they may leave its arrival counters and slots, which the kernels expect at zero and return to zero, at other values; hq_shutdown()
  * and calls (and captures) anew start from fresh ones.
  * No counterpart in the reference. */
